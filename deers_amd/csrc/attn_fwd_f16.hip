@@ -74,7 +74,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_f16_kernel(FwdParams p, int B
   const int T = p.T;
 
   int bh, rank;
-  if (!map_block(blockIdx.x, n_qtiles, heads_per_xcd, BH, &bh, &rank)) return;
+  // A scalar block id makes every operand base scalar; the compiler then hoists address arithmetic
+  // into vector registers until the D = 128 kernel spills (164 of them): kept in a vector register.
+  if (!map_block((int)opaque(blockIdx.x), n_qtiles, heads_per_xcd, BH, &bh, &rank)) return;
   const int qtile = n_qtiles - 1 - rank;  // longest rows first
   const int b = bh / p.H, h = bh % p.H;
 

@@ -54,6 +54,9 @@ __global__ __launch_bounds__(256, (D == 32 ? 3 : 2)) void attn_fwd_f32_kernel(Fw
   const int g = lane >> 5;
   const int T = p.T;
 
+  // a vector register on purpose: with a scalar block id the compiler hoists address arithmetic
+  // until the D = 64 and D = 128 kernels spill
+  const uint32_t block_id = opaque(blockIdx.x);
   // (head, query tile) of list position `item`, or bh = -1 past the end of the list.  Without
   // lists a workgroup has the one tile its id names (every tile of a head on one XCD, each
   // XCD's tiles longest first).  List entries of heads past the last one are skipped.
@@ -61,7 +64,7 @@ __global__ __launch_bounds__(256, (D == 32 ? 3 : 2)) void attn_fwd_f32_kernel(Fw
     *bh = -1;
     if (!lists) {
       int rank;
-      if (item == 0 && map_block(blockIdx.x, n_qtiles, heads_per_xcd, BH, bh, &rank))
+      if (item == 0 && map_block((int)block_id, n_qtiles, heads_per_xcd, BH, bh, &rank))
         *qtile = n_qtiles - 1 - rank;
       else
         *bh = -1;
@@ -70,9 +73,9 @@ __global__ __launch_bounds__(256, (D == 32 ? 3 : 2)) void attn_fwd_f32_kernel(Fw
     for (; item < max_len; ++item) {
       // the same in every lane: a scalar, so that the trip counts and causal tests that
       // derive from it are scalar too
-      const int code = __builtin_amdgcn_readfirstlane(lists[(blockIdx.x >> 3) * max_len + item]);
+      const int code = __builtin_amdgcn_readfirstlane(lists[(block_id >> 3) * max_len + item]);
       if (code < 0) return;
-      const int head = (code >> 16) * 8 + (blockIdx.x & 7);
+      const int head = (code >> 16) * 8 + (int)(block_id & 7);
       if (head < BH) {
         *bh = head;
         *qtile = code & 0xffff;
