@@ -33,47 +33,33 @@ __global__ __launch_bounds__(256) void neg_kernel(const T* a, T* out, size_t n) 
     out[i] = (T)(-to_f32(a[i]));
 }
 
-struct View6 {
-  int64_t shape[6];
-  int64_t stride[6];
+// A strided copy: up to six dimensions, outermost first, each with its extent and the
+// element (or 16-byte chunk) stride on either side.
+template <typename I>
+struct CopyView {
+  I shape[6];
+  I src[6];
+  I dst[6];
+  int ndim;
 };
 
-// dst (compact, row-major over `shape`) <- src viewed through `stride`.
-template <typename T>
-__global__ __launch_bounds__(256) void copy_strided_kernel(const T* src, T* dst, View6 v,
-                                                           size_t n) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    size_t rem = i;
-    int64_t off = 0;
-#pragma unroll
-    for (int d = 5; d >= 0; --d) {
-      const size_t idx = rem % (size_t)v.shape[d];
-      rem /= (size_t)v.shape[d];
-      off += (int64_t)idx * v.stride[d];
-    }
-    dst[i] = src[off];
-  }
-}
-
-// Fast path of copy_strided for views whose rows are contiguous runs of 16-byte
-// chunks (unit innermost stride, everything 16-byte aligned): one thread moves one
-// chunk, index arithmetic is 32-bit and runs once per 16 bytes instead of once per
-// element.  `v` describes the view in chunks.
-struct View6u {
-  uint32_t shape[6];
-  uint32_t stride[6];
-};
-__global__ __launch_bounds__(256) void copy_chunks_kernel(const uint4* src, uint4* dst, View6u v,
-                                                          uint32_t n) {
-  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-    uint32_t rem = i, off = 0;
-#pragma unroll
-    for (int d = 5; d >= 0; --d) {
-      const uint32_t q = rem / v.shape[d];
-      off += (rem - q * v.shape[d]) * v.stride[d];
+// dst viewed through v.dst <- src viewed through v.src, `n` units of E in all.  E is uint4
+// where both sides are whole aligned 16-byte chunks, else the element; I is 32-bit where every
+// offset fits.  The index arithmetic (a division per dimension) is what an element-wise 64-bit
+// form was bound by: 32 prompts of 512 x 12 heads x 64 halves into a KV cache, 25 MB each way,
+// took 79 us = 0.6 TB/s; one division chain per 16 bytes, in 32 bits, over dimensions the host
+// has merged: 10.8 us = 4.7 TB/s.
+template <typename E, typename I>
+__global__ __launch_bounds__(256) void copy_view_kernel(const E* src, E* dst, CopyView<I> v, I n) {
+  for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < n; i += (I)gridDim.x * 256) {
+    I rem = i, so = 0, dof = 0;
+    for (int d = v.ndim - 1; d > 0; --d) {
+      const I q = rem / v.shape[d], idx = rem - q * v.shape[d];
+      so += idx * v.src[d];
+      dof += idx * v.dst[d];
       rem = q;
     }
-    dst[i] = src[off];
+    dst[dof + rem * v.dst[0]] = src[so + rem * v.src[0]];
   }
 }
 
@@ -110,85 +96,91 @@ void launch_neg(int dtype_f16, const void* a, void* out, size_t n, hipStream_t s
                        (const float*)a, (float*)out, n);
 }
 
-// dst viewed through dst_strides <- src viewed through src_strides, same shape
-// (element-wise; used for small scatters such as a KV-cache append).
-template <typename T>
-__global__ __launch_bounds__(256) void copy_view_kernel(const T* src, T* dst, View6 v, View6 w,
-                                                        size_t n) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-    size_t rem = i;
-    int64_t so = 0, dof = 0;
-#pragma unroll
-    for (int d = 5; d >= 0; --d) {
-      const size_t idx = rem % (size_t)v.shape[d];
-      rem /= (size_t)v.shape[d];
-      so += (int64_t)idx * v.stride[d];
-      dof += (int64_t)idx * w.stride[d];
-    }
-    dst[dof] = src[so];
+template <typename E, typename I>
+static void copy_view_as(const void* src, void* dst, const CopyView<int64_t>& v, int64_t n, hipStream_t stream) {
+  CopyView<I> u;
+  u.ndim = v.ndim;
+  for (int d = 0; d < v.ndim; ++d) {
+    u.shape[d] = (I)v.shape[d];
+    u.src[d] = (I)v.src[d];
+    u.dst[d] = (I)v.dst[d];
   }
+  hipLaunchKernelGGL((copy_view_kernel<E, I>), dim3(grid_for((size_t)n)), dim3(256), 0, stream, (const E*)src,
+                     (E*)dst, u, (I)n);
 }
 
+// dst viewed through dst_strides <- src viewed through src_strides, same shape.
 void launch_copy_view(int dtype_f16, const void* src, const int64_t* src_strides, void* dst,
                       const int64_t* dst_strides, const int64_t* shape, int ndim,
                       hipStream_t stream) {
-  View6 v, w;
-  size_t n = 1;
-  for (int d = 0; d < 6; ++d) {
-    const int s = d - (6 - ndim);
-    v.shape[d] = w.shape[d] = s >= 0 ? shape[s] : 1;
-    v.stride[d] = s >= 0 ? src_strides[s] : 0;
-    w.stride[d] = s >= 0 ? dst_strides[s] : 0;
-    n *= (size_t)v.shape[d];
+  // extents of one vanish, neighbouring dimensions that step alike on both sides become one
+  CopyView<int64_t> v;
+  v.ndim = 0;
+  int64_t n = 1;
+  for (int d = 0; d < ndim; ++d) {
+    n *= shape[d];
+    if (shape[d] == 1) continue;
+    const int last = v.ndim - 1;
+    if (last >= 0 && v.src[last] == src_strides[d] * shape[d] && v.dst[last] == dst_strides[d] * shape[d]) {
+      v.shape[last] *= shape[d];
+    } else {
+      v.shape[v.ndim++] = shape[d];
+    }
+    v.src[v.ndim - 1] = src_strides[d];
+    v.dst[v.ndim - 1] = dst_strides[d];
   }
   if (n == 0) return;
-  if (dtype_f16)
-    hipLaunchKernelGGL(copy_view_kernel<half_t>, dim3(grid_for(n)), dim3(256), 0, stream,
-                       (const half_t*)src, (half_t*)dst, v, w, n);
-  else
-    hipLaunchKernelGGL(copy_view_kernel<float>, dim3(grid_for(n)), dim3(256), 0, stream,
-                       (const float*)src, (float*)dst, v, w, n);
+  if (v.ndim == 0) {
+    v.shape[0] = 1;
+    v.src[0] = v.dst[0] = 1;
+    v.ndim = 1;
+  }
+  // Whole 16-byte chunks: unit innermost strides, and every other step, the innermost extent
+  // and both addresses multiples of 16 bytes.
+  const int64_t per16 = dtype_f16 ? 8 : 4;
+  const int in = v.ndim - 1;
+  bool chunked = v.src[in] == 1 && v.dst[in] == 1 && v.shape[in] % per16 == 0 &&
+                 ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0;
+  int64_t src_span = 1, dst_span = 1;
+  for (int d = 0; d <= in; ++d) {
+    if (d < in) chunked = chunked && v.src[d] % per16 == 0 && v.dst[d] % per16 == 0;
+    src_span += (v.shape[d] - 1) * v.src[d];
+    dst_span += (v.shape[d] - 1) * v.dst[d];
+  }
+  int64_t span = src_span > dst_span ? src_span : dst_span;
+  if (n > span) span = n;
+  if (chunked) {
+    for (int d = 0; d < in; ++d) {
+      v.src[d] /= per16;
+      v.dst[d] /= per16;
+    }
+    v.shape[in] /= per16;
+    n /= per16;
+    span /= per16;
+  }
+  // 32-bit indices, with room for the grid stride past the last unit
+  const bool narrow = span < (int64_t(1) << 31);
+  if (chunked) {
+    if (narrow) copy_view_as<uint4, uint32_t>(src, dst, v, n, stream);
+    else copy_view_as<uint4, int64_t>(src, dst, v, n, stream);
+  } else if (dtype_f16) {
+    if (narrow) copy_view_as<uint16_t, uint32_t>(src, dst, v, n, stream);
+    else copy_view_as<uint16_t, int64_t>(src, dst, v, n, stream);
+  } else {
+    if (narrow) copy_view_as<uint32_t, uint32_t>(src, dst, v, n, stream);
+    else copy_view_as<uint32_t, int64_t>(src, dst, v, n, stream);
+  }
 }
 
+// dst (compact, row-major over `shape`) <- src viewed through `strides`.
 void launch_copy_strided(int dtype_f16, const void* src, const int64_t* shape,
                          const int64_t* strides, int ndim, void* dst, hipStream_t stream) {
-  View6 v;
-  size_t n = 1;
-  for (int d = 0; d < 6; ++d) {  // right-align the view in six dimensions
-    const int s = d - (6 - ndim);
-    v.shape[d] = s >= 0 ? shape[s] : 1;
-    v.stride[d] = s >= 0 ? strides[s] : 0;
-    n *= (size_t)v.shape[d];
+  int64_t compact[6], run = 1;
+  for (int d = ndim - 1; d >= 0; --d) {
+    compact[d] = run;
+    run *= shape[d];
   }
-  if (n == 0) return;
-  // rows of whole 16-byte chunks, everything aligned, offsets within 32 bits
-  const int64_t per16 = dtype_f16 ? 8 : 4;
-  bool chunked = v.stride[5] == 1 && v.shape[5] % per16 == 0 && n / per16 < (size_t(1) << 31) &&
-                 ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0;
-  int64_t span = 0;
-  for (int d = 0; d < 5 && chunked; ++d) {
-    chunked = v.stride[d] % per16 == 0;
-    span += (v.shape[d] - 1) * v.stride[d];
-  }
-  if (chunked && (span + v.shape[5]) / per16 < (int64_t(1) << 32)) {
-    View6u u;
-    for (int d = 0; d < 5; ++d) {
-      u.shape[d] = (uint32_t)v.shape[d];
-      u.stride[d] = (uint32_t)(v.stride[d] / per16);
-    }
-    u.shape[5] = (uint32_t)(v.shape[5] / per16);
-    u.stride[5] = 1;
-    const uint32_t nc = (uint32_t)(n / per16);
-    hipLaunchKernelGGL(copy_chunks_kernel, dim3(grid_for(nc)), dim3(256), 0, stream,
-                       (const uint4*)src, (uint4*)dst, u, nc);
-    return;
-  }
-  if (dtype_f16)
-    hipLaunchKernelGGL(copy_strided_kernel<half_t>, dim3(grid_for(n)), dim3(256), 0, stream,
-                       (const half_t*)src, (half_t*)dst, v, n);
-  else
-    hipLaunchKernelGGL(copy_strided_kernel<float>, dim3(grid_for(n)), dim3(256), 0, stream,
-                       (const float*)src, (float*)dst, v, n);
+  launch_copy_view(dtype_f16, src, strides, dst, compact, shape, ndim, stream);
 }
 
 }  // namespace deers

@@ -232,3 +232,33 @@ def test_attn_decode_append_is_decode_qkv_then_attn_decode(B, H, D, cap, pos):
     with pytest.raises(rocm.RocmError):
         rocm.attn_decode_append_raw(dtype, at(dqkv, 0), at(dqkv, C), at(dqkv, 2 * C), (3 * C, D), cos_row, sin_row,
                                     k1.ptr, v1.ptr, kv_strides, o1.ptr, cap, cap, B, H, D, scale)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("shape,src_perm,dst_perm,offset", [
+    ((3, 5, 4, 16), (0, 2, 1, 3), (0, 1, 2, 3), 0),   # whole 16-byte chunks, two strided dimensions
+    ((3, 5, 4, 16), (0, 1, 2, 3), (2, 0, 1, 3), 0),   # scattered
+    ((3, 5, 4, 16), (0, 2, 1, 3), (0, 1, 2, 3), 1),   # off a 16-byte boundary
+    ((3, 5, 4, 6), (0, 2, 1, 3), (1, 0, 2, 3), 0),    # rows that are not whole chunks
+    ((2, 1, 7, 8), (0, 1, 2, 3), (0, 1, 2, 3), 0),    # compact on both sides: one dimension
+    ((4, 3, 5), (2, 1, 0), (0, 1, 2), 0),             # innermost stride not one
+    ((1, 1, 1), (0, 1, 2), (0, 1, 2), 0),
+])
+def test_copy_view_layouts(dtype, shape, src_perm, dst_perm, offset):
+    import ctypes
+    def strides(perm):  # of a tensor stored compactly in the order of `perm`
+        out, run = [0] * len(shape), 1
+        for d in reversed(perm):
+            out[d], run = run, run * shape[d]
+        return out
+    n = int(np.prod(shape))
+    stored = lambda a, perm: np.ascontiguousarray(a.transpose(perm)).reshape(-1)
+    x = synth.normal(shape, synth.tensor_seed(29, "view", "x"), 1.0).astype(dtype)
+    src = rocm.DeviceBuffer.from_numpy(np.concatenate([np.zeros(offset, dtype), stored(x, src_perm)]))
+    dst = rocm.DeviceBuffer.from_numpy(np.full(n + offset + 8, 7.0, dtype))
+    at = lambda b: ctypes.c_void_p(b.ptr.value + offset * np.dtype(dtype).itemsize)
+    rocm.copy_view_raw(dtype, at(src), strides(src_perm), at(dst), strides(dst_perm), shape)
+    got = dst.numpy()
+    assert np.array_equal(got[offset:offset + n], stored(x, dst_perm))
+    assert (got[:offset] == 7).all() and (got[offset + n:] == 7).all()
