@@ -80,7 +80,8 @@ void launch_sumsq(int dtype_f16, const void* g, int64_t n, float* partial, float
                   int accumulate, hipStream_t stream);
 void launch_scale(int dtype_f16, void* x, int64_t n, double scale, hipStream_t stream);
 int multi_max_tensors();
-int64_t multi_blocks(int dtype_f16, int64_t n);
+int64_t adamw_multi_blocks(int dtype_f16, int64_t n);
+int64_t sumsq_multi_blocks(int dtype_f16, int64_t n);
 void launch_adamw_multi(int dtype_f16, int count, void* const* w, const void* const* g, void* const* m,
                         void* const* v, const int64_t* sizes, double lr, double beta1, double beta2,
                         double eps, double weight_decay, int step, double grad_scale,
@@ -1391,7 +1392,7 @@ int deers_rocm_adamw_step_multi(int dtype, int n_tensors, void* const* w, const 
     if (sizes[i] == 0) continue;
     if (multi_ok(w[i], sizes[i]) && multi_ok(grad[i], sizes[i]) && multi_ok(m[i], sizes[i]) &&
         multi_ok(v[i], sizes[i])) {
-      const int64_t nb = deers::multi_blocks(f16, sizes[i]);
+      const int64_t nb = deers::adamw_multi_blocks(f16, sizes[i]);
       if ((int)gw.size() == cap || group_blocks + nb > INT32_MAX / 2) flush();
       gw.push_back(w[i]); gg.push_back(grad[i]); gm.push_back(m[i]); gv.push_back(v[i]); gn.push_back(sizes[i]);
       group_blocks += nb;
@@ -1421,7 +1422,7 @@ int deers_rocm_sum_squares_multi(int dtype, int n_tensors, const void* const* x,
     if (sizes[i] > 0 && ((uintptr_t)x[i] & 15))
       return fail(DEERS_ROCM_ERR_LAYOUT, "sum_squares_multi: tensor %d is not 16-byte aligned; use "
                   "deers_rocm_sum_squares for it", i);
-    blocks += deers::multi_blocks(f16, sizes[i]);
+    blocks += deers::sumsq_multi_blocks(f16, sizes[i]);
   }
   if (blocks > INT32_MAX / 2) return fail(DEERS_ROCM_ERR_ARG, "sum_squares_multi: too many elements for one call");
   void* ws = nullptr;  // one partial per block of every tensor, then one fixed-order sum

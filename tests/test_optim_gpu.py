@@ -219,3 +219,16 @@ def test_multi_tensor_step_and_norm_equal_the_single_tensor_calls(dtype):
         rocm.sum_squares_multi_raw(dtype, [at(a[0][1], 1)], [4], total.ptr)
     rocm.sum_squares_multi_raw(dtype, [], [], total.ptr)
     assert total.numpy()[0] == 0.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_sum_squares_multi_at_slab_edges(dtype):
+    slab = 65536 // np.dtype(dtype).itemsize  # elements one block of the reduction owns
+    sizes = [1, slab - 1, slab, slab + 1, 2 * slab + 7, 3]
+    xs = [synth.normal((n,), synth.tensor_seed(68, "sumsq", str(n)), 1.0).astype(dtype) for n in sizes]
+    bufs = [rocm.DeviceBuffer.from_numpy(x) for x in xs]
+    total = rocm.DeviceBuffer((1,), np.float32)
+    rocm.sum_squares_multi_raw(dtype, [b.ptr for b in bufs], sizes, total.ptr)
+    want = sum(float((x.astype(np.float64) ** 2).sum()) for x in xs)
+    assert abs(float(total.numpy()[0]) - want) <= 1e-6 * want
