@@ -72,65 +72,145 @@ __global__ __launch_bounds__(256) void index_select_kernel(const T* table, const
 }
 
 // ---- index_add (dim 0): dst[idx[i], :] += src[i, :], in ascending i ----
-// The order of additions is the reference's (src/storage/cpu.rs:954-975), so the result
-// is the same bits and the same from run to run: workgroup i owns the destination row
-// idx[i] if no earlier position names it, finds every later position that does (a
-// bitmap in LDS, built from the index vector, which stays in L2), and adds their source
-// rows in order.  Other workgroups leave at once.  A launch covers at most
-// kIndexAddChunk positions (every workgroup scans its launch's whole index slice, so the
-// cost of a launch grows with the square of its length); longer index vectors take one
-// launch per slice, in order, which keeps the order of additions: a later slice adds to
-// what the earlier ones left.
-constexpr int kIndexAddChunk = 1 << 14;  // bitmap of 2 KB of dynamic LDS
+// The order of additions is the reference's (src/storage/cpu.rs:954-975), so the result is the
+// same bits and the same from run to run.  Destination rows are dealt to the workgroups by a hash:
+// a workgroup reads the whole index vector once (it stays in L2), keeps the positions that name
+// its rows in ascending order in LDS, and applies them.  With a workgroup per position instead,
+// each scanning the vector to find out whether it is the first to name its row, 8192 tokens of
+// 768 floats read 512 MB of indices through L2 and took 171 us; with at most 1024 workgroups the
+// scan is 64 MB and the launch, 22 us, is mostly the rows' own traffic (three streams of 25 MB).
+// A launch covers at most kIndexAddChunk positions (one 64-bit word of the LDS bitmap per
+// thread); longer index vectors take one launch per slice, in order, which keeps the order of
+// additions: a later slice adds to what the earlier ones left.
+constexpr int kIndexAddChunk = 1 << 14;
+constexpr int kIndexAddOwners = 1024;  // workgroups at most: four per CU, all resident
+constexpr int kIndexAddBatch = 4;      // source rows in flight per column group
+constexpr int kIndexAddCols = 4;       // column groups of 64 units a wave has in flight
 
-template <typename T>
+// dst row `out` += the source rows at positions list[64 * w + b] for every bit b of hits(w),
+// w = w0, w0 + 1, ..., in that order, for the columns c_first + lane, + c_step, ... of the row's
+// units of EPU elements (16 bytes, or one element where rows are not whole aligned chunks).  The
+// loops are uniform over the wave: `hits` may be a ballot.
+template <typename T, int EPU, typename Hits>
+__device__ __forceinline__ void add_rows(const T* src, T* out, const uint16_t* list, int words, int w0, int width,
+                                         int c_first, int c_step, int lane, Hits hits) {
+  struct alignas(sizeof(T) * EPU) Unit { T e[EPU]; };
+  const int n_units = width / EPU;
+  for (int base = c_first; base < n_units; base += c_step * kIndexAddCols) {
+    const int c0 = base + lane;
+    Unit acc[kIndexAddCols];
+#pragma unroll
+    for (int k = 0; k < kIndexAddCols; ++k)
+      if (c0 + k * c_step < n_units) acc[k] = *(const Unit*)(out + (int64_t)(c0 + k * c_step) * EPU);
+    for (int w = w0; w < words; ++w) {
+      unsigned long long bits = hits(w);
+      while (bits) {
+        Unit x[kIndexAddBatch][kIndexAddCols];
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < kIndexAddBatch; ++u) {
+          if (!bits) break;
+          const T* row = src + (int64_t)list[64 * w + __builtin_ctzll(bits)] * width;
+          bits &= bits - 1;
+          ++n;
+#pragma unroll
+          for (int k = 0; k < kIndexAddCols; ++k)
+            if (c0 + k * c_step < n_units) x[u][k] = *(const Unit*)(row + (int64_t)(c0 + k * c_step) * EPU);
+        }
+#pragma unroll
+        for (int u = 0; u < kIndexAddBatch; ++u) {
+          if (u >= n) break;
+#pragma unroll
+          for (int k = 0; k < kIndexAddCols; ++k)
+#pragma unroll
+            for (int e = 0; e < EPU; ++e)  // rounded to T after each addition, as `+=` on the storage type
+              acc[k].e[e] = (T)((float)acc[k].e[e] + (float)x[u][k].e[e]);
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kIndexAddCols; ++k)
+      if (c0 + k * c_step < n_units) *(Unit*)(out + (int64_t)(c0 + k * c_step) * EPU) = acc[k];
+  }
+}
+
+template <typename T, int EPU>
 __global__ __launch_bounds__(256) void index_add_kernel(const T* src, const int64_t* idx, T* dst,
                                                         int64_t n_rows, int n_idx, int width,
                                                         int* error_flag) {
-  extern __shared__ unsigned int bitmap[];  // one bit per position, 2 words per 64 positions
-  __shared__ int not_leader;
-  const int i = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t r = idx[i];
-  if (r < 0 || r >= n_rows) {
-    if (tid == 0) atomicOr(error_flag, 1);
-    return;
-  }
-  if (tid == 0) not_leader = 0;
-  __syncthreads();
-  // each wavefront compares 64 consecutive positions per step (one coalesced load)
-  const int groups = (n_idx + 63) / 64;
-  for (int gq = wave; gq < groups; gq += 4) {
-    const int pos = gq * 64 + lane;
-    const bool match = pos < n_idx && idx[pos] == r;
-    const unsigned long long mask = __ballot(match);
-    if (lane == 0) {
-      bitmap[2 * gq] = (unsigned int)mask;
-      bitmap[2 * gq + 1] = (unsigned int)(mask >> 32);
-      const int base = gq * 64;
-      if (base < i) {
-        const unsigned long long before =
-            base + 64 <= i ? mask : mask & ((1ull << (i - base)) - 1ull);
-        if (before) not_leader = 1;  // benign race: every writer stores 1
-      }
+  extern __shared__ uint16_t list[];  // this workgroup's positions, ascending (room for n_idx)
+  __shared__ unsigned long long bitmap[kIndexAddChunk / 64];
+  __shared__ int wave_total[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned owner_mask = gridDim.x - 1;  // a power of two of workgroups
+  const int groups = (n_idx + 63) / 64;       // at most 256
+  constexpr int kInFlight = 8;
+  for (int g0 = wave; g0 < groups; g0 += 4 * kInFlight) {
+    int64_t r[kInFlight];
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const int pos = (g0 + 4 * u) * 64 + lane;
+      r[u] = pos < n_idx ? idx[pos] : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const int g = g0 + 4 * u;
+      if (g >= groups) break;
+      const bool ok = r[u] >= 0 && r[u] < n_rows;
+      const unsigned owner = ((unsigned)r[u] * 0x9E3779B1u) >> 16;
+      const unsigned long long mask = __ballot(ok && (owner & owner_mask) == blockIdx.x);
+      if (lane == 0) bitmap[g] = mask;
+      if (blockIdx.x == 0 && !ok && g * 64 + lane < n_idx) atomicOr(error_flag, 1);
     }
   }
   __syncthreads();
-  if (not_leader) return;
-  const int words = 2 * groups;
-  T* out = dst + r * width;
-  for (int c = tid; c < width; c += 256) {
-    float acc = (float)out[c];
-    for (int w = i / 32; w < words; ++w) {
-      unsigned int bits = bitmap[w];
-      while (bits) {
-        const int b = __builtin_ctz(bits);
-        bits &= bits - 1;
-        // rounding to T after each addition, as `+=` on the storage type does
-        acc = (float)(T)(acc + (float)src[(int64_t)(w * 32 + b) * width + c]);
-      }
+  // the set bits' positions, in order: a prefix sum over the words' counts, one word per thread
+  const unsigned long long mine = tid < groups ? bitmap[tid] : 0;
+  const int count = __popcll(mine);
+  int before = count;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int other = __shfl_up(before, off, 64);
+    if (lane >= off) before += other;
+  }
+  if (lane == 63) wave_total[wave] = before;
+  __syncthreads();
+  int at = before - count, total = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) at += wave_total[w];
+    total += wave_total[w];
+  }
+  for (unsigned long long bits = mine; bits; bits &= bits - 1)
+    list[at++] = (uint16_t)(tid * 64 + __builtin_ctzll(bits));
+  __syncthreads();
+  if (total <= 64) {
+    // the usual case: the list fits a wave's lanes, the waves share out its rows
+    const int64_t row = lane < total ? idx[list[lane]] : -1;
+    for (int j = wave; j < total; j += 4) {
+      const int64_t rj = idx[list[j]];
+      const unsigned long long hits = __ballot(row == rj);
+      if (hits & ((1ull << j) - 1)) continue;  // an earlier entry names this row
+      add_rows<T, EPU>(src, dst + rj * width, list, 1, 0, width, 0, 64, lane, [&](int) { return hits; });
     }
-    out[c] = (T)acc;
+  } else {
+    // a row that many positions name (or an unlucky hash): every wave takes its columns of every row
+    const int words = (total + 63) / 64;
+    auto hits_of = [&](int w, int64_t rj) {
+      const int e = 64 * w + lane;
+      return __ballot(e < total && idx[list[e < total ? e : 0]] == rj);
+    };
+    for (int j = 0; j < total; ++j) {
+      const int64_t rj = idx[list[j]];
+      bool first = true;
+      for (int w = 0; w <= j / 64 && first; ++w) {
+        const unsigned long long hits = hits_of(w, rj);
+        first = !(w == j / 64 ? hits & ((1ull << (j & 63)) - 1) : hits);
+      }
+      if (!first) continue;
+      add_rows<T, EPU>(src, dst + rj * width, list, words, j / 64, width, wave * 64, 256, lane,
+                       [&](int w) { return hits_of(w, rj); });
+    }
   }
 }
 
@@ -692,21 +772,32 @@ void launch_index_select(int dtype_f16, const void* table, const int64_t* idx, v
     index_select_t((const float*)table, idx, (float*)out, n_rows, n_idx, width, flag, stream);
 }
 
+template <typename T>
+static void index_add_t(const T* src, const int64_t* idx, T* dst, int64_t n_rows, int64_t n_idx, int width,
+                        int* flag, hipStream_t stream) {
+  constexpr int kEpc = 16 / sizeof(T);
+  const bool vec = aligned16(src) && aligned16(dst) && width % kEpc == 0;
+  for (int64_t first = 0; first < n_idx; first += kIndexAddChunk) {
+    const int n = (int)(n_idx - first < kIndexAddChunk ? n_idx - first : kIndexAddChunk);
+    unsigned owners = 1;
+    while (owners < (unsigned)n && owners < kIndexAddOwners) owners *= 2;
+    const size_t lds = (size_t)n * sizeof(uint16_t);
+    if (vec)
+      hipLaunchKernelGGL((index_add_kernel<T, kEpc>), dim3(owners), dim3(256), lds, stream, src + first * width,
+                         idx + first, dst, n_rows, n, width, flag);
+    else
+      hipLaunchKernelGGL((index_add_kernel<T, 1>), dim3(owners), dim3(256), lds, stream, src + first * width,
+                         idx + first, dst, n_rows, n, width, flag);
+  }
+}
+
 void launch_index_add(int dtype_f16, const void* src, const int64_t* idx, void* dst, int64_t n_rows,
                       int64_t n_idx, int width, int* flag, hipStream_t stream) {
   LaunchScope scope("index_add", stream);
-  for (int64_t first = 0; first < n_idx; first += kIndexAddChunk) {
-    const int n = (int)(n_idx - first < kIndexAddChunk ? n_idx - first : kIndexAddChunk);
-    const size_t lds = (size_t)((n + 63) / 64) * 2 * sizeof(unsigned int);
-    if (dtype_f16)
-      hipLaunchKernelGGL(index_add_kernel<half_t>, dim3((unsigned)n), dim3(256), lds, stream,
-                         (const half_t*)src + first * width, idx + first, (half_t*)dst, n_rows, n, width,
-                         flag);
-    else
-      hipLaunchKernelGGL(index_add_kernel<float>, dim3((unsigned)n), dim3(256), lds, stream,
-                         (const float*)src + first * width, idx + first, (float*)dst, n_rows, n, width,
-                         flag);
-  }
+  if (dtype_f16)
+    index_add_t((const half_t*)src, idx, (half_t*)dst, n_rows, n_idx, width, flag, stream);
+  else
+    index_add_t((const float*)src, idx, (float*)dst, n_rows, n_idx, width, flag, stream);
 }
 
 template <typename T>

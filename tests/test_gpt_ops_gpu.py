@@ -279,3 +279,20 @@ def test_index_add_over_several_index_slices(n):
     want = np.zeros((vocab, width), np.float32)
     np.add.at(want, idx, g)  # unbuffered, in position order: the same sequence of f32 additions
     assert np.array_equal(dst.numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("vocab,width,n", [
+    (3, 4100, 70),        # a list longer than a wave's lanes, more column units than the workgroup has threads
+    (2, 5, 300),          # the same with rows that are not whole chunks
+    (4096, 8, 1 << 14),   # the longest slice of one launch
+    (50000, 1288, 5),     # more columns than one pass of a wave, fewer positions than a wave
+])
+def test_index_add_list_lengths_and_column_passes(dtype, vocab, width, n):
+    idx = _tokens(n, vocab, 78)
+    g = synth.normal((n, width), synth.tensor_seed(78, "emb", "g"), 1.0).astype(dtype)
+    dg, di = _dev(g), _dev(idx)
+    dst = rocm.DeviceBuffer((vocab, width), dtype, zeros=True)
+    rocm.index_add_raw(dtype, dg.ptr, di.ptr, dst.ptr, vocab, n, width)
+    assert np.array_equal(dst.numpy(), oracle.index_add(vocab, g, idx))
