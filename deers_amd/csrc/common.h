@@ -150,6 +150,18 @@ __device__ __forceinline__ void async_load16_to_lds(const void* uniform_base, ui
                "s"(uniform)
                : "memory");
 }
+// The same for data that is used once (a non-temporal access).
+__device__ __forceinline__ void async_load16_to_lds_nt(const void* uniform_base, uint32_t lane_off,
+                                                       uint32_t lds_addr) {
+  const uint32_t uniform = __builtin_amdgcn_readfirstlane(lds_addr);
+  const uint64_t b = (uint64_t)uniform_base;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  const uint64_t sbase = ((uint64_t)hi << 32) | (uint64_t)lo;
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(lane_off), "s"(sbase),
+               "s"(uniform)
+               : "memory");
+}
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");

@@ -10,13 +10,12 @@
 // The reference composes the last three from primitive tensor ops (4, 3 and 5 kernels
 // with as many intermediate tensors); here each is one pass forward and one backward.
 // All are HBM-bound.  Arithmetic is f32 whatever the storage type, rounded once.
-#include "common.h"
+#include "row_regs.h"
 
 namespace deers {
 
 namespace {
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 template <typename T> struct alignas(16) Vec16 { T e[16 / sizeof(T)]; };
 
 template <typename T>
@@ -428,37 +427,138 @@ __global__ __launch_bounds__(256) void relu_sq_unaligned_kernel(const T* x, cons
 }
 
 // ---- cross entropy ----
-// Forward: one workgroup per row streams the logits once with an online (max, sum)
-// pair and keeps lse_i = ln sum exp(x_i) and loss_i = lse_i - x_i[target_i]; a second
-// tiny kernel averages the per-row losses in a fixed order.  The log-probabilities are
-// never written.  Rows start at any element (50257 is odd): the sweep runs over 16-byte
-// chunks counted from the 16-byte boundary at or before the row start, with the two
-// edge chunks masked.
+// Forward: lse_i = ln sum exp(x_i) and loss_i = lse_i - x_i[target_i] per row; a second tiny
+// kernel averages the per-row losses in a fixed order.  The log-probabilities are never written.
+// With GRAD also dlogits[r, c] = (exp(x - lse) - [c == target]) * inv_n, the gradient of the mean
+// loss for an upstream gradient of one: same expression, same bits as cross_entropy_bwd_kernel's.
+// A row is held on chip by the thread group that owns it, reduced there and written from there,
+// so the logits cross HBM once (row_regs.h); with and without GRAD the reduction is the same, so
+// are lse and loss.  HBM-bound: [8192, 50257] f32, 1.65 GB in and 1.65 GB out.
+//   A workgroup only reads until its row has arrived and only writes after that, so a CU needs two
+// of them to keep both directions busy: the widest rows leave NLDS of their chunks in LDS, where
+// the loads put them without passing through registers, so that the rest and the arithmetic fit
+// the 64 registers two 1024-thread workgroups leave each thread: 585 us = 5.6 TB/s, where one
+// workgroup of 512 threads holding 28 chunks each took 694 us = 4.7 TB/s.
+template <typename T, int GROUP, int NREG, int NLDS, bool GRAD>
+__global__ __launch_bounds__(kRegBlockOf(GROUP), NLDS ? 8 : 1) void cross_entropy_fwd_kernel(
+    const T* logits, const int64_t* targets, float* row_lse, float* row_loss, T* dlogits, float inv_n,
+    int64_t n_rows, int width, int* error_flag) {
+  __shared__ float red_m[16], red_s[16];
+  extern __shared__ u32x4 parked[];  // [NLDS][GROUP]
+  constexpr int kRows = kRegBlockOf(GROUP) / GROUP;
+  constexpr int kEpc = 16 / sizeof(T);
+  static_assert(NLDS == 0 || kRows == 1, "one row per workgroup where LDS holds a part of it");
+  const int t = threadIdx.x % GROUP;
+  const int64_t r = (int64_t)blockIdx.x * kRows + threadIdx.x / GROUP;
+  const bool live = r < n_rows;  // whole groups only: GROUP == 64 when kRows > 1
+  const T* row = logits + (live ? r : 0) * width;
+  const RowGeom<T> geo(row, width);
+  const int n_chunks = live ? geo.n_chunks : 0;  // a dead group's descriptors cover nothing
+  // Row position of this thread's chunk 0, element 0.  Chunk u is looked at as chunk 0 of the row's
+  // rest from u * GROUP chunks on (`left` elements, uniform): one register tells where all of them lie.
+  const int lo0 = t * kEpc - geo.head;
+  auto left = [&](int u) { return width - u * GROUP * kEpc; };
+  if constexpr (NLDS > 0) {
+    const uint32_t wave_lds = lds_address(parked) + (threadIdx.x & ~63) * 16;
+#pragma unroll
+    for (int u = 0; u < NLDS; ++u) {  // chunks past the row's end repeat its last one and are patched below
+      const int chunk = min(t + (NREG + u) * GROUP, n_chunks - 1);
+      async_load16_to_lds_nt(geo.base_of(row), (uint32_t)chunk * 16, wave_lds + u * GROUP * 16);
+    }
+  }
+  u32x4 c[NREG];
+#pragma unroll
+  for (int u = 0; u < NREG; ++u) {
+    c[u] = u32x4{0u, 0u, 0u, 0u};
+    // chunks wholly before the row (slice 0 only) are not read
+    if (u > 0 || lo0 + kEpc > 0) c[u] = chunk_load(slice_rsrc(geo.base_of(row), n_chunks, u * GROUP), t * 16);
+  }
+  const int64_t target = live ? targets[r] : 0;
+  const bool ok = target >= 0 && target < width;
+  const float x_target = ok ? (float)row[target] : 0.f;
+#pragma unroll
+  for (int u = 0; u < NREG; ++u) {
+    if ((u == 0 && lo0 < 0) || lo0 + kEpc > left(u)) c[u] = patch_outside<T>(c[u], lo0, left(u), -INFINITY, u == 0);
+  }
+  if constexpr (NLDS > 0) wait_all_vmem();  // a thread reads only what its own wave loaded: no barrier
+  auto chunk_of = [&](int u, float(&f)[kEpc]) {
+    if (u < NREG) {
+      keep_packed<T>(c[u < NREG ? u : 0]);
+      unpack<T>(c[u < NREG ? u : 0], f);
+    } else {
+      u32x4 x = parked[(u - NREG) * GROUP + threadIdx.x];
+      if (lo0 + kEpc > left(u)) x = patch_outside<T>(x, lo0, left(u), -INFINITY, false);
+      unpack<T>(x, f);
+    }
+  };
+  // ends a chunk's work before the next one's begins: no registers for more than one beside the row
+  auto settle = [](float& x) {
+    asm volatile("" : "+v"(x));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  float m = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < NREG + NLDS; ++u) {
+    float f[kEpc];
+    chunk_of(u, f);
+#pragma unroll
+    for (int e = 0; e < kEpc; ++e) m = fmaxf(m, f[e]);
+    if (NLDS > 0) settle(m);
+  }
+  float s = 0.f;
+  if (m != -INFINITY) {
+#pragma unroll
+    for (int u = 0; u < NREG + NLDS; ++u) {
+      float f[kEpc];
+      chunk_of(u, f);
+#pragma unroll
+      for (int e = 0; e < kEpc; ++e) s += __expf(f[e] - m);
+      if (NLDS > 0) settle(s);
+    }
+  }
+  group_reduce_ms<GROUP>(m, s, red_m, red_s, t);
+  if (!live) return;
+  const float lse = __logf(s) + m;
+  if (t == 0) {
+    if (!ok) atomicOr(error_flag, 1);
+    row_lse[r] = lse;
+    row_loss[r] = ok ? lse - x_target : 0.f;
+  }
+  if constexpr (GRAD) {
+    T* orow = dlogits + r * width;
+    // 16-byte stores need the output row at the input row's offset from a 16-byte boundary
+    const bool same = same_phase(orow, row);
+    const char* obase = geo.base_of(orow);
+    const int hit = ok ? (int)target : INT32_MIN / 2;
+#pragma unroll
+    for (int u = 0; u < NREG + NLDS; ++u) {
+      const int hit_u = hit - u * GROUP * kEpc;
+      float f[kEpc];
+      chunk_of(u, f);
+#pragma unroll
+      for (int e = 0; e < kEpc; ++e) {
+        const float pr = __expf(f[e] - lse);
+        f[e] = (pr - (hit_u == lo0 + e ? 1.0f : 0.0f)) * inv_n;
+      }
+      if (same && (u > 0 || lo0 >= 0) && lo0 + kEpc <= left(u))
+        chunk_store(pack<T>(f), slice_rsrc(obase, n_chunks, u * GROUP), t * 16);
+      else
+        store_inside<T>(f, orow + u * GROUP * kEpc, lo0, left(u), u == 0);
+      if (NLDS > 0) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+}
+
+// The same for rows that no group's registers hold: one workgroup walks the row with an online
+// (max, sum) pair, and a second time for the gradient.
 constexpr int kCeThreads = 512;
 constexpr int kCeInFlight = 4;
 
-__device__ __forceinline__ void merge_ms(float& m, float& s, float m2, float s2) {
-  const float mn = fmaxf(m, m2);
-  const float a = (m == -INFINITY) ? 0.f : __expf(m - mn);
-  const float b = (m2 == -INFINITY) ? 0.f : __expf(m2 - mn);
-  s = s * a + s2 * b;
-  m = mn;
-}
-
-// MODE 0: the forward.  MODE 1 and 2 also write dlogits[r, c] = (exp(x - lse) - [c == target]) *
-// inv_n, the gradient of the mean loss for an upstream gradient of one: same expression, same
-// bits as cross_entropy_bwd_kernel's.  In MODE 2 the workgroup keeps the whole row in registers
-// between the reduction and the gradient (rows of up to kCeThreads * ce_keep<T>() 16-byte chunks:
-// 57344 floats or 65536 halves), so the logits are read once; MODE 1 walks longer rows a second
-// time.  The reduction takes the chunks in the same groups and order in every mode: same lse,
-// same loss.
-template <typename T>
-constexpr int ce_keep() {  // chunks per thread MODE 2 holds (a multiple of kCeInFlight)
-  return sizeof(T) == 2 ? 16 : 28;
-}
-
-template <typename T, int MODE>
-__global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(
+template <typename T, bool GRAD>
+__global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_wide_kernel(
     const T* logits, const int64_t* targets, float* row_lse, float* row_loss, T* dlogits, float inv_n,
     int width, int* error_flag) {
   __shared__ float red_m[kCeThreads / 64], red_s[kCeThreads / 64];
@@ -470,13 +570,17 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(
   const int head = (int)((uintptr_t)row & 15) / (int)sizeof(T);
   const T* base = row - head;  // 16-byte aligned
   const int n_chunks = (head + width + kEpc - 1) / kEpc;
-  constexpr int kCeKeep = ce_keep<T>();
-  static_assert(kCeKeep % kCeInFlight == 0, "whole groups");
   float m = -INFINITY, s = 0.f;
-  // one group of kCeInFlight chunks: the running maximum and sum take them in
-  auto take_group = [&](int c0, const Vec16<T>* v) {
+  for (int c0 = tid; c0 < n_chunks; c0 += kCeThreads * kCeInFlight) {
+    Vec16<T> v[kCeInFlight];
     float f[kCeInFlight][kEpc];
     float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < kCeInFlight; ++u) {
+      const int c = c0 + u * kCeThreads;
+      v[u] = Vec16<T>{};
+      if (c < n_chunks) v[u] = GRAD ? load16(base + c * kEpc) : load16_stream(base + c * kEpc);
+    }
 #pragma unroll
     for (int u = 0; u < kCeInFlight; ++u) {
       const int lo = (c0 + u * kCeThreads) * kEpc - head;  // row position of element 0
@@ -496,31 +600,6 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(
       for (int u = 0; u < kCeInFlight; ++u)
 #pragma unroll
         for (int e = 0; e < kEpc; ++e) s += __expf(f[u][e] - m);
-    }
-  };
-  Vec16<T> keep[MODE == 2 ? kCeKeep : 1];
-  if constexpr (MODE == 2) {
-#pragma unroll
-    for (int i = 0; i < kCeKeep; ++i) {  // every load of the row is in flight at once
-      const int c = tid + i * kCeThreads;
-      keep[i] = Vec16<T>{};
-      if (c < n_chunks) keep[i] = load16_stream(base + c * kEpc);
-    }
-#pragma unroll
-    for (int gq = 0; gq < kCeKeep / kCeInFlight; ++gq) {
-      const int c0 = tid + gq * kCeInFlight * kCeThreads;
-      if (c0 < n_chunks) take_group(c0, keep + gq * kCeInFlight);
-    }
-  } else {
-    for (int c0 = tid; c0 < n_chunks; c0 += kCeThreads * kCeInFlight) {
-      Vec16<T> v[kCeInFlight];
-#pragma unroll
-      for (int u = 0; u < kCeInFlight; ++u) {
-        const int c = c0 + u * kCeThreads;
-        v[u] = Vec16<T>{};
-        if (c < n_chunks) v[u] = MODE == 1 ? load16(base + c * kEpc) : load16_stream(base + c * kEpc);
-      }
-      take_group(c0, v);
     }
   }
 #pragma unroll
@@ -543,16 +622,16 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(
     if (!ok) atomicOr(error_flag, 1);
     row_lse[r] = lse;
     row_loss[r] = ok ? lse - (float)row[t] : 0.f;
-    if (MODE != 0) lse_all = lse;
+    lse_all = lse;
   }
-  if constexpr (MODE != 0) {
+  if constexpr (GRAD) {
     __syncthreads();
     const float lse = lse_all;
     const int64_t t = targets[r];
     T* obase = dlogits + r * width - head;  // the chunk grid of the input row
-    // 16-byte stores need the output row at the input row's offset from a 16-byte boundary
-    const bool same_phase = (((uintptr_t)(dlogits + r * width)) & 15) == ((uintptr_t)row & 15);
-    auto write_chunk = [&](int c, const Vec16<T>& v) {
+    const bool same = same_phase(dlogits + r * width, row);
+    for (int c = tid; c < n_chunks; c += kCeThreads) {
+      const Vec16<T> v = load16(base + c * kEpc);
       const int lo = c * kEpc - head;  // row position of element 0
       Vec16<T> o;
 #pragma unroll
@@ -560,22 +639,13 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_fwd_kernel(
         const float pr = __expf((float)v.e[e] - lse);
         o.e[e] = (T)((pr - (t == lo + e ? 1.0f : 0.0f)) * inv_n);
       }
-      if (same_phase && lo >= 0 && lo + kEpc <= width) {
+      if (same && lo >= 0 && lo + kEpc <= width) {
         store16_stream(o, obase + c * kEpc);
       } else {  // an edge chunk shares its 16 bytes with the neighbouring row
 #pragma unroll
         for (int e = 0; e < kEpc; ++e)
           if (lo + e >= 0 && lo + e < width) obase[c * kEpc + e] = o.e[e];
       }
-    };
-    if constexpr (MODE == 2) {
-#pragma unroll
-      for (int i = 0; i < kCeKeep; ++i) {
-        const int c = tid + i * kCeThreads;
-        if (c < n_chunks) write_chunk(c, keep[i]);
-      }
-    } else {
-      for (int c = tid; c < n_chunks; c += kCeThreads) write_chunk(c, load16(base + c * kEpc));
     }
   }
 }
@@ -590,16 +660,32 @@ __global__ __launch_bounds__(256) void scale_by_device_scalar_kernel(T* x, int64
     x[i] = (T)((float)x[i] * f);
 }
 
-// loss = scale * sum(row_loss), additions in a fixed order
-__global__ __launch_bounds__(256) void mean_rows_kernel(const float* row_loss, int64_t n, float scale,
-                                                        float* loss) {
-  __shared__ float red[4];
+// loss = scale * sum(row_loss), additions in a fixed order.  One workgroup: 8 loads in flight on
+// each of 1024 threads make 8192 rows one round trip (8.6 -> 4.5 us against 256 threads with one).
+constexpr int kMeanThreads = 1024, kMeanInFlight = 8;
+
+__global__ __launch_bounds__(kMeanThreads) void mean_rows_kernel(const float* row_loss, int64_t n, float scale,
+                                                                 float* loss) {
+  __shared__ float red[kMeanThreads / 64];
   float s = 0.f;
-  for (int64_t i = threadIdx.x; i < n; i += 256) s += row_loss[i];
+  for (int64_t i0 = threadIdx.x; i0 < n; i0 += kMeanThreads * kMeanInFlight) {
+    float x[kMeanInFlight];
+#pragma unroll
+    for (int u = 0; u < kMeanInFlight; ++u) {
+      const int64_t i = i0 + u * kMeanThreads;
+      x[u] = i < n ? row_loss[i] : 0.f;
+    }
+    s += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+  }
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) *loss = ((red[0] + red[1]) + (red[2] + red[3])) * scale;
+  if (threadIdx.x == 0) {
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kMeanThreads / 64; ++w) total += red[w];
+    *loss = total * scale;
+  }
 }
 
 // Backward: dlogits[i, c] = (exp(x[i, c] - lse_i) - [c == target_i]) * upstream / N, one
@@ -875,31 +961,58 @@ void launch_argmax_rows(int dtype_f16, const void* x, int64_t* out, int64_t oute
                        (const float*)x, out, width);
 }
 
+// The narrowest group that holds a row on chip: few lanes without work, and as many workgroups
+// per CU as the row's size allows.
+template <typename T, int GROUP, int NREG, int NLDS, bool GRAD>
+static void cross_entropy_fwd_go(const T* x, const int64_t* targets, float* row_lse, float* row_loss, T* dx,
+                                 int64_t n_rows, int width, int* flag, hipStream_t stream) {
+  constexpr int kBlock = kRegBlockOf(GROUP), kRows = kBlock / GROUP, kLds = NLDS * GROUP * 16;
+  const auto kernel = cross_entropy_fwd_kernel<T, GROUP, NREG, NLDS, GRAD>;
+  if constexpr (kLds > 0) {
+    static bool attr_set = false;  // launches are serialised by the caller
+    if (!attr_set) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((n_rows + kRows - 1) / kRows)), dim3(kBlock), kLds, stream, x, targets,
+                     row_lse, row_loss, dx, (float)(1.0 / (double)n_rows), n_rows, width, flag);
+}
+
+template <typename T, bool GRAD>
+static void cross_entropy_fwd_t(const T* x, const int64_t* targets, float* row_lse, float* row_loss, T* dx,
+                                int64_t n_rows, int width, int* flag, hipStream_t stream) {
+  const int64_t n = worst_chunks<T>(x, width);
+#define DEERS_CE_TIER(GROUP, NREG, NLDS)                                                                          \
+  if (n <= GROUP * (NREG + NLDS))                                                                                 \
+    return cross_entropy_fwd_go<T, GROUP, NREG, NLDS, GRAD>(x, targets, row_lse, row_loss, dx, n_rows, width, flag, \
+                                                            stream);
+  DEERS_CE_TIER(64, 1, 0)
+  DEERS_CE_TIER(64, 4, 0)
+  DEERS_CE_TIER(256, 4, 0)
+  DEERS_CE_TIER(256, 8, 0)
+  DEERS_CE_TIER(1024, 4, 0)
+  if constexpr (sizeof(T) == 4) {
+    DEERS_CE_TIER(1024, 6, 2)
+    DEERS_CE_TIER(1024, 9, 4)
+    DEERS_CE_TIER(1024, 10, 4)
+  } else {
+    DEERS_CE_TIER(1024, 8, 0)
+  }
+#undef DEERS_CE_TIER
+  hipLaunchKernelGGL((cross_entropy_fwd_wide_kernel<T, GRAD>), dim3((unsigned)n_rows), dim3(kCeThreads), 0, stream,
+                     x, targets, row_lse, row_loss, dx, (float)(1.0 / (double)n_rows), width, flag);
+}
+
 void launch_cross_entropy_fwd(int dtype_f16, const void* logits, const int64_t* targets, float* row_lse,
                               float* row_loss, float* loss, void* dlogits, int64_t n_rows, int width,
                               int* flag, hipStream_t stream) {
   LaunchScope scope(dlogits ? "cross_entropy_fwd_grad" : "cross_entropy_fwd", stream);
-  const float inv_n = (float)(1.0 / (double)n_rows);
-  const dim3 grid((unsigned)n_rows), block(kCeThreads);
-  // a row and its possible lead-in fit the registers of a workgroup?
-  const bool resident = (int64_t)width + 16 <= (int64_t)kCeThreads * (dtype_f16 ? ce_keep<half_t>() * 8 : ce_keep<float>() * 4);
-  auto go = [&](auto kernel, auto* x, auto* dx) {
-    hipLaunchKernelGGL(kernel, grid, block, 0, stream, x, targets, row_lse, row_loss, dx, inv_n, width, flag);
+  auto go = [&](auto* x, auto* dx) {
+    if (dx) cross_entropy_fwd_t<std::decay_t<decltype(*dx)>, true>(x, targets, row_lse, row_loss, dx, n_rows, width, flag, stream);
+    else cross_entropy_fwd_t<std::decay_t<decltype(*dx)>, false>(x, targets, row_lse, row_loss, dx, n_rows, width, flag, stream);
   };
-  if (dtype_f16) {
-    const half_t* x = (const half_t*)logits;
-    half_t* dx = (half_t*)dlogits;
-    if (!dlogits) go(cross_entropy_fwd_kernel<half_t, 0>, x, dx);
-    else if (resident) go(cross_entropy_fwd_kernel<half_t, 2>, x, dx);
-    else go(cross_entropy_fwd_kernel<half_t, 1>, x, dx);
-  } else {
-    const float* x = (const float*)logits;
-    float* dx = (float*)dlogits;
-    if (!dlogits) go(cross_entropy_fwd_kernel<float, 0>, x, dx);
-    else if (resident) go(cross_entropy_fwd_kernel<float, 2>, x, dx);
-    else go(cross_entropy_fwd_kernel<float, 1>, x, dx);
-  }
-  hipLaunchKernelGGL(mean_rows_kernel, dim3(1), dim3(256), 0, stream, row_loss, n_rows,
+  if (dtype_f16) go((const half_t*)logits, (half_t*)dlogits);
+  else go((const float*)logits, (float*)dlogits);
+  hipLaunchKernelGGL(mean_rows_kernel, dim3(1), dim3(kMeanThreads), 0, stream, row_loss, n_rows,
                      (float)(1.0 / (double)n_rows), loss);
 }
 

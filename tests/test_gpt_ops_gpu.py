@@ -296,3 +296,25 @@ def test_index_add_list_lengths_and_column_passes(dtype, vocab, width, n):
     dst = rocm.DeviceBuffer((vocab, width), dtype, zeros=True)
     rocm.index_add_raw(dtype, dg.ptr, di.ptr, dst.ptr, vocab, n, width)
     assert np.array_equal(dst.numpy(), oracle.index_add(vocab, g, idx))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,v", [
+    (np.float32, 225), (np.float32, 993), (np.float32, 4065), (np.float32, 8161), (np.float32, 16353),
+    (np.float32, 32737), (np.float32, 32769), (np.float32, 53217), (np.float32, 57313), (np.float32, 57345),
+    (np.float16, 449), (np.float16, 16321), (np.float16, 65473), (np.float16, 65537)])
+def test_cross_entropy_at_the_edges_of_its_tiers(dtype, v):
+    # odd widths: rows start anywhere in a 128-byte line, so a width near a tier's end has rows on both sides
+    n = 5
+    x = synth.normal((n, v), synth.tensor_seed(79, "ce", "x"), 3.0).astype(dtype)
+    t = np.int64([0, v - 1, v // 2, 1, v - 2])
+    bx, bt = _dev(x), _dev(t)
+    lse, loss = rocm.DeviceBuffer((n,), np.float32), rocm.DeviceBuffer((1,), np.float32)
+    d = _dev(np.full((n, v), 9.0, dtype=dtype))
+    rocm.cross_entropy_fwd_grad_raw(dtype, bx.ptr, bt.ptr, lse.ptr, loss.ptr, d.ptr, n, v)
+    x32 = x.astype(np.float32)
+    want_lse = np.log(np.exp(x32.astype(np.float64)).sum(axis=1))
+    assert np.abs(lse.numpy() - want_lse).max() <= 1e-5 * np.abs(want_lse).max()
+    assert abs(float(loss.numpy()[0]) - float(oracle.cross_entropy_fwd(x32, t))) <= 1e-4
+    tol = 1e-6 if dtype == np.float32 else 5e-4
+    assert np.abs(d.numpy().astype(np.float32) - oracle.cross_entropy_bwd(x32, t)).max() <= tol
