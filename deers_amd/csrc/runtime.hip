@@ -14,6 +14,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <unordered_map>
 #include <mutex>
@@ -121,6 +122,9 @@ struct Runtime {
   // whether the next single-launch backward leaves out the workgroups that publish
   int bwd_spin_limit = 1 << 20;
   int bwd_skip_producers = 0;
+  // Pinned host memory that small device-to-host copies land in: a copy to pageable memory goes
+  // through the driver's own staging with a wait of its own
+  void* host_staging = nullptr;
   // sticky "an index was out of range" flag that index kernels raise; read back by the
   // next synchronising call after one of them has been launched
   int* index_flag = nullptr;
@@ -144,6 +148,7 @@ struct Runtime {
 
 Runtime g_rt;
 std::mutex g_mu;
+constexpr size_t kHostStagingBytes = 4096;
 
 // Device memory that exists without any allocation call: the split partials of
 // deers_rocm_attn_decode_noalloc live here.  Each GPU the library is loaded on holds its
@@ -349,6 +354,7 @@ int deers_rocm_init(int ordinal) {
   HIP_TRY(hipSetDevice(ordinal));
   HIP_TRY(hipStreamCreateWithFlags(&g_rt.stream, hipStreamNonBlocking));
   HIP_TRY(hipGetSymbolAddress(&g_scratch_ptr, HIP_SYMBOL(scratch)));
+  HIP_TRY(hipHostMalloc(&g_rt.host_staging, kHostStagingBytes, hipHostMallocDefault));
   {
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, ordinal));
@@ -542,8 +548,11 @@ int deers_rocm_dtoh(void* dst_host, const void* src_device, size_t bytes) {
   NEED_INIT();
   if (bytes == 0) return DEERS_ROCM_OK;
   if (!dst_host || !src_device) return fail(DEERS_ROCM_ERR_ARG, "dtoh: null pointer");
-  HIP_TRY(hipMemcpyAsync(dst_host, src_device, bytes, hipMemcpyDeviceToHost, g_rt.stream));
+  const bool staged = bytes <= kHostStagingBytes;
+  HIP_TRY(hipMemcpyAsync(staged ? g_rt.host_staging : dst_host, src_device, bytes, hipMemcpyDeviceToHost,
+                         g_rt.stream));
   HIP_TRY(hipStreamSynchronize(g_rt.stream));
+  if (staged) memcpy(dst_host, g_rt.host_staging, bytes);
   return check_device_flags();
 }
 

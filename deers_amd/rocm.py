@@ -392,7 +392,9 @@ def sum_squares_raw(dtype, x, n, total, accumulate=False):
 
 
 def _ptr_table(ptrs):
-    return (ctypes.c_void_p * len(ptrs))(*[p.value if isinstance(p, ctypes.c_void_p) else p for p in ptrs])
+    """Addresses or c_void_p, as the array's constructor takes both: an AdamW call over 74 tensors
+    converts 296 of them while the device waits."""
+    return (ctypes.c_void_p * len(ptrs))(*ptrs)
 
 
 def adamw_step_multi_raw(dtype, w, grad, m, v, sizes, lr, beta1, beta2, eps, weight_decay, step,
