@@ -28,6 +28,10 @@ namespace deers {
 void launch_attn_fwd_f16(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_fwd_f32(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, hipStream_t stream);
+bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
+bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
+void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream);
+void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f32(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_decode_f16(const DecodeParams& p, int B, int D, bool append, hipStream_t stream);
 int decode_pick_splits(int64_t BH, int64_t L, int* chunk);
@@ -674,7 +678,9 @@ int deers_rocm_attn_fwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
   p.H = (int)H; p.T = (int)T;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
-  if (dtype == DEERS_ROCM_F16)
+  if (dtype == DEERS_ROCM_F16 && deers::attn_fwd_f16_split_takes(B * H, T, D))
+    deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+  else if (dtype == DEERS_ROCM_F16)
     deers::launch_attn_fwd_f16(p, (int)B, (int)D, g_rt.stream);
   else
     deers::launch_attn_fwd_f32(p, (int)B, (int)D, g_rt.stream);
@@ -704,6 +710,18 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   if (int rc = resolve_strides("dq", dq, dq_strides, H, T, D, elem, &p.sdq)) return rc;
   if (int rc = resolve_strides("dk", dk, dk_strides, H, T, D, elem, &p.sdk)) return rc;
   if (int rc = resolve_strides("dv", dv, dv_strides, H, T, D, elem, &p.sdv)) return rc;
+  p.q = q; p.k = k; p.v = v; p.o = o; p.d_o = d_o; p.lse = lse;
+  p.dq = dq; p.dk = dk; p.dv = dv;
+  p.H = (int)H; p.T = (int)T;
+  p.scale = scale;
+  p.scale_log2 = (float)((double)scale * 1.4426950408889634);
+  // the form for launches that cannot fill the device needs no workspace and hands nothing over
+  // (the test hook of the hand-over asks for the form that does)
+  if (dtype == DEERS_ROCM_F16 && !g_rt.bwd_skip_producers && deers::attn_bwd_f16_split_takes(B * H, T, D)) {
+    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+    HIP_TRY(hipGetLastError());
+    return DEERS_ROCM_OK;
+  }
   // f32: delta[B,H,T].  f16: lse2 and negdelta, rows padded to a multiple of 64 per head.
   const int64_t t_pad = (T + 63) / 64 * 64;
   // f16: + 64 floats, the block-pipelined dK/dV role loads row vectors 64 floats at a time
@@ -712,7 +730,6 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   // f16: behind them the dQ role's scaled queries, [B*H][t_pad][D] f16
   const size_t ws_qs = dtype == DEERS_ROCM_F16 ? (size_t)(B * H * t_pad * D) * 2 : 0;
   if (int rc = workspace(ws_floats * sizeof(float) + ws_qs, &ws)) return rc;
-  p.q = q; p.k = k; p.v = v; p.o = o; p.d_o = d_o; p.lse = lse;
   p.delta = static_cast<float*>(ws);
   // A launch that is being captured into a graph gets no fresh epoch on replay: it takes the
   // two-launch form with the flags switched off (epoch 0).  The workspace and the flags must
@@ -752,10 +769,6 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.negdelta = static_cast<float*>(ws) + B * H * t_pad;
   p.qs = static_cast<float*>(ws) + ws_floats;
   p.t_pad = (int)t_pad;
-  p.dq = dq; p.dk = dk; p.dv = dv;
-  p.H = (int)H; p.T = (int)T;
-  p.scale = scale;
-  p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   if (dtype == DEERS_ROCM_F16) {
     if (single_launch) g_rt.bwd_error_armed = true;
     const int mode = !single_launch ? 0 : (g_rt.bwd_skip_producers ? 2 : 1);

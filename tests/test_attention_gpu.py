@@ -382,3 +382,39 @@ def test_elementwise_helper_errors():
         rocm.copy_compact_raw(np.float32, buf.ptr, (8,), (-1,), buf.ptr)  # negative stride
     with pytest.raises(rocm.RocmError):
         rocm.add_raw(np.float32, None, buf.ptr, buf.ptr, 8)  # null pointer
+
+
+# ---- f16 launches on either side of the line between the two forms (few heads: 32 rows per
+# workgroup, the walk divided among its waves; many heads: 128 rows per workgroup) ----
+
+@pytest.mark.parametrize("B,H,T,D", [
+    (1, 1, 2, 32), (2, 3, 65, 64), (1, 5, 95, 128), (1, 2, 128, 32), (1, 3, 129, 128), (2, 2, 161, 64),
+    (1, 2, 513, 32), (1, 1, 700, 128),                                           # few heads
+    (60, 7, 33, 64), (60, 7, 97, 32), (60, 7, 64, 128), (60, 7, 130, 32), (50, 8, 159, 64)])  # many
+def test_f16_forms_at_the_edges_of_their_blocks(B, H, T, D):
+    x = synth.attention_inputs(f"forms-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=21)
+    out = check_case(x, TOL[np.dtype(np.float16)], f"forms {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
+    again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for a, b in zip(out, again):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_f16_few_heads_rows_interleaved_over_heads():
+    """[B,T,H,D] memory under the logical [B,H,T,D], every operand: same bits as compact."""
+    import ctypes
+    B, H, T, D = 2, 3, 150, 64
+    x = synth.attention_inputs("forms-strided", B, H, T, D, np.float16, base_seed=22)
+    want = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    st = (T * H * D, D, H * D, 1)
+    bufs = {n: rocm.DeviceBuffer.from_numpy(np.ascontiguousarray(x[n].transpose(0, 2, 1, 3))) for n in x}
+    outs = {n: rocm.DeviceBuffer((B, T, H, D), np.float16) for n in ("o", "dq", "dk", "dv")}
+    lse = rocm.DeviceBuffer((B, H, T), np.float32)
+    scale = rocm.default_scale(D)
+    rocm.attn_fwd_raw(np.float16, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, B, H, T, D,
+                      scale, q_strides=st, k_strides=st, v_strides=st, o_strides=st)
+    rocm.attn_bwd_raw(np.float16, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, bufs["do"].ptr,
+                      outs["dq"].ptr, outs["dk"].ptr, outs["dv"].ptr, B, H, T, D, scale,
+                      strides={n: st for n in ("q", "k", "v", "o", "do", "dq", "dk", "dv")})
+    for name, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:])):
+        np.testing.assert_array_equal(outs[name].numpy().transpose(0, 2, 1, 3), ref, err_msg=name)
+    np.testing.assert_array_equal(lse.numpy(), want[1])
