@@ -134,6 +134,7 @@ struct Runtime {
   int* index_flag = nullptr;
   bool index_flag_armed = false;
   deers::SkinnyPrefetch skinny_next;  // one-shot hint for the next few-rows product (decode_linear_hint)
+  int* decode_counters = nullptr;  // arrival counters of split decode heads (all zero between launches)
   int* skinny_counters = nullptr;  // arrival counters of the few-rows GEMM's K splits (all zero between launches)
   // Block cache behind deers_rocm_alloc / _free.  Every kernel and copy of this library
   // runs on `stream`, in order, so a block handed back by free can be handed out again
@@ -152,6 +153,7 @@ struct Runtime {
 
 Runtime g_rt;
 std::mutex g_mu;
+constexpr int kDecodeCounters = 1024;  // heads of a decode call that may be split
 constexpr size_t kHostStagingBytes = 4096;
 
 // Device memory that exists without any allocation call: the split partials of
@@ -780,6 +782,24 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   return DEERS_ROCM_OK;
 }
 
+// Arrival counters for a decode call whose split heads are merged inside the launch; null where
+// they are merged by a second one: nothing to merge, splits that may not share an XCD, or a call
+// that may run beside another one (a captured graph; deers_rocm_attn_decode_noalloc asks for
+// null itself), since calls that overlap would count each other's arrivals.
+static int decode_counters(int64_t BH, int splits, int** out) {
+  *out = nullptr;
+  if (splits == 1 || BH > kDecodeCounters || !same_xcd_handover_now()) return DEERS_ROCM_OK;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
+  if (cs != hipStreamCaptureStatusNone) return DEERS_ROCM_OK;
+  if (!g_rt.decode_counters) {  // zero once; the kernel leaves every counter at zero
+    HIP_TRY(hipMalloc(&g_rt.decode_counters, kDecodeCounters * sizeof(int)));
+    HIP_TRY(hipMemsetAsync(g_rt.decode_counters, 0, kDecodeCounters * sizeof(int), g_rt.stream));
+  }
+  *out = g_rt.decode_counters;
+  return DEERS_ROCM_OK;
+}
+
 // Argument checks and launch shared by deers_rocm_attn_decode (partials in the growing
 // workspace) and deers_rocm_attn_decode_noalloc (partials in the static scratch array).
 static int attn_decode_impl(const char* what, bool no_alloc, int dtype, const void* q,
@@ -821,7 +841,9 @@ static int attn_decode_impl(const char* what, bool no_alloc, int dtype, const vo
   p.q = q; p.k = k_cache; p.v = v_cache; p.o = o;
   p.part_o = static_cast<float*>(ws);
   p.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
-  p.H = (int)H; p.L = (int)L; p.splits = splits; p.chunk = chunk;
+  p.BH = (int)(B * H); p.H = (int)H; p.L = (int)L; p.splits = splits; p.chunk = chunk;
+  if (!no_alloc)
+    if (int rc = decode_counters(B * H, splits, &p.arrived)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, false, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -888,7 +910,8 @@ int deers_rocm_attn_decode_append(int dtype, const void* q, const void* k, const
   p.in_b = in_strides[0]; p.in_h = in_strides[1];
   p.part_o = static_cast<float*>(ws);
   p.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
-  p.H = (int)H; p.L = (int)pos; p.splits = splits; p.chunk = chunk;
+  p.BH = (int)(B * H); p.H = (int)H; p.L = (int)pos; p.splits = splits; p.chunk = chunk;
+  if (int rc = decode_counters(B * H, splits, &p.arrived)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, true, g_rt.stream);
   HIP_TRY(hipGetLastError());

@@ -104,6 +104,22 @@ def test_unsplit_few_rows_gemm_matches_split_within_rounding(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,H,L,D", [(1, 1, 129, 64), (1, 7, 1500, 64), (1, 12, 257, 128), (2, 8, 4111, 32),
+                                     (11, 12, 300, 64), (16, 16, 130, 64), (17, 16, 130, 64)])
+def test_decode_splits_merged_in_the_launch_or_after_it_give_the_same_bits(gpu, B, H, L, D):
+    """Few heads with many splits, a last split of one row, as many workgroups as CUs and more."""
+    x = synth.attention_inputs(f"handover-dec-{B}-{H}-{L}-{D}", B, H, 1, D, np.float16, base_seed=13, kv_len=L,
+                               names=("q", "k", "v"))
+    outs = []
+    for mode in (rocm.HANDOVER_SAME_XCD, rocm.HANDOVER_STREAM_ORDER, rocm.HANDOVER_SAME_XCD):
+        rocm.set_handover_mode(mode)
+        outs.append(rocm.attn_decode(x["q"][:, :, 0], x["k"], x["v"]))
+    want = oracle.attn_fwd(x["q"], x["k"], x["v"])[:, :, 0]
+    assert np.max(np.abs(outs[0].astype(np.float64) - want)) <= 5e-3
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
+
+
+@pytest.mark.gpu
 def test_a_wait_that_runs_out_is_reported_and_then_cleared(gpu):
     B, H, T, D = 1, 2, 200, 64
     x = synth.attention_inputs("handover-giveup", B, H, T, D, np.float16, base_seed=12)
