@@ -47,6 +47,7 @@ constexpr int kSkStepBytes = 2048;            // W tile [16 k x 32 n] + x tile [
 constexpr int kSkChunkBytes = kSkStepsPerChunk * kSkStepBytes;
 constexpr int kSkWaveBytes = kSkRing * kSkChunkBytes;
 constexpr int kSkLds = kSkWaves * kSkWaveBytes;  // 96 KB
+constexpr int kSkGather = 4;                     // splits whose partials the last arrival has in flight
 constexpr int kSkPieceBytes = 256 * 64;          // prefetch unit: 256 rows of a packed tile
 
 template <bool ACCUMULATE, int PROLOGUE>
@@ -105,9 +106,13 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
   const int w_row = lane >> 2;
   const int w_piece = min(lane & 3, (N - n0) / 8 - 1);
   const uint32_t w_lane_off = (uint32_t)((w_row * ldw + 8 * w_piece) * 2);
-  // x tile of a step: lane -> row lane/2 of 32 (clamped to M-1), 16-byte piece lane%2
-  const int x_row = min(lane >> 1, M - 1);
-  const uint32_t x_lane_off = (uint32_t)((x_row * ldx + 8 * (lane & 1)) * 2);
+  // x part of a chunk [32 m][64 k]: 8 rows of 128 bytes per load (clamped to row M-1), so that a
+  // load touches 8 cache lines.  Row r's 16-byte piece c sits at position c ^ (r % 8): the
+  // fragment reads below take one piece of 32 rows at a time and would otherwise share banks.
+  uint32_t x_lane_off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    x_lane_off[i] = (uint32_t)((min(8 * i + (lane >> 3), M - 1) * ldx + 8 * ((lane & 7) ^ (lane >> 3))) * 2);
   // row-major W: the block's 32 columns start 32 elements after the previous block's, rows
   // ldw apart; packed W ([column block][K][32]): blocks K*32 apart, rows 32 apart
   const half_t* w_base = W + col_block * w_block_stride;
@@ -117,10 +122,21 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
 #pragma unroll
     for (int i = 0; i < kSkStepsPerChunk; ++i) {
       const int k0 = k_begin + (chunk * kSkStepsPerChunk + i) * 16;
-      async_load16_to_lds(w_base + (int64_t)k0 * ldw, w_lane_off, dst + i * kSkStepBytes);
-      async_load16_to_lds(x + k0, x_lane_off, dst + i * kSkStepBytes + 1024);
+      async_load16_to_lds(w_base + (int64_t)k0 * ldw, w_lane_off, dst + i * 1024);
+      async_load16_to_lds(x + k_begin + chunk * 64, x_lane_off[i], dst + 4096 + i * 1024);
     }
   };
+  // the addend of the columns this lane will hold at the end: requested first, so that its trip
+  // to memory is over by then
+  const int rp = wave & 1;  // waves 0 and 1 sum and store output columns n0 + 16 rp .. + 15
+  const int c_lo = n0 + 16 * rp + 4 * g, c_hi = c_lo + 8;
+  half4 old_lo = {0, 0, 0, 0}, old_hi = {0, 0, 0, 0};
+  if constexpr (ACCUMULATE) {
+    if (wave < 2 && (lane & 31) < M) {
+      if (c_lo < N) old_lo = *(const half4*)(y + (int64_t)(lane & 31) * ldy + c_lo);
+      if (c_hi < N) old_hi = *(const half4*)(y + (int64_t)(lane & 31) * ldy + c_hi);
+    }
+  }
   issue(0);
   if (n_chunks > 1) issue(1);
 
@@ -138,12 +154,12 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
     const char* chunk = smem + wave * kSkWaveBytes + (c % kSkRing) * kSkChunkBytes;
 #pragma unroll
     for (int i = 0; i < kSkStepsPerChunk; ++i) {
-      const half_t* wt = (const half_t*)(chunk + i * kSkStepBytes);          // [16][32]
-      const half_t* xt = (const half_t*)(chunk + i * kSkStepBytes + 1024);   // [32][16]
-      const half8 a = lds_frag_transposed(wt, 32, 0, 0, lane);  // column lane%32; k = 4g..4g+3, 8+4g..
-      const half4 b_lo = *(const half4*)(xt + (lane & 31) * 16 + 4 * g);
-      const half4 b_hi = *(const half4*)(xt + (lane & 31) * 16 + 8 + 4 * g);
-      half8 b = __builtin_shufflevector(b_lo, b_hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      // k of slot e of lane half g in step i: 16 i + 8 g + e
+      const half_t* wt = (const half_t*)chunk + (16 * i + 8 * g + ((lane & 15) >> 2)) * 32 + 4 * (lane & 3) +
+                         ((lane >> 4) & 1) * 16;
+      const half4 a_lo = lds_read_tr16(wt), a_hi = lds_read_tr16(wt + 4 * 32);
+      const half8 a = __builtin_shufflevector(a_lo, a_hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      half8 b = *(const half8*)(chunk + 4096 + (lane & 31) * 128 + (((2 * i + g) ^ (lane & 7)) * 16));
       if constexpr (PROLOGUE == kSkinnyReluSq) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -170,7 +186,6 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
   if constexpr (PROLOGUE == kSkinnyRmsNorm) red_sq[wave * 64 + lane] = sum_sq;
   __syncthreads();
   float s[8];
-  const int rp = wave & 1;  // waves 0 and 1 sum and store output columns n0 + 16 rp .. + 15
   if (wave < 2) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -190,11 +205,14 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
     }
   }
   if (S > 1) {
-    // this workgroup's partial tile: [column block][split][rp][lane][8] floats
-    float* mine = partial + ((((int64_t)col_block * S + split) * 2 + rp) * 64 + lane) * 8;
+    // a partial tile: [column block][split][rp][pair of sums][lane], so that a wave's accesses are
+    // 512-byte runs
+    typedef unsigned long long u64;
+    u64* tiles = (u64*)partial + ((int64_t)col_block * S * 2 + rp) * 4 * 64 + lane;
     if (wave < 2) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) mine[e] = s[e];
+      for (int e = 0; e < 4; ++e)
+        tiles[(split * 8 + e) * 64] = __builtin_bit_cast(u64, floatx2{s[2 * e], s[2 * e + 1]});
     }
     // The S workgroups of a column block share one XCD and so one L2: a completed store
     // (vmcnt 0) is in that L2, and relaxed device-scope atomics, which bypass the CU's
@@ -214,11 +232,23 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
     if (wave < 2) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) s[e] = 0.f;
-      for (int sp = 0; sp < S; ++sp) {  // index order, whoever arrived last
-        const float* theirs = partial + ((((int64_t)col_block * S + sp) * 2 + rp) * 64 + lane) * 8;
+      for (int sp = 0; sp < S; sp += kSkGather) {  // index order, whoever arrived last
+        u64 t[kSkGather][4];  // requested together: one trip to L2, not one per split
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          s[e] += __hip_atomic_load(theirs + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int i = 0; i < kSkGather; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            t[i][e] = __hip_atomic_load(tiles + (min(sp + i, S - 1) * 8 + e) * 64, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < kSkGather; ++i)
+          if (sp + i < S)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const floatx2 f = __builtin_bit_cast(floatx2, t[i][e]);
+              s[2 * e] += f[0];
+              s[2 * e + 1] += f[1];
+            }
       }
     }
   }
@@ -235,20 +265,11 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
       lo[e] = (half_t)s[e];
       hi[e] = (half_t)s[4 + e];
     }
-    if constexpr (ACCUMULATE) {
-      // the addend is added in f32 before the one rounding: fetch the lane's own columns
-      if (m < M) {
-        const int c_lo = n0 + 16 * rp + 4 * g, c_hi = c_lo + 8;
-        if (c_lo < N) {
-          const half4 old = *(const half4*)(y + (int64_t)m * ldy + c_lo);
+    if constexpr (ACCUMULATE) {  // in f32, before the one rounding
 #pragma unroll
-          for (int e = 0; e < 4; ++e) lo[e] = (half_t)(s[e] + (float)old[e]);
-        }
-        if (c_hi < N) {
-          const half4 old = *(const half4*)(y + (int64_t)m * ldy + c_hi);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) hi[e] = (half_t)(s[4 + e] + (float)old[e]);
-        }
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = (half_t)(s[e] + (float)old_lo[e]);
+        hi[e] = (half_t)(s[4 + e] + (float)old_hi[e]);
       }
     }
     const u32x2 xu = __builtin_bit_cast(u32x2, lo), yu = __builtin_bit_cast(u32x2, hi);
