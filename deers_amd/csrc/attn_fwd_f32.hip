@@ -1,4 +1,5 @@
-// Fused causal attention forward, f32 storage and arithmetic, gfx950.
+// Fused causal attention forward, f32 storage and arithmetic, gfx950: the large launches of head
+// widths 64 and 128 (attn_split_f32.hip has the others and the rule).
 //
 // Same decomposition as the f16 kernel (one query column per lane, S^T = K Q^T,
 // O^T += V^T P^T, online softmax in the log2 domain) on v_mfma_f32_32x32x2_f32.
@@ -35,7 +36,7 @@ struct Fwd32Lists {
 };
 
 template <int D, int BN>
-__global__ __launch_bounds__(256, (D == 32 ? 3 : 2)) void attn_fwd_f32_kernel(FwdParams p, int BH, int n_qtiles,
+__global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(FwdParams p, int BH, int n_qtiles,
                                                            int heads_per_xcd, const int* lists,
                                                            int max_len) {
   constexpr int LD = D + 4;   // LDS row stride in floats
@@ -375,7 +376,6 @@ void launch_attn_fwd_f32(const FwdParams& p, int B, int D, hipStream_t stream) {
   const int n_qtiles = (p.T + kFwd32BM - 1) / kFwd32BM;
   const int heads_per_xcd = (BH + 7) / 8;
   switch (D) {
-    case 32: launch_fwd32_d<32, 64>(p, BH, n_qtiles, heads_per_xcd, stream); break;
     case 64: launch_fwd32_d<64, 64>(p, BH, n_qtiles, heads_per_xcd, stream); break;
     case 128: launch_fwd32_d<128, 32>(p, BH, n_qtiles, heads_per_xcd, stream); break;
   }

@@ -166,8 +166,7 @@ constexpr size_t split_fwd_lds() {  // two V blocks per wave, or the merge; then
 }
 
 template <int D, int W>
-__global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams p, int BH, int n_blocks,
-                                                                        int heads_per_xcd) {
+__global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams p, int BH, int n_blocks) {
   using C = SplitCfg<D>;
   constexpr int KS = C::KS, DB = C::DB;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -175,7 +174,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5, T = p.T;
   int bh, rank;
-  if (!map_block(blockIdx.x, n_blocks, heads_per_xcd, BH, &bh, &rank)) return;
+  if (!map_block_even(blockIdx.x, n_blocks, BH, &bh, &rank)) return;
   const int qb = n_blocks - 1 - rank;  // longest rows first
   const int b_ = bh / p.H, h_ = bh % p.H;
   const half_t* K = (const half_t*)p.k + b_ * p.sk.b + h_ * p.sk.h;
@@ -424,14 +423,12 @@ __device__ __forceinline__ void split_dkdv_body(const BwdParams& p, int bh, int 
 // Ranks alternate between the roles, longest first: rank 2 r is the dK/dV block of keys 32 r ..,
 // rank 2 r + 1 the dQ block as many rows from the end.
 template <int D, int W>
-__global__ __launch_bounds__(64 * W, D == 128 ? 1 : 2) void attn_bwd_f16_split_kernel(BwdParams p, int BH,
-                                                                                       int n_blocks,
-                                                                                       int heads_per_xcd) {
+__global__ __launch_bounds__(64 * W, D == 128 ? 1 : 2) void attn_bwd_f16_split_kernel(BwdParams p, int BH, int n_blocks) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bh, rank;
-  if (!map_block(blockIdx.x, 2 * n_blocks, heads_per_xcd, BH, &bh, &rank)) return;
+  if (!map_block_even(blockIdx.x, 2 * n_blocks, BH, &bh, &rank)) return;
   if (rank & 1)
     split_dq_body<D, W>(p, bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
   else
@@ -451,9 +448,8 @@ void launch_fwd_split(const FwdParams& p, int BH, hipStream_t stream) {
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
-  const int n_blocks = (p.T + kSplitRows - 1) / kSplitRows, heads_per_xcd = (BH + 7) / 8;
-  hipLaunchKernelGGL(kernel, dim3(8 * n_blocks * heads_per_xcd), dim3(64 * W), lds, stream, p, BH, n_blocks,
-                     heads_per_xcd);
+  const int n_blocks = (p.T + kSplitRows - 1) / kSplitRows;
+  hipLaunchKernelGGL(kernel, dim3(map_even_blocks(n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
 }
 template <int D, int W>
 void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
@@ -462,9 +458,8 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
-  const int n_blocks = (p.T + kSplitRows - 1) / kSplitRows, heads_per_xcd = (BH + 7) / 8;
-  hipLaunchKernelGGL(kernel, dim3(16 * n_blocks * heads_per_xcd), dim3(64 * W), lds, stream, p, BH, n_blocks,
-                     heads_per_xcd);
+  const int n_blocks = (p.T + kSplitRows - 1) / kSplitRows;
+  hipLaunchKernelGGL(kernel, dim3(map_even_blocks(2 * n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
 }
 
 }  // namespace

@@ -302,6 +302,28 @@ __device__ __forceinline__ bool map_block(int block_id, int n_blocks, int heads_
   return *bh < BH;
 }
 
+// The same for launches of few heads, where whole heads per XCD leave XCDs idle (12 heads: 2, 2, 2, 2,
+// 1, 1, 1, 1): BH / 8 whole heads per XCD, and the blocks of the BH % 8 remaining heads dealt to all
+// XCDs in turn.  An XCD's list is still ordered by rank.  The grid is map_even_blocks(n_ranks, BH).
+__device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH, int* bh, int* rank) {
+  const int xcd = block_id & 7, idx = block_id >> 3;
+  const int whole = BH >> 3, rest = BH & 7;
+  // remaining heads' blocks of rank < k on this XCD: t = rank * rest + head, dealt to XCD t % 8
+  auto dealt = [&](int k) { return k * rest > xcd ? (k * rest - xcd + 7) >> 3 : 0; };
+  int k = (int)((int64_t)idx * 8 / BH);
+  while (whole * (k + 1) + dealt(k + 1) <= idx) ++k;
+  while (k > 0 && whole * k + dealt(k) > idx) --k;
+  if (k >= n_ranks) return false;
+  const int in_rank = idx - (whole * k + dealt(k)), extra = dealt(k + 1) - dealt(k);
+  if (in_rank < extra)
+    *bh = 8 * whole + (8 * (dealt(k) + in_rank) + xcd) % rest;
+  else
+    *bh = (in_rank - extra) * 8 + xcd;
+  *rank = k;
+  return true;
+}
+inline int map_even_blocks(int n_ranks, int BH) { return 8 * (n_ranks * (BH >> 3) + (n_ranks * (BH & 7) + 7) / 8); }
+
 // Brackets one kernel launch with a hipEvent pair when per-kernel profiling is
 // switched on (deers_rocm_profile_enable); a no-op otherwise.  Defined in
 // runtime.hip.

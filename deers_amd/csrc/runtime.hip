@@ -33,6 +33,10 @@ bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f32(const BwdParams& p, int B, int D, hipStream_t stream);
+bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
+bool attn_bwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
+void launch_attn_fwd_f32_split(const FwdParams& p, int B, int D, hipStream_t stream);
+void launch_attn_bwd_f32_split(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_decode_f16(const DecodeParams& p, int B, int D, bool append, hipStream_t stream);
 int decode_pick_splits(int64_t BH, int64_t L, int* chunk);
 void launch_fill(int dtype_f16, void* dst, size_t n, float value, hipStream_t stream);
@@ -684,6 +688,8 @@ int deers_rocm_attn_fwd(int dtype, const void* q, const int64_t* q_strides, cons
     deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, g_rt.stream);
   else if (dtype == DEERS_ROCM_F16)
     deers::launch_attn_fwd_f16(p, (int)B, (int)D, g_rt.stream);
+  else if (deers::attn_fwd_f32_split_takes(B * H, T, D))
+    deers::launch_attn_fwd_f32_split(p, (int)B, (int)D, g_rt.stream);
   else
     deers::launch_attn_fwd_f32(p, (int)B, (int)D, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -717,10 +723,15 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.H = (int)H; p.T = (int)T;
   p.scale = scale;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
-  // the form for launches that cannot fill the device needs no workspace and hands nothing over
+  // the forms for launches that cannot fill the device need no workspace and hand nothing over
   // (the test hook of the hand-over asks for the form that does)
   if (dtype == DEERS_ROCM_F16 && !g_rt.bwd_skip_producers && deers::attn_bwd_f16_split_takes(B * H, T, D)) {
     deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+    HIP_TRY(hipGetLastError());
+    return DEERS_ROCM_OK;
+  }
+  if (dtype == DEERS_ROCM_F32 && deers::attn_bwd_f32_split_takes(B * H, T, D)) {
+    deers::launch_attn_bwd_f32_split(p, (int)B, (int)D, g_rt.stream);
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }

@@ -418,3 +418,38 @@ def test_f16_few_heads_rows_interleaved_over_heads():
     for name, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:])):
         np.testing.assert_array_equal(outs[name].numpy().transpose(0, 2, 1, 3), ref, err_msg=name)
     np.testing.assert_array_equal(lse.numpy(), want[1])
+
+
+# ---- f32 launches: 32 rows per workgroup in one, two and four waves, and the 128-row kernels ----
+
+@pytest.mark.parametrize("B,H,T,D", [
+    (1, 1, 2, 32), (2, 3, 33, 64), (1, 5, 95, 128), (1, 2, 128, 32), (1, 3, 129, 64), (2, 2, 161, 128), (1, 9, 257, 32),
+    (1, 1, 700, 128),                                                             # four waves, or a wave per block
+    (60, 7, 63, 64), (25, 8, 130, 32), (25, 5, 193, 128), (60, 7, 97, 128), (100, 8, 159, 64),  # two and one
+    (40, 10, 700, 32), (20, 4, 990, 64), (19, 10, 641, 128)])                     # 128 rows
+def test_f32_forms_at_the_edges_of_their_blocks(B, H, T, D):
+    x = synth.attention_inputs(f"forms32-{B}-{H}-{T}-{D}", B, H, T, D, np.float32, base_seed=23)
+    out = check_case(x, TOL[np.dtype(np.float32)], f"f32 forms {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
+    again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for a, b in zip((out[0], out[1], out[3], out[4]), (again[0], again[1], again[3], again[4])):
+        np.testing.assert_array_equal(a, b)  # dQ of the one-pass backward is summed in arrival order
+
+
+def test_f32_few_heads_rows_interleaved_over_heads():
+    """[B,T,H,D] memory under the logical [B,H,T,D], every operand: same bits as compact."""
+    B, H, T, D = 2, 3, 150, 64
+    x = synth.attention_inputs("forms32-strided", B, H, T, D, np.float32, base_seed=24)
+    want = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    st = (T * H * D, D, H * D, 1)
+    bufs = {n: rocm.DeviceBuffer.from_numpy(np.ascontiguousarray(x[n].transpose(0, 2, 1, 3))) for n in x}
+    outs = {n: rocm.DeviceBuffer((B, T, H, D), np.float32) for n in ("o", "dq", "dk", "dv")}
+    lse = rocm.DeviceBuffer((B, H, T), np.float32)
+    scale = rocm.default_scale(D)
+    rocm.attn_fwd_raw(np.float32, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, B, H, T, D,
+                      scale, q_strides=st, k_strides=st, v_strides=st, o_strides=st)
+    rocm.attn_bwd_raw(np.float32, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, bufs["do"].ptr,
+                      outs["dq"].ptr, outs["dk"].ptr, outs["dv"].ptr, B, H, T, D, scale,
+                      strides={n: st for n in ("q", "k", "v", "o", "do", "dq", "dk", "dv")})
+    for name, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:])):
+        np.testing.assert_array_equal(outs[name].numpy().transpose(0, 2, 1, 3), ref, err_msg=name)
+    np.testing.assert_array_equal(lse.numpy(), want[1])
