@@ -6,7 +6,7 @@
 // The kernels of those files give a workgroup 128 rows and let its four waves walk the other
 // operand together: one dependent chain of T / 32 stages with a barrier in each.  With few heads
 // or short sequences the launch is nothing but that chain (12 heads of 512 x 64: 48 workgroups on
-// 256 CUs, forward 10.1 us and backward 17.5 us; here 6.6 and 11.3).  Here a workgroup owns 32 rows,
+// 256 CUs, forward 10.1 us and backward 17.5 us; here 6.4 and 10.9).  Here a workgroup owns 32 rows,
 // so there are four times as many of them, and its W waves divide the blocks of 32 rows of the
 // other operand among themselves (wave w takes blocks w, w + W, ...), each with its own loads,
 // its own slice of LDS and no barrier; their partial results meet once, at the end, in LDS.  The
@@ -14,8 +14,8 @@
 // 32 rows read all of the other operand through L1 (64 bytes per clock and CU), so launches that
 // fill the device anyway stay with the 128-row kernels (the rule is above split_takes, below).
 //
-//   forward  S^T = K Q^T, one query per lane, K fragments straight from global memory, V through
-//            LDS for its transposed fragments; online softmax per wave; O, m and l are merged.
+//   forward  S^T = K Q^T, one query per lane; V through LDS for its transposed fragments, K through
+//            LDS or straight into registers; online softmax per wave; O, m and l are merged.
 //   dQ       the same walk: S^T and dP^T = V dO^T, dQ^T += K^T dS^T with K in LDS; sums merged.
 //   dK/dV    a workgroup owns 32 keys, one per lane; Q and dO blocks in LDS (row and transposed
 //            fragments).  It forms each query block's row sums dO . O itself, so it waits for
@@ -30,8 +30,6 @@ namespace deers {
 
 namespace {
 
-constexpr int kSplitRows = 32;
-
 template <int D>
 struct SplitCfg {
   static constexpr int KS = D / 16;         // contraction steps over D
@@ -39,12 +37,19 @@ struct SplitCfg {
   static constexpr int RB = 2 * D;          // bytes per row
   static constexpr int CH = D / 8;          // 16-byte chunks per row
   static constexpr int BB = 32 * RB;        // bytes of a 32-row block
+  static constexpr int NI = BB / 1024;      // loads per block
   static constexpr int kRound = DB > 2 ? 4 : 2 * DB;  // 16-column units merged per round
 };
 
 // Every load of this wave has landed, those into LDS included; LDS reads stay behind it.
 __device__ __forceinline__ void settle_loads() {
   wait_all_vmem();
+  asm volatile("" ::: "memory");
+}
+
+// Before the loads into a block that earlier LDS reads of this wave have used: those have returned.
+__device__ __forceinline__ void settle_lds_reads() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   asm volatile("" ::: "memory");
 }
 
@@ -56,12 +61,20 @@ template <int D>
 __device__ __forceinline__ void split_load_block(const half_t* base, int row_stride, int r0, int T, uint32_t dst,
                                                  int lane) {
   using C = SplitCfg<D>;
-  constexpr int RPW = 1024 / C::RB;
+  constexpr int RPL = 1024 / C::RB;  // rows per load
+  const int lane_row = lane / C::CH;
+  if (r0 + 32 <= T) {  // the row of a load goes into its scalar base
+    const uint32_t row_off = opaque((uint32_t)lane_row * (uint32_t)row_stride * 2);
+    const half_t* row = base + (int64_t)r0 * row_stride;
 #pragma unroll
-  for (int i = 0; i < C::BB / 1024; ++i) {
-    const int row = i * RPW + lane / C::CH;
-    const uint32_t col = 16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(row));
-    async_load16_to_lds(base, (uint32_t)(min(r0 + row, T - 1) * row_stride * 2) + col, dst + i * 1024);
+    for (int i = 0; i < C::NI; ++i)
+      async_load16_to_lds(row + (int64_t)(i * RPL) * row_stride,
+                          row_off + 16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(i * RPL + lane_row)), dst + i * 1024);
+  } else {
+#pragma unroll
+    for (int i = 0; i < C::NI; ++i)
+      async_load16_to_lds(base, (uint32_t)min(r0 + i * RPL + lane_row, T - 1) * (uint32_t)row_stride * 2 +
+                                    16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(i * RPL + lane_row)), dst + i * 1024);
   }
 }
 
@@ -159,13 +172,16 @@ constexpr size_t merge_bytes() { return (size_t)W * SplitCfg<D>::kRound * 8 * 64
 
 // ---- forward ----
 
-template <int D, int W>
-constexpr size_t split_fwd_lds() {  // two V blocks per wave, or the merge; then m and l of every wave
-  const size_t ring = (size_t)W * 2 * SplitCfg<D>::BB;
-  return std::max(ring, merge_bytes<D, W>()) + W * 32 * 2 * sizeof(float);
+// KREGS: the wave's next K fragments wait in registers, straight from global memory, and V has two
+// blocks in LDS: the shortest stage.  Otherwise K and V have one block each in LDS, filled by whole
+// cache lines and asked for again as soon as they have been read: half the LDS and a quarter of the lines
+// per load, for launches in which several waves of a SIMD cover each other's waits.
+template <int D, int W, bool KREGS>
+constexpr size_t split_fwd_lds() {  // two blocks per wave, or the merge; then m and l of every wave
+  return std::max((size_t)W * 2 * SplitCfg<D>::BB, merge_bytes<D, W>()) + W * 32 * 2 * sizeof(float);
 }
 
-template <int D, int W>
+template <int D, int W, bool KREGS>
 __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams p, int BH, int n_blocks) {
   using C = SplitCfg<D>;
   constexpr int KS = C::KS, DB = C::DB;
@@ -182,28 +198,50 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
   const int skt = (int)p.sk.t, svt = (int)p.sv.t;
   const int qrow = 32 * qb + (lane & 31);
   const uint32_t ring = lds_address(smem) + wave * 2 * C::BB;
+  const uint32_t k_blk = ring + C::BB;
+  uint32_t v_blk = ring;
 
-  half8 kf[KS], qf[KS];
+  half8 kf[KREGS ? KS : 1], qf[KS];
   int kb = wave;
+  auto request_k = [&](int block) {
+    if constexpr (KREGS)
+      split_global_frags<D>(kf, K, skt, min(32 * block + (lane & 31), T - 1), g);
+    else
+      split_load_block<D>(K, skt, 32 * block, T, k_blk, lane);
+  };
   if (kb <= qb) {
-    split_load_block<D>(V, svt, 32 * kb, T, ring, lane);
-    split_global_frags<D>(kf, K, skt, min(32 * kb + (lane & 31), T - 1), g);
+    if (KREGS) split_load_block<D>(V, svt, 32 * kb, T, v_blk, lane);
+    request_k(kb);
   }
   split_global_frags<D>(qf, (const half_t*)p.q + b_ * p.sq.b + h_ * p.sq.h, (int)p.sq.t, min(qrow, T - 1), g);
+  if (!KREGS && kb <= qb) split_load_block<D>(V, svt, 32 * kb, T, v_blk, lane);
+  if (!KREGS) wait_all_vmem();
   scale_frags<KS>(qf, p.scale_log2);
 
   floatx16 oacc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) oacc[db] = ZERO16S;
   float m = -INFINITY, l = 0.f;
-  for (uint32_t slot = 0; kb <= qb; kb += W, slot ^= C::BB) {
-    settle_loads();  // K and V of this block
+  for (; kb <= qb; kb += W) {
+    const bool more = kb + W <= qb;
+    if constexpr (KREGS)
+      settle_loads();  // K and V of this block
+    else
+      wait_vmcnt<C::NI>();  // K; V's block may be on its way
     floatx16 s = ZERO16S;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) s = mfma_f16(kf[ks], qf[ks], s);
-    if (kb + W <= qb) {  // the next block's, under this block's work
-      split_load_block<D>(V, svt, 32 * (kb + W), T, ring + (slot ^ C::BB), lane);
-      split_global_frags<D>(kf, K, skt, min(32 * (kb + W) + (lane & 31), T - 1), g);
+    for (int ks = 0; ks < KS; ++ks) {
+      half8 k;
+      if constexpr (KREGS) k = kf[ks];
+      else k = split_row_frag<D>(k_blk, ks, lane);
+      s = mfma_f16(k, qf[ks], s);
+    }
+    if (more) {  // the next block's, under this block's work
+      if constexpr (KREGS)
+        split_load_block<D>(V, svt, 32 * (kb + W), T, v_blk ^ C::BB, lane);
+      else
+        settle_lds_reads();
+      request_k(kb + W);
     }
     if (kb == qb) {  // the diagonal block (its keys past T - 1 lie in the future of every stored row)
 #pragma unroll
@@ -228,16 +266,28 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
       sum[r & 1] += s[r];
     }
     l += sum[0] + sum[1];
+    if constexpr (!KREGS) {
+      if (more)
+        wait_vmcnt<C::NI>();  // V
+      else
+        wait_vmcnt<0>();
+    }
 #pragma unroll
     for (int ms = 0; ms < 2; ++ms) {
       const half8 pf = pack_regs(s, ms);
 #pragma unroll
-      for (int db = 0; db < DB; ++db) oacc[db] = mfma_f16(split_col_frag<D>(ring + slot, ms, db, lane), pf, oacc[db]);
+      for (int db = 0; db < DB; ++db) oacc[db] = mfma_f16(split_col_frag<D>(v_blk, ms, db, lane), pf, oacc[db]);
+    }
+    if constexpr (KREGS) {
+      v_blk ^= C::BB;
+    } else if (more) {
+      settle_lds_reads();
+      split_load_block<D>(V, svt, 32 * (kb + W), T, v_blk, lane);
     }
   }
 
   // ---- the waves' (m, l, O) become one; a wave without a block has m = -inf and weight 0 ----
-  float* stat_m = (float*)(smem + split_fwd_lds<D, W>() - W * 32 * 2 * sizeof(float));
+  float* stat_m = (float*)(smem + split_fwd_lds<D, W, KREGS>() - W * 32 * 2 * sizeof(float));
   float* stat_l = stat_m + W * 32;
   l = pair_sum(l);
   if (g == 0) {
@@ -441,14 +491,14 @@ void allow_lds(Kernel kernel, size_t bytes) {
     (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-template <int D, int W>
+template <int D, int W, bool KREGS>
 void launch_fwd_split(const FwdParams& p, int BH, hipStream_t stream) {
-  const auto kernel = attn_fwd_f16_split_kernel<D, W>;
-  constexpr size_t lds = split_fwd_lds<D, W>();
+  const auto kernel = attn_fwd_f16_split_kernel<D, W, KREGS>;
+  constexpr size_t lds = split_fwd_lds<D, W, KREGS>();
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
-  const int n_blocks = (p.T + kSplitRows - 1) / kSplitRows;
+  const int n_blocks = (p.T + 31) / 32;
   hipLaunchKernelGGL(kernel, dim3(map_even_blocks(n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
 }
 template <int D, int W>
@@ -458,44 +508,95 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
-  const int n_blocks = (p.T + kSplitRows - 1) / kSplitRows;
+  const int n_blocks = (p.T + 31) / 32;
   hipLaunchKernelGGL(kernel, dim3(map_even_blocks(2 * n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
 }
 
 }  // namespace
 
-// Where the lines lie (measured on grids of T = 32 .. 2048, 1 .. 384 heads and the three head
-// widths, us per launch, 128-row kernels -> these; n = heads * T / 32 workgroups):
-//   forward   a win while the workgroups' reads of the whole other operand stay few: n * D / 32 up
-//             to about 1152 (D = 64: 12 x 1024 16.3 -> 11.4, 24 x 512 10.3 -> 7.9; n = 768: 17.9 ->
-//             23.0).  Short sequences are one or two stages either way and only win while nearly
-//             everything runs at once (48 x 128 5.6 -> 5.1, 96 x 128 5.7 -> 5.7).
-//   backward  the dK/dV role reads three operands per block, so the line is lower, and it falls with
-//             the length of the walk (D = 64: 24 x 256 14.3 -> 9.0, 12 x 512 17.5 -> 11.3, 12 x 768 21.2 ->
-//             20.1, 12 x 1024 23.8 -> 25.3; 12 x 256 x 128 20.8 -> 11.6).
+// Which launches come here and in which form, measured on T = 32 .. 8192, 3 .. 800 heads and the three
+// head widths against the 128-row kernels and between 1, 2 and 4 waves.  nb = T / 32 is the length of a
+// walk, n = heads * nb the number of workgroups, u = n * D / 64 their number weighted by what a block
+// of the other operand weighs.
+//
+// Waves: four while the workgroups are few, and for long walks (forward D = 64, us in 4 / 2 / 1 waves:
+// 12 x 512 6.8 / 9.2 / 13.7, 24 x 1024 11.0 / 15.1 / 24.9, 96 x 256 7.3 / 7.1 / 9.1; backward 12 x 512
+// 11 / 12 / 18, 384 x 64 17 / 13 / 10); never more than blocks to walk.  KREGS where one wave per SIMD is
+// all there is, and at head width 32, whose fragments are two loads (3 x 4096 x 32 15.1 us against 19.2,
+// 12 x 256 x 64 5.5 against 6.0, 24 x 1024 x 64 14.3 against 11.0).
+//
+// Takes, 128-row kernels -> these: short walks gain throughout, what the others do for 128 rows that
+// are not there (forward 800 x 64 x 64 10.2 -> 7.2, 384 x 256 x 64 13.8 -> 12.9; backward 384 x 64 x 64 16.0 -> 10.2,
+// 384 x 256 x 32 24.1 -> 18.9).  Longer walks gain while the device is not full: forward 15 x 777 x 128 18.3 ->
+// 12.6, 36 x 1024 x 64 17.4 -> 16.2, 16 x 2048 x 128 38.7 -> 36.7 (48 x 1024 x 64 18.1 -> 18.5); backward, which streams
+// three operands per block, 3 x 4096 x 64 86 -> 47, 12 x 1024 x 64 24.1 -> 21.4, 24 x 400 x 128 25.5 -> 21.4 (16 x 2048 x
+// 64 36.4 -> 37.6, 24 x 1024 x 64 27.6 -> 27.7).
+struct SplitSize {
+  int64_t nb, u;
+  SplitSize(int64_t BH, int64_t T, int64_t D) : nb((T + 31) / 32), u(BH * nb * D / 64) {}
+};
 bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
-  const int64_t n = BH * ((T + kSplitRows - 1) / kSplitRows) * (D / 32);
-  return T > 64 && n <= (T >= 256 ? 1152 : 384);
+  const SplitSize z(BH, T, D);
+  return z.nb <= 8 ? z.u <= 3200 : z.u <= (D == 128 ? 2048 : 1200);
 }
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
-  const int64_t blocks = (T + kSplitRows - 1) / kSplitRows;
-  return BH * blocks * (D / 32) <= 768 && BH * blocks * blocks * (D / 32) <= 16384 && T * D <= 98304;
+  const SplitSize z(BH, T, D);
+  return z.u <= (z.nb <= 4 ? 3200 : z.nb <= 8 ? 1600 : z.nb <= 16 || D == 128 ? 768 : 448);
+}
+static int fwd_waves(const SplitSize& z) {
+  const int64_t most = z.u <= 320 ? z.nb : z.u <= 1200 ? z.nb / 2 : z.nb / 4;
+  const int64_t w = z.u <= 640 || (z.nb >= 16 && z.u <= 1152) || z.nb >= 64 ? 4 : z.u <= 1536 ? 2 : 1;
+  return (int)std::min(w, most);
+}
+static int bwd_waves(const SplitSize& z) {
+  const int64_t w = z.u <= 256 || z.nb >= 28 ? 4 : z.u <= (z.nb <= 8 ? 512 : 768) ? 2 : 1;
+  return (int)std::min(w, z.u <= 256 ? z.nb : z.nb / 4);
+}
+
+template <int D, int W>
+static void launch_fwd(const FwdParams& p, int BH, bool kregs, hipStream_t stream) {
+  if constexpr (D != 32) {
+    if (!kregs) return launch_fwd_split<D, W, false>(p, BH, stream);
+  }
+  launch_fwd_split<D, W, true>(p, BH, stream);
+}
+template <int D>
+static void launch_fwd(const FwdParams& p, int BH, hipStream_t stream) {
+  const SplitSize z(BH, p.T, D);
+  const int w = fwd_waves(z);
+  const bool kregs = z.u <= 192;
+  if (w >= 4)
+    launch_fwd<D, 4>(p, BH, kregs, stream);
+  else if (w >= 2)
+    launch_fwd<D, 2>(p, BH, kregs, stream);
+  else
+    launch_fwd<D, 1>(p, BH, kregs, stream);
+}
+template <int D>
+static void launch_bwd(const BwdParams& p, int BH, hipStream_t stream) {
+  const int w = bwd_waves(SplitSize(BH, p.T, D));
+  if (w >= 4)
+    launch_bwd_split<D, 4>(p, BH, stream);
+  else if (w >= 2)
+    launch_bwd_split<D, 2>(p, BH, stream);
+  else
+    launch_bwd_split<D, 1>(p, BH, stream);
 }
 
 void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream) {
   LaunchScope scope("attn_fwd_f16", stream);
   switch (D) {
-    case 32: launch_fwd_split<32, 4>(p, B * p.H, stream); break;
-    case 64: launch_fwd_split<64, 4>(p, B * p.H, stream); break;
-    case 128: launch_fwd_split<128, 4>(p, B * p.H, stream); break;
+    case 32: launch_fwd<32>(p, B * p.H, stream); break;
+    case 64: launch_fwd<64>(p, B * p.H, stream); break;
+    case 128: launch_fwd<128>(p, B * p.H, stream); break;
   }
 }
 void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream) {
   LaunchScope scope("attn_bwd_f16", stream);
   switch (D) {
-    case 32: launch_bwd_split<32, 4>(p, B * p.H, stream); break;
-    case 64: launch_bwd_split<64, 4>(p, B * p.H, stream); break;
-    case 128: launch_bwd_split<128, 4>(p, B * p.H, stream); break;
+    case 32: launch_bwd<32>(p, B * p.H, stream); break;
+    case 64: launch_bwd<64>(p, B * p.H, stream); break;
+    case 128: launch_bwd<128>(p, B * p.H, stream); break;
   }
 }
 
