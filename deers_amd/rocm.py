@@ -1,4 +1,5 @@
-"""Python binding of the C ABI in include/deers_rocm.h (ctypes, no torch).
+"""Python binding of the C ABI in include/deers_rocm.h (no torch).  The calls that a training step or
+a generated token consists of go through the extension module `_calls`, the others through ctypes.
 
 This is host-side plumbing for tests and the benchmark: device buffers, copies,
 timers and the three attention entry points, called exactly the way a
@@ -9,6 +10,7 @@ present, every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 
 import numpy as np
@@ -21,13 +23,24 @@ _lib = None
 _inited = False
 
 
+class _NotLoaded:
+    """Stands in for the extension until the first call through it."""
+
+    def __getattr__(self, name):
+        load()
+        return getattr(_calls, name)
+
+
+_calls = _NotLoaded()
+
+
 class RocmError(RuntimeError):
     """A non-zero return code from the library (the role of deers' backend error variant)."""
 
 
 def load() -> ctypes.CDLL:
-    """Loads libdeers_rocm.so; raises if it has not been built."""
-    global _lib
+    """Loads libdeers_rocm.so and the extension module; raises if they have not been built."""
+    global _lib, _calls
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RocmError(
@@ -36,7 +49,13 @@ def load() -> ctypes.CDLL:
         lib = ctypes.CDLL(LIB_PATH)
         lib.deers_rocm_last_error.restype = ctypes.c_char_p
         lib.deers_rocm_stream.restype = ctypes.c_void_p
-        _lib = lib
+        try:
+            calls = importlib.import_module("deers_amd._calls")
+        except ImportError as e:
+            raise RocmError(f"the extension module deers_amd._calls is missing ({e}): build it with "
+                            "`make -C deers_amd/csrc` (or __graft_entry__.build())") from e
+        calls.bind(LIB_PATH, ctypes.c_void_p, RocmError)
+        _lib, _calls = lib, calls
     return _lib
 
 
@@ -82,7 +101,13 @@ def debug_bwd_wait(spin_limit: int = 1 << 20, skip_producers: bool = False):
     _check(load().deers_rocm_debug_bwd_wait(ctypes.c_int(spin_limit), ctypes.c_int(int(skip_producers))))
 
 
+_CODES = {np.float16: F16, np.float32: F32}
+
+
 def dtype_code(dtype) -> int:
+    code = _CODES.get(dtype)
+    if code is not None:
+        return code
     dtype = np.dtype(dtype)
     if dtype == np.float16:
         return F16
@@ -114,8 +139,7 @@ class DeviceBuffer:
 
     def numpy(self) -> np.ndarray:
         out = np.empty(self.shape, dtype=self.dtype)
-        _check(load().deers_rocm_dtoh(out.ctypes.data_as(ctypes.c_void_p), self.ptr,
-                                      ctypes.c_size_t(self.nbytes)))
+        _calls.dtoh(out, self.ptr, self.nbytes)
         return out
 
     def free(self):
@@ -183,36 +207,21 @@ def profile_collect() -> dict:
     return out
 
 
-def _strides(s):
-    if s is None:
-        return None
-    return (ctypes.c_int64 * 4)(*[int(x) for x in s])
-
-
 def attn_fwd_raw(dtype, q, k, v, o, lse, B, H, T, D, scale, q_strides=None, k_strides=None,
                  v_strides=None, o_strides=None):
     """deers_rocm_attn_fwd on raw device pointers (DeviceBuffer.ptr)."""
-    _check(load().deers_rocm_attn_fwd(
-        ctypes.c_int(dtype_code(dtype)), q, _strides(q_strides), k, _strides(k_strides), v,
-        _strides(v_strides), o, _strides(o_strides), lse, ctypes.c_int64(B), ctypes.c_int64(H),
-        ctypes.c_int64(T), ctypes.c_int64(D), ctypes.c_float(scale)))
+    _calls.attn_fwd(dtype_code(dtype), q, q_strides, k, k_strides, v, v_strides, o, o_strides, lse, B, H, T, D, scale)
 
 
 def attn_bwd_raw(dtype, q, k, v, o, lse, do, dq, dk, dv, B, H, T, D, scale, strides=None):
     """deers_rocm_attn_bwd on raw device pointers; `strides` maps tensor name -> 4 strides."""
-    s = strides or {}
-    g = lambda n: _strides(s.get(n))  # noqa: E731
-    _check(load().deers_rocm_attn_bwd(
-        ctypes.c_int(dtype_code(dtype)), q, g("q"), k, g("k"), v, g("v"), o, g("o"), lse, do,
-        g("do"), dq, g("dq"), dk, g("dk"), dv, g("dv"), ctypes.c_int64(B), ctypes.c_int64(H),
-        ctypes.c_int64(T), ctypes.c_int64(D), ctypes.c_float(scale)))
+    g = (strides or {}).get
+    _calls.attn_bwd(dtype_code(dtype), q, g("q"), k, g("k"), v, g("v"), o, g("o"), lse, do, g("do"), dq, g("dq"), dk,
+                    g("dk"), dv, g("dv"), B, H, T, D, scale)
 
 
 def attn_decode_raw(dtype, q, k_cache, v_cache, o, B, H, L, D, scale, kv_strides=None):
-    ks = None if kv_strides is None else (ctypes.c_int64 * 3)(*[int(x) for x in kv_strides])
-    _check(load().deers_rocm_attn_decode(
-        ctypes.c_int(dtype_code(dtype)), q, k_cache, v_cache, ks, o, ctypes.c_int64(B),
-        ctypes.c_int64(H), ctypes.c_int64(L), ctypes.c_int64(D), ctypes.c_float(scale)))
+    _calls.attn_decode(dtype_code(dtype), q, k_cache, v_cache, kv_strides, o, B, H, L, D, scale)
 
 
 def attn_decode_noalloc_raw(dtype, q, k_cache, v_cache, o, B, H, L, D, scale, kv_strides=None):
@@ -226,16 +235,12 @@ def attn_decode_noalloc_raw(dtype, q, k_cache, v_cache, o, B, H, L, D, scale, kv
 def attn_decode_append_raw(dtype, q, k, v, in_strides, cos_row, sin_row, k_cache, v_cache, cache_strides,
                            o, pos, capacity, B, H, D, scale):
     """deers_rocm_attn_decode_append: rotate q, k at `pos`, append k, v as cache row pos, attend over [0,pos]."""
-    i64 = ctypes.c_int64
-    _check(load().deers_rocm_attn_decode_append(
-        ctypes.c_int(dtype_code(dtype)), q, k, v, (i64 * 2)(*[int(x) for x in in_strides]), cos_row,
-        sin_row, k_cache, v_cache, (i64 * 3)(*[int(x) for x in cache_strides]), o, i64(pos),
-        i64(capacity), i64(B), i64(H), i64(D), ctypes.c_float(scale)))
+    _calls.attn_decode_append(dtype_code(dtype), q, k, v, in_strides, cos_row, sin_row, k_cache, v_cache, cache_strides,
+                              o, pos, capacity, B, H, D, scale)
 
 
 def fill_raw(dtype, dst, n, value):
-    _check(load().deers_rocm_fill(ctypes.c_int(dtype_code(dtype)), dst, ctypes.c_size_t(n),
-                                  ctypes.c_float(value)))
+    _calls.fill(dtype_code(dtype), dst, n, value)
 
 
 def add_raw(dtype, a, b, out, n):
@@ -266,66 +271,51 @@ def log_softmax_bwd_raw(dtype, grad, lsm, out, outer, inner):
 
 
 def index_select_raw(dtype, table, indices, out, n_rows, n_indices, width):
-    _check(load().deers_rocm_index_select(ctypes.c_int(dtype_code(dtype)), table, indices, out,
-                                          ctypes.c_int64(n_rows), ctypes.c_int64(n_indices),
-                                          ctypes.c_int64(width)))
+    _calls.index_select(dtype_code(dtype), table, indices, out, n_rows, n_indices, width)
 
 
 def index_add_raw(dtype, src, indices, dst, n_rows, n_indices, width):
-    _check(load().deers_rocm_index_add(ctypes.c_int(dtype_code(dtype)), src, indices, dst,
-                                       ctypes.c_int64(n_rows), ctypes.c_int64(n_indices),
-                                       ctypes.c_int64(width)))
+    _calls.index_add(dtype_code(dtype), src, indices, dst, n_rows, n_indices, width)
 
 
 def rms_norm_fwd_raw(dtype, x, y, outer, inner, eps):
-    _check(load().deers_rocm_rms_norm_fwd(ctypes.c_int(dtype_code(dtype)), x, y, ctypes.c_int64(outer),
-                                          ctypes.c_int64(inner), ctypes.c_double(eps)))
+    _calls.rms_norm_fwd(dtype_code(dtype), x, y, outer, inner, eps)
 
 
 def rms_norm_bwd_raw(dtype, x, dy, dx, outer, inner, eps):
-    _check(load().deers_rocm_rms_norm_bwd(ctypes.c_int(dtype_code(dtype)), x, dy, dx,
-                                          ctypes.c_int64(outer), ctypes.c_int64(inner),
-                                          ctypes.c_double(eps)))
+    _calls.rms_norm_bwd(dtype_code(dtype), x, dy, dx, outer, inner, eps)
 
 
 def rms_norm_bwd_add_raw(dtype, x, dy, addend, dx, outer, inner, eps):
-    _check(load().deers_rocm_rms_norm_bwd_add(ctypes.c_int(dtype_code(dtype)), x, dy, addend, dx,
-                                              ctypes.c_int64(outer), ctypes.c_int64(inner),
-                                              ctypes.c_double(eps)))
+    _calls.rms_norm_bwd_add(dtype_code(dtype), x, dy, addend, dx, outer, inner, eps)
 
 
 def relu_sq_fwd_raw(dtype, x, y, n):
-    _check(load().deers_rocm_relu_sq_fwd(ctypes.c_int(dtype_code(dtype)), x, y, ctypes.c_int64(n)))
+    _calls.relu_sq_fwd(dtype_code(dtype), x, y, n)
 
 
 def relu_sq_bwd_raw(dtype, x, dy, dx, n):
-    _check(load().deers_rocm_relu_sq_bwd(ctypes.c_int(dtype_code(dtype)), x, dy, dx, ctypes.c_int64(n)))
+    _calls.relu_sq_bwd(dtype_code(dtype), x, dy, dx, n)
 
 
 def argmax_rows_raw(dtype, x, out, outer, inner):
-    _check(load().deers_rocm_argmax_rows(ctypes.c_int(dtype_code(dtype)), x, out, ctypes.c_int64(outer),
-                                         ctypes.c_int64(inner)))
+    _calls.argmax_rows(dtype_code(dtype), x, out, outer, inner)
 
 
 def cross_entropy_fwd_raw(dtype, logits, targets, row_lse, loss, n_rows, n_classes):
-    _check(load().deers_rocm_cross_entropy_fwd(ctypes.c_int(dtype_code(dtype)), logits, targets, row_lse,
-                                               loss, ctypes.c_int64(n_rows), ctypes.c_int64(n_classes)))
+    _calls.cross_entropy_fwd(dtype_code(dtype), logits, targets, row_lse, loss, n_rows, n_classes)
 
 
 def cross_entropy_fwd_grad_raw(dtype, logits, targets, row_lse, loss, dlogits, n_rows, n_classes):
-    _check(load().deers_rocm_cross_entropy_fwd_grad(ctypes.c_int(dtype_code(dtype)), logits, targets, row_lse,
-                                                    loss, dlogits, ctypes.c_int64(n_rows),
-                                                    ctypes.c_int64(n_classes)))
+    _calls.cross_entropy_fwd_grad(dtype_code(dtype), logits, targets, row_lse, loss, dlogits, n_rows, n_classes)
 
 
 def scale_by_scalar_raw(dtype, x, n, factor):
-    _check(load().deers_rocm_scale_by_scalar(ctypes.c_int(dtype_code(dtype)), x, ctypes.c_int64(n), factor))
+    _calls.scale_by_scalar(dtype_code(dtype), x, n, factor)
 
 
 def cross_entropy_bwd_raw(dtype, logits, targets, row_lse, upstream, dlogits, n_rows, n_classes):
-    _check(load().deers_rocm_cross_entropy_bwd(ctypes.c_int(dtype_code(dtype)), logits, targets, row_lse,
-                                               upstream, dlogits, ctypes.c_int64(n_rows),
-                                               ctypes.c_int64(n_classes)))
+    _calls.cross_entropy_bwd(dtype_code(dtype), logits, targets, row_lse, upstream, dlogits, n_rows, n_classes)
 
 
 # op codes of deers_rocm_unary / deers_rocm_binary / deers_rocm_reduce (include/deers_rocm.h)
@@ -391,27 +381,20 @@ def sum_squares_raw(dtype, x, n, total, accumulate=False):
                                          total, ctypes.c_int(1 if accumulate else 0)))
 
 
-def _ptr_table(ptrs):
-    """Addresses or c_void_p, as the array's constructor takes both: an AdamW call over 74 tensors
-    converts 296 of them while the device waits."""
-    return (ctypes.c_void_p * len(ptrs))(*ptrs)
-
-
 def adamw_step_multi_raw(dtype, w, grad, m, v, sizes, lr, beta1, beta2, eps, weight_decay, step,
                          grad_scale=1.0):
     n = len(sizes)
-    _check(load().deers_rocm_adamw_step_multi(
-        ctypes.c_int(dtype_code(dtype)), ctypes.c_int(n), _ptr_table(w), _ptr_table(grad), _ptr_table(m),
-        _ptr_table(v), (ctypes.c_int64 * n)(*sizes), ctypes.c_double(lr), ctypes.c_double(beta1),
-        ctypes.c_double(beta2), ctypes.c_double(eps), ctypes.c_double(weight_decay), ctypes.c_int64(step),
-        ctypes.c_double(grad_scale)))
+    if not n == len(w) == len(grad) == len(m) == len(v):
+        raise ValueError("as many weights, gradients and moments as sizes are needed")
+    _calls.adamw_step_multi(dtype_code(dtype), n, w, grad, m, v, sizes, lr, beta1, beta2, eps, weight_decay, step,
+                            grad_scale)
 
 
 def sum_squares_multi_raw(dtype, x, sizes, total, accumulate=False):
     n = len(sizes)
-    _check(load().deers_rocm_sum_squares_multi(ctypes.c_int(dtype_code(dtype)), ctypes.c_int(n),
-                                               _ptr_table(x), (ctypes.c_int64 * n)(*sizes), total,
-                                               ctypes.c_int(1 if accumulate else 0)))
+    if n != len(x):
+        raise ValueError("as many tensors as sizes are needed")
+    _calls.sum_squares_multi(dtype_code(dtype), n, x, sizes, total, 1 if accumulate else 0)
 
 
 def scale_raw(dtype, x, n, scale):
@@ -421,29 +404,17 @@ def scale_raw(dtype, x, n, scale):
 
 def matmul_raw(dtype, a, a_strides, b, b_strides, c, batch, m, n, k):
     """deers_rocm_matmul: c[batch,m,n] = a @ b; strides are (row, col, batch) in elements."""
-    i64 = ctypes.c_int64
-    _check(load().deers_rocm_matmul(
-        ctypes.c_int(dtype_code(dtype)), a, i64(a_strides[0]), i64(a_strides[1]), i64(a_strides[2]),
-        b, i64(b_strides[0]), i64(b_strides[1]), i64(b_strides[2]), c, i64(batch), i64(m), i64(n),
-        i64(k)))
+    _calls.matmul(dtype_code(dtype), a, *a_strides[:3], b, *b_strides[:3], c, batch, m, n, k)
 
 
 def matmul_acc_raw(dtype, a, a_strides, b, b_strides, c, batch, m, n, k):
     """deers_rocm_matmul_acc: c[batch,m,n] += a @ b; strides are (row, col, batch) in elements."""
-    i64 = ctypes.c_int64
-    _check(load().deers_rocm_matmul_acc(
-        ctypes.c_int(dtype_code(dtype)), a, i64(a_strides[0]), i64(a_strides[1]), i64(a_strides[2]),
-        b, i64(b_strides[0]), i64(b_strides[1]), i64(b_strides[2]), c, i64(batch), i64(m), i64(n),
-        i64(k)))
+    _calls.matmul_acc(dtype_code(dtype), a, *a_strides[:3], b, *b_strides[:3], c, batch, m, n, k)
 
 
 def matmul_add_raw(dtype, a, a_strides, b, b_strides, addend, c, batch, m, n, k):
     """deers_rocm_matmul_add: c[batch,m,n] = a @ b + addend; strides are (row, col, batch) in elements."""
-    i64 = ctypes.c_int64
-    _check(load().deers_rocm_matmul_add(
-        ctypes.c_int(dtype_code(dtype)), a, i64(a_strides[0]), i64(a_strides[1]), i64(a_strides[2]),
-        b, i64(b_strides[0]), i64(b_strides[1]), i64(b_strides[2]), addend, c, i64(batch), i64(m), i64(n),
-        i64(k)))
+    _calls.matmul_add(dtype_code(dtype), a, *a_strides[:3], b, *b_strides[:3], addend, c, batch, m, n, k)
 
 
 LINEAR_PROLOGUES = {"plain": 0, "rms_norm": 1, "relu_sq": 2}
@@ -452,46 +423,37 @@ LINEAR_W_PACKED = -32  # DEERS_ROCM_LINEAR_W_PACKED: pass as ldw for a [n/32][k]
 
 def decode_linear_raw(dtype, prologue, eps, x, ldx, w, ldw, y, accumulate, m, n, k):
     """deers_rocm_decode_linear: y[m,n] (+)= f(x)[m,k] @ w[k,n], m <= 32, f one of LINEAR_PROLOGUES."""
-    i64 = ctypes.c_int64
-    _check(load().deers_rocm_decode_linear(
-        ctypes.c_int(dtype_code(dtype)), ctypes.c_int(LINEAR_PROLOGUES[prologue]), ctypes.c_float(eps), x,
-        i64(ldx), w, i64(ldw), y, ctypes.c_int(1 if accumulate else 0), i64(m), i64(n), i64(k)))
+    _calls.decode_linear(dtype_code(dtype), LINEAR_PROLOGUES[prologue], eps, x, ldx, w, ldw, y, 1 if accumulate else 0, m,
+                         n, k)
 
 
 def decode_linear_hint_raw(next_w_packed, n, k):
     """deers_rocm_decode_linear_hint: the packed weight of the product after the next one (None clears)."""
-    _check(load().deers_rocm_decode_linear_hint(next_w_packed, ctypes.c_int64(n), ctypes.c_int64(k)))
+    _calls.decode_linear_hint(next_w_packed, n, k)
 
 
 def decode_qkv_raw(dtype, q, k, v, in_strides, cos_row, sin_row, q_out, k_cache, v_cache, cache_strides,
                    pos, capacity, B, H, D):
     """deers_rocm_decode_qkv: rotate q, k at `pos`; q -> q_out [B,H,D]; k, v -> row pos of the caches."""
-    i64 = ctypes.c_int64
-    _check(load().deers_rocm_decode_qkv(
-        ctypes.c_int(dtype_code(dtype)), q, k, v, (i64 * 2)(*[int(x) for x in in_strides]), cos_row,
-        sin_row, q_out, k_cache, v_cache, (i64 * 3)(*[int(x) for x in cache_strides]), i64(pos),
-        i64(capacity), i64(B), i64(H), i64(D)))
+    _calls.decode_qkv(dtype_code(dtype), q, k, v, in_strides, cos_row, sin_row, q_out, k_cache, v_cache, cache_strides,
+                      pos, capacity, B, H, D)
 
 
 def rope_fwd_raw(dtype, x, cos, sin, y, B, T, H, D, x_strides=None, y_strides=None):
     """deers_rocm_rope_fwd: x logical [B,T,H,D] -> y [B,H,T,D] (compact unless y_strides)."""
-    _check(load().deers_rocm_rope_fwd(
-        ctypes.c_int(dtype_code(dtype)), x, _strides(x_strides), cos, sin, y, _strides(y_strides),
-        ctypes.c_int64(B), ctypes.c_int64(T), ctypes.c_int64(H), ctypes.c_int64(D)))
+    _calls.rope_fwd(dtype_code(dtype), x, x_strides, cos, sin, y, y_strides, B, T, H, D)
 
 
 def copy_view_raw(dtype, src, src_strides, dst, dst_strides, shape):
     nd = len(shape)
-    arr = lambda v: (ctypes.c_int64 * nd)(*[int(x) for x in v])  # noqa: E731
-    _check(load().deers_rocm_copy_view(ctypes.c_int(dtype_code(dtype)), src, arr(src_strides), dst,
-                                       arr(dst_strides), arr(shape), ctypes.c_int(nd)))
+    if not nd == len(src_strides) == len(dst_strides):
+        raise ValueError("as many strides as dimensions are needed")
+    _calls.copy_view(dtype_code(dtype), src, src_strides, dst, dst_strides, shape, nd)
 
 
 def rope_bwd_raw(dtype, dy, cos, sin, dx, B, T, H, D, dy_strides=None):
     """deers_rocm_rope_bwd: dy logical [B,H,T,D] -> dx compact [B,T,H,D]."""
-    _check(load().deers_rocm_rope_bwd(
-        ctypes.c_int(dtype_code(dtype)), dy, _strides(dy_strides), cos, sin, dx, ctypes.c_int64(B),
-        ctypes.c_int64(T), ctypes.c_int64(H), ctypes.c_int64(D)))
+    _calls.rope_bwd(dtype_code(dtype), dy, dy_strides, cos, sin, dx, B, T, H, D)
 
 
 def default_scale(D: int) -> float:
