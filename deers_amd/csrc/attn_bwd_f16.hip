@@ -71,13 +71,13 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void attn_bwd_f16_bp_kernel(
                                                                                  int heads_per_xcd, int first_id,
                                                                                  int dq_short_first) {
   const int group_wgs = 8 * heads_per_xcd;
-  const int per_role = n_blocks * group_wgs;
+  const int per_role = heads_per_xcd ? n_blocks * group_wgs : map_even_blocks(n_blocks, BH);
   const int id = (int)blockIdx.x + first_id;
   int bh, rank;
   if (id < per_role) {
-    const int group = id / group_wgs;
-    const int r = dq_short_first ? n_blocks - 1 - group : group;
-    if (map_block(r * group_wgs + id % group_wgs, n_blocks, heads_per_xcd, BH, &bh, &rank))
+    int at = id;
+    if (dq_short_first) at = (n_blocks - 1 - id / group_wgs) * group_wgs + id % group_wgs;
+    if (map_block(at, n_blocks, heads_per_xcd, BH, &bh, &rank))
       bwd_dq_f16_bp_body<D>(p, __builtin_amdgcn_readfirstlane(bh), n_blocks - 1 - __builtin_amdgcn_readfirstlane(rank),
                             n_blocks, blockIdx.x);
   } else {
@@ -87,12 +87,22 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void attn_bwd_f16_bp_kernel(
   }
 }
 
+// Whether the blocks of heads that the XCDs cannot share out whole are dealt to all XCDs.  The
+// hand-over inside one launch needs a head on one XCD, so this takes the two launches in stream
+// order, 7-10 us more: for long walks only (9 x 8192 x 128: 743 -> 556 us, 12 x 4096 x 64 123 -> 120; 12 x 2048 x
+// 128 72 -> 96, 10 x 4096 x 32 70 -> 79), where XCDs would idle for a tenth of the time or more.
+static bool bwd_even(int BH, int T, int D) {
+  return T >= 4096 && (int64_t)T * D >= 262144 && 80 * ((BH + 7) / 8) >= 11 * BH;
+}
+
 template <int D>
 static void launch_bwd_f16_d(const BwdParams& p, int B, int mode, hipStream_t stream) {
   const int BH = B * p.H;
   const int n_blocks = (p.T + kBwdBlk - 1) / kBwdBlk;
-  const int heads_per_xcd = (BH + 7) / 8;
-  const int per_role = 8 * n_blocks * heads_per_xcd;
+  const bool even = mode != 2 && bwd_even(BH, p.T, D);
+  if (even) mode = 0;
+  const int heads_per_xcd = even ? 0 : (BH + 7) / 8;
+  const int per_role = even ? map_even_blocks(n_blocks, BH) : 8 * n_blocks * heads_per_xcd;
   typedef void (*Kernel)(BwdParams, int, int, int, int, int);
   const Kernel kernel = attn_bwd_f16_bp_kernel<D>;
   const size_t lds = BwdBpCfg<D>::kLds;

@@ -502,7 +502,11 @@ template <int D>
 static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
   const int BH = B * p.H;
   const int n_qtiles = (p.T + kFwdBM - 1) / kFwdBM;
-  const int heads_per_xcd = (BH + 7) / 8;
+  // heads that the XCDs cannot share out whole (9 x 8192 x 128: 218 us with two heads on one XCD, 163
+  // with the ninth head's tiles dealt to all; 25 x 4096 x 64 74 -> 65, 20 x 2048 x 64 30.6 -> 29.8)
+  const bool even = BH % 8 != 0;
+  const int heads_per_xcd = even ? 0 : (BH + 7) / 8;
+  const int grid = even ? map_even_blocks(n_qtiles, BH) : 8 * n_qtiles * heads_per_xcd;
   const size_t lds = FwdCfg<D>::kLds;
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) {
@@ -523,19 +527,20 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
     // first.  Smaller launches are faster on the tile-pipelined kernel (2x12x2048x64: 33.6
     // against 34.6 us).
     bool use_resident = false;
-    const TileOrder* table = resident_order<D>(heads_per_xcd, p.T, &use_resident);
+    const TileOrder* table = resident_order<D>((BH + 7) / 8, p.T, &use_resident);
+    if (even) table = nullptr;  // the table places whole heads
     static const TileOrder kNoTable = [] {
       TileOrder t{};
       t.code[0] = -1;
       return t;
     }();
     if (const TileOrder* order = use_resident ? (table ? table : &kNoTable) : nullptr) {
-      hipLaunchKernelGGL(attn_fwd_f16_bp_kernel<D>, dim3(8 * n_qtiles * heads_per_xcd), dim3(256), BpCfg<D>::kLds,
+      hipLaunchKernelGGL(attn_fwd_f16_bp_kernel<D>, dim3(grid), dim3(256), BpCfg<D>::kLds,
                          stream, p, BH, n_qtiles, heads_per_xcd, *order);
       return;
     }
   }
-  hipLaunchKernelGGL(attn_fwd_f16_kernel<D>, dim3(8 * n_qtiles * heads_per_xcd), dim3(256), lds,
+  hipLaunchKernelGGL(attn_fwd_f16_kernel<D>, dim3(grid), dim3(256), lds,
                      stream, p, BH, n_qtiles, heads_per_xcd);
 }
 

@@ -284,25 +284,7 @@ struct SkinnyPrefetch {
   int64_t n = 0, k = 0;
 };
 
-// Maps a block id (blockIdx.x, or blockIdx.x minus a multiple of 8) to (head, block
-// rank).  Workgroups are dealt round-robin to the 8 XCDs, so id % 8 is the XCD: every block of one head is given to one XCD
-// (its operands stay in that XCD's L2) and each XCD's list is ordered longest
-// first (rank 0 = the block with the most iterations), which is what the
-// dispatcher's in-order hand-out to free slots needs for an even finish.
-// Returns false for padding ids.
-// (The head and rank stay in vector registers on purpose: forcing them into scalar
-// registers with readfirstlane was measured and raises the kernels' vector register
-// count through the address arithmetic the compiler then hoists out of the loops.)
-__device__ __forceinline__ bool map_block(int block_id, int n_blocks, int heads_per_xcd, int BH,
-                                          int* bh, int* rank) {
-  const int xcd = block_id & 7;
-  const int idx = block_id >> 3;
-  *bh = (idx % heads_per_xcd) * 8 + xcd;
-  *rank = idx / heads_per_xcd;
-  return *bh < BH;
-}
-
-// The same for launches of few heads, where whole heads per XCD leave XCDs idle (12 heads: 2, 2, 2, 2,
+// Block ids for launches of few heads, where whole heads per XCD leave XCDs idle (12 heads: 2, 2, 2, 2,
 // 1, 1, 1, 1): BH / 8 whole heads per XCD, and the blocks of the BH % 8 remaining heads dealt to all
 // XCDs in turn.  An XCD's list is still ordered by rank.  The grid is map_even_blocks(n_ranks, BH).
 __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH, int* bh, int* rank) {
@@ -322,7 +304,26 @@ __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH
   *rank = k;
   return true;
 }
-inline int map_even_blocks(int n_ranks, int BH) { return 8 * (n_ranks * (BH >> 3) + (n_ranks * (BH & 7) + 7) / 8); }
+__host__ __device__ inline int map_even_blocks(int n_ranks, int BH) { return 8 * (n_ranks * (BH >> 3) + (n_ranks * (BH & 7) + 7) / 8); }
+
+// Maps a block id (blockIdx.x, or blockIdx.x minus a multiple of 8) to (head, block
+// rank).  Workgroups are dealt round-robin to the 8 XCDs, so id % 8 is the XCD: every block of one head is given to one XCD
+// (its operands stay in that XCD's L2) and each XCD's list is ordered longest
+// first (rank 0 = the block with the most iterations), which is what the
+// dispatcher's in-order hand-out to free slots needs for an even finish.
+// Returns false for padding ids.  heads_per_xcd == 0: map_block_even.
+// (The head and rank stay in vector registers on purpose: forcing them into scalar
+// registers with readfirstlane was measured and raises the kernels' vector register
+// count through the address arithmetic the compiler then hoists out of the loops.)
+__device__ __forceinline__ bool map_block(int block_id, int n_blocks, int heads_per_xcd, int BH,
+                                          int* bh, int* rank) {
+  if (heads_per_xcd == 0) return map_block_even(block_id, n_blocks, BH, bh, rank);
+  const int xcd = block_id & 7;
+  const int idx = block_id >> 3;
+  *bh = (idx % heads_per_xcd) * 8 + xcd;
+  *rank = idx / heads_per_xcd;
+  return *bh < BH;
+}
 
 // Brackets one kernel launch with a hipEvent pair when per-kernel profiling is
 // switched on (deers_rocm_profile_enable); a no-op otherwise.  Defined in

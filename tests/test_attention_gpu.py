@@ -390,7 +390,8 @@ def test_elementwise_helper_errors():
 @pytest.mark.parametrize("B,H,T,D", [
     (1, 1, 2, 32), (2, 3, 65, 64), (1, 5, 95, 128), (1, 2, 128, 32), (1, 3, 129, 128), (2, 2, 161, 64),
     (1, 2, 513, 32), (1, 1, 700, 128),                                           # few heads
-    (60, 7, 33, 64), (60, 7, 97, 32), (60, 7, 64, 128), (60, 7, 130, 32), (50, 8, 159, 64)])  # many
+    (60, 7, 33, 64), (60, 7, 97, 32), (60, 7, 64, 128), (60, 7, 130, 32), (50, 8, 159, 64),  # many
+    (3, 25, 650, 64), (3, 19, 400, 128), (1, 9, 4161, 64)])                      # not whole heads per XCD
 def test_f16_forms_at_the_edges_of_their_blocks(B, H, T, D):
     x = synth.attention_inputs(f"forms-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=21)
     out = check_case(x, TOL[np.dtype(np.float16)], f"forms {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
