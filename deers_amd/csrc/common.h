@@ -131,9 +131,15 @@ __device__ __forceinline__ half8 lds_frag_transposed(const half_t* tile, int ld,
 // lane i's 16 bytes land at lds_addr + 16*i, where lds_addr is a wave-uniform LDS
 // byte address.  Completion is tracked by vmcnt; pair with wait_vmcnt<N>() and a
 // barrier before other waves read the data.
+// The compiler sees neither the use of m0 nor that of a scalar base inside the asm text, so what the
+// ISA leaves to software stands there: one wait state between the write of m0 and a load into LDS,
+// five between a vector instruction that writes a scalar register (readfirstlane; readlane, where
+// scalars were spilled) and a memory access through that register.  A scalar move of the base is
+// both: a register that a scalar instruction has written is waited for by the hardware.  (Without it
+// a kernel whose bases came from readfirstlane right before their use has faulted.)
 __device__ __forceinline__ void async_load16_to_lds(const void* gptr, uint32_t lds_addr) {
   const uint32_t uniform = __builtin_amdgcn_readfirstlane(lds_addr);
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(uniform)
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(uniform)
                : "memory");
 }
 // Same copy with the address split into a wave-uniform 64-bit base (SGPR pair) and a
@@ -146,8 +152,10 @@ __device__ __forceinline__ void async_load16_to_lds(const void* uniform_base, ui
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
   const uint64_t sbase = ((uint64_t)hi << 32) | (uint64_t)lo;
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(sbase),
-               "s"(uniform)
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+               : "=&s"(base)
+               : "v"(lane_off), "s"(sbase), "s"(uniform)
                : "memory");
 }
 // The same for data that is used once (a non-temporal access).
@@ -158,8 +166,10 @@ __device__ __forceinline__ void async_load16_to_lds_nt(const void* uniform_base,
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
   const uint64_t sbase = ((uint64_t)hi << 32) | (uint64_t)lo;
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(lane_off), "s"(sbase),
-               "s"(uniform)
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0 nt"
+               : "=&s"(base)
+               : "v"(lane_off), "s"(sbase), "s"(uniform)
                : "memory");
 }
 template <int N>
@@ -207,8 +217,10 @@ __device__ __forceinline__ void async_load4_to_lds(const void* uniform_base, uin
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
   const uint64_t sbase = ((uint64_t)hi << 32) | (uint64_t)lo;
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(lane_off), "s"(sbase),
-               "s"(uniform)
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dword %1, %0"
+               : "=&s"(base)
+               : "v"(lane_off), "s"(sbase), "s"(uniform)
                : "memory");
 }
 
