@@ -256,10 +256,10 @@ inline bool bwd_dq_short_first(int group_wgs, int capacity) { return 8 * group_w
 
 struct BwdParams {
   const void* q; const void* k; const void* v; const void* o; const void* d_o;
-  const float* lse; float* delta;  // delta: [B,H,T] workspace, rowsum(dO o O)
-  // f16 path workspace, rows padded to a multiple of 64 per head (t_pad), written by the dQ
-  // role and read by the dK/dV role: lse2 = -LSE*log2(e) (-inf in the padding), negdelta =
-  // -rowsum(dO o O) (0 in the padding), and qs = f16(Q * scale * log2(e)), [B*H][t_pad][D]
+  const float* lse;
+  // workspace, rows padded to a multiple of 64 per head (t_pad), written by the dQ role (f32: by a
+  // launch of its own) and read by the dK/dV role: lse2 = -LSE*log2(e) (-inf in the padding), negdelta =
+  // -rowsum(dO o O) (0 in the padding), and, f16, qs = f16(Q * scale * log2(e)), [B*H][t_pad][D]
   // compact: the scaled queries the forward and the dQ role form their scores from, so that
   // all three kernels exponentiate the same scores
   float* lse2; float* negdelta; void* qs; int t_pad;

@@ -32,9 +32,10 @@ bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream);
-void launch_attn_bwd_f32(const BwdParams& p, int B, int D, hipStream_t stream);
+bool attn_bwd_f32_takes(int64_t BH, int64_t T, int64_t D);
+size_t attn_bwd_f32_ds_bytes(int64_t BH, int64_t T, int* heads);
+void launch_attn_bwd_f32(const BwdParams& p, int B, int D, int heads, void* ds, hipStream_t stream);
 bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
-bool attn_bwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f32_split(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f32_split(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_decode_f16(const DecodeParams& p, int B, int D, bool append, hipStream_t stream);
@@ -730,65 +731,75 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }
-  if (dtype == DEERS_ROCM_F32 && deers::attn_bwd_f32_split_takes(B * H, T, D)) {
-    deers::launch_attn_bwd_f32_split(p, (int)B, (int)D, g_rt.stream);
+  // row statistics lse2 and negdelta, rows padded to a multiple of 64 per head (+ 64 floats: the
+  // block-pipelined f16 dK/dV role loads row vectors 64 floats at a time)
+  const int64_t t_pad = (T + 63) / 64 * 64;
+  const size_t ws_floats = (size_t)(2 * B * H * t_pad + 64);
+  void* ws = nullptr;
+  if (dtype == DEERS_ROCM_F32) {
+    int heads = 0;
+    // behind them dS of `heads` heads at a time; without the memory for it, or while a capture forbids
+    // to get it, the form that computes S and dP twice
+    bool two_pass = deers::attn_bwd_f32_takes(B * H, T, D);
+    if (two_pass) {
+      const size_t bytes = ws_floats * sizeof(float) + deers::attn_bwd_f32_ds_bytes(B * H, T, &heads);
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (bytes > g_rt.workspace_bytes) HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
+      two_pass = cs == hipStreamCaptureStatusNone && workspace(bytes, &ws) == DEERS_ROCM_OK;
+      if (!two_pass) (void)hipGetLastError();
+    }
+    if (two_pass) {
+      p.lse2 = static_cast<float*>(ws);
+      p.negdelta = p.lse2 + B * H * t_pad;
+      p.t_pad = (int)t_pad;
+      deers::launch_attn_bwd_f32(p, (int)B, (int)D, heads, static_cast<float*>(ws) + ws_floats, g_rt.stream);
+    } else {
+      deers::launch_attn_bwd_f32_split(p, (int)B, (int)D, g_rt.stream);
+    }
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }
-  // f32: delta[B,H,T].  f16: lse2 and negdelta, rows padded to a multiple of 64 per head.
-  const int64_t t_pad = (T + 63) / 64 * 64;
-  // f16: + 64 floats, the block-pipelined dK/dV role loads row vectors 64 floats at a time
-  const size_t ws_floats = dtype == DEERS_ROCM_F16 ? (size_t)(2 * B * H * t_pad + 64) : (size_t)(B * H * T);
-  void* ws = nullptr;
-  // f16: behind them the dQ role's scaled queries, [B*H][t_pad][D] f16
-  const size_t ws_qs = dtype == DEERS_ROCM_F16 ? (size_t)(B * H * t_pad * D) * 2 : 0;
+  // behind them the dQ role's scaled queries, [B*H][t_pad][D] f16
+  const size_t ws_qs = (size_t)(B * H * t_pad * D) * 2;
   if (int rc = workspace(ws_floats * sizeof(float) + ws_qs, &ws)) return rc;
-  p.delta = static_cast<float*>(ws);
   // A launch that is being captured into a graph gets no fresh epoch on replay: it takes the
   // two-launch form with the flags switched off (epoch 0).  The workspace and the flags must
   // have been grown by an earlier, eager call of the same geometry: capture allows neither
   // the synchronisation nor the allocation.
-  bool capturing = false;
-  if (dtype == DEERS_ROCM_F16) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
-    capturing = cs != hipStreamCaptureStatusNone;
-    const size_t n_flags = (size_t)(B * H) * (size_t)((T + 127) / 128);
-    if (n_flags > g_rt.bwd_ready_len || g_rt.bwd_epoch == INT32_MAX) {
-      if (capturing)
-        return fail(DEERS_ROCM_ERR_ARG,
-                    "attn_bwd: call once outside stream capture with this geometry first (the "
-                    "hand-over flags have to grow)");
-      if (g_rt.bwd_ready) {
-        HIP_TRY(hipStreamSynchronize(g_rt.stream));
-        // an error raised by a launch before this point is reported by this call
-        if (int rc = check_handover_error()) return rc;
-        HIP_TRY(hipFree(g_rt.bwd_ready));
-        g_rt.bwd_ready = nullptr;
-      }
-      const size_t want = n_flags > g_rt.bwd_ready_len ? n_flags : g_rt.bwd_ready_len;
-      HIP_TRY(hipMalloc(&g_rt.bwd_ready, (want + 1) * sizeof(int)));  // [error word][flags]
-      HIP_TRY(hipMemsetAsync(g_rt.bwd_ready, 0, (want + 1) * sizeof(int), g_rt.stream));
-      g_rt.bwd_ready_len = want;
-      g_rt.bwd_epoch = 0;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
+  const bool capturing = cs != hipStreamCaptureStatusNone;
+  const size_t n_flags = (size_t)(B * H) * (size_t)((T + 127) / 128);
+  if (n_flags > g_rt.bwd_ready_len || g_rt.bwd_epoch == INT32_MAX) {
+    if (capturing)
+      return fail(DEERS_ROCM_ERR_ARG,
+                  "attn_bwd: call once outside stream capture with this geometry first (the "
+                  "hand-over flags have to grow)");
+    if (g_rt.bwd_ready) {
+      HIP_TRY(hipStreamSynchronize(g_rt.stream));
+      // an error raised by a launch before this point is reported by this call
+      if (int rc = check_handover_error()) return rc;
+      HIP_TRY(hipFree(g_rt.bwd_ready));
+      g_rt.bwd_ready = nullptr;
     }
-    p.error = g_rt.bwd_ready;
-    p.ready = g_rt.bwd_ready + 1;
-    p.epoch = capturing ? 0 : ++g_rt.bwd_epoch;
-    p.spin_limit = g_rt.bwd_spin_limit;
+    const size_t want = n_flags > g_rt.bwd_ready_len ? n_flags : g_rt.bwd_ready_len;
+    HIP_TRY(hipMalloc(&g_rt.bwd_ready, (want + 1) * sizeof(int)));  // [error word][flags]
+    HIP_TRY(hipMemsetAsync(g_rt.bwd_ready, 0, (want + 1) * sizeof(int), g_rt.stream));
+    g_rt.bwd_ready_len = want;
+    g_rt.bwd_epoch = 0;
   }
+  p.error = g_rt.bwd_ready;
+  p.ready = g_rt.bwd_ready + 1;
+  p.epoch = capturing ? 0 : ++g_rt.bwd_epoch;
+  p.spin_limit = g_rt.bwd_spin_limit;
   const bool single_launch = !capturing && same_xcd_handover_now();
   p.lse2 = static_cast<float*>(ws);
   p.negdelta = static_cast<float*>(ws) + B * H * t_pad;
   p.qs = static_cast<float*>(ws) + ws_floats;
   p.t_pad = (int)t_pad;
-  if (dtype == DEERS_ROCM_F16) {
-    if (single_launch) g_rt.bwd_error_armed = true;
-    const int mode = !single_launch ? 0 : (g_rt.bwd_skip_producers ? 2 : 1);
-    deers::launch_attn_bwd_f16(p, (int)B, (int)D, mode, g_rt.stream);
-  } else {
-    deers::launch_attn_bwd_f32(p, (int)B, (int)D, g_rt.stream);
-  }
+  if (single_launch) g_rt.bwd_error_armed = true;
+  const int mode = !single_launch ? 0 : (g_rt.bwd_skip_producers ? 2 : 1);
+  deers::launch_attn_bwd_f16(p, (int)B, (int)D, mode, g_rt.stream);
   HIP_TRY(hipGetLastError());
   return DEERS_ROCM_OK;
 }

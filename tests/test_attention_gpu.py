@@ -454,3 +454,27 @@ def test_f32_few_heads_rows_interleaved_over_heads():
     for name, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:])):
         np.testing.assert_array_equal(outs[name].numpy().transpose(0, 2, 1, 3), ref, err_msg=name)
     np.testing.assert_array_equal(lse.numpy(), want[1])
+
+
+@pytest.mark.parametrize("B,H,T,D", [
+    (6, 10, 353, 32), (5, 9, 384, 64), (5, 6, 415, 128),         # four waves
+    (21, 8, 415, 32), (24, 8, 225, 64), (10, 8, 250, 128),       # two
+    (198, 8, 65, 32), (123, 8, 33, 64), (78, 8, 63, 128)])       # one
+def test_f32_backward_with_ds_in_memory(B, H, T, D):
+    """The two-pass backward at the ends of its blocks and of its rules; every gradient bit for bit again."""
+    x = synth.attention_inputs(f"ds32-{B}-{H}-{T}-{D}", B, H, T, D, np.float32, base_seed=29)
+    out = check_case(x, TOL[np.dtype(np.float32)], f"f32 dS in memory {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
+    again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for a, b in zip(out, again):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_f32_backward_with_ds_of_some_heads_at_a_time():
+    """Heads that do not fit the workspace together give the bits they give two at a time."""
+    H, T, D = 5, 16384, 32
+    x = synth.attention_inputs("ds32-shares", 1, H, T, D, np.float32, base_seed=30)
+    got = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for h in (0, 3):
+        pair = rocm.attn_fwd_bwd(*(np.ascontiguousarray(x[n][:, h:h + 2]) for n in ("q", "k", "v", "do")))
+        for a, b in zip(got[2:], pair[2:]):
+            np.testing.assert_array_equal(a[:, h:h + 2], b)
