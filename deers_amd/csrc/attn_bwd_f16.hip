@@ -78,11 +78,11 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void attn_bwd_f16_bp_kernel(
     int at = id;
     if (dq_short_first) at = (n_blocks - 1 - id / group_wgs) * group_wgs + id % group_wgs;
     if (map_block(at, n_blocks, heads_per_xcd, BH, &bh, &rank))
-      bwd_dq_f16_bp_body<D>(p, __builtin_amdgcn_readfirstlane(bh), n_blocks - 1 - __builtin_amdgcn_readfirstlane(rank),
+      bwd_dq_f16_bp_body<D>(first_argument<BwdParams>(), __builtin_amdgcn_readfirstlane(bh), n_blocks - 1 - __builtin_amdgcn_readfirstlane(rank),
                             n_blocks, blockIdx.x);
   } else {
     if (map_block(id - per_role, n_blocks, heads_per_xcd, BH, &bh, &rank))
-      bwd_dkdv_f16_bp_body<D>(p, __builtin_amdgcn_readfirstlane(bh), __builtin_amdgcn_readfirstlane(rank), n_blocks,
+      bwd_dkdv_f16_bp_body<D>(first_argument<BwdParams>(), __builtin_amdgcn_readfirstlane(bh), __builtin_amdgcn_readfirstlane(rank), n_blocks,
                               blockIdx.x);
   }
 }

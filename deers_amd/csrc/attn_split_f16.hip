@@ -480,9 +480,9 @@ __global__ __launch_bounds__(64 * W, D == 128 ? 1 : 2) void attn_bwd_f16_split_k
   int bh, rank;
   if (!map_block_even(blockIdx.x, 2 * n_blocks, BH, &bh, &rank)) return;
   if (rank & 1)
-    split_dq_body<D, W>(p, bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
+    split_dq_body<D, W>(first_argument<BwdParams>(), bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
   else
-    split_dkdv_body<D, W>(p, bh, rank >> 1, n_blocks, smem, wave, lane);
+    split_dkdv_body<D, W>(first_argument<BwdParams>(), bh, rank >> 1, n_blocks, smem, wave, lane);
 }
 
 template <typename Kernel>

@@ -290,17 +290,10 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f3
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bh, rank;
   if (!map_block_even(blockIdx.x, 2 * n_blocks, BH, &bh, &rank)) return;
-  // each role fetches the arguments it needs: those of both, fetched before the branch, do not fit the
-  // scalar registers
-  const auto args = [] {
-    auto ptr = (const __attribute__((address_space(4))) BwdParams*)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(ptr));
-    return (const BwdParams*)ptr;
-  };
   if (rank & 1)
-    split32_dq<D, W>(*args(), bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
+    split32_dq<D, W>(first_argument<BwdParams>(), bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
   else
-    split32_dkdv<D, W>(*args(), bh, rank >> 1, n_blocks, smem, wave, lane);
+    split32_dkdv<D, W>(first_argument<BwdParams>(), bh, rank >> 1, n_blocks, smem, wave, lane);
 }
 
 template <int D, int W>

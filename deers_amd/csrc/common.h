@@ -318,6 +318,16 @@ __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH
 }
 __host__ __device__ inline int map_even_blocks(int n_ranks, int BH) { return 8 * (n_ranks * (BH >> 3) + (n_ranks * (BH & 7) + 7) / 8); }
 
+// The kernel's first argument, fetched where it is asked for.  In a kernel whose branches are roles with
+// arguments of their own, the arguments of all roles fetched before the branch do not fit the scalar
+// registers and come back by hundreds of readlane instructions.
+template <typename Params>
+__device__ __forceinline__ const Params& first_argument() {
+  auto ptr = (const __attribute__((address_space(4))) Params*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ptr));
+  return *(const Params*)ptr;
+}
+
 // Maps a block id (blockIdx.x, or blockIdx.x minus a multiple of 8) to (head, block
 // rank).  Workgroups are dealt round-robin to the 8 XCDs, so id % 8 is the XCD: every block of one head is given to one XCD
 // (its operands stay in that XCD's L2) and each XCD's list is ordered longest
