@@ -478,3 +478,22 @@ def test_f32_backward_with_ds_of_some_heads_at_a_time():
         pair = rocm.attn_fwd_bwd(*(np.ascontiguousarray(x[n][:, h:h + 2]) for n in ("q", "k", "v", "do")))
         for a, b in zip(got[2:], pair[2:]):
             np.testing.assert_array_equal(a[:, h:h + 2], b)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("beta", [0.3, 1.5, -14.0])
+def test_f32_forward_when_the_row_maximum_grows_late(beta, D):
+    """As test_forward_when_the_row_maximum_grows_late, for the 32-row f32 forward: later keys within the
+    head-room of the reference, beyond it, and (negative: the first block has them) far below it."""
+    B, H, T = 2, 3, 355
+    x = synth.attention_inputs(f"late-max32-{beta}-{D}", B, H, T, D, np.float32, base_seed=31)
+    base = x["q"][:, :, :1, :]
+    q, k = base + 0.5 * x["q"], x["k"].copy()
+    for t in ((0, 1, 31) if beta < 0 else (40, 133, 331, 354)):
+        k[:, :, t, :] = abs(beta) * base[:, :, 0, :]
+    if beta < 0:
+        k[:, :, 32:, :] -= base
+    o, lse = rocm.attn_fwd(q, k, x["v"])
+    ro, rlse = oracle.attn_fwd(q, k, x["v"], return_lse=True, heads_per_call=1)
+    assert max_err(o, ro) <= TOL[np.dtype(np.float32)]
+    assert np.max(np.abs(lse - rlse) / (1e-4 + 1e-6 * np.abs(rlse))) <= 1.0
