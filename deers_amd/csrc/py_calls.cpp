@@ -7,11 +7,15 @@
 // token (32 sequences, 12 blocks) 433 -> 378 us, of a forward and backward of attention 11-13 -> 9 us.  The functions raise the binding's error class on a
 // non-zero return code and release the interpreter lock during the call, as ctypes does.
 //
-//   pointers    None, an int, a ctypes.c_void_p (its value), or any object with a buffer (its address)
-//   dimensions  None or a sequence of ints, copied for the duration of the call
+//   pointers    None, an int or a ctypes.c_void_p; for anything else the binding's `address` says which
+//               address it stands for, or refuses it.  An object's own storage is host memory, which a
+//               kernel must not be given.
+//   dimensions  None or a sequence of what int() takes, copied for the duration of the call
+//   sizes       a sequence of ints
 //   tables      a sequence of pointers
+//   dtoh's destination, the one host buffer: an object with a writable buffer that holds the bytes
 //
-// The library is the one the binding has loaded: bind(path, c_void_p, error class) looks the
+// The library is the one the binding has loaded: bind(path, c_void_p, error class, address) looks the
 // functions up in it, so that the path can be chosen at run time.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -28,11 +32,20 @@ namespace {
 
 PyTypeObject* g_void_p = nullptr;  // ctypes.c_void_p
 PyObject* g_error = nullptr;       // the exception class for a non-zero return code
+PyObject* g_address = nullptr;     // address(object) -> int
 decltype(&deers_rocm_last_error) g_last_error = nullptr;
 
 bool to_int64(PyObject* o, int64_t* out) {
   *out = PyLong_AsLongLong(o);
   return *out != -1 || !PyErr_Occurred();
+}
+// As int(o), which strides have always been passed through.
+bool to_dimension(PyObject* o, int64_t* out) {
+  if (PyLong_Check(o)) return to_int64(o, out);
+  PyObject* i = PyNumber_Long(o);
+  const bool ok = i && to_int64(i, out);
+  Py_XDECREF(i);
+  return ok;
 }
 bool to_address(PyObject* o, void** out) {
   if (o == Py_None) {
@@ -43,11 +56,18 @@ bool to_address(PyObject* o, void** out) {
     *out = PyLong_AsVoidPtr(o);
     return *out || !PyErr_Occurred();
   }
-  Py_buffer view;
-  if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) != 0) return false;
-  *out = Py_IS_TYPE(o, g_void_p) ? *(void**)view.buf : view.buf;
-  PyBuffer_Release(&view);
-  return true;
+  if (Py_IS_TYPE(o, g_void_p)) {
+    Py_buffer view;  // of the eight bytes that hold the address
+    if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) != 0) return false;
+    *out = *(void**)view.buf;
+    PyBuffer_Release(&view);
+    return true;
+  }
+  PyObject* address = PyObject_CallOneArg(g_address, o);
+  if (!address) return false;
+  *out = PyLong_AsVoidPtr(address);
+  Py_DECREF(address);
+  return *out || !PyErr_Occurred();
 }
 
 // One converter per kind of parameter: from() fills it, get() is what the C function takes.
@@ -90,6 +110,19 @@ struct Ptr {
   bool from(PyObject* o) { return to_address(o, &v); }
   T* get() { return static_cast<T*>(v); }
 };
+// Host memory to be written, held until the call is over.
+struct HostOut {
+  Py_buffer view{};
+  bool from(PyObject* o) {
+    if (PyObject_TypeCheck(o, g_void_p)) {  // its buffer is the address it holds
+      PyErr_SetString(PyExc_TypeError, "the destination is an object with a writable buffer, not an address");
+      return false;
+    }
+    return PyObject_GetBuffer(o, &view, PyBUF_WRITABLE) == 0;
+  }
+  void* get() { return view.buf; }
+  ~HostOut() { PyBuffer_Release(&view); }
+};
 
 // A sequence as a tuple or list, checked for its length (N = 0: any).
 PyObject* sequence(PyObject* o, size_t n) {
@@ -108,27 +141,57 @@ struct Items {
   bool from(PyObject* o) {
     PyObject* s = sequence(o, N);
     if (!s) return false;
-    const size_t n = (size_t)PySequence_Fast_GET_SIZE(s);
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(s);
     v = few.data();
-    if (n > few.size()) {
-      many.resize(n);
+    if ((size_t)n > few.size()) {
+      many.resize((size_t)n);
       v = many.data();
     }
     bool ok = true;
-    for (size_t i = 0; ok && i < n; ++i) ok = CONVERT(PySequence_Fast_GET_ITEM(s, i), v + i);
+    for (Py_ssize_t i = 0; ok && i < n; ++i) {
+      if (i >= PySequence_Fast_GET_SIZE(s)) {  // a conversion may run code that changes a list
+        PyErr_SetString(PyExc_RuntimeError, "a list changed its size while it was read");
+        ok = false;
+        break;
+      }
+      PyObject* item = PySequence_Fast_GET_ITEM(s, i);
+      Py_INCREF(item);
+      ok = CONVERT(item, v + i);
+      Py_DECREF(item);
+    }
     Py_DECREF(s);
     return ok;
   }
 };
 template <size_t N>
-struct Dims : Items<int64_t, to_int64, N> {  // None: null
-  bool from(PyObject* o) { return o == Py_None || Items<int64_t, to_int64, N>::from(o); }
+struct Dims : Items<int64_t, to_dimension, N> {  // None: null
+  bool from(PyObject* o) { return o == Py_None || Items<int64_t, to_dimension, N>::from(o); }
   const int64_t* get() { return this->v; }
+};
+struct Sizes : Items<int64_t, to_int64, 0> {
+  const int64_t* get() { return v; }
 };
 template <class T>
 struct Table : Items<void*, to_address, 0> {
   T get() { return (T)this->v; }
 };
+
+using CP = Ptr<const void>;
+using MP = Ptr<void>;
+using FP = Ptr<float>;
+using CFP = Ptr<const float>;
+using IP = Ptr<const int64_t>;  // index vectors in device memory
+using I64 = Int64;
+
+template <class... Kinds>
+bool fits(std::tuple<Kinds...>&) {
+  return true;
+}
+bool fits(std::tuple<HostOut, CP, Size>& k) {
+  if (std::get<0>(k).view.len >= 0 && (size_t)std::get<0>(k).view.len >= std::get<2>(k).get()) return true;
+  PyErr_Format(PyExc_ValueError, "%zu bytes do not fit a buffer of %zd", std::get<2>(k).get(), std::get<0>(k).view.len);
+  return false;
+}
 
 template <class Kinds, class Fn, size_t... I>
 PyObject* call(Fn fn, PyObject* const* args, Py_ssize_t n, std::index_sequence<I...>) {
@@ -138,7 +201,7 @@ PyObject* call(Fn fn, PyObject* const* args, Py_ssize_t n, std::index_sequence<I
   }
   if (!fn) return PyErr_Format(PyExc_RuntimeError, "bind() comes first");
   Kinds k;
-  if (!(std::get<I>(k).from(args[I]) && ...)) return nullptr;
+  if (!((std::get<I>(k).from(args[I]) && ...) && fits(k))) return nullptr;
   PyThreadState* state = PyEval_SaveThread();
   const int rc = fn(std::get<I>(k).get()...);
   PyEval_RestoreThread(state);
@@ -148,13 +211,6 @@ PyObject* call(Fn fn, PyObject* const* args, Py_ssize_t n, std::index_sequence<I
   }
   Py_RETURN_NONE;
 }
-
-using CP = Ptr<const void>;
-using MP = Ptr<void>;
-using FP = Ptr<float>;
-using CFP = Ptr<const float>;
-using IP = Ptr<const int64_t>;  // index vectors in device memory
-using I64 = Int64;
 
 // X(name, parameter kinds ...)
 #define CALLS(X)                                                                                                    \
@@ -177,8 +233,8 @@ using I64 = Int64;
   X(cross_entropy_bwd, Int, CP, IP, CFP, CFP, MP, I64, I64)                                                         \
   X(scale_by_scalar, Int, MP, I64, CFP)                                                                             \
   X(adamw_step_multi, Int, Int, Table<void* const*>, Table<const void* const*>, Table<void* const*>,                \
-    Table<void* const*>, Dims<0>, Double, Double, Double, Double, Double, I64, Double)                              \
-  X(sum_squares_multi, Int, Int, Table<const void* const*>, Dims<0>, FP, Int)                                       \
+    Table<void* const*>, Sizes, Double, Double, Double, Double, Double, I64, Double)                              \
+  X(sum_squares_multi, Int, Int, Table<const void* const*>, Sizes, FP, Int)                                       \
   X(copy_view, Int, CP, Dims<0>, MP, Dims<0>, Dims<0>, Int)                                                         \
   X(matmul, Int, CP, I64, I64, I64, CP, I64, I64, I64, MP, I64, I64, I64, I64)                                      \
   X(matmul_acc, Int, CP, I64, I64, I64, CP, I64, I64, I64, MP, I64, I64, I64, I64)                                  \
@@ -188,7 +244,7 @@ using I64 = Int64;
   X(decode_qkv, Int, CP, CP, CP, Dims<2>, CP, CP, MP, MP, MP, Dims<3>, I64, I64, I64, I64, I64)                     \
   X(rope_fwd, Int, CP, Dims<4>, CP, CP, MP, Dims<4>, I64, I64, I64, I64)                                            \
   X(rope_bwd, Int, CP, Dims<4>, CP, CP, MP, I64, I64, I64, I64)                                                     \
-  X(dtoh, MP, CP, Size)
+  X(dtoh, HostOut, CP, Size)
 
 #define DEFINE(name, ...)                                                                       \
   decltype(&deers_rocm_##name) p_##name = nullptr;                                              \
@@ -201,8 +257,8 @@ CALLS(DEFINE)
 
 PyObject* bind(PyObject*, PyObject* args) {
   const char* path;
-  PyObject *void_p, *error;
-  if (!PyArg_ParseTuple(args, "sOO", &path, &void_p, &error)) return nullptr;
+  PyObject *void_p, *error, *address;
+  if (!PyArg_ParseTuple(args, "sOOO", &path, &void_p, &error, &address)) return nullptr;
   if (!PyType_Check(void_p)) return PyErr_Format(PyExc_TypeError, "c_void_p is needed");
   void* lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
   if (!lib) return PyErr_Format(PyExc_OSError, "%s", dlerror());
@@ -215,11 +271,13 @@ PyObject* bind(PyObject*, PyObject* args) {
   Py_XSETREF(g_void_p, (PyTypeObject*)void_p);
   Py_INCREF(error);
   Py_XSETREF(g_error, error);
+  Py_INCREF(address);
+  Py_XSETREF(g_address, address);
   Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {
-    {"bind", bind, METH_VARARGS, "bind(path, c_void_p, error): look the functions up in the library at `path`"},
+    {"bind", bind, METH_VARARGS, "bind(path, c_void_p, error, address): look the functions up in the library at `path`"},
 #define METHOD(name, ...) {#name, (PyCFunction)(void (*)(void))call_##name, METH_FASTCALL, "deers_rocm_" #name},
     CALLS(METHOD)
 #undef METHOD

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import importlib
+import operator
 import os
 
 import numpy as np
@@ -38,6 +39,28 @@ class RocmError(RuntimeError):
     """A non-zero return code from the library (the role of deers' backend error variant)."""
 
 
+_BYREF = type(ctypes.byref(ctypes.c_int()))
+_INTEGER_CODES = "bBhHiIlLqQ"  # of ctypes' simple types
+
+
+def _address(o) -> int:
+    """The address that a pointer argument stands for, if it is no None, int or c_void_p: what ctypes passes
+    for its own pointers, integers and arrays and for byref(), an object's `_as_parameter_`, or an integer
+    of another type.  Everything else is refused, a numpy array or a tensor above all: its storage may be
+    host memory, and its one element is no address."""
+    if isinstance(o, ctypes._SimpleCData):
+        if isinstance(o, ctypes.c_void_p) or o._type_ in _INTEGER_CODES:
+            return o.value or 0
+    elif isinstance(o, (ctypes._Pointer, ctypes.Array, _BYREF)):
+        return ctypes.cast(o, ctypes.c_void_p).value or 0
+    elif hasattr(o, "_as_parameter_"):
+        p = o._as_parameter_
+        return 0 if p is None else p if isinstance(p, int) else _address(p)
+    elif hasattr(o, "__index__") and not hasattr(o, "__len__"):
+        return operator.index(o)
+    raise ctypes.ArgumentError(f"a pointer argument cannot be of type {type(o).__name__}")
+
+
 def load() -> ctypes.CDLL:
     """Loads libdeers_rocm.so and the extension module; raises if they have not been built."""
     global _lib, _calls
@@ -54,7 +77,7 @@ def load() -> ctypes.CDLL:
         except ImportError as e:
             raise RocmError(f"the extension module deers_amd._calls is missing ({e}): build it with "
                             "`make -C deers_amd/csrc` (or __graft_entry__.build())") from e
-        calls.bind(LIB_PATH, ctypes.c_void_p, RocmError)
+        calls.bind(LIB_PATH, ctypes.c_void_p, RocmError, _address)
         _lib, _calls = lib, calls
     return _lib
 
