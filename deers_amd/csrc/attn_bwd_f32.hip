@@ -18,6 +18,11 @@
 //   these: 1037.
 // Every sum is taken in a fixed order: dQ, dK and dV are reproducible bit for bit.
 //
+// The products start from zero and the row statistics are added to the finished sums.  Starting them from
+// the statistics saves 32 additions per block (8 x 12 x 1024 x 64, forward and backward: 442 us, 446 this way)
+// but rounds every element's term at the size of the LSE: relative error of dQ against 64 bits 1.0e-6 instead
+// of 0.43e-6 at T = 1024, D = 64, of dK 1.06e-6 instead of 0.53e-6.
+//
 // us, before -> now: 8 x 12 x 1024 x 64 366 -> 302, 400 x 512 x 64 427 -> 345, 8 x 2048 x 64 162 -> 136, 48 x 1024 x 128
 // 499 -> 379, 400 x 512 x 128 1225 -> 765, 96 x 1024 x 32 199 -> 167.
 #include <algorithm>
@@ -106,14 +111,11 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f3
   for (; qb < n_blocks; qb += W) {
     const bool more = qb + W < n_blocks;
     wait_vmcnt<C::NI>();  // dS written, statistics, Q
-    floatx16 s = product<D>(q_blk, kf, D == 128 ? ZERO16S : stat_rows(stat, g), lane);
-    floatx16 dp = D == 128 ? ZERO16S : stat_rows(stat + 32, g);
+    floatx16 s = product<D>(q_blk, kf, ZERO16S, lane);
     wait_vmcnt<0>();  // dO
-    dp = product<D>(do_blk, vf, dp, lane);
-    if constexpr (D == 128) {
-      s += stat_rows(stat, g);
-      dp += stat_rows(stat + 32, g);
-    }
+    floatx16 dp = product<D>(do_blk, vf, ZERO16S, lane);
+    s += stat_rows(stat, g);
+    dp += stat_rows(stat + 32, g);
     if (qb == kb) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)

@@ -189,14 +189,9 @@ __device__ __forceinline__ void split32_dq(const BwdParams& p, int bh, int qb, c
   for (int db = 0; db < DB; ++db) dq[db] = ZERO16S;
   for (; kb <= qb; kb += W) {
     const bool more = kb + W <= qb;
-    floatx16 s, dp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = lse2;
-      dp[r] = nd;
-    }
     wait_vmcnt<C::NI>();  // V; K's block may be on its way
-    dp = product<D>(v_blk, dof, dp, lane);
+    // (from zero, not from the row statistics: see the error figures in attn_bwd_f32.hip)
+    const floatx16 dp = product<D>(v_blk, dof, ZERO16S, lane);
     if (more) {
       settle_lds_reads();
       load_block<D>(V, svt, 32 * (kb + W), T, v_blk, lane);
@@ -204,14 +199,14 @@ __device__ __forceinline__ void split32_dq(const BwdParams& p, int bh, int qb, c
     } else {
       wait_vmcnt<0>();
     }
-    s = product<D>(k_blk, qf, s, lane);
+    floatx16 s = product<D>(k_blk, qf, ZERO16S, lane);
     if (kb == qb) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         if (8 * (r >> 2) + 4 * g + (r & 3) > (lane & 31)) s[r] = -INFINITY;
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r]) * dp[r];
+    for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r] + lse2) * (dp[r] + nd);
     accumulate<D>(dq, k_blk, s, lane);
     if (more) {
       settle_lds_reads();

@@ -497,3 +497,31 @@ def test_f32_forward_when_the_row_maximum_grows_late(beta, D):
     ro, rlse = oracle.attn_fwd(q, k, x["v"], return_lse=True, heads_per_call=1)
     assert max_err(o, ro) <= TOL[np.dtype(np.float32)]
     assert np.max(np.abs(lse - rlse) / (1e-4 + 1e-6 * np.abs(rlse))) <= 1.0
+
+
+@pytest.mark.parametrize("B,H,T,D", [
+    (1, 3, 1024, 64), (1, 2, 777, 128), (1, 4, 1024, 32),       # S and dP computed twice
+    (2, 8, 1024, 64), (2, 12, 1024, 32), (24, 8, 225, 64)])     # dS in memory
+def test_f32_gradients_round_at_the_size_of_the_lse_once(B, H, T, D):
+    """Relative 2-norm error of the gradients against 64 bits.  A probability's exponent S - LSE may be
+    rounded twice at the size of the LSE (8 to 16 in base 2: an rms of 2^-20 / sqrt(12) each), for LSE * log2(e)
+    and for the difference; times ln 2 that is 2.7e-7, the error of dP - dO . O is smaller, and the sums over up
+    to 1024 rows add about as much again (0.3 to 0.6e-6 in all).  A product that starts from the LSE rounds at
+    that size for every element of D: sqrt(D) * 1.9e-7, 1.1e-6 at D = 32.  The bound is 12 * 2^-24."""
+    x = synth.attention_inputs(f"acc32-{B}-{H}-{T}-{D}", B, H, T, D, np.float32, base_seed=37)
+    got = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])[2:]
+    future = np.triu(np.ones((T, T), bool), 1)
+    scale = float(rocm.default_scale(D))
+    off, size = np.zeros(3), np.zeros(3)
+    for b, h in {(0, 0), (B - 1, H - 1), (B // 2, 0)}:
+        q, k, v, do = (x[n][b, h].astype(np.float64) for n in ("q", "k", "v", "do"))
+        s = np.where(future, -np.inf, q @ k.T * scale)
+        p = np.exp(s - np.max(s, 1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        ds = p * (do @ v.T - np.sum(do * (p @ v), 1, keepdims=True))
+        for i, want in enumerate((ds @ k * scale, ds.T @ q * scale, p.T @ do)):
+            off[i] += np.sum((got[i][b, h] - want) ** 2)
+            size[i] += np.sum(want ** 2)
+    rel = np.sqrt(off / size)
+    say(f"f32 {B}x{H}x{T}x{D}: dq={rel[0]:.2e} dk={rel[1]:.2e} dv={rel[2]:.2e}")
+    assert (rel <= 12 * 2.0 ** -24).all(), rel
