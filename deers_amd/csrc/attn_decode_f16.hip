@@ -49,8 +49,17 @@ constexpr int kDecSplitRows = 128;  // a split's smallest share of the cache
 // another start-up and another partial to merge (12 heads x 6000 x 64: 9.6 us in 16 splits, 10.5
 // in 21, 13.9 in 47); below kDecSplitRows rows the merge costs what the shorter stream saves
 // (12 x 1500 x 64: 6.1 us in 12 splits, 9.1 in 24).
-int decode_pick_splits(int64_t BH, int64_t L, int* chunk) {
-  const int64_t by_cus = 32 / ((BH + 7) / 8), by_rows = (L + kDecSplitRows - 1) / kDecSplitRows;
+// Where that leaves three CUs of ten without a workgroup (11 heads of an XCD in two splits, 17 to 21 in
+// one) a CU gets two, if the caches are long enough for the stream to be what counts (us in one per CU /
+// two per CU: 132 x 1024 x 64 10.1 / 9.8, 132 x 8192 x 64 54.6 / 44.6, 160 x 8192 x 64 56.3 / 50.3, 88 x 8192 x 128 60.1 /
+// 54.8; but 160 x 768 x 64 8.7 / 9.0).  With fewer idle ones it gains nothing (12 heads, three of four CUs:
+// 96 x 16384 x 64 60.9 / 59.9).
+// Spreading fewer than eight heads over all XCDs, to be merged by a second launch, gains only beyond any
+// cache of interest (2 x 65536 x 64: 19.5 us on two XCDs, 17.4 on eight; 2 x 16384: 9.0 / 13.6).
+int decode_pick_splits(int64_t BH, int64_t L, int64_t D, int* chunk) {
+  const int64_t heads = (BH + 7) / 8, by_rows = (L + kDecSplitRows - 1) / kDecSplitRows;
+  int64_t by_cus = 32 / heads;
+  if (L * D >= 65536 && 10 * heads * by_cus < 7 * 32 && 64 / heads > 2 * by_cus) by_cus = 64 / heads;
   const int64_t want = std::max<int64_t>(1, std::min(by_cus, by_rows));
   const int64_t c = std::max<int64_t>(16, ((L + want - 1) / want + 15) / 16 * 16);
   *chunk = (int)c;

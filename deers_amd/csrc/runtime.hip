@@ -39,7 +39,7 @@ bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f32_split(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f32_split(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_decode_f16(const DecodeParams& p, int B, int D, bool append, hipStream_t stream);
-int decode_pick_splits(int64_t BH, int64_t L, int* chunk);
+int decode_pick_splits(int64_t BH, int64_t L, int64_t D, int* chunk);
 void launch_fill(int dtype_f16, void* dst, size_t n, float value, hipStream_t stream);
 void launch_add(int dtype_f16, const void* a, const void* b, void* out, size_t n,
                 hipStream_t stream);
@@ -139,7 +139,6 @@ struct Runtime {
   int* index_flag = nullptr;
   bool index_flag_armed = false;
   deers::SkinnyPrefetch skinny_next;  // one-shot hint for the next few-rows product (decode_linear_hint)
-  int* decode_counters = nullptr;  // arrival counters of split decode heads (all zero between launches)
   int* skinny_counters = nullptr;  // arrival counters of the few-rows GEMM's K splits (all zero between launches)
   // Block cache behind deers_rocm_alloc / _free.  Every kernel and copy of this library
   // runs on `stream`, in order, so a block handed back by free can be handed out again
@@ -169,6 +168,10 @@ constexpr size_t kHostStagingBytes = 4096;
 constexpr size_t kScratchBytes = 512 * 1024;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 void* g_scratch_ptr = nullptr;  // device address of `scratch` on g_rt.ordinal
+// Arrival counters of split decode heads, all zero between launches; the same kind of memory, since
+// the entry point that allocates nothing uses them too.
+static __device__ int decode_arrivals[kDecodeCounters];
+int* g_decode_arrivals = nullptr;
 thread_local std::string t_err;
 
 int fail(int code, const char* fmt, ...) {
@@ -365,6 +368,7 @@ int deers_rocm_init(int ordinal) {
   HIP_TRY(hipSetDevice(ordinal));
   HIP_TRY(hipStreamCreateWithFlags(&g_rt.stream, hipStreamNonBlocking));
   HIP_TRY(hipGetSymbolAddress(&g_scratch_ptr, HIP_SYMBOL(scratch)));
+  HIP_TRY(hipGetSymbolAddress((void**)&g_decode_arrivals, HIP_SYMBOL(decode_arrivals)));
   HIP_TRY(hipHostMalloc(&g_rt.host_staging, kHostStagingBytes, hipHostMallocDefault));
   {
     hipDeviceProp_t prop;
@@ -806,19 +810,14 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
 
 // Arrival counters for a decode call whose split heads are merged inside the launch; null where
 // they are merged by a second one: nothing to merge, splits that may not share an XCD, or a call
-// that may run beside another one (a captured graph; deers_rocm_attn_decode_noalloc asks for
-// null itself), since calls that overlap would count each other's arrivals.
+// that may run beside another one (a captured graph), since calls that overlap would count each other's
+// arrivals.
 static int decode_counters(int64_t BH, int splits, int** out) {
   *out = nullptr;
   if (splits == 1 || BH > kDecodeCounters || !same_xcd_handover_now()) return DEERS_ROCM_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
-  if (cs != hipStreamCaptureStatusNone) return DEERS_ROCM_OK;
-  if (!g_rt.decode_counters) {  // zero once; the kernel leaves every counter at zero
-    HIP_TRY(hipMalloc(&g_rt.decode_counters, kDecodeCounters * sizeof(int)));
-    HIP_TRY(hipMemsetAsync(g_rt.decode_counters, 0, kDecodeCounters * sizeof(int), g_rt.stream));
-  }
-  *out = g_rt.decode_counters;
+  if (cs == hipStreamCaptureStatusNone) *out = g_decode_arrivals;
   return DEERS_ROCM_OK;
 }
 
@@ -845,7 +844,7 @@ static int attn_decode_impl(const char* what, bool no_alloc, int dtype, const vo
       (reinterpret_cast<uintptr_t>(o) & 15))
     return fail(DEERS_ROCM_ERR_LAYOUT, "%s: cache rows, q and o must be 16-byte aligned", what);
   int chunk = 0;
-  const int splits = deers::decode_pick_splits(B * H, L, &chunk);
+  const int splits = deers::decode_pick_splits(B * H, L, D, &chunk);
   void* ws = nullptr;
   const size_t part_o = (size_t)(B * H) * splits * D * sizeof(float);
   const size_t part_ml = (size_t)(B * H) * splits * 2 * sizeof(float);
@@ -864,7 +863,10 @@ static int attn_decode_impl(const char* what, bool no_alloc, int dtype, const vo
   p.part_o = static_cast<float*>(ws);
   p.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
   p.BH = (int)(B * H); p.H = (int)H; p.L = (int)L; p.splits = splits; p.chunk = chunk;
-  if (!no_alloc)
+  // The entry point that allocates nothing has merged by a second launch from the beginning; inside the
+  // launch pays for up to four splits (1 head x 500 x 64 6.5 -> 4.0 us, 48 x 2000 x 64 9.2 -> 8.9), and with many
+  // short ones it does not (12 x 2000 x 64 in 16 splits 6.2 -> 7.1).
+  if (!no_alloc || splits <= 4)
     if (int rc = decode_counters(B * H, splits, &p.arrived)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, false, g_rt.stream);
@@ -922,7 +924,7 @@ int deers_rocm_attn_decode_append(int dtype, const void* q, const void* k, const
   deers::DecodeParams p{};
   p.skb = cache_strides[0]; p.skh = cache_strides[1]; p.skl = cache_strides[2];
   int chunk = 0;
-  const int splits = deers::decode_pick_splits(B * H, pos, &chunk);  // over the rows already cached
+  const int splits = deers::decode_pick_splits(B * H, pos, D, &chunk);  // over the rows already cached
   void* ws = nullptr;
   const size_t part_o = (size_t)(B * H) * splits * D * sizeof(float);
   const size_t part_ml = (size_t)(B * H) * splits * 2 * sizeof(float);

@@ -213,7 +213,7 @@ int deers_rocm_attn_decode(int dtype,
  * the split partial results live in a fixed 512 KiB device array that is part of the
  * library image, so the call performs no hipMalloc / hipFree and never grows a
  * workspace.  A problem whose partials (B*H*splits*(D+2) floats, only when heads are
- * split over workgroups, i.e. B*H < 256) would not fit is rejected with
+ * split over workgroups, i.e. B*H <= 168) would not fit is rejected with
  * DEERS_ROCM_ERR_ARG.  All calls on a device share the one array: calls that overlap
  * on the device (other streams, other processes' copies aside) would race; the library
  * stream runs them in order. */

@@ -188,3 +188,42 @@ def test_captured_backward_replays_correctly(gpu):
     finally:
         hip.hipGraphExecDestroy(graph_exec)
         hip.hipGraphDestroy(graph)
+
+
+def test_decode_splits_leave_few_compute_units_idle_on_long_caches():
+    """The rule alone, on the host: at most three of an XCD's ten compute units without a workgroup, at most
+    two workgroups on one, and every row of the cache in exactly one split that has rows."""
+    import ctypes
+    rule = rocm.load()["_ZN5deers18decode_pick_splitsElllPi"]
+    chunk = ctypes.c_int()
+    i64 = ctypes.c_int64
+    for D, L in ((64, 1), (64, 300), (32, 2047), (64, 1023), (64, 1024), (64, 8192), (128, 512), (128, 16000)):
+        for heads in range(1, 400):
+            splits = rule(i64(heads), i64(L), i64(D), ctypes.byref(chunk))
+            per_xcd = (heads + 7) // 8 * splits
+            assert splits * chunk.value >= L > (splits - 1) * chunk.value, (D, L, heads)
+            assert heads > 256 or per_xcd <= 64, (D, L, heads)
+            assert heads * splits * (D + 2) * 4 <= 512 * 1024 or splits == 1, (D, L, heads)
+            if L >= 8192 and heads > 7:
+                assert per_xcd >= 0.65 * 32, (D, L, heads, splits)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,L,D", [(12, 11, 1023, 64), (12, 11, 1025, 64), (21, 8, 513, 128), (11, 8, 2063, 32)])
+def test_decode_with_two_workgroups_on_a_compute_unit(gpu, B, H, L, D):
+    """Either side of the cache length from which 17 to 21 heads of an XCD are split in three, and 11 in five;
+    merged in the launch, after it, and in the static memory of the entry point that allocates nothing."""
+    x = synth.attention_inputs(f"handover-dec2-{B}-{H}-{L}-{D}", B, H, 1, D, np.float16, base_seed=17, kv_len=L,
+                               names=("q", "k", "v"))
+    outs = []
+    for mode in (rocm.HANDOVER_SAME_XCD, rocm.HANDOVER_STREAM_ORDER, rocm.HANDOVER_SAME_XCD):
+        rocm.set_handover_mode(mode)
+        outs.append(rocm.attn_decode(x["q"][:, :, 0], x["k"], x["v"]))
+        q, k, v = (rocm.DeviceBuffer.from_numpy(x[n]) for n in ("q", "k", "v"))
+        o = rocm.DeviceBuffer.from_numpy(np.full((B, H, D), np.nan, np.float16))
+        rocm.attn_decode_noalloc_raw(np.float16, q.ptr, k.ptr, v.ptr, o.ptr, B, H, L, D, rocm.default_scale(D))
+        outs.append(o.numpy())
+    want = oracle.attn_fwd(x["q"], x["k"], x["v"])[:, :, 0]
+    assert np.max(np.abs(outs[0].astype(np.float64) - want)) <= 5e-3
+    for other in outs[1:]:
+        np.testing.assert_array_equal(outs[0], other)
