@@ -257,12 +257,6 @@ void launch_bwd(const BwdParams& p, int BH, int heads, char* ds, hipStream_t str
   }
 }
 
-// dS of as many heads as this holds (a head of 34 K rows) is in memory at a time.  Larger is better until
-// a share of the heads fills the device many times over: every share has an end at which CUs are idle
-// (128 MB, which the memory-side cache would hold, instead of 1 GB: 96 x 1024 x 64 316 -> 336 us, 24 x 4096 x 64
-// 1065 -> 1857).
-constexpr int64_t kMaxDsBytes = (int64_t)2304 << 20;
-
 int64_t ds_bytes(int64_t T) {
   const int64_t nb = (T + 31) / 32;
   return nb * (nb + 1) / 2 * kDsBlock;
@@ -270,25 +264,33 @@ int64_t ds_bytes(int64_t T) {
 
 }  // namespace
 
+// dS of as many heads as the limit holds (by default a head of 34 K rows) is in memory at a time.  Larger is
+// better until a share of the heads fills the device many times over: every share has an end at which CUs are
+// idle (128 MB, which the memory-side cache would hold, instead of 1 GB: 96 x 1024 x 64 316 -> 336 us, 24 x 4096 x
+// 64 1065 -> 1857).
+int64_t attn_bwd_f32_default_ds_limit() { return (int64_t)2304 << 20; }
+
 // Which launches come here (the others: attn_split_f32.hip, S and dP twice but one launch).  Three
 // launches and a workspace pay from enough workgroups on to fill the device, n = heads * T / 32 (D = 64: at
 // 512 of them, 8 x 2048, 136 us against 162; at 384, 12 x 1024, 71 against 66).  The shorter the walks, the
 // more the launches weigh: below twelve blocks several times as many workgroups (192 x 256 x 64 72 against
 // 75, 96 x 256 x 64 47 against 44), below eight only with one wave per workgroup (800 x 128 x 64: 86 against
 // 97; 4000 x 64 x 128: 350 against 455).
-bool attn_bwd_f32_takes(int64_t BH, int64_t T, int64_t D) {
+static bool takes(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb;
-  if (ds_bytes(T) > kMaxDsBytes) return false;
   if (nb >= 12) return n >= (D == 32 ? 640 : D == 64 ? 512 : 384);
   if (nb >= 8) return n >= (D == 128 ? 640 : 1536);
   return nb >= 2 && attn_f32_one_wave(n, nb, D);
 }
-// Bytes for the dS of `heads` heads: all of them, or an even share of those that fit.
-size_t attn_bwd_f32_ds_bytes(int64_t BH, int64_t T, int* heads) {
-  const int64_t most = std::min(BH, kMaxDsBytes / ds_bytes(T)), shares = (BH + most - 1) / most;
-  *heads = (int)((BH + shares - 1) / shares);
-  return (size_t)(*heads * ds_bytes(T));
+// Returns how many heads at a time: all of them, or an even share of those whose dS the limit holds; 0: the
+// launch goes elsewhere, for a share that cannot fill the device too.
+int attn_bwd_f32_heads(int64_t BH, int64_t T, int64_t D, int64_t limit) {
+  const int64_t most = std::min(BH, limit / ds_bytes(T));
+  if (most == 0) return 0;
+  const int64_t shares = (BH + most - 1) / most, heads = (BH + shares - 1) / shares;
+  return takes(heads, T, D) ? (int)heads : 0;
 }
+size_t attn_bwd_f32_ds_bytes(int heads, int64_t T) { return (size_t)(heads * ds_bytes(T)); }
 
 void launch_attn_bwd_f32(const BwdParams& p, int B, int D, int heads, void* ds, hipStream_t stream) {
   switch (D) {

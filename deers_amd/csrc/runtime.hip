@@ -32,8 +32,9 @@ bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream);
-bool attn_bwd_f32_takes(int64_t BH, int64_t T, int64_t D);
-size_t attn_bwd_f32_ds_bytes(int64_t BH, int64_t T, int* heads);
+int64_t attn_bwd_f32_default_ds_limit();
+int attn_bwd_f32_heads(int64_t BH, int64_t T, int64_t D, int64_t limit);
+size_t attn_bwd_f32_ds_bytes(int heads, int64_t T);
 void launch_attn_bwd_f32(const BwdParams& p, int B, int D, int heads, void* ds, hipStream_t stream);
 bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f32_split(const FwdParams& p, int B, int D, hipStream_t stream);
@@ -113,6 +114,13 @@ struct Runtime {
   hipStream_t stream = nullptr;
   void* workspace = nullptr;  // grows on demand, freed never (process lifetime)
   size_t workspace_bytes = 0;
+  // dS of the f32 backward and its row statistics: grows on demand, its dS up to the limit; given back by
+  // empty_cache, by a lower limit and when an allocation fails.  Once a captured launch has used it, it stays
+  // for the graph's replays, and a larger one is a new one beside it.
+  void* ds = nullptr;
+  size_t ds_bytes = 0;
+  bool ds_captured = false;
+  int64_t ds_limit = deers::attn_bwd_f32_default_ds_limit();
   rocblas_handle blas = nullptr;  // created by the first matmul, bound to `stream`
   // per (head, 128-row query block) publication flags of the single-launch f16
   // backward; a flag equals the current epoch once its rows are published
@@ -234,6 +242,43 @@ int workspace(size_t bytes, void** out) {
     g_rt.workspace_bytes = want;
   }
   *out = g_rt.workspace;
+  return DEERS_ROCM_OK;
+}
+
+// Returns the f32 backward's dS memory to the driver (after the stream has drained), unless a captured
+// graph uses it.
+int release_ds() {
+  if (!g_rt.ds || g_rt.ds_captured) return DEERS_ROCM_OK;
+  HIP_TRY(hipStreamSynchronize(g_rt.stream));
+  HIP_TRY(hipFree(g_rt.ds));
+  g_rt.ds = nullptr;
+  g_rt.ds_bytes = 0;
+  return DEERS_ROCM_OK;
+}
+
+// That memory with at least `bytes`, or null: there is not as much, or a capture, which allows no
+// allocation, would have to get it.
+int ds_memory(size_t bytes, void** out) {
+  *out = nullptr;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
+  const bool capturing = cs != hipStreamCaptureStatusNone;
+  if (bytes > g_rt.ds_bytes) {
+    if (capturing) return DEERS_ROCM_OK;
+    if (int rc = release_ds()) return rc;
+    g_rt.ds = nullptr;  // a captured graph's is its own from here on
+    g_rt.ds_bytes = 0;
+    g_rt.ds_captured = false;
+    const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
+    if (hipMalloc(&g_rt.ds, want) != hipSuccess) {
+      (void)hipGetLastError();
+      g_rt.ds = nullptr;
+      return DEERS_ROCM_OK;
+    }
+    g_rt.ds_bytes = want;
+  }
+  g_rt.ds_captured |= capturing;
+  *out = g_rt.ds;
   return DEERS_ROCM_OK;
 }
 
@@ -494,7 +539,15 @@ static int release_cached_blocks() {
 int deers_rocm_empty_cache(void) {
   std::lock_guard<std::mutex> lock(g_mu);
   NEED_INIT();
+  if (int rc = release_ds()) return rc;
   return release_cached_blocks();
+}
+
+int deers_rocm_set_bwd_workspace_limit(int64_t bytes) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  NEED_INIT();
+  g_rt.ds_limit = bytes < 0 ? deers::attn_bwd_f32_default_ds_limit() : bytes;
+  return (int64_t)g_rt.ds_bytes > g_rt.ds_limit ? release_ds() : DEERS_ROCM_OK;
 }
 
 int deers_rocm_alloc(size_t bytes, void** out_ptr) {
@@ -516,6 +569,7 @@ int deers_rocm_alloc(size_t bytes, void** out_ptr) {
   hipError_t e = hipMalloc(out_ptr, size);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
+    if (int rc = release_ds()) return rc;
     if (int rc = release_cached_blocks()) return rc;
     e = hipMalloc(out_ptr, size);
   }
@@ -741,18 +795,11 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   const size_t ws_floats = (size_t)(2 * B * H * t_pad + 64);
   void* ws = nullptr;
   if (dtype == DEERS_ROCM_F32) {
-    int heads = 0;
-    // behind them dS of `heads` heads at a time; without the memory for it, or while a capture forbids
-    // to get it, the form that computes S and dP twice
-    bool two_pass = deers::attn_bwd_f32_takes(B * H, T, D);
-    if (two_pass) {
-      const size_t bytes = ws_floats * sizeof(float) + deers::attn_bwd_f32_ds_bytes(B * H, T, &heads);
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      if (bytes > g_rt.workspace_bytes) HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
-      two_pass = cs == hipStreamCaptureStatusNone && workspace(bytes, &ws) == DEERS_ROCM_OK;
-      if (!two_pass) (void)hipGetLastError();
-    }
-    if (two_pass) {
+    // behind them dS of `heads` heads at a time; without that memory the form that computes S and dP twice
+    const int heads = deers::attn_bwd_f32_heads(B * H, T, D, g_rt.ds_limit);
+    if (heads)
+      if (int rc = ds_memory(ws_floats * sizeof(float) + deers::attn_bwd_f32_ds_bytes(heads, T), &ws)) return rc;
+    if (ws) {
       p.lse2 = static_cast<float*>(ws);
       p.negdelta = p.lse2 + B * H * t_pad;
       p.t_pad = (int)t_pad;

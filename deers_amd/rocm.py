@@ -217,6 +217,12 @@ def empty_cache():
     _check(load().deers_rocm_empty_cache())
 
 
+def set_bwd_workspace_limit(nbytes: int = -1):
+    """deers_rocm_set_bwd_workspace_limit: memory for the f32 backward's dS (-1: the default, 0: none)."""
+    init()
+    _check(load().deers_rocm_set_bwd_workspace_limit(ctypes.c_int64(nbytes)))
+
+
 def profile_collect() -> dict:
     """{kernel name: (calls, total_ms)} for launches since profile_enable(True)."""
     n = ctypes.c_int()

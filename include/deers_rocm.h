@@ -117,7 +117,8 @@ int deers_rocm_alloc_zeros(size_t bytes, void** out_ptr);
  * a later alloc of the same size reuses the block.  That is safe because all of the
  * library's work runs in order on one stream (a buffer the caller also uses on another
  * stream must be ordered by the caller).  A block leaves the cache when hipMalloc runs
- * out of memory or deers_rocm_empty_cache is called. */
+ * out of memory or deers_rocm_empty_cache is called; both also give back the memory of
+ * deers_rocm_set_bwd_workspace_limit. */
 int deers_rocm_free(void* ptr);
 int deers_rocm_empty_cache(void);
 
@@ -179,7 +180,10 @@ int deers_rocm_attn_fwd(int dtype,
  *     dS = P o (dP - rowsum(dO o O));  dQ = scale dS K;  dK = scale dS^T Q.
  * o and lse are the forward outputs.  dq,dk,dv are overwritten (not
  * accumulated into); the caller's GradientStore::accumulate
- * (src/backprop.rs:101-112) adds them to existing gradients. */
+ * (src/backprop.rs:101-112) adds them to existing gradients.
+ * f32 launches that fill the device keep dS in device memory between two passes (see
+ * deers_rocm_set_bwd_workspace_limit); the others, and all where there is no memory for it,
+ * compute it twice.  Every gradient is reproducible bit for bit on the same one of the two. */
 int deers_rocm_attn_bwd(int dtype,
                         const void* q, const int64_t* q_strides,
                         const void* k, const int64_t* k_strides,
@@ -191,6 +195,15 @@ int deers_rocm_attn_bwd(int dtype,
                         void* dk, const int64_t* dk_strides,
                         void* dv, const int64_t* dv_strides,
                         int64_t B, int64_t H, int64_t T, int64_t D, float scale);
+
+/* Device memory that the f32 backward may keep dS in: 4 KiB per 32 x 32 block at or below the
+ * diagonal and head (8 x 12 x 1024: 217 MB), of so many heads at a time that it stays within
+ * `bytes`; -1: the default of 2.25 GiB, 0: none.  The library takes it at the first call that
+ * uses it and keeps it for the next; deers_rocm_empty_cache, a lower limit and a failed
+ * deers_rocm_alloc give it back, unless a HIP graph was captured with it: then it stays for the
+ * graph's replays.  A call that is being captured uses the memory that is there and otherwise
+ * computes dS twice. */
+int deers_rocm_set_bwd_workspace_limit(int64_t bytes);
 
 /* Decode: one query token per (b,h) against a KV cache of length L.  Same math
  * as the forward with tgt_len = 1 and seqlen_offset = L-1, where the mask row

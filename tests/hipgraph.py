@@ -1,0 +1,27 @@
+"""Stream capture of the library's stream for tests."""
+import ctypes
+
+from deers_amd import rocm
+
+
+class Graph:
+    """What `calls()` enqueues, captured; launch() replays it on the library's stream."""
+
+    def __init__(self, calls):
+        self.hip = ctypes.CDLL("libamdhip64.so")
+        self.stream = ctypes.c_void_p(rocm.load().deers_rocm_stream())
+        self.graph, self.exec = ctypes.c_void_p(), ctypes.c_void_p()
+        assert self.hip.hipStreamBeginCapture(self.stream, 2) == 0  # hipStreamCaptureModeRelaxed
+        try:
+            calls()
+        finally:
+            assert self.hip.hipStreamEndCapture(self.stream, ctypes.byref(self.graph)) == 0
+        assert self.hip.hipGraphInstantiate(ctypes.byref(self.exec), self.graph, None, None, ctypes.c_size_t(0)) == 0
+
+    def launch(self):
+        assert self.hip.hipGraphLaunch(self.exec, self.stream) == 0
+
+    def close(self):
+        rocm.sync()
+        self.hip.hipGraphExecDestroy(self.exec)
+        self.hip.hipGraphDestroy(self.graph)
