@@ -108,18 +108,22 @@ void launch_copy_view(int dtype_f16, const void* src, const int64_t* src_strides
 
 namespace {
 
+// Device memory of the library's own.  Once a captured launch has used it, it stays allocated for the graph's
+// replays, and a larger one is a new one beside it.
+struct Region {
+  void* p = nullptr;
+  size_t bytes = 0;
+  bool captured = false;
+};
+
 struct Runtime {
   bool ready = false;
   int ordinal = -1;
   hipStream_t stream = nullptr;
-  void* workspace = nullptr;  // grows on demand, freed never (process lifetime)
-  size_t workspace_bytes = 0;
+  Region workspace;  // grows on demand, freed never (process lifetime)
   // dS of the f32 backward and its row statistics: grows on demand, its dS up to the limit; given back by
-  // empty_cache, by a lower limit and when an allocation fails.  Once a captured launch has used it, it stays
-  // for the graph's replays, and a larger one is a new one beside it.
-  void* ds = nullptr;
-  size_t ds_bytes = 0;
-  bool ds_captured = false;
+  // empty_cache, by a lower limit and when an allocation fails
+  Region ds;
   int64_t ds_limit = deers::attn_bwd_f32_default_ds_limit();
   rocblas_handle blas = nullptr;  // created by the first matmul, bound to `stream`
   // per (head, 128-row query block) publication flags of the single-launch f16
@@ -228,57 +232,66 @@ bool device_is_gfx950(int ordinal) {
   return std::string(prop.gcnArchName).rfind("gfx950", 0) == 0;
 }
 
-// Workspace that only grows; callers hold g_mu.
-int workspace(size_t bytes, void** out) {
-  if (bytes > g_rt.workspace_bytes) {
-    if (g_rt.workspace) {
-      HIP_TRY(hipStreamSynchronize(g_rt.stream));
-      HIP_TRY(hipFree(g_rt.workspace));
-      g_rt.workspace = nullptr;
-      g_rt.workspace_bytes = 0;
-    }
-    const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-    HIP_TRY(hipMalloc(&g_rt.workspace, want));
-    g_rt.workspace_bytes = want;
-  }
-  *out = g_rt.workspace;
-  return DEERS_ROCM_OK;
-}
-
-// Returns the f32 backward's dS memory to the driver (after the stream has drained), unless a captured
-// graph uses it.
-int release_ds() {
-  if (!g_rt.ds || g_rt.ds_captured) return DEERS_ROCM_OK;
-  HIP_TRY(hipStreamSynchronize(g_rt.stream));
-  HIP_TRY(hipFree(g_rt.ds));
-  g_rt.ds = nullptr;
-  g_rt.ds_bytes = 0;
-  return DEERS_ROCM_OK;
-}
-
-// That memory with at least `bytes`, or null: there is not as much, or a capture, which allows no
-// allocation, would have to get it.
-int ds_memory(size_t bytes, void** out) {
-  *out = nullptr;
+int stream_captures(bool* out) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
-  const bool capturing = cs != hipStreamCaptureStatusNone;
-  if (bytes > g_rt.ds_bytes) {
+  *out = cs != hipStreamCaptureStatusNone;
+  return DEERS_ROCM_OK;
+}
+
+// Returns a region to the driver (after the stream has drained), unless a captured graph uses it.
+int release(Region& r) {
+  if (!r.p || r.captured) return DEERS_ROCM_OK;
+  HIP_TRY(hipStreamSynchronize(g_rt.stream));
+  HIP_TRY(hipFree(r.p));
+  r = Region{};
+  return DEERS_ROCM_OK;
+}
+
+// Gives a region that holds less than `bytes` new memory.
+int grow(Region& r, size_t bytes) {
+  if (int rc = release(r)) return rc;
+  r = Region{};  // a captured graph's memory is its own from here on
+  const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
+  void* p = nullptr;
+  HIP_TRY(hipMalloc(&p, want));
+  r.p = p;
+  r.bytes = want;
+  return DEERS_ROCM_OK;
+}
+
+// Workspace that only grows; callers hold g_mu.
+int workspace(size_t bytes, void** out) {
+  Region& r = g_rt.workspace;
+  bool capturing;
+  if (int rc = stream_captures(&capturing)) return rc;
+  if (bytes > r.bytes) {
+    if (capturing && r.p)
+      return fail(DEERS_ROCM_ERR_ARG,
+                  "the workspace has to grow: call once outside stream capture with this geometry first");
+    if (int rc = grow(r, bytes)) return rc;
+  }
+  r.captured |= capturing;
+  *out = r.p;
+  return DEERS_ROCM_OK;
+}
+
+// The f32 backward's memory with at least `bytes`, or null: there is not as much, or a capture, which allows
+// no allocation, would have to get it.
+int ds_memory(size_t bytes, void** out) {
+  Region& r = g_rt.ds;
+  *out = nullptr;
+  bool capturing;
+  if (int rc = stream_captures(&capturing)) return rc;
+  if (bytes > r.bytes) {
     if (capturing) return DEERS_ROCM_OK;
-    if (int rc = release_ds()) return rc;
-    g_rt.ds = nullptr;  // a captured graph's is its own from here on
-    g_rt.ds_bytes = 0;
-    g_rt.ds_captured = false;
-    const size_t want = (bytes + (size_t(1) << 20) - 1) & ~((size_t(1) << 20) - 1);
-    if (hipMalloc(&g_rt.ds, want) != hipSuccess) {
+    if (grow(r, bytes) != DEERS_ROCM_OK) {
       (void)hipGetLastError();
-      g_rt.ds = nullptr;
       return DEERS_ROCM_OK;
     }
-    g_rt.ds_bytes = want;
   }
-  g_rt.ds_captured |= capturing;
-  *out = g_rt.ds;
+  r.captured |= capturing;
+  *out = r.p;
   return DEERS_ROCM_OK;
 }
 
@@ -539,7 +552,7 @@ static int release_cached_blocks() {
 int deers_rocm_empty_cache(void) {
   std::lock_guard<std::mutex> lock(g_mu);
   NEED_INIT();
-  if (int rc = release_ds()) return rc;
+  if (int rc = release(g_rt.ds)) return rc;
   return release_cached_blocks();
 }
 
@@ -547,7 +560,7 @@ int deers_rocm_set_bwd_workspace_limit(int64_t bytes) {
   std::lock_guard<std::mutex> lock(g_mu);
   NEED_INIT();
   g_rt.ds_limit = bytes < 0 ? deers::attn_bwd_f32_default_ds_limit() : bytes;
-  return (int64_t)g_rt.ds_bytes > g_rt.ds_limit ? release_ds() : DEERS_ROCM_OK;
+  return (int64_t)g_rt.ds.bytes > g_rt.ds_limit ? release(g_rt.ds) : DEERS_ROCM_OK;
 }
 
 int deers_rocm_alloc(size_t bytes, void** out_ptr) {
@@ -569,7 +582,7 @@ int deers_rocm_alloc(size_t bytes, void** out_ptr) {
   hipError_t e = hipMalloc(out_ptr, size);
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
-    if (int rc = release_ds()) return rc;
+    if (int rc = release(g_rt.ds)) return rc;
     if (int rc = release_cached_blocks()) return rc;
     e = hipMalloc(out_ptr, size);
   }
@@ -817,9 +830,8 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   // two-launch form with the flags switched off (epoch 0).  The workspace and the flags must
   // have been grown by an earlier, eager call of the same geometry: capture allows neither
   // the synchronisation nor the allocation.
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
-  const bool capturing = cs != hipStreamCaptureStatusNone;
+  bool capturing;
+  if (int rc = stream_captures(&capturing)) return rc;
   const size_t n_flags = (size_t)(B * H) * (size_t)((T + 127) / 128);
   if (n_flags > g_rt.bwd_ready_len || g_rt.bwd_epoch == INT32_MAX) {
     if (capturing)
@@ -862,9 +874,9 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
 static int decode_counters(int64_t BH, int splits, int** out) {
   *out = nullptr;
   if (splits == 1 || BH > kDecodeCounters || !same_xcd_handover_now()) return DEERS_ROCM_OK;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(g_rt.stream, &cs));
-  if (cs == hipStreamCaptureStatusNone) *out = g_decode_arrivals;
+  bool capturing;
+  if (int rc = stream_captures(&capturing)) return rc;
+  if (!capturing) *out = g_decode_arrivals;
   return DEERS_ROCM_OK;
 }
 
