@@ -148,10 +148,8 @@ struct Runtime {
   void* host_staging = nullptr;
   // sticky "an index was out of range" flag that index kernels raise; read back by the
   // next synchronising call after one of them has been launched
-  int* index_flag = nullptr;
   bool index_flag_armed = false;
   deers::SkinnyPrefetch skinny_next;  // one-shot hint for the next few-rows product (decode_linear_hint)
-  int* skinny_counters = nullptr;  // arrival counters of the few-rows GEMM's K splits (all zero between launches)
   // Block cache behind deers_rocm_alloc / _free.  Every kernel and copy of this library
   // runs on `stream`, in order, so a block handed back by free can be handed out again
   // without waiting for the device: whatever still reads it was enqueued earlier than
@@ -170,6 +168,7 @@ struct Runtime {
 Runtime g_rt;
 std::mutex g_mu;
 constexpr int kDecodeCounters = 1024;  // heads of a decode call that may be split
+constexpr int kSkinnyCounters = 4096;  // column blocks a K-split launch of the few-rows GEMM may have
 constexpr size_t kHostStagingBytes = 4096;
 
 // Device memory that exists without any allocation call: the split partials of
@@ -180,10 +179,11 @@ constexpr size_t kHostStagingBytes = 4096;
 constexpr size_t kScratchBytes = 512 * 1024;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 void* g_scratch_ptr = nullptr;  // device address of `scratch` on g_rt.ordinal
-// Arrival counters of split decode heads, all zero between launches; the same kind of memory, since
-// the entry point that allocates nothing uses them too.
-static __device__ int decode_arrivals[kDecodeCounters];
-int* g_decode_arrivals = nullptr;
+// The same kind of memory, zero from the start, so that a first call needs no allocation and no memset (which
+// a capture would record): arrival counters of split decode heads and of the few-rows GEMM's K splits, all zero
+// between launches, and the index flag.
+static __device__ int decode_arrivals[kDecodeCounters], skinny_arrivals[kSkinnyCounters], index_flag_word;
+int *g_decode_arrivals = nullptr, *g_skinny_arrivals = nullptr, *g_index_flag = nullptr;
 thread_local std::string t_err;
 
 int fail(int code, const char* fmt, ...) {
@@ -427,6 +427,8 @@ int deers_rocm_init(int ordinal) {
   HIP_TRY(hipStreamCreateWithFlags(&g_rt.stream, hipStreamNonBlocking));
   HIP_TRY(hipGetSymbolAddress(&g_scratch_ptr, HIP_SYMBOL(scratch)));
   HIP_TRY(hipGetSymbolAddress((void**)&g_decode_arrivals, HIP_SYMBOL(decode_arrivals)));
+  HIP_TRY(hipGetSymbolAddress((void**)&g_skinny_arrivals, HIP_SYMBOL(skinny_arrivals)));
+  HIP_TRY(hipGetSymbolAddress((void**)&g_index_flag, HIP_SYMBOL(index_flag_word)));
   HIP_TRY(hipHostMalloc(&g_rt.host_staging, kHostStagingBytes, hipHostMallocDefault));
   {
     hipDeviceProp_t prop;
@@ -440,15 +442,10 @@ int deers_rocm_init(int ordinal) {
   return DEERS_ROCM_OK;
 }
 
-// Device memory for the index flag, created by the first call that needs it.
-int index_flag(int** out) {
-  if (!g_rt.index_flag) {
-    HIP_TRY(hipMalloc((void**)&g_rt.index_flag, sizeof(int)));
-    HIP_TRY(hipMemsetAsync(g_rt.index_flag, 0, sizeof(int), g_rt.stream));
-  }
+// The index flag for a kernel that may raise it.
+int* index_flag() {
   g_rt.index_flag_armed = true;
-  *out = g_rt.index_flag;
-  return DEERS_ROCM_OK;
+  return g_index_flag;
 }
 
 // After the stream has drained: reports (once) an out-of-range index seen by any index
@@ -457,11 +454,11 @@ int check_index_flag() {
   if (!g_rt.index_flag_armed) return DEERS_ROCM_OK;
   g_rt.index_flag_armed = false;
   int seen = 0;
-  HIP_TRY(hipMemcpyAsync(&seen, g_rt.index_flag, sizeof(int), hipMemcpyDeviceToHost, g_rt.stream));
+  HIP_TRY(hipMemcpyAsync(&seen, g_index_flag, sizeof(int), hipMemcpyDeviceToHost, g_rt.stream));
   HIP_TRY(hipStreamSynchronize(g_rt.stream));
   if (!seen) return DEERS_ROCM_OK;
   // on the library stream, so that the reset is ordered with the kernels that raise the flag
-  HIP_TRY(hipMemsetAsync(g_rt.index_flag, 0, sizeof(int), g_rt.stream));
+  HIP_TRY(hipMemsetAsync(g_index_flag, 0, sizeof(int), g_rt.stream));
   HIP_TRY(hipStreamSynchronize(g_rt.stream));
   return fail(DEERS_ROCM_ERR_INDEX,
               "an index was out of bounds in an index_select / index_add / cross_entropy call "
@@ -1123,8 +1120,7 @@ int deers_rocm_index_select(int dtype, const void* table, const int64_t* indices
   if (n_rows < 0) return fail(DEERS_ROCM_ERR_ARG, "index_select: negative table size");
   if (n_indices == 0) return DEERS_ROCM_OK;
   if (!table || !indices || !out) return fail(DEERS_ROCM_ERR_ARG, "index_select: null pointer");
-  int* flag = nullptr;
-  if (int rc = index_flag(&flag)) return rc;
+  int* flag = index_flag();
   deers::launch_index_select(dtype == DEERS_ROCM_F16, table, indices, out, n_rows, n_indices,
                              (int)width, flag, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -1139,8 +1135,7 @@ int deers_rocm_index_add(int dtype, const void* src, const int64_t* indices, voi
   if (n_rows < 0) return fail(DEERS_ROCM_ERR_ARG, "index_add: negative destination size");
   if (n_indices == 0) return DEERS_ROCM_OK;
   if (!src || !indices || !dst) return fail(DEERS_ROCM_ERR_ARG, "index_add: null pointer");
-  int* flag = nullptr;
-  if (int rc = index_flag(&flag)) return rc;
+  int* flag = index_flag();
   deers::launch_index_add(dtype == DEERS_ROCM_F16, src, indices, dst, n_rows, n_indices,
                           (int)width, flag, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -1231,8 +1226,7 @@ static int cross_entropy_fwd_locked(const char* what, int dtype, const void* log
   if (!logits || !targets || !row_lse || !loss) return fail(DEERS_ROCM_ERR_ARG, "%s: null pointer", what);
   void* ws = nullptr;  // per-row losses
   if (int rc = workspace((size_t)n_rows * sizeof(float), &ws)) return rc;
-  int* flag = nullptr;
-  if (int rc = index_flag(&flag)) return rc;
+  int* flag = index_flag();
   deers::launch_cross_entropy_fwd(dtype == DEERS_ROCM_F16, logits, targets, row_lse, (float*)ws, loss, dlogits,
                                   n_rows, (int)n_classes, flag, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -1424,8 +1418,7 @@ int deers_rocm_gather(int dtype, const void* src, const int64_t* indices, void* 
   if (int rc = dim_check("gather", left, src_dim, index_len, right)) return rc;
   if (left * index_len * right == 0) return DEERS_ROCM_OK;
   if (!src || !indices || !out) return fail(DEERS_ROCM_ERR_ARG, "gather: null pointer");
-  int* flag = nullptr;
-  if (int rc = index_flag(&flag)) return rc;
+  int* flag = index_flag();
   const int bytes = dtype == DEERS_ROCM_F16 ? 2 : dtype == DEERS_ROCM_F32 ? 4 : 8;
   deers::launch_gather(bytes, src, indices, out, left, src_dim, index_len, right, flag, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -1442,8 +1435,7 @@ int deers_rocm_scatter_add(int dtype, const void* src, const int64_t* indices, v
   if (!src || !indices || !dst) return fail(DEERS_ROCM_ERR_ARG, "scatter_add: null pointer");
   if (left * right > (int64_t)INT32_MAX * 256)
     return fail(DEERS_ROCM_ERR_ARG, "scatter_add: too many columns for one call");
-  int* flag = nullptr;
-  if (int rc = index_flag(&flag)) return rc;
+  int* flag = index_flag();
   deers::launch_scatter_add(dtype == DEERS_ROCM_F16, src, indices, dst, left, dst_dim, index_len, right,
                             flag, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -1610,7 +1602,6 @@ int deers_rocm_matmul_tune(int on) {
 }
 
 constexpr size_t kTuneScratchMax = (size_t)256 << 20;  // largest output a tuned product with an addend may have
-constexpr int kSkinnyCounters = 4096;  // column blocks a K-split launch of the few-rows GEMM may have
 
 // The few-rows GEMM on operands skinny_gemm_takes() accepted; prologue 0 none, 1 rms_norm
 // of x's rows, 2 relu(x)^2.  The caller holds g_mu.
@@ -1621,18 +1612,13 @@ static int skinny_locked(const void* x, int64_t ldx, const void* w, int64_t ldw,
   int splits = (prologue == 1 || !same_xcd_handover_now()) ? 1 : deers::skinny_gemm_splits(n, k);
   void* ws = nullptr;
   if (splits > 1 && (n + 31) / 32 > kSkinnyCounters) splits = 1;
-  if (splits > 1) {
+  if (splits > 1)
     if (int rc = workspace(deers::skinny_gemm_workspace_bytes(n, splits), &ws)) return rc;
-    if (!g_rt.skinny_counters) {  // zero once; the kernel leaves every counter at zero
-      HIP_TRY(hipMalloc(&g_rt.skinny_counters, kSkinnyCounters * sizeof(int)));
-      HIP_TRY(hipMemsetAsync(g_rt.skinny_counters, 0, kSkinnyCounters * sizeof(int), g_rt.stream));
-    }
-  }
   const deers::SkinnyPrefetch next = g_rt.skinny_next;
   g_rt.skinny_next = deers::SkinnyPrefetch{};  // a hint serves one launch
   deers::LaunchScope scope("matmul", g_rt.stream);
   deers::launch_skinny_gemm_f16(x, ldx, w, ldw, y, n, (int)m, (int)n, (int)k, accumulate, prologue, eps, packed,
-                                splits, (float*)ws, g_rt.skinny_counters, next, g_rt.stream);
+                                splits, (float*)ws, g_skinny_arrivals, next, g_rt.stream);
   HIP_TRY(hipGetLastError());
   return DEERS_ROCM_OK;
 }

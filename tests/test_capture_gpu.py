@@ -60,3 +60,38 @@ def test_a_captured_decode_with_splits_replays_when_the_workspace_has_grown(B, H
     finally:
         graph.close()
         noalloc.close()
+
+
+def test_a_captured_few_rows_product_and_lookup_replay():
+    """K split over workgroups (3072 in four) and an index kernel; index 99 is out of range and reported by the
+    eager call that raises the flag, not by the replays of a graph without it."""
+    m, n, k = 5, 768, 3072
+    rng = np.random.default_rng(47)
+    x = rocm.DeviceBuffer.from_numpy(rng.standard_normal((m, k)).astype(np.float16))
+    w = rocm.DeviceBuffer.from_numpy((rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float16))
+    y = rocm.DeviceBuffer((m, n), np.float16)
+    table = rocm.DeviceBuffer.from_numpy(rng.standard_normal((50, 64)).astype(np.float16))
+    good, bad = (rocm.DeviceBuffer.from_numpy(np.array(i, np.int64)) for i in ([3, 49, 0], [3, 99, 0]))
+    rows = rocm.DeviceBuffer((3, 64), np.float16)
+
+    def calls():
+        rocm.decode_linear_raw(np.float16, "plain", 0.0, x.ptr, k, w.ptr, n, y.ptr, False, m, n, k)
+        rocm.index_select_raw(np.float16, table.ptr, good.ptr, rows.ptr, 50, 3, 64)
+
+    graph = Graph(calls)
+    try:
+        calls()
+        want = y.numpy(), rows.numpy()
+        np.testing.assert_array_equal(want[1], table.numpy()[[3, 49, 0]])
+        for _ in range(3):
+            rocm.fill_raw(np.float16, y.ptr, m * n, float("nan"))
+            graph.launch()
+            np.testing.assert_array_equal(y.numpy(), want[0])
+            np.testing.assert_array_equal(rows.numpy(), want[1])
+            rocm.index_select_raw(np.float16, table.ptr, bad.ptr, rows.ptr, 50, 3, 64)
+            with pytest.raises(rocm.RocmError, match="out of bounds"):
+                rocm.sync()
+            calls()
+            np.testing.assert_array_equal(y.numpy(), want[0])
+    finally:
+        graph.close()
