@@ -197,7 +197,7 @@ int deers_rocm_attn_bwd(int dtype,
                         int64_t B, int64_t H, int64_t T, int64_t D, float scale);
 
 /* Device memory that the f32 backward may keep dS in: 4 KiB per 32 x 32 block at or below the
- * diagonal and head (8 x 12 x 1024: 217 MB), of so many heads at a time that it stays within
+ * diagonal and head (8 x 12 x 1024: 198 MiB), of so many heads at a time that it stays within
  * `bytes`; -1: the default of 2.25 GiB, 0: none.  The library takes it at the first call that
  * uses it and keeps it for the next; deers_rocm_empty_cache, a lower limit and a failed
  * deers_rocm_alloc give it back, unless a HIP graph was captured with it: then it stays for the

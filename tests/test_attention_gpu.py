@@ -432,8 +432,8 @@ def test_f32_forms_at_the_edges_of_their_blocks(B, H, T, D):
     x = synth.attention_inputs(f"forms32-{B}-{H}-{T}-{D}", B, H, T, D, np.float32, base_seed=23)
     out = check_case(x, TOL[np.dtype(np.float32)], f"f32 forms {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
     again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
-    for a, b in zip((out[0], out[1], out[3], out[4]), (again[0], again[1], again[3], again[4])):
-        np.testing.assert_array_equal(a, b)  # dQ of the one-pass backward is summed in arrival order
+    for a, b in zip(out, again):
+        np.testing.assert_array_equal(a, b)
 
 
 def test_f32_few_heads_rows_interleaved_over_heads():
@@ -525,3 +525,72 @@ def test_f32_gradients_round_at_the_size_of_the_lse_once(B, H, T, D):
     rel = np.sqrt(off / size)
     say(f"f32 {B}x{H}x{T}x{D}: dq={rel[0]:.2e} dk={rel[1]:.2e} dv={rel[2]:.2e}")
     assert (rel <= 12 * 2.0 ** -24).all(), rel
+
+
+# ---- forms by name: the shapes above were chosen before small launches had forms of their own ----
+
+def takes_split(direction, dtype, B, H, T, D):
+    """The library's own rule: whether this launch takes the 32-row form (for the f32 backward: whether it
+    computes S and dP twice)."""
+    import ctypes
+    i64 = ctypes.c_int64
+    if direction == "bwd" and dtype == np.float32:
+        return rocm.load()["_ZN5deers18attn_bwd_f32_headsEllll"](i64(B * H), i64(T), i64(D), i64(2304 << 20)) == 0
+    rule = rocm.load()[f"_ZN5deers24attn_{direction}_f{16 if dtype == np.float16 else 32}_split_takesElll"]
+    rule.restype = ctypes.c_bool
+    return rule(i64(B * H), i64(T), i64(D))
+
+
+@pytest.mark.parametrize("dtype,B,H,T,D", [
+    (np.float16, 11, 11, 300, 64), (np.float16, 8, 13, 300, 128), (np.float16, 4, 19, 1000, 32),
+    (np.float16, 9, 13, 1500, 64),                              # tile-pipelined, then block-pipelined forward
+    (np.float32, 17, 4, 990, 64), (np.float32, 13, 8, 500, 128)])
+def test_128_row_kernels_rows_interleaved_over_heads(dtype, B, H, T, D):
+    """[B,T,H,D] memory under the logical [B,H,T,D], every operand, in launches that fill the device (f32: the
+    backward with dS in memory): same bits as compact."""
+    assert not takes_split("fwd", dtype, B, H, T, D) and not takes_split("bwd", dtype, B, H, T, D)
+    strided_equals_compact(dtype, B, H, T, D)
+
+
+@pytest.mark.parametrize("B,H,T,D", [(4, 10, 500, 32), (4, 8, 500, 64), (3, 8, 500, 128)])
+def test_f32_backward_with_ds_in_memory_rows_interleaved_over_heads(B, H, T, D):
+    assert not takes_split("bwd", np.float32, B, H, T, D)
+    strided_equals_compact(np.float32, B, H, T, D)
+
+
+def strided_equals_compact(dtype, B, H, T, D):
+    x = synth.attention_inputs(f"strided-{np.dtype(dtype).name}-{B}-{H}-{T}-{D}", B, H, T, D, dtype, base_seed=51)
+    want = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    st = (T * H * D, D, H * D, 1)
+    bufs = {n: rocm.DeviceBuffer.from_numpy(np.ascontiguousarray(x[n].transpose(0, 2, 1, 3))) for n in x}
+    outs = {n: rocm.DeviceBuffer((B, T, H, D), dtype) for n in ("o", "dq", "dk", "dv")}
+    lse = rocm.DeviceBuffer((B, H, T), np.float32)
+    scale = rocm.default_scale(D)
+    rocm.attn_fwd_raw(dtype, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, B, H, T, D, scale,
+                      q_strides=st, k_strides=st, v_strides=st, o_strides=st)
+    rocm.attn_bwd_raw(dtype, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, bufs["do"].ptr,
+                      outs["dq"].ptr, outs["dk"].ptr, outs["dv"].ptr, B, H, T, D, scale,
+                      strides={n: st for n in ("q", "k", "v", "o", "do", "dq", "dk", "dv")})
+    for name, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:])):
+        np.testing.assert_array_equal(outs[name].numpy().transpose(0, 2, 1, 3), ref, err_msg=name)
+    np.testing.assert_array_equal(lse.numpy(), want[1])
+    one = (slice(B - 1, B), slice(H - 1, H))
+    o = oracle.attn_fwd(x["q"][one], x["k"][one], x["v"][one])
+    refs = (o, *oracle.attn_bwd(x["q"][one], x["k"][one], x["v"][one], x["do"][one]))
+    for name, got, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:]), refs):
+        assert max_err(got[one], ref) <= TOL[np.dtype(dtype)], name
+
+
+def test_f16_backward_of_heads_dealt_to_all_xcds_at_head_width_128():
+    """Nine heads of a long walk: the blocks of the ninth go to every XCD, in two launches."""
+    B, H, T, D = 1, 9, 4161, 128
+    assert not takes_split("bwd", np.float16, B, H, T, D)
+    x = synth.attention_inputs("even-bwd-128", B, H, T, D, np.float16, base_seed=53)
+    rocm.profile_enable(True)
+    out = check_case(x, TOL[np.dtype(np.float16)], "nine heads of 4161 x 128", heads=(slice(0, 1), slice(7, 9)))
+    names = rocm.profile_collect()
+    rocm.profile_enable(False)
+    assert "attn_bwd_f16_dq" in names and "attn_bwd_f16_dkdv" in names
+    again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for a, b in zip(out, again):
+        np.testing.assert_array_equal(a, b)

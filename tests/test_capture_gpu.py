@@ -95,3 +95,30 @@ def test_a_captured_few_rows_product_and_lookup_replay():
             np.testing.assert_array_equal(y.numpy(), want[0])
     finally:
         graph.close()
+
+
+@pytest.mark.parametrize("dtype,B,H,T,D", [(np.float16, 7, 12, 300, 64), (np.float16, 4, 11, 257, 128),
+                                           (np.float16, 2, 3, 300, 64)])
+def test_a_captured_f16_backward_replays(dtype, B, H, T, D):
+    """The first two are launches whose kernels hand statistics over: captured, they are two launches without
+    flags (a replay could be given no fresh epoch); the last is the 32-row form.  Eager backwards of the same and
+    of another geometry between the replays move the epochs on."""
+    x = synth.attention_inputs(f"cap-bwd-{B}-{H}-{T}-{D}", B, H, T, D, dtype, base_seed=45)
+    want = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    ins = [rocm.DeviceBuffer.from_numpy(a) for a in (x["q"], x["k"], x["v"], want[0], want[1], x["do"])]
+    grads = [rocm.DeviceBuffer((B, H, T, D), dtype) for _ in range(3)]
+
+    def backward():
+        rocm.attn_bwd_raw(dtype, *(b.ptr for b in ins + grads), B, H, T, D, rocm.default_scale(D))
+
+    graph = Graph(backward)
+    try:
+        for between in (lambda: None, backward, grow_the_workspace, backward):
+            between()
+            for g in grads:
+                rocm.fill_raw(dtype, g.ptr, B * H * T * D, float("nan"))
+            graph.launch()
+            for got, ref in zip(grads, want[2:]):
+                np.testing.assert_array_equal(got.numpy(), ref)
+    finally:
+        graph.close()

@@ -1,4 +1,4 @@
-"""BASELINE configs[4] at its real size: the f32 attention kernels at B=8 H=12 T=1024 D=64 and
+"""The f32 attention kernels at B=8 H=12 T=1024 D=64 and
 the whole GPT training step at 12 layers x 12 heads x 768, vocabulary 50257, T=1024, B=8.
 
 The reference's counterpart is its training loop (examples/tinystories_train.rs:188-218) and
@@ -49,11 +49,8 @@ def test_f32_attention_at_config5_size_matches_oracle_and_is_reproducible():
     np.testing.assert_array_equal(o[:, :, 0], v[:, :, 0])  # the first query sees only itself
     assert np.max(np.abs(dq[:, :, 0])) <= 1e-5             # ... so dS = P (dP - delta) cancels to rounding
     o2, lse2, dq2, dk2, dv2 = rocm.attn_fwd_bwd(q, k, v, do)
-    for a, b_ in ((o, o2), (lse, lse2), (dk, dk2), (dv, dv2)):
-        np.testing.assert_array_equal(a, b_)               # bit-reproducible
-    # dQ adds the contributions of its (up to 8) key blocks with f32 atomics in arrival order:
-    # reproducible to f32 rounding of that sum
-    assert np.max(np.abs(dq - dq2)) <= 1e-6
+    for a, b_ in ((o, o2), (lse, lse2), (dq, dq2), (dk, dk2), (dv, dv2)):
+        np.testing.assert_array_equal(a, b_)               # every sum in a fixed order
 
 
 def test_f32_attention_with_ragged_heads_and_several_tiles_per_workgroup():
@@ -78,8 +75,8 @@ def test_f32_attention_with_ragged_heads_and_several_tiles_per_workgroup():
         for n, e in errs.items():
             assert e <= 1e-4, f"(b={b}, h={h}) {n}: max abs err {e:.3e} > 1e-4"
     np.testing.assert_array_equal(o[:, :, 0], v[:, :, 0])
-    o2, lse2, _, dk2, dv2 = rocm.attn_fwd_bwd(q, k, v, do)
-    for a, b_ in ((o, o2), (lse, lse2), (dk, dk2), (dv, dv2)):
+    o2, lse2, dq2, dk2, dv2 = rocm.attn_fwd_bwd(q, k, v, do)
+    for a, b_ in ((o, o2), (lse, lse2), (dq, dq2), (dk, dk2), (dv, dv2)):
         np.testing.assert_array_equal(a, b_)
 
 

@@ -227,3 +227,25 @@ def test_decode_with_two_workgroups_on_a_compute_unit(gpu, B, H, L, D):
     assert np.max(np.abs(outs[0].astype(np.float64) - want)) <= 5e-3
     for other in outs[1:]:
         np.testing.assert_array_equal(outs[0], other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,T,D", [(14, 11, 300, 32), (6, 9, 520, 32), (7, 12, 300, 64), (4, 11, 257, 128),
+                                     (2, 9, 700, 128)])
+def test_backward_kernels_with_a_hand_over_give_the_same_bits_in_two_launches(gpu, B, H, T, D):
+    """Launches beyond the 32-row form, which hands nothing over, at every head width; the kernels are named by
+    what they were launched as."""
+    x = synth.attention_inputs(f"handover128-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=18)
+    outs = []
+    for mode, names in ((rocm.HANDOVER_SAME_XCD, {"attn_bwd_f16"}),
+                        (rocm.HANDOVER_STREAM_ORDER, {"attn_bwd_f16_dq", "attn_bwd_f16_dkdv"})):
+        rocm.set_handover_mode(mode)
+        rocm.profile_enable(True)
+        outs.append(rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"]))
+        assert set(rocm.profile_collect()) - {"attn_fwd_f16"} == names
+        rocm.profile_enable(False)
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)
+    one = (slice(B - 1, B), slice(H - 1, H))
+    for got, want in zip(outs[0][2:], oracle.attn_bwd(*(x[n][one] for n in ("q", "k", "v", "do")))):
+        assert np.max(np.abs(got[one].astype(np.float64) - want)) <= 5e-3
