@@ -191,7 +191,7 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_f32_dq_kernel(BwdParams p, in
   for (int kb = wave; kb <= qb; kb += W) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      async_load16_to_lds(ds_row + (int64_t)kb * kDsBlock + 1024 * i, lane * 16, lds + C::BB + i * kDsPitch);
+      async_load16_to_lds(ds_row + (int64_t)kb * kDsBlock + 1024 * i, lane * 16, lds, C::BB + i * kDsPitch);
     load_block<D>(K, skt, 32 * kb, T, lds, lane);
     wait_vmcnt<0>();
     floatx16 x;

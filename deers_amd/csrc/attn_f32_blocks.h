@@ -59,12 +59,12 @@ __device__ __forceinline__ void load_block(const float* base, int row_stride, in
     asm volatile("" : "+s"(step));
     const uint32_t off = (uint32_t)lane_row * (uint32_t)row_stride * 4 + col_off;
 #pragma unroll
-    for (int i = 0; i < C::NI; ++i, row += step) async_load16_to_lds(row, off, dst + i * C::GP);
+    for (int i = 0; i < C::NI; ++i, row += step) async_load16_to_lds(row, off, dst, i * C::GP);
   } else {
 #pragma unroll
     for (int i = 0; i < C::NI; ++i)
       async_load16_to_lds(row, (uint32_t)min(i * C::kLoadStep + lane_row, T - 1 - r0) * (uint32_t)row_stride * 4 + col_off,
-                          dst + i * C::GP);
+                          dst, i * C::GP);
   }
 }
 

@@ -69,12 +69,12 @@ __device__ __forceinline__ void split_load_block(const half_t* base, int row_str
 #pragma unroll
     for (int i = 0; i < C::NI; ++i)
       async_load16_to_lds(row + (int64_t)(i * RPL) * row_stride,
-                          row_off + 16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(i * RPL + lane_row)), dst + i * 1024);
+                          row_off + 16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(i * RPL + lane_row)), dst, i * 1024);
   } else {
 #pragma unroll
     for (int i = 0; i < C::NI; ++i)
       async_load16_to_lds(base, (uint32_t)min(r0 + i * RPL + lane_row, T - 1) * (uint32_t)row_stride * 2 +
-                                    16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(i * RPL + lane_row)), dst + i * 1024);
+                                    16 * ((lane % C::CH) ^ lds_swizzle<C::CH>(i * RPL + lane_row)), dst, i * 1024);
   }
 }
 

@@ -463,7 +463,7 @@ __global__ __launch_bounds__(kRegBlockOf(GROUP), NLDS ? 8 : 1) void cross_entrop
 #pragma unroll
     for (int u = 0; u < NLDS; ++u) {  // chunks past the row's end repeat its last one and are patched below
       const int chunk = min(t + (NREG + u) * GROUP, n_chunks - 1);
-      async_load16_to_lds_nt(geo.base_of(row), (uint32_t)chunk * 16, wave_lds + u * GROUP * 16);
+      async_load16_to_lds_nt(geo.base_of(row), (uint32_t)chunk * 16, wave_lds, u * GROUP * 16);
     }
   }
   u32x4 c[NREG];

@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
 #pragma unroll
     for (int i = 0; i < kSkStepsPerChunk; ++i) {
       const int k0 = k_begin + (chunk * kSkStepsPerChunk + i) * 16;
-      async_load16_to_lds(w_base + (int64_t)k0 * ldw, w_lane_off, dst + i * 1024);
-      async_load16_to_lds(x + k_begin + chunk * 64, x_lane_off[i], dst + 4096 + i * 1024);
+      async_load16_to_lds(w_base + (int64_t)k0 * ldw, w_lane_off, dst, i * 1024);
+      async_load16_to_lds(x + k_begin + chunk * 64, x_lane_off[i], dst, 4096 + i * 1024);
     }
   };
   // the addend of the columns this lane will hold at the end: requested first, so that its trip
