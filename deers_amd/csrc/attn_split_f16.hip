@@ -530,7 +530,11 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 384 x 256 x 32 24.1 -> 18.9).  Longer walks gain while the device is not full: forward 15 x 777 x 128 18.3 ->
 // 12.6, 36 x 1024 x 64 17.4 -> 16.2, 16 x 2048 x 128 38.7 -> 36.7 (48 x 1024 x 64 18.1 -> 18.5); backward, which streams
 // three operands per block, 3 x 4096 x 64 86 -> 47, 12 x 1024 x 64 24.1 -> 21.4, 24 x 400 x 128 25.5 -> 21.4 (16 x 2048 x
-// 64 36.4 -> 37.6, 24 x 1024 x 64 27.6 -> 27.7).
+// 64 36.4 -> 37.6, 24 x 1024 x 64 27.6 -> 27.7).  The backward's line at head width 128, 128-row kernels / these, us,
+// u in parentheses: below 28 blocks 24 x 512 (768) 27.7 / 23.0, 16 x 768 (768) 32.7 / 29.4, 18 x 700 (792, in four
+// waves) 31.3 / 47.6; from 28 on 11 x 896 (616) 35.0 / 32.8, 12 x 896 (672) 35.2 / 36.5, 9 x 1024 (576) 37.0 / 32.9,
+// 11 x 1024 (704) 37.3 / 38.8, 8 x 1280 (640) 42.7 / 46.2; from 48 on 7 x 1536 (672) 48.5 / 47.5, 8 x 1536 (768) 49.2 / 56.9,
+// 6 x 2048 (768) 60.3 / 63.7, 4 x 3072 (768) 87.3 / 93.9; from 128 on 3 x 4096 (768) 171 / 106, 2 x 6144 (768) 247 / 167.
 struct SplitSize {
   int64_t nb, u;
   SplitSize(int64_t BH, int64_t T, int64_t D) : nb((T + 31) / 32), u(BH * nb * D / 64) {}
@@ -541,7 +545,8 @@ bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
 }
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   const SplitSize z(BH, T, D);
-  return z.u <= (z.nb <= 4 ? 3200 : z.nb <= 8 ? 1600 : z.nb <= 16 || D == 128 ? 768 : 448);
+  if (D == 128 && z.nb > 8) return z.u <= (z.nb < 28 || z.nb >= 128 ? 768 : z.nb < 48 ? 624 : 672);
+  return z.u <= (z.nb <= 4 ? 3200 : z.nb <= 8 ? 1600 : z.nb <= 16 ? 768 : 448);
 }
 static int fwd_waves(const SplitSize& z) {
   const int64_t most = z.u <= 320 ? z.nb : z.u <= 1200 ? z.nb / 2 : z.nb / 4;
