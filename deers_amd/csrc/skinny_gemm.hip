@@ -291,19 +291,24 @@ bool skinny_gemm_takes(int64_t m, int64_t n, int64_t k, int64_t ldx, int64_t ldw
   return true;
 }
 
-// Number of K splits per column block for this shape.  A split costs a trip through the
-// workspace and the arrival counter (~1.5 us), so it only pays when one workgroup's share
-// of K is long: every split keeps at least 768 of K (32x768x3072: 12.0 us unsplit, 8.5 us
-// in four splits; 32x768x768: 4.0 us unsplit, 5.6 us in three).
+// Number of K splits per column block for this shape.  A split costs a trip through the workspace and
+// the arrival counter, 0.5 to 0.9 us (1024 x 1024: 4.17 us unsplit, 4.91 in two; 768 x 768 3.81, 4.53 in three;
+// 1280 x 1280 4.80, 5.79 in five), and saves the time in which a workgroup streams what it gives away.  That
+// pays from K = 1536 on with shares of 512 or more (packed weights, one row; 32 rows alike): 1536 x 768 5.00 us
+// unsplit, 5.19 in two, 4.97 in three; 2048 x 512 5.65, 5.34 in two, 4.93 in four; 2560 x 640 6.66, 6.01 in two, 5.51 in
+// five; 3072 x 768 7.45, 5.80 in three, 5.55 in four, 5.95 in six; 4096 x 1024 8.91, 6.35 in four, 7.22 in eight.
+// With 48 column blocks or more the device streams fast enough up to K = 2048 (1536 x 1536 5.21 unsplit, 5.61 in
+// two; 1536 x 2304 5.22, 5.85; 2048 x 2048 5.98, 6.20; but 3072 x 2304 7.67, 7.11), and with 96 at any.
 int skinny_gemm_splits(int64_t n, int64_t k) {
   const int64_t col_blocks = (n + 31) / 32, units = k / 256;  // a split owns whole 256-deep units
+  if (units < 6 || col_blocks >= (units <= 8 ? 48 : 96)) return 1;
   int best = 1;
-  for (int sp = 2; sp <= units / 3 && sp <= 16; ++sp)
+  for (int sp = 2; sp <= units / 2 && sp <= 16; ++sp)
     if (units % sp == 0) {
       best = sp;
       if (col_blocks * sp >= 96) break;
     }
-  return col_blocks >= 96 ? 1 : best;
+  return best;
 }
 size_t skinny_gemm_workspace_bytes(int64_t n, int splits) {
   return splits > 1 ? (size_t)((n + 31) / 32) * splits * 2 * 64 * 8 * sizeof(float) : 0;

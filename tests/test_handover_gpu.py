@@ -249,3 +249,26 @@ def test_backward_kernels_with_a_hand_over_give_the_same_bits_in_two_launches(gp
     one = (slice(B - 1, B), slice(H - 1, H))
     for got, want in zip(outs[0][2:], oracle.attn_bwd(*(x[n][one] for n in ("q", "k", "v", "do")))):
         assert np.max(np.abs(got[one].astype(np.float64) - want)) <= 5e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,n", [(1536, 768), (2048, 512), (2560, 640), (1536, 1536), (1280, 256)])
+@pytest.mark.parametrize("m", [1, 32])
+def test_few_rows_products_in_shares_of_512(gpu, m, k, n):
+    """K in three, four and five shares, and unsplit on the other side of either line: against 64 bits, the
+    stream-order form (unsplit) within the rounding of two fixed orders, the same bits again."""
+    rng = np.random.default_rng(k + n + m)
+    x = rng.standard_normal((m, k)).astype(np.float16)
+    w = (rng.standard_normal((k, n)) / np.sqrt(k)).astype(np.float16)
+    want = x.astype(np.float64) @ w.astype(np.float64)
+    dx, dw = rocm.DeviceBuffer.from_numpy(x), rocm.DeviceBuffer.from_numpy(w)
+    outs = []
+    for mode in (rocm.HANDOVER_SAME_XCD, rocm.HANDOVER_STREAM_ORDER, rocm.HANDOVER_SAME_XCD):
+        rocm.set_handover_mode(mode)
+        dy = rocm.DeviceBuffer.from_numpy(np.full((m, n), np.nan, np.float16))
+        rocm.decode_linear_raw(np.float16, "plain", 0.0, dx.ptr, k, dw.ptr, n, dy.ptr, False, m, n, k)
+        outs.append(dy.numpy().astype(np.float64))
+    # one rounding to f16 (2^-11 relative; values up to 4: 2^-9 at most) on top of f32 sums
+    assert np.max(np.abs(outs[0] - want)) <= 2.0 ** -9 + 1e-4
+    assert np.max(np.abs(outs[1] - want)) <= 2.0 ** -9 + 1e-4
+    np.testing.assert_array_equal(outs[0], outs[2])
