@@ -107,11 +107,8 @@ static void launch_bwd_f16_d(const BwdParams& p, int B, int mode, hipStream_t st
   const Kernel kernel = attn_bwd_f16_bp_kernel<D>;
   const size_t lds = BwdBpCfg<D>::kLds;
   static bool attr_set = false;  // launches are serialised by the caller
-  if (!attr_set) {
-    if (lds > 64 * 1024)
-      (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    attr_set = true;
-  }
+  if (!attr_set) allow_lds(kernel, lds);
+  attr_set = true;
   if (mode == 2) {  // test hook: consumers only, so that their bounded wait runs out
     LaunchScope scope("attn_bwd_f16_dkdv", stream);
     hipLaunchKernelGGL(kernel, dim3(per_role), dim3(256), lds, stream, p, BH, n_blocks, heads_per_xcd, per_role, 0);

@@ -34,10 +34,6 @@
 
 namespace deers {
 
-#ifndef ZERO16
-#define ZERO16 floatx16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}
-#endif
-
 // Hook for a timestamp-tracing build of these bodies; expands to nothing in the library.
 #ifndef DEERS_TRACE_POINT
 #define DEERS_TRACE_POINT(slot)

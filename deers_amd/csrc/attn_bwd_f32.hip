@@ -107,13 +107,13 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f3
 
   floatx16 dk[DB], dv[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16;
   for (; qb < n_blocks; qb += W) {
     const bool more = qb + W < n_blocks;
     wait_vmcnt<C::NI>();  // dS written, statistics, Q
-    floatx16 s = product<D>(q_blk, kf, ZERO16S, lane);
+    floatx16 s = product<D>(q_blk, kf, ZERO16, lane);
     wait_vmcnt<0>();  // dO
-    floatx16 dp = product<D>(do_blk, vf, ZERO16S, lane);
+    floatx16 dp = product<D>(do_blk, vf, ZERO16, lane);
     s += stat_rows(stat, g);
     dp += stat_rows(stat + 32, g);
     if (qb == kb) {
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_f32_dq_kernel(BwdParams p, in
 
   floatx16 acc[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) acc[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) acc[db] = ZERO16;
   for (int kb = wave; kb <= qb; kb += W) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)

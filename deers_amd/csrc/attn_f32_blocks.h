@@ -13,8 +13,6 @@
 
 namespace deers {
 
-#define ZERO16S floatx16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}
-
 template <int D>
 struct Split32 {
   static constexpr int KH = D / 2;         // elements of D a lane contracts over
@@ -38,12 +36,6 @@ struct Split32 {
 // rows which a quarter of a wave reads together at most two share banks; at 32 it has eight rows in
 // sequence, four of which do: what a load fetches is then 1 KB in sequence (96 x 1024 x 32 backward 166 us
 // against 171).
-
-// Before the loads into a block that earlier LDS reads of this wave have used: those have returned.
-__device__ __forceinline__ void settle_lds_reads() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-}
 
 // Requests rows r0 .. r0 + 31 (rows past T - 1 read row T - 1) of a [T, D] matrix into the block at
 // LDS address `dst`.
@@ -175,12 +167,6 @@ __device__ __forceinline__ floatx16 stat_rows(const float* stat, int g) {
     for (int e = 0; e < 4; ++e) v[4 * r4 + e] = a[e];
   }
   return v;
-}
-
-template <typename Kernel>
-inline void allow_lds(Kernel kernel, size_t bytes) {
-  if (bytes > 64 * 1024)
-    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 }  // namespace deers

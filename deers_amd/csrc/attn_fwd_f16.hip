@@ -36,7 +36,6 @@
 // XOR-swizzled by 16-byte chunk.  One barrier per iteration.
 #include <algorithm>
 #include <map>
-#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -431,50 +430,42 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_f16_kernel(FwdParams p, int B
 }
 
 
-// Builds the TileOrder of a launch whose workgroups are all resident at once (their
+// What the device holds of the block-pipelined kernel: CUs of an XCD and workgroups of a CU.
+template <int D>
+static void resident_capacity(int* n_cu, int* per_cu) {
+  static int cus = 0, wgs = 0;  // launches are serialised by the caller
+  if (cus == 0) {
+    int dev = 0, all = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&all, hipDeviceAttributeMultiprocessorCount, dev);
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&wgs, attn_fwd_f16_bp_kernel<D>, 256, BpCfg<D>::kLds);
+    cus = std::max(all / 8, 1);
+  }
+  *n_cu = cus;
+  *per_cu = wgs;
+}
+
+// Builds the TileOrder of a launch of whole heads per XCD whose workgroups are all resident at once (their
 // number does not exceed what the chip holds).  Workgroup position p of an XCD (id / 8)
 // lands on CU p % cus_per_xcd when the dispatcher fills an empty chip, so positions p,
 // p + cus, p + 2 cus share a CU and its issue ports: tiles are dealt longest first to the
 // CU with the smallest total that still has a free slot.  Returns nullptr when the tiles
 // do not all fit (then the dispatcher's own longest-first hand-out is the better order).
-// *use_resident_kernel tells whether the launch is large enough for the plain kernel at
-// all.  Built at the first launch of a geometry and kept on the host for the life of the
+// Built at the first launch of a geometry and kept on the host for the life of the
 // process; no device memory.
 template <int D>
-static const TileOrder* resident_order(int heads_per_xcd, int T, bool* use_resident_kernel) {
-  struct Key {
-    int dev, heads, T;
-    bool operator<(const Key& o) const { return std::tie(dev, heads, T) < std::tie(o.dev, o.heads, o.T); }
-  };
-  struct Entry {
-    bool usable = false;    // the table is filled in
-    bool resident = false;  // the launch is large enough for the plain kernel
-    TileOrder order{};
-  };
-  static std::map<Key, Entry> cache;  // launches are serialised by the caller
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  const Key key{dev, heads_per_xcd, T};
-  auto it = cache.find(key);
-  if (it != cache.end()) {
-    *use_resident_kernel = it->second.resident;
-    return it->second.usable ? &it->second.order : nullptr;
-  }
-  Entry& entry = cache[key];
-  *use_resident_kernel = false;
-  int cus = 0, per_cu = 0;
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_fwd_f16_bp_kernel<D>, 256,
-                                                     BpCfg<D>::kLds);
-  const int n_cu = std::max(cus / 8, 1);
+static const TileOrder* resident_order(int heads_per_xcd, int T, int n_cu, int per_cu) {
   const int n_qtiles = (T + kFwdBM - 1) / kFwdBM;
   const int n_items = heads_per_xcd * n_qtiles;
-  // launches that fit the pipelined kernel's two workgroups per CU are faster there
-  // (head width 128: both kernels hold two workgroups per CU and the block-pipelined one is the
-  // faster from the same size on: 1x16x8192x128 267 against 296 us)
-  entry.resident = (D == 128 ? per_cu >= 2 : per_cu > 2) && n_items > 2 * n_cu;
-  *use_resident_kernel = entry.resident;
-  if (!entry.resident || n_items > n_cu * per_cu || n_items > kMaxResidentTiles) return nullptr;
+  if (n_items > n_cu * per_cu || n_items > kMaxResidentTiles) return nullptr;
+  struct Entry {
+    bool usable = false;  // the table is filled in
+    TileOrder order{};
+  };
+  static std::map<std::pair<int, int>, Entry> cache;  // launches are serialised by the caller
+  const auto found = cache.find({heads_per_xcd, T});
+  if (found != cache.end()) return found->second.usable ? &found->second.order : nullptr;
+  Entry& entry = cache[{heads_per_xcd, T}];
   std::vector<long> load(n_cu, 0);
   std::vector<int> used(n_cu, 0);
   std::vector<char> filled((size_t)n_items, 0);
@@ -510,12 +501,8 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
   const size_t lds = FwdCfg<D>::kLds;
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) {
-    if (lds > 64 * 1024)
-      (void)hipFuncSetAttribute((const void*)attn_fwd_f16_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds);
-    if (BpCfg<D>::kLds > 64 * 1024)
-      (void)hipFuncSetAttribute((const void*)attn_fwd_f16_bp_kernel<D>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)BpCfg<D>::kLds);
+    allow_lds(attn_fwd_f16_kernel<D>, lds);
+    allow_lds(attn_fwd_f16_bp_kernel<D>, BpCfg<D>::kLds);
     attr_set = true;
   }
   LaunchScope scope("attn_fwd_f16", stream);
@@ -523,20 +510,21 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
     // More tiles than the tile-pipelined kernel holds at once (two workgroups per CU): the
     // block-pipelined kernel, at three workgroups per CU for head widths 32 and 64.  While they all fit, every workgroup
     // is resident from the start, placed for even CU totals, and nothing is left to a tail of
-    // late, short workgroups; beyond that the dispatcher hands out each XCD's list longest
-    // first.  Smaller launches are faster on the tile-pipelined kernel (2x12x2048x64: 33.6
-    // against 34.6 us).
-    bool use_resident = false;
-    const TileOrder* table = resident_order<D>((BH + 7) / 8, p.T, &use_resident);
-    if (even) table = nullptr;  // the table places whole heads
-    static const TileOrder kNoTable = [] {
-      TileOrder t{};
-      t.code[0] = -1;
-      return t;
-    }();
-    if (const TileOrder* order = use_resident ? (table ? table : &kNoTable) : nullptr) {
+    // late, short workgroups; beyond that, and where the tiles of some heads are dealt to all XCDs, the dispatcher
+    // hands out each XCD's list longest first.  Smaller launches are faster on the tile-pipelined kernel (2x12x2048x64:
+    // 33.6 against 34.6 us).  Head width 128: both kernels hold two workgroups per CU and the block-pipelined one is
+    // the faster from the same size on (1x16x8192x128 267 against 296 us).
+    int n_cu, per_cu;
+    resident_capacity<D>(&n_cu, &per_cu);
+    if ((D == 128 ? per_cu >= 2 : per_cu > 2) && (BH + 7) / 8 * n_qtiles > 2 * n_cu) {
+      static const TileOrder kNoTable = [] {
+        TileOrder t{};
+        t.code[0] = -1;
+        return t;
+      }();
+      const TileOrder* order = even ? nullptr : resident_order<D>(heads_per_xcd, p.T, n_cu, per_cu);
       hipLaunchKernelGGL(attn_fwd_f16_bp_kernel<D>, dim3(grid), dim3(256), BpCfg<D>::kLds,
-                         stream, p, BH, n_qtiles, heads_per_xcd, *order);
+                         stream, p, BH, n_qtiles, heads_per_xcd, order ? *order : kNoTable);
       return;
     }
   }

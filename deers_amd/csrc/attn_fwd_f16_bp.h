@@ -11,10 +11,6 @@ namespace deers {
 constexpr int kFwdBM = 128;  // query rows per workgroup
 constexpr int kFwdBN = 64;   // key/value rows per tile
 
-#ifndef ZERO16
-#define ZERO16 floatx16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}
-#endif
-
 template <int D>
 struct FwdCfg {
   // prefetch distance in tiles; D = 128 keeps one tile less in flight so that two

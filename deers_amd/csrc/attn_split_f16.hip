@@ -47,14 +47,6 @@ __device__ __forceinline__ void settle_loads() {
   asm volatile("" ::: "memory");
 }
 
-// Before the loads into a block that earlier LDS reads of this wave have used: those have returned.
-__device__ __forceinline__ void settle_lds_reads() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-  asm volatile("" ::: "memory");
-}
-
-#define ZERO16S floatx16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}
-
 // Requests rows r0 .. r0 + 31 (rows past T - 1 read row T - 1) of a [T, D] matrix into the 32-row
 // block at LDS address `dst`: 16-byte chunks, swizzled.
 template <int D>
@@ -220,7 +212,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
 
   floatx16 oacc[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) oacc[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) oacc[db] = ZERO16;
   float m = -INFINITY, l = 0.f;
   for (; kb <= qb; kb += W) {
     const bool more = kb + W <= qb;
@@ -228,7 +220,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
       settle_loads();  // K and V of this block
     else
       wait_vmcnt<C::NI>();  // K; V's block may be on its way
-    floatx16 s = ZERO16S;
+    floatx16 s = ZERO16;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       half8 k;
@@ -344,7 +336,7 @@ __device__ __forceinline__ void split_dq_body(const BwdParams& p, int bh, int qb
 
   floatx16 dq[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dq[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) dq[db] = ZERO16;
   for (uint32_t slot = 0; kb <= qb; kb += W, slot ^= C::BB) {
     settle_loads();
     floatx16 s, dp;
@@ -412,7 +404,7 @@ __device__ __forceinline__ void split_dkdv_body(const BwdParams& p, int bh, int 
 
   floatx16 dk[DB], dv[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16;
   for (uint32_t slot = 0; qb < n_blocks; qb += W, slot ^= 2 * C::BB) {
     settle_loads();
     const uint32_t q_blk = ring + slot, do_blk = q_blk + C::BB;
@@ -483,12 +475,6 @@ __global__ __launch_bounds__(64 * W, D == 128 ? 1 : 2) void attn_bwd_f16_split_k
     split_dq_body<D, W>(first_argument<BwdParams>(), bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
   else
     split_dkdv_body<D, W>(first_argument<BwdParams>(), bh, rank >> 1, n_blocks, smem, wave, lane);
-}
-
-template <typename Kernel>
-void allow_lds(Kernel kernel, size_t bytes) {
-  if (bytes > 64 * 1024)
-    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 template <int D, int W, bool KREGS>

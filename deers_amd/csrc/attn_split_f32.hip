@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
 
   floatx16 oacc[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) oacc[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) oacc[db] = ZERO16;
   // The reference m of a row's exponentials is the maximum of its first block, and moves when a later
   // score exceeds it by more than 2^8: `ref` is -m in the layout of the products, which start from it, so
   // that the usual stage has no subtraction and no rescaling (some 60 of 110 vector instructions).
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
   constexpr bool kLazy = D < 128;
   const bool any = kb <= qb;
   bool first = true;
-  floatx16 ref = ZERO16S;
+  floatx16 ref = ZERO16;
   float m = kLazy ? 0.f : -INFINITY, l = 0.f;
   for (; kb <= qb; kb += W) {
     const bool more = kb + W <= qb;
@@ -186,12 +186,12 @@ __device__ __forceinline__ void split32_dq(const BwdParams& p, int bh, int qb, c
 
   floatx16 dq[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dq[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) dq[db] = ZERO16;
   for (; kb <= qb; kb += W) {
     const bool more = kb + W <= qb;
     wait_vmcnt<C::NI>();  // V; K's block may be on its way
     // (from zero, not from the row statistics: see the error figures in attn_bwd_f32.hip)
-    const floatx16 dp = product<D>(v_blk, dof, ZERO16S, lane);
+    const floatx16 dp = product<D>(v_blk, dof, ZERO16, lane);
     if (more) {
       settle_lds_reads();
       load_block<D>(V, svt, 32 * (kb + W), T, v_blk, lane);
@@ -199,7 +199,7 @@ __device__ __forceinline__ void split32_dq(const BwdParams& p, int bh, int qb, c
     } else {
       wait_vmcnt<0>();
     }
-    floatx16 s = product<D>(k_blk, qf, ZERO16S, lane);
+    floatx16 s = product<D>(k_blk, qf, ZERO16, lane);
     if (kb == qb) {
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -248,7 +248,7 @@ __device__ __forceinline__ void split32_dkdv(const BwdParams& p, int bh, int kb,
 
   floatx16 dk[DB], dv[DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16S;
+  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16;
   for (; qb < n_blocks; qb += W) {
     const bool more = qb + W < n_blocks;
     const int row = 32 * qb + (lane & 31), read = min(row, T - 1);
@@ -257,9 +257,9 @@ __device__ __forceinline__ void split32_dkdv(const BwdParams& p, int bh, int kb,
     if (g == 0) stat[lane] = row < T ? -lse_row * kLog2e : -INFINITY;  // a padded query's probabilities are zero
     wait_vmcnt<2 * C::NI>();  // Q; dO's block may be on its way
     // (the statistics later: as the first product's accumulator they would be waited for)
-    floatx16 s = product<D>(q_blk, kf, ZERO16S, lane);
+    floatx16 s = product<D>(q_blk, kf, ZERO16, lane);
     wait_vmcnt<C::NI>();  // dO
-    floatx16 dp = product<D, true>(do_blk, vf, ZERO16S, lane, of, &sum);
+    floatx16 dp = product<D, true>(do_blk, vf, ZERO16, lane, of, &sum);
     sum = pair_sum(sum);
     if (g == 0) stat[32 + lane] = -sum;
     if (qb == kb) {

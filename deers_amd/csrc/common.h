@@ -26,6 +26,7 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((__vector_size__(4 * sizeof(__fp16)))) __fp16 fp16x4_raw;
 
 #define DEERS_LDS __attribute__((address_space(3)))
+#define ZERO16 floatx16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -182,6 +183,11 @@ __device__ __forceinline__ void wait_vmcnt() {
 __device__ __forceinline__ void wait_all_vmem() {
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), expcnt and lgkmcnt untouched
 }
+// Before the loads into an LDS block that earlier LDS reads of this wave have used: those have returned.
+__device__ __forceinline__ void settle_lds_reads() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  asm volatile("" ::: "memory");
+}
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return (uint32_t)(size_t)(DEERS_LDS const void*)p;
 }
@@ -326,6 +332,13 @@ __device__ __forceinline__ bool map_block(int block_id, int n_blocks, int heads_
   *bh = (idx % heads_per_xcd) * 8 + xcd;
   *rank = idx / heads_per_xcd;
   return *bh < BH;
+}
+
+// A kernel that takes more dynamic LDS than a launch may have by default.
+template <typename Kernel>
+inline void allow_lds(Kernel kernel, size_t bytes) {
+  if (bytes > 64 * 1024)
+    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
 // Brackets one kernel launch with a hipEvent pair when per-kernel profiling is

@@ -48,7 +48,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
       exit(1);                                                             \
     }                                                                      \
   } while (0)
-#define ZERO16 floatx16{0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}
 #define MF(acc) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b))
 #define FM(v) asm volatile("v_fma_f32 %0, %0, %1, %2" : "+v"(v) : "v"(c1), "v"(c2))
 #define EX(v) asm volatile("v_exp_f32 %0, %0" : "+v"(v))
