@@ -81,16 +81,17 @@ const char* deers_rocm_last_error(void);
 void* deers_rocm_stream(void);
 
 /* ---- hand-overs between workgroups ----------------------------------------
- * Two kernels pass data between workgroups inside one launch: the f16 attention backward
- * (row statistics published by one half of the grid, read by the other) and the few-rows
- * GEMM (K splits summed by the last workgroup to arrive).  Both publish with a drained
+ * Three kernels pass data between workgroups inside one launch: the f16 attention backward
+ * of larger launches (row statistics published by one half of the grid, read by the other),
+ * the few-rows GEMM (K splits summed by the last workgroup to arrive) and the decode (the
+ * splits of a head, likewise).  All publish with a drained
  * store plus a relaxed flag / counter, which is sufficient only while producer and
  * consumer run on the same XCD (one L2); the kernels arrange that by workgroup id % 8.
  * deers_rocm_init checks what that mapping assumes, in the spirit of the capability
  * checks of the reference's runtime construction (src/storage/cuda.rs:492-528), and
  * otherwise selects forms without such a hand-over: the backward as two launches in
- * stream order, the few-rows GEMM unsplit.  Same results either way (the backward bit for
- * bit). */
+ * stream order, the few-rows GEMM unsplit, the decode's splits merged by a second launch.
+ * Same results either way (the backward and the decode bit for bit). */
 #define DEERS_ROCM_HANDOVER_STREAM_ORDER 0
 #define DEERS_ROCM_HANDOVER_SAME_XCD 1
 /* The rule itself, callable without a device: SAME_XCD only for an unpartitioned MI355X
