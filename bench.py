@@ -172,10 +172,10 @@ def bench_attention_config(dtype, B, H, T, D, launches=50, sigma=1.0):
 
 
 EXTRA_CONFIGS = {
-    "c1": dict(dtype=np.float32, B=4, H=6, T=256, D=32),
-    "c3": dict(dtype=np.float16, B=1, H=16, T=8192, D=128, sigma=0.5),
-    "c2_d128": dict(dtype=np.float16, B=8, H=12, T=1024, D=128),            # configs[1] at head width 128
-    "c5_attn": dict(dtype=np.float32, B=8, H=12, T=1024, D=64),             # one layer's attention of configs[4]
+    "c1": dict(dtype=np.float32, B=4, H=6, T=256, D=32),                    # the reference's CPU-runnable size
+    "c3": dict(dtype=np.float16, B=1, H=16, T=8192, D=128, sigma=0.5),      # long context, wide heads
+    "c2_d128": dict(dtype=np.float16, B=8, H=12, T=1024, D=128),            # the headline shape at head width 128
+    "c5_attn": dict(dtype=np.float32, B=8, H=12, T=1024, D=64),             # one layer's attention of the GPT training step
 }
 
 
@@ -437,7 +437,7 @@ def bench_adamw(steps: int, warmup: int):
 
 
 def bench_gpt(steps: int, warmup: int):
-    """End-to-end GPT training step (BASELINE configs[4]): f32 parameters, 12 layers,
+    """End-to-end GPT training step: f32 parameters, 12 layers,
     12 heads, n_embd 768, MLP 3072, vocabulary 50257, sequence 1024, batch 8; forward,
     cross-entropy, backward, gradient-norm clipping, AdamW, all on the device through the
     C++ host (deers_amd/host/gpt_step), with the library's GEMM kernel picked per problem by
@@ -463,7 +463,7 @@ def bench_gpt(steps: int, warmup: int):
     fwd_f, bwd_f = attn_flops(cfg["batch"], cfg["n_head"], cfg["seq_len"], cfg["n_embd"] // cfg["n_head"])
     attn = cfg["n_layer"] * (fwd_f + bwd_f)
     out["workload"] = ("GPT training step, f32, 12 layers x 12 heads x 768, MLP 3072, vocab 50257, "
-                       "seq 1024, batch 8 (BASELINE configs[4]); synthetic token ids, random-init weights")
+                       "seq 1024, batch 8; synthetic token ids, random-init weights")
     out["flops_per_step"] = {"matmul": gemm_flops, "attention": attn}
     out["model_tflops"] = (gemm_flops + attn) / (out["ms_per_step"] * 1e-3) / 1e12
     # greedy generation with KV caches on the same architecture in f16 (32 sequences, 512 cached
@@ -622,7 +622,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f16", "data": "synthetic",
         "config": {"workload": "causal self-attention fwd+bwd, f16 in / f32 accumulate, "
-                               "B=8 H=12 T=1024 D=64 (BASELINE configs[1])",
+                               "B=8 H=12 T=1024 D=64",
                    "flops_per_step": fwd_f + bwd_f, "flop_convention": "7*B*H*T^2*D"},
         "frac_mfma_peak": tflops / PEAK_F16_TFLOPS,
         "peak_tflops_f16_dense": PEAK_F16_TFLOPS,
@@ -634,7 +634,7 @@ def main():
         "step_us_event_pairs": tr["step_us"],
         "kernels": kern,
         "roofline": roofline,
-        "decode": {"workload": "decode f16 B=32 H=12 L=4096 D=64 (BASELINE configs[3]), "
+        "decode": {"workload": "decode f16 B=32 H=12 L=4096 D=64, "
                                "4 KV caches in rotation",
                    "timing": "one event pair around %d back-to-back calls" % dec_calls,
                    "bytes_per_call": dec["bytes"], "kernel_us": dec["kernel_us"],
@@ -642,7 +642,7 @@ def main():
                    "GB/s_whole_call": dec["gbs_call"], "peak_GB/s": PEAK_HBM_GBS,
                    "frac_hbm_peak": dec["gbs_kernel"] / PEAK_HBM_GBS},
     }
-    # BASELINE configs[0] and configs[2] (and configs[1]'s shape at head width 128), reported
+    # the small f32 size, the long f16 one and the headline shape at head width 128, reported
     # beside the headline, never part of `value`
     for name, cfg in EXTRA_CONFIGS.items():
         try:
@@ -650,7 +650,7 @@ def main():
         except Exception as e:  # the headline line must not depend on them
             out[name] = {"error": str(e)}
     if not args.no_gpt:
-        # BASELINE configs[4], reported beside the headline (never part of `value`)
+        # the GPT training step, reported beside the headline (never part of `value`)
         try:
             g = bench_gpt(5, 2)
             out["gpt_train_step"] = {k: g[k] for k in ("workload", "ms_per_step", "tokens_per_s",
