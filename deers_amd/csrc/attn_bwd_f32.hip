@@ -15,7 +15,7 @@
 //   the same with 128 keys per workgroup in lockstep and their dQ summed through LDS first, a quarter of the
 //     adds: 1160.  Kernels of that kind with swizzled LDS addresses stood here before: 1222.
 //   S and dP computed again for dQ, 7 products (attn_split_f32.hip): better where the launch is small.
-//   these: 1037.
+//   these: 1037 with products that started from the row statistics (below), 1060 now.
 // Every sum is taken in a fixed order: dQ, dK and dV are reproducible bit for bit.
 //
 // The products start from zero and the row statistics are added to the finished sums.  Starting them from
@@ -23,8 +23,8 @@
 // but rounds every element's term at the size of the LSE: relative error of dQ against 64 bits 1.0e-6 instead
 // of 0.43e-6 at T = 1024, D = 64, of dK 1.06e-6 instead of 0.53e-6.
 //
-// us, before -> now: 8 x 12 x 1024 x 64 366 -> 302, 400 x 512 x 64 427 -> 345, 8 x 2048 x 64 162 -> 136, 48 x 1024 x 128
-// 499 -> 379, 400 x 512 x 128 1225 -> 765, 96 x 1024 x 32 199 -> 167.
+// us, kernels of that kind -> these: 8 x 12 x 1024 x 64 366 -> 305, 400 x 512 x 64 427 -> 352, 8 x 2048 x 64 162 -> 132, 48 x
+// 1024 x 128 499 -> 370, 400 x 512 x 128 1225 -> 747, 96 x 1024 x 32 199 -> 168.
 #include <algorithm>
 
 #include "attn_f32_blocks.h"
@@ -234,9 +234,9 @@ bool attn_f32_one_wave(int64_t n, int64_t nb, int64_t D);  // attn_split_f32.hip
 namespace {
 
 // Waves per workgroup of both passes, for n workgroups that walk up to nb blocks.  As in
-// attn_split_f32.hip: one where many workgroups of short walks cover the SIMDs (400 x 512 x 64: 418 us in
-// four waves, 376 in two, 354 in one), four where the longest walk would be alone at the end (24 x 4096 x 64
-// 1065 / 1123 / 1270), two between (192 x 384 x 64 133 / 122 / 134; 48 x 512 x 128 141 / 127 / 206).
+// attn_split_f32.hip: one where many workgroups of short walks cover the SIMDs (400 x 512 x 64: 412 us in
+// four waves, 374 in two, 353 in one), four where the longest walk would be alone at the end (24 x 4096 x 64
+// 1058 / 1085 / 1206), two between (192 x 384 x 64 129 / 118 / 127; 48 x 512 x 128 138 / 124 / 199).
 int bwd_waves(int64_t n, int64_t nb, int64_t D) {
   if (attn_f32_one_wave(n, nb, D)) return 1;
   return n >= (D == 32 ? 1792 + 24 * nb : D == 64 ? 384 + 72 * nb : 256 + 24 * nb) ? 2 : 4;
@@ -272,10 +272,10 @@ int64_t attn_bwd_f32_default_ds_limit() { return (int64_t)2304 << 20; }
 
 // Which launches come here (the others: attn_split_f32.hip, S and dP twice but one launch).  Three
 // launches and a workspace pay from enough workgroups on to fill the device, n = heads * T / 32 (D = 64: at
-// 512 of them, 8 x 2048, 136 us against 162; at 384, 12 x 1024, 71 against 66).  The shorter the walks, the
-// more the launches weigh: below twelve blocks several times as many workgroups (192 x 256 x 64 72 against
-// 75, 96 x 256 x 64 47 against 44), below eight only with one wave per workgroup (800 x 128 x 64: 86 against
-// 97; 4000 x 64 x 128: 350 against 455).
+// 512 of them, 8 x 2048, 132 us against 157; at 384, 12 x 1024, 69 against 67).  The shorter the walks, the
+// more the launches weigh: below twelve blocks several times as many workgroups (192 x 256 x 64 69 against
+// 71, 96 x 256 x 64 47 against 42), below eight only with one wave per workgroup (800 x 128 x 64: 81 against
+// 91; 4000 x 64 x 128: 347 against 460).
 static bool takes(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb;
   if (nb >= 12) return n >= (D == 32 ? 640 : D == 64 ? 512 : 384);

@@ -24,8 +24,8 @@
 // last is the one that the next stage needs second, so that both requests are covered by a product
 // (2048 clocks at D = 64).
 //
-// us, forward / backward, 128-row kernels -> these: 24 heads x 256 x 32 15.4 / 26.1 -> 6.1 / 12.9, 12 x 512 x 64
-// 41 / 66 -> 14 / 32, 12 x 1024 x 64 77 / 121 -> 29 / 66, 3 x 4096 x 32 191 / 337 -> 55 / 129, 8 x 256 x 128 48 / 98
+// us, forward / backward, 128-row kernels -> these: 24 heads x 256 x 32 15.6 / 26.9 -> 5.9 / 11.3, 12 x 512 x 64
+// 41 / 66 -> 14 / 32, 12 x 1024 x 64 77 / 119 -> 28 / 67, 3 x 4096 x 32 191 / 337 -> 55 / 129, 8 x 256 x 128 48 / 98
 // -> 16 / 31.
 #include <algorithm>
 
