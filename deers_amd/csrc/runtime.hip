@@ -128,8 +128,7 @@ struct Runtime {
   rocblas_handle blas = nullptr;  // created by the first matmul, bound to `stream`
   // per (head, 128-row query block) publication flags of the single-launch f16
   // backward; a flag equals the current epoch once its rows are published
-  int* bwd_ready = nullptr;  // allocation: [error word][flags ...]; kernels get the address of flags[0]
-  size_t bwd_ready_len = 0;
+  Region bwd_flags;  // [error word][flags ...]; kernels get the address of flags[0]
   int bwd_epoch = 0;
   bool bwd_error_armed = false;  // a single-launch backward ran since the error word was last read
   // Hand-overs between workgroups inside one launch (the f16 backward's row statistics,
@@ -468,13 +467,13 @@ int check_index_flag() {
 // After the stream has drained: reports (once) that a dK/dV workgroup of a single-launch
 // backward gave up waiting for its row statistics since the last check.
 int check_handover_error() {
-  if (!g_rt.bwd_error_armed || !g_rt.bwd_ready) return DEERS_ROCM_OK;
+  if (!g_rt.bwd_error_armed || !g_rt.bwd_flags.p) return DEERS_ROCM_OK;
   g_rt.bwd_error_armed = false;
   int seen = 0;
-  HIP_TRY(hipMemcpyAsync(&seen, g_rt.bwd_ready, sizeof(int), hipMemcpyDeviceToHost, g_rt.stream));
+  HIP_TRY(hipMemcpyAsync(&seen, g_rt.bwd_flags.p, sizeof(int), hipMemcpyDeviceToHost, g_rt.stream));
   HIP_TRY(hipStreamSynchronize(g_rt.stream));
   if (!seen) return DEERS_ROCM_OK;
-  HIP_TRY(hipMemsetAsync(g_rt.bwd_ready, 0, sizeof(int), g_rt.stream));
+  HIP_TRY(hipMemsetAsync(g_rt.bwd_flags.p, 0, sizeof(int), g_rt.stream));
   HIP_TRY(hipStreamSynchronize(g_rt.stream));
   return fail(DEERS_ROCM_ERR_HANDOVER,
               "attn_bwd: a workgroup gave up waiting for another workgroup's row statistics "
@@ -821,35 +820,34 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
     return DEERS_ROCM_OK;
   }
   // behind them the dQ role's scaled queries, [B*H][t_pad][D] f16
-  const size_t ws_qs = (size_t)(B * H * t_pad * D) * 2;
-  if (int rc = workspace(ws_floats * sizeof(float) + ws_qs, &ws)) return rc;
+  const size_t ws_bytes = ws_floats * sizeof(float) + (size_t)(B * H * t_pad * D) * 2;
+  const size_t flag_bytes = ((size_t)(B * H) * (size_t)((T + 127) / 128) + 1) * sizeof(int);
+  Region& flags = g_rt.bwd_flags;
+  const bool flags_grow = flag_bytes > flags.bytes || g_rt.bwd_epoch == INT32_MAX;
   // A launch that is being captured into a graph gets no fresh epoch on replay: it takes the
-  // two-launch form with the flags switched off (epoch 0).  The workspace and the flags must
-  // have been grown by an earlier, eager call of the same geometry: capture allows neither
-  // the synchronisation nor the allocation.
+  // two-launch form with the flags switched off (epoch 0; the dQ role still clears its flags).  Where the
+  // workspace or the flags would have to grow, which a capture does not allow, the form that needs neither.
   bool capturing;
   if (int rc = stream_captures(&capturing)) return rc;
-  const size_t n_flags = (size_t)(B * H) * (size_t)((T + 127) / 128);
-  if (n_flags > g_rt.bwd_ready_len || g_rt.bwd_epoch == INT32_MAX) {
-    if (capturing)
-      return fail(DEERS_ROCM_ERR_ARG,
-                  "attn_bwd: call once outside stream capture with this geometry first (the "
-                  "hand-over flags have to grow)");
-    if (g_rt.bwd_ready) {
+  if (capturing && (flags_grow || ws_bytes > g_rt.workspace.bytes)) {
+    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+    HIP_TRY(hipGetLastError());
+    return DEERS_ROCM_OK;
+  }
+  if (int rc = workspace(ws_bytes, &ws)) return rc;
+  if (flags_grow) {
+    if (flags.p) {
       HIP_TRY(hipStreamSynchronize(g_rt.stream));
       // an error raised by a launch before this point is reported by this call
       if (int rc = check_handover_error()) return rc;
-      HIP_TRY(hipFree(g_rt.bwd_ready));
-      g_rt.bwd_ready = nullptr;
     }
-    const size_t want = n_flags > g_rt.bwd_ready_len ? n_flags : g_rt.bwd_ready_len;
-    HIP_TRY(hipMalloc(&g_rt.bwd_ready, (want + 1) * sizeof(int)));  // [error word][flags]
-    HIP_TRY(hipMemsetAsync(g_rt.bwd_ready, 0, (want + 1) * sizeof(int), g_rt.stream));
-    g_rt.bwd_ready_len = want;
+    if (int rc = grow(flags, std::max(flag_bytes, flags.bytes))) return rc;
+    HIP_TRY(hipMemsetAsync(flags.p, 0, flags.bytes, g_rt.stream));
     g_rt.bwd_epoch = 0;
   }
-  p.error = g_rt.bwd_ready;
-  p.ready = g_rt.bwd_ready + 1;
+  flags.captured |= capturing;
+  p.error = static_cast<int*>(flags.p);
+  p.ready = p.error + 1;
   p.epoch = capturing ? 0 : ++g_rt.bwd_epoch;
   p.spin_limit = g_rt.bwd_spin_limit;
   const bool single_launch = !capturing && same_xcd_handover_now();

@@ -102,9 +102,10 @@ int deers_rocm_handover_policy(int cu_count, int cu_mask_set);
  * STREAM_ORDER is refused with DEERS_ROCM_ERR_ARG (the hand-over through one L2 is not valid
  * there).  A backward call made while the library stream is being captured into a HIP graph
  * takes the two-launch form without flags by itself: the single launch's flag epoch is a
- * kernel argument, so a replayed launch would find its flags already set.  Such a call must
- * have been made once outside capture with the same geometry (workspace and flags grow
- * there). */
+ * kernel argument, so a replayed launch would find its flags already set.  Where workspace
+ * or flags would have to grow for that (no call with the geometry, or a larger one, has been
+ * made outside capture) it takes the form that needs neither, which small launches always
+ * take: the same gradients to rounding, slower for large launches. */
 int deers_rocm_handover_mode(void);
 int deers_rocm_set_handover_mode(int mode);
 
