@@ -259,11 +259,12 @@ int grow(Region& r, size_t bytes) {
   return DEERS_ROCM_OK;
 }
 
-// Workspace that only grows; callers hold g_mu.
-int workspace(size_t bytes, void** out) {
+// Workspace that only grows; callers hold g_mu.  *captures: whether the stream is being captured.
+int workspace(size_t bytes, void** out, bool* captures = nullptr) {
   Region& r = g_rt.workspace;
   bool capturing;
   if (int rc = stream_captures(&capturing)) return rc;
+  if (captures) *captures = capturing;
   if (bytes > r.bytes) {
     if (capturing && r.p)
       return fail(DEERS_ROCM_ERR_ARG,
@@ -862,16 +863,29 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   return DEERS_ROCM_OK;
 }
 
-// Arrival counters for a decode call whose split heads are merged inside the launch; null where
-// they are merged by a second one: nothing to merge, splits that may not share an XCD, or a call
-// that may run beside another one (a captured graph), since calls that overlap would count each other's
-// arrivals.
-static int decode_counters(int64_t BH, int splits, int** out) {
-  *out = nullptr;
-  if (splits == 1 || BH > kDecodeCounters || !same_xcd_handover_now()) return DEERS_ROCM_OK;
+// Where the splits of a decode call's heads meet: the partials in the workspace (or in `ws`, if that is given),
+// and the arrival counters for a merge inside the launch.  Those are null where a second launch merges:
+// splits that may not share an XCD, more of them than `merge_most`, or a call that may run beside another one (a
+// captured graph), since calls that overlap would count each other's arrivals.
+static int decode_meeting(deers::DecodeParams* p, int64_t D, void* ws, int merge_most) {
+  if (p->splits == 1) return DEERS_ROCM_OK;  // nothing to merge
+  const size_t part_o = (size_t)p->BH * p->splits * D * sizeof(float);
+  const size_t part_ml = (size_t)p->BH * p->splits * 2 * sizeof(float);
   bool capturing;
-  if (int rc = stream_captures(&capturing)) return rc;
-  if (!capturing) *out = g_decode_arrivals;
+  if (ws) {
+    if (part_o + part_ml > kScratchBytes)
+      return fail(DEERS_ROCM_ERR_ARG,
+                  "attn_decode_noalloc: the split partials of this problem need %zu bytes, the static scratch "
+                  "holds %zu; use deers_rocm_attn_decode",
+                  part_o + part_ml, kScratchBytes);
+    if (int rc = stream_captures(&capturing)) return rc;
+  } else {
+    if (int rc = workspace(part_o + part_ml, &ws, &capturing)) return rc;
+  }
+  p->part_o = static_cast<float*>(ws);
+  p->part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
+  if (p->BH <= kDecodeCounters && p->splits <= merge_most && !capturing && same_xcd_handover_now())
+    p->arrived = g_decode_arrivals;
   return DEERS_ROCM_OK;
 }
 
@@ -899,29 +913,12 @@ static int attn_decode_impl(const char* what, bool no_alloc, int dtype, const vo
     return fail(DEERS_ROCM_ERR_LAYOUT, "%s: cache rows, q and o must be 16-byte aligned", what);
   int chunk = 0;
   const int splits = deers::decode_pick_splits(B * H, L, D, &chunk);
-  void* ws = nullptr;
-  const size_t part_o = (size_t)(B * H) * splits * D * sizeof(float);
-  const size_t part_ml = (size_t)(B * H) * splits * 2 * sizeof(float);
-  if (no_alloc) {
-    // a head that is not split writes its output itself and touches no scratch
-    if (splits > 1 && part_o + part_ml > kScratchBytes)
-      return fail(DEERS_ROCM_ERR_ARG,
-                  "%s: the split partials of this problem need %zu bytes, the static scratch "
-                  "holds %zu; use deers_rocm_attn_decode",
-                  what, part_o + part_ml, kScratchBytes);
-    ws = g_scratch_ptr;
-  } else {
-    if (int rc = workspace(part_o + part_ml, &ws)) return rc;
-  }
   p.q = q; p.k = k_cache; p.v = v_cache; p.o = o;
-  p.part_o = static_cast<float*>(ws);
-  p.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
   p.BH = (int)(B * H); p.H = (int)H; p.L = (int)L; p.splits = splits; p.chunk = chunk;
   // The entry point that allocates nothing has merged by a second launch from the beginning; inside the
   // launch pays for up to four splits (1 head x 500 x 64 6.5 -> 4.0 us, 48 x 2000 x 64 9.2 -> 8.9), and with many
   // short ones it does not (12 x 2000 x 64 in 16 splits 6.2 -> 7.1).
-  if (!no_alloc || splits <= 4)
-    if (int rc = decode_counters(B * H, splits, &p.arrived)) return rc;
+  if (int rc = decode_meeting(&p, D, no_alloc ? g_scratch_ptr : nullptr, no_alloc ? 4 : splits)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, false, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -979,17 +976,11 @@ int deers_rocm_attn_decode_append(int dtype, const void* q, const void* k, const
   p.skb = cache_strides[0]; p.skh = cache_strides[1]; p.skl = cache_strides[2];
   int chunk = 0;
   const int splits = deers::decode_pick_splits(B * H, pos, D, &chunk);  // over the rows already cached
-  void* ws = nullptr;
-  const size_t part_o = (size_t)(B * H) * splits * D * sizeof(float);
-  const size_t part_ml = (size_t)(B * H) * splits * 2 * sizeof(float);
-  if (int rc = workspace(part_o + part_ml, &ws)) return rc;
   p.k = k_cache; p.v = v_cache; p.o = o;
   p.q_in = q; p.k_in = k; p.v_in = v; p.cos_row = cos_row; p.sin_row = sin_row;
   p.in_b = in_strides[0]; p.in_h = in_strides[1];
-  p.part_o = static_cast<float*>(ws);
-  p.part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
   p.BH = (int)(B * H); p.H = (int)H; p.L = (int)pos; p.splits = splits; p.chunk = chunk;
-  if (int rc = decode_counters(B * H, splits, &p.arrived)) return rc;
+  if (int rc = decode_meeting(&p, D, nullptr, splits)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, true, g_rt.stream);
   HIP_TRY(hipGetLastError());
