@@ -144,26 +144,40 @@ __device__ __forceinline__ void async_load16_to_lds(const void* gptr, uint32_t l
                : "memory");
 }
 // Same copy with the address split into a wave-uniform 64-bit base (SGPR pair) and a
-// per-lane unsigned 32-bit byte offset, so advancing to the next tile is scalar work.  The LDS address is
-// given as two terms, which the write of m0 adds up: where one is a register and the other a constant, that
+// per-lane unsigned 32-bit byte offset, so advancing to the next tile is scalar work.  The form whose LDS address
+// has two terms adds them up in the write of m0: where one is a register and the other a constant, that
 // saves a scalar instruction per load, what the move of the base costs (15 heads x 777 x 128 forward and backward
-// 45.15 -> 44.85 us, a generated token of 32 sequences 426.4 -> 424.9).  The block-pipelined f16 loops pass one
-// term: with two, the compiler's other choices made the forward of 8 x 12 x 1024 x 64 20.4 -> 20.7 us.
-#define DEERS_ASYNC_LOAD_TO_LDS(name, load)                                                                      \
-  __device__ __forceinline__ void name(const void* uniform_base, uint32_t lane_off, uint32_t lds_addr,           \
-                                       uint32_t lds_add = 0) {                                                   \
-    const uint32_t at = __builtin_amdgcn_readfirstlane(lds_addr), add = __builtin_amdgcn_readfirstlane(lds_add); \
-    const uint64_t b = (uint64_t)uniform_base;                                                                   \
-    /* readfirstlane returns a signed int: widen through uint32_t, never sign-extend */                          \
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);                                   \
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));                           \
-    const uint64_t sbase = ((uint64_t)hi << 32) | (uint64_t)lo;                                                  \
-    uint64_t base;                                                                                               \
-    asm volatile("s_add_u32 m0, %3, %4\n\ts_mov_b64 %0, %2\n\t" load                                            \
-                 : "=&s"(base)                                                                                   \
-                 : "v"(lane_off), "s"(sbase), "s"(at), "ri"(add)                                                 \
-                 : "memory", "scc");                                                                             \
+// 45.15 -> 44.85 us, a generated token of 32 sequences 426.4 -> 424.9).  It changes the scalar condition code, which
+// the compiler works around: the pipelined f16 loops pass one term (with two, the forward of 8 x 12 x 1024 x 64 20.4 ->
+// 20.7 us).
+#define DEERS_ASYNC_LOAD_TO_LDS(name, load)                                                                     \
+  __device__ __forceinline__ void name(const void* uniform_base, uint32_t lane_off, uint32_t lds_addr) {        \
+    const uint32_t at = __builtin_amdgcn_readfirstlane(lds_addr);                                               \
+    const uint64_t sbase = uniform_address(uniform_base);                                                       \
+    uint64_t base;                                                                                              \
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\t" load                                               \
+                 : "=&s"(base)                                                                                  \
+                 : "v"(lane_off), "s"(sbase), "s"(at)                                                           \
+                 : "memory");                                                                                   \
+  }                                                                                                             \
+  __device__ __forceinline__ void name(const void* uniform_base, uint32_t lane_off, uint32_t lds_addr,          \
+                                       uint32_t lds_add) {                                                      \
+    const uint32_t at = __builtin_amdgcn_readfirstlane(lds_addr);                                               \
+    const uint32_t add = __builtin_amdgcn_readfirstlane(lds_add);                                               \
+    const uint64_t sbase = uniform_address(uniform_base);                                                       \
+    uint64_t base;                                                                                              \
+    asm volatile("s_add_u32 m0, %3, %4\n\ts_mov_b64 %0, %2\n\t" load                                           \
+                 : "=&s"(base)                                                                                  \
+                 : "v"(lane_off), "s"(sbase), "s"(at), "ri"(add)                                                \
+                 : "memory", "scc");                                                                            \
   }
+__device__ __forceinline__ uint64_t uniform_address(const void* p) {
+  const uint64_t b = (uint64_t)p;
+  // readfirstlane returns a signed int: widen through uint32_t, never sign-extend
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  return ((uint64_t)hi << 32) | (uint64_t)lo;
+}
 DEERS_ASYNC_LOAD_TO_LDS(async_load16_to_lds, "global_load_lds_dwordx4 %1, %0")
 // for data that is used once (a non-temporal access)
 DEERS_ASYNC_LOAD_TO_LDS(async_load16_to_lds_nt, "global_load_lds_dwordx4 %1, %0 nt")
