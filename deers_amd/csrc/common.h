@@ -248,6 +248,7 @@ struct FwdParams {
   Strides3 sq, sk, sv, so;
   int H, T;
   float scale_log2;  // scale * log2(e)
+  int scaled_q;      // f16, 32 rows per workgroup: scores from f16(Q * scale_log2), not from Q
 };
 
 // Whether the single-launch f16 backward runs its dQ groups shortest first: when a group
@@ -273,6 +274,7 @@ struct BwdParams {
   Strides3 sq, sk, sv, so, sdo, sdq, sdk, sdv;
   int H, T;
   float scale, scale_log2;
+  int scaled_q;  // as in FwdParams: what the forward that made lse did
 };
 
 struct DecodeParams {
@@ -305,7 +307,7 @@ __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH
   const int whole = BH >> 3, rest = BH & 7;
   // remaining heads' blocks of rank < k on this XCD: t = rank * rest + head, dealt to XCD t % 8
   auto dealt = [&](int k) { return k * rest > xcd ? (k * rest - xcd + 7) >> 3 : 0; };
-  int k = (int)((int64_t)idx * 8 / BH);
+  int k = (int)((unsigned)idx * 8u / (unsigned)BH);  // idx * 8 <= the block id, which fits
   while (whole * (k + 1) + dealt(k + 1) <= idx) ++k;
   while (k > 0 && whole * k + dealt(k) > idx) --k;
   if (k >= n_ranks) return false;

@@ -753,6 +753,7 @@ int deers_rocm_attn_fwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
   p.H = (int)H; p.T = (int)T;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
+  p.scaled_q = !deers::attn_bwd_f16_split_takes(B * H, T, D);
   if (dtype == DEERS_ROCM_F16 && deers::attn_fwd_f16_split_takes(B * H, T, D))
     deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, g_rt.stream);
   else if (dtype == DEERS_ROCM_F16)
@@ -792,6 +793,7 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.H = (int)H; p.T = (int)T;
   p.scale = scale;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
+  p.scaled_q = !deers::attn_bwd_f16_split_takes(B * H, T, D);
   // the forms for launches that cannot fill the device need no workspace and hand nothing over
   // (the test hook of the hand-over asks for the form that does)
   if (dtype == DEERS_ROCM_F16 && !g_rt.bwd_skip_producers && deers::attn_bwd_f16_split_takes(B * H, T, D)) {

@@ -1,0 +1,89 @@
+"""The f16 attention kernels that give a workgroup 32 rows: every form at the sizes where it can go wrong (a walk of one
+block, of as many blocks as waves and one more, rows past the end of the last block), and the rule that chooses them."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from deers_amd import rocm, synth
+
+# relative 2-norm error of a result against the f32 oracle on the same f16 inputs: three roundings to f16 on the way
+# (scores' operand or probability, score gradient, result), each 2^-12 / sqrt(3) in the root mean square, and the
+# same again for what they do to small sums
+REL = 2 * 3 ** 0.5 * 2.0 ** -12 / 3 ** 0.5
+
+
+def takes(direction, BH, T, D):
+    rule = rocm.load()[f"_ZN5deers24attn_{direction}_f16_split_takesElll"]
+    rule.restype = ctypes.c_bool
+    return rule(*(ctypes.c_int64(v) for v in (BH, T, D)))
+
+
+def test_what_the_backward_takes_the_forward_takes_too():
+    """Both then form their scores from Q itself; otherwise a probability would be recomputed from another score than
+    the one it was normalised with."""
+    for D in (32, 64, 128):
+        for T in [32 * nb for nb in range(1, 140)] + [8192]:
+            for BH in [int(1.15 ** i) for i in range(70)]:
+                assert not takes("bwd", BH, T, D) or takes("fwd", BH, T, D), (BH, T, D)
+
+
+def rel(got, want):
+    return float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want))
+
+
+# BH, T: forms by waves (4 with K and V twice in LDS, 4, 2, 1), remainders of T / 32 and of the blocks by the waves
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("BH,T", [(3, 1), (2, 31), (5, 33), (4, 97), (3, 129), (2, 160), (9, 417), (30, 255), (61, 250),
+                                  (130, 200), (300, 65), (500, 100)])
+def test_every_form_matches_the_oracle(BH, T, D):
+    assert takes("fwd", BH, T, D)
+    x = synth.attention_inputs(f"split-{BH}-{T}-{D}", 1, BH, T, D, np.float16, base_seed=61)
+    print(f"{BH} x {T} x {D}", flush=True)
+    got = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for a, b in zip(got, again):
+        np.testing.assert_array_equal(a, b)
+    few = (slice(None), sorted({0, BH // 2, BH - 1}))
+    o, lse = oracle.attn_fwd(x["q"][few], x["k"][few], x["v"][few], return_lse=True)
+    refs = (o, lse, *oracle.attn_bwd(x["q"][few], x["k"][few], x["v"][few], x["do"][few]))
+    for name, g, want in zip(("o", "lse", "dq", "dk", "dv"), got, refs):
+        if name == "dq" and T == 1:  # one key: exactly zero but for the rounding of dO . (O - V)
+            assert np.max(np.abs(g[few])) <= 2.0 ** -8
+        elif name == "dk" and T == 1:
+            assert np.max(np.abs(g[few])) <= 2.0 ** -8
+        else:
+            assert rel(g[few], want) <= REL, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D,stride", [(3, 64, 1 << 20), (40, 128, 1 << 14), (70, 32, 1 << 13)])
+def test_rows_far_apart_give_the_same_bits(T, D, stride):
+    """Row strides at which 32 rows reach past what a block's rows span; between the rows NaN."""
+    H = 2
+    x = synth.attention_inputs(f"split-far-{T}-{D}", 1, H, T, D, np.float16, base_seed=62)
+    want = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    st = (T * stride, D, stride, 1)
+
+    def spread(a):
+        buf = np.full((T, stride), np.nan, np.float16)
+        for h in range(H):
+            buf[:, h * D:h * D + D] = a[0, h]
+        return rocm.DeviceBuffer.from_numpy(buf)
+
+    bufs = {n: spread(x[n]) for n in ("q", "k", "v", "do")}
+    outs = {n: rocm.DeviceBuffer((T, stride), np.float16) for n in ("o", "dq", "dk", "dv")}
+    lse = rocm.DeviceBuffer((1, H, T), np.float32)
+    scale = rocm.default_scale(D)
+    rocm.attn_fwd_raw(np.float16, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, 1, H, T, D, scale,
+                      q_strides=st, k_strides=st, v_strides=st, o_strides=st)
+    rocm.attn_bwd_raw(np.float16, bufs["q"].ptr, bufs["k"].ptr, bufs["v"].ptr, outs["o"].ptr, lse.ptr, bufs["do"].ptr,
+                      outs["dq"].ptr, outs["dk"].ptr, outs["dv"].ptr, 1, H, T, D, scale,
+                      strides={n: st for n in ("q", "k", "v", "o", "do", "dq", "dk", "dv")})
+    for name, ref in zip(("o", "dq", "dk", "dv"), (want[0], *want[2:])):
+        got = outs[name].numpy()
+        for h in range(H):
+            np.testing.assert_array_equal(got[:, h * D:h * D + D], ref[0, h], err_msg=name)
+    np.testing.assert_array_equal(lse.numpy(), want[1])
