@@ -105,9 +105,9 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f3
 #pragma unroll
   for (int k = 0; k < KH; ++k) kf[k] *= p.scale_log2;
 
-  floatx16 dk[DB], dv[DB];
+  floatx16 acc[2][DB];  // dK, dV
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16;
+  for (int db = 0; db < DB; ++db) acc[0][db] = acc[1][db] = ZERO16;
   for (; qb < n_blocks; qb += W) {
     const bool more = qb + W < n_blocks;
     wait_vmcnt<C::NI>();  // dS written, statistics, Q
@@ -134,22 +134,24 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f3
             floatx4{dp[4 * r4], dp[4 * r4 + 1], dp[4 * r4 + 2], dp[4 * r4 + 3]};
       asm volatile("" ::: "memory");
     }
-    accumulate<D>(dk, q_blk, dp, lane);
+    accumulate<D>(acc[0], q_blk, dp, lane);
     if (more) {
       settle_lds_reads();
       async_load4_to_lds(stats + 32 * (qb + W), stat_off, stat_lds);
       load_block<D>(Q, sqt, 32 * (qb + W), T, q_blk, lane);
     }
-    accumulate<D>(dv, do_blk, s, lane);
+    accumulate<D>(acc[1], do_blk, s, lane);
     if (more) {
       settle_lds_reads();
       load_block<D>(dO, sdot, 32 * (qb + W), T, do_blk, lane);
     }
   }
-  float* dv_row = (float*)p.dv + b * p.sdv.b + h * p.sdv.h + (int64_t)kread * p.sdv.t;
-  float* dk_row = (float*)p.dk + b * p.sdk.b + h * p.sdk.h + (int64_t)kread * p.sdk.t;
-  merge_store<D, W>(dv, 1.f, 1.f, dv_row, krow < T, (float*)smem, wave, lane);
-  merge_store<D, W>(dk, 1.f, p.scale, dk_row, krow < T, (float*)smem, wave, lane);
+  float* const row[2] = {(float*)p.dk + b * p.sdk.b + h * p.sdk.h + (int64_t)kread * p.sdk.t,
+                         (float*)p.dv + b * p.sdv.b + h * p.sdv.h + (int64_t)kread * p.sdv.t};
+  const float mul[2] = {p.scale, 1.f};
+  settle_lds_reads();
+  leave_sums<D, W, 2, 2 * C::BB>(acc, q_blk, lane);
+  store_sums<D, W, 2, 2 * C::BB>(acc, lds_address(smem), nullptr, mul, row, krow < T, wave, lane);
 }
 
 // A wave of the dQ pass has one K block and one block of dS in LDS (12.5 KB at D = 64): three to a SIMD
@@ -158,7 +160,7 @@ template <int D, int W>
 struct DqPass {
   using C = Split32<D>;
   static constexpr int WAVE = C::BB + 4 * kDsPitch;
-  static constexpr int LDS = std::max(W * WAVE, W * (D / 2) * 64 * 4);
+  static constexpr int LDS = W * WAVE;
 };
 
 template <int D, int W>
@@ -185,9 +187,9 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_f32_dq_kernel(BwdParams p, in
   const int q = lane & 31;
   const uint32_t ds_at = C::BB + (q >> 3) * kDsPitch + ((q >> 2) & 1) * 512 + (q & 3) * 4 + g * 64;
 
-  floatx16 acc[DB];
+  floatx16 acc[1][DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) acc[db] = ZERO16;
+  for (int db = 0; db < DB; ++db) acc[0][db] = ZERO16;
   for (int kb = wave; kb <= qb; kb += W) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -198,12 +200,14 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_f32_dq_kernel(BwdParams p, in
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       x[r] = *(DEERS_LDS const float*)(uintptr_t)(lds + ds_at + (8 * (r >> 2) + (r & 3)) * 16);
-    accumulate<D>(acc, lds, x, lane);
+    accumulate<D>(acc[0], lds, x, lane);
     settle_lds_reads();
   }
   const int qrow = 32 * qb + q;
-  float* row = (float*)p.dq + b * p.sdq.b + h * p.sdq.h + (int64_t)min(qrow, T - 1) * p.sdq.t;
-  merge_store<D, W>(acc, 1.f, p.scale, row, qrow < T, (float*)smem, wave, lane);
+  float* const row = (float*)p.dq + b * p.sdq.b + h * p.sdq.h + (int64_t)min(qrow, T - 1) * p.sdq.t;
+  const float mul = p.scale;
+  leave_sums<D, W, 1, S::WAVE>(acc, lds, lane);
+  store_sums<D, W, 1, S::WAVE>(acc, lds_address(smem), nullptr, &mul, &row, qrow < T, wave, lane);
 }
 
 template <int D, int W>

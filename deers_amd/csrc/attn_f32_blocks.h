@@ -123,34 +123,58 @@ __device__ __forceinline__ void accumulate(floatx16 (&acc)[D / 32], uint32_t blo
   }
 }
 
-// Adds the W waves' accumulators of a [32 rows, D] result (row = lane % 32), each scaled by its
-// wave's `weight` first, in wave order, multiplies by `mul` and writes rows at dst (this lane's
-// row; not where !store).  `red` is LDS for W * D / 2 * 64 floats.  Starts with a barrier.
-template <int D, int W>
-__device__ __forceinline__ void merge_store(const floatx16 (&acc)[D / 32], float weight, float mul, float* dst,
-                                            bool store, float* red, int wave, int lane) {
-  __syncthreads();
+// N results of [32 rows, D] (row = lane % 32) meet by four columns, four registers: every wave leaves its accumulators
+// in its own LDS, `own_lds` and on (N * D / 8 KB, no more than its blocks took), and after one barrier wave w adds
+// columns w, w + W, .. of all results in wave order, each times its wave's weight where there are any, multiplies by
+// mul[n] and writes rows at dst[n] (this lane's row; not where !store).  first_lds: wave 0's, the others' WAVE_BYTES apart.
+// 16 bytes per lane both ways; two barriers per result and four bytes took 0.3 us more at D = 32.
+template <int D, int W, int N, int WAVE_BYTES>
+__device__ __forceinline__ void leave_sums(const floatx16 (&acc)[N][D / 32], uint32_t own_lds, int lane) {
+  static_assert(WAVE_BYTES >= N * D * 128, "a wave's sums take its blocks' place");
+  if constexpr (W > 1) {
 #pragma unroll
-  for (int r = 0; r < D / 2; ++r) red[(wave * (D / 2) + r) * 64 + lane] = acc[r / 16][r % 16] * weight;
+    for (int u = 0; u < N * D / 8; ++u) {
+      const floatx16& a = acc[u / (D / 8)][u % (D / 8) / 4];
+      const int r = u % 4 * 4;
+      *(DEERS_LDS floatx4*)(uintptr_t)(own_lds + lane * 16 + u * 1024) = floatx4{a[r], a[r + 1], a[r + 2], a[r + 3]};
+    }
+  }
   __syncthreads();
+}
+template <int D, int W, int N, int WAVE_BYTES, bool WEIGHTED = false>
+__device__ __forceinline__ void store_sums(const floatx16 (&acc)[N][D / 32], uint32_t first_lds, const float* weight,
+                                           const float* mul, float* const* dst, bool store, int wave, int lane) {
+  constexpr int U = D / 8;
 #pragma unroll
-  for (int i = 0; i < D / 8 / W; ++i) {
-    const int u = wave + i * W;  // registers 4 u .. 4 u + 3: four columns
+  for (int i = 0; i < N * U / W; ++i) {
+    const int u = W == 1 ? i : wave + i * W;
     floatx4 s;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float t = red[(4 * u + e) * 64 + lane];
+    for (int w = 0; w < W; ++w) {
+      floatx4 t;
+      if constexpr (W == 1) {
+        const floatx16& a = acc[i / U][i % U / 4];
+        const int r = i % 4 * 4;
+        t = floatx4{a[r], a[r + 1], a[r + 2], a[r + 3]};
+      } else {
+        t = lds_read_float4_at(first_lds + w * WAVE_BYTES + u * 1024 + lane * 16);
+      }
 #pragma unroll
-      for (int w = 1; w < W; ++w) t += red[(w * (D / 2) + 4 * u + e) * 64 + lane];
-      s[e] = t * mul;
+      for (int e = 0; e < 4; ++e) {
+        const float x = WEIGHTED ? t[e] * weight[w] : t[e];
+        s[e] = w ? s[e] + x : x;
+      }
     }
-    if (store) *(floatx4*)(dst + 32 * (u / 4) + 8 * (u % 4) + 4 * (lane >> 5)) = s;
+    const bool second = N > 1 && u >= U;
+    s *= second ? mul[N - 1] : mul[0];
+    float* const row = second ? dst[N - 1] : dst[0];
+    if (store) *(floatx4*)(row + 32 * (u % U / 4) + 8 * (u % 4) + 4 * (lane >> 5)) = s;
   }
 }
 
 template <int D, int W>
-constexpr size_t split32_lds() {  // a block of each of two operands per wave, or the merge; row statistics
-  return std::max((size_t)W * 2 * Split32<D>::BB, (size_t)W * (D / 2) * 64 * sizeof(float)) + W * 64 * sizeof(float);
+constexpr size_t split32_lds() {  // a block of each of two operands per wave, or its sums; row statistics
+  return (size_t)W * 2 * Split32<D>::BB + W * 64 * sizeof(float);
 }
 template <int D, int W>
 __device__ __forceinline__ float* split32_stats(char* smem) {

@@ -396,7 +396,8 @@ constexpr size_t split_fwd_lds() {  // blocks of every wave, as large as its acc
 }
 
 template <int D, int W, bool DOUBLE>
-__global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams p, int BH, int n_blocks) {
+__global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams p, int BH, int n_blocks, int cus,
+                                                                      int scaled_q) {
   using C = SplitCfg<D>;
   constexpr int KS = C::KS, DB = C::DB, A = kSplitAhead, kWave = (DOUBLE ? 4 : 2) * C::BB;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5, T = p.T;
   int bh, rank;
-  if (!map_block_even(blockIdx.x, n_blocks, BH, &bh, &rank)) return;
+  if (!map_block_even(paired_block(blockIdx.x, gridDim.x, cus), n_blocks, BH, &bh, &rank)) return;
   const int qb = n_blocks - 1 - rank;  // longest rows first
   const int b_ = bh / p.H, h_ = bh % p.H;
   const int qrow = 32 * qb + (lane & 31);
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
     K.request_all(kb, p.k, p.sk, b_, h_, T, ring, lane);
     if (!kQInV) V.request_all(kb, p.v, p.sv, b_, h_, T, ring + C::BB, lane);
   }
-  const float c = p.scaled_q ? 1.f : p.scale_log2;
+  const float c = scaled_q ? 1.f : p.scale_log2;
   floatx16 oacc[1][DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) oacc[0][db] = ZERO16;
@@ -438,7 +439,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
     settle_lds_reads();
     V.request_all(kb, p.v, p.sv, b_, h_, T, ring + C::BB, lane);
   }
-  if (p.scaled_q) scale_frags<KS>(qf, p.scale_log2);
+  if (scaled_q) scale_frags<KS>(qf, p.scale_log2);
 
   float m = -INFINITY, l = 0.f;
   SplitFrags<D> at(ring, lane);
@@ -862,14 +863,19 @@ __global__ __launch_bounds__(64 * W, D == 128 ? 1 : 2) void attn_bwd_f16_split_k
 }
 
 template <int D, int W, bool DOUBLE>
-void launch_fwd_split(const FwdParams& p, int BH, hipStream_t stream) {
+void launch_fwd_split(const FwdParams& p, int BH, bool scaled_q, hipStream_t stream) {
   const auto kernel = attn_fwd_f16_split_kernel<D, W, DOUBLE>;
   constexpr size_t lds = split_fwd_lds<D, W, DOUBLE>();
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
   const int n_blocks = (p.T + 31) / 32;
-  hipLaunchKernelGGL(kernel, dim3(map_even_blocks(n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
+  const int grid = map_even_blocks(n_blocks, BH);
+  // even CU totals at D = 128 (15 x 777 10.6 -> 10.3 us, 9 x 1500 15.2 -> 14.6); below it the launch is the chain of its
+  // longest wave, which should start first (9 x 1500 x 64 10.3 -> 11.0)
+  static PairedState paired;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), lds, stream, p, BH, n_blocks,
+                     D == 128 ? paired_cus(paired, kernel, 64 * W, lds, grid) : 0, (int)scaled_q);
 }
 template <int D, int W, bool SCALED_Q = false>
 void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
@@ -904,7 +910,7 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // From 9 blocks on some lines lie lower than the times would have them: at 9 to 12 blocks, in the backward at D = 128 up
 // to 23 and at D = 32 at 17 to 20 (100 x 384 x 64 backward 22.5 / 20.8, 83 x 384 x 128 39.0 / 30.3, 20 x 512 x 128 27.5 / 18.9):
 // the tests of what the 128-row kernels hand over, and of strided rows in them, have their shapes just above.
-// What the backward takes the forward takes too: then both form their scores from Q itself (FwdParams::scaled_q).
+// What the backward takes the forward takes too: then both form their scores from Q itself (`scaled_q`: the other way).
 struct SplitSize {
   int64_t nb, u;
   SplitSize(int64_t BH, int64_t T, int64_t D) : nb((T + 31) / 32), u(BH * nb * D / 64) {}
@@ -949,28 +955,28 @@ static int bwd_waves(const SplitSize& z, int64_t D) {
 }
 
 template <int D, int W>
-static void launch_fwd(const FwdParams& p, int BH, bool twice, hipStream_t stream) {
+static void launch_fwd(const FwdParams& p, int BH, bool twice, bool scaled_q, hipStream_t stream) {
   if constexpr (W == 4) {
-    if (twice) return launch_fwd_split<D, W, true>(p, BH, stream);
+    if (twice) return launch_fwd_split<D, W, true>(p, BH, scaled_q, stream);
   }
-  launch_fwd_split<D, W, false>(p, BH, stream);
+  launch_fwd_split<D, W, false>(p, BH, scaled_q, stream);
 }
 template <int D>
-static void launch_fwd(const FwdParams& p, int BH, hipStream_t stream) {
+static void launch_fwd(const FwdParams& p, int BH, bool scaled_q, hipStream_t stream) {
   const SplitSize z(BH, p.T, D);
   const int w = fwd_waves(z, D);
   const bool twice = w >= 4 && fwd_twice(z, D);
   if (w >= 4)
-    launch_fwd<D, 4>(p, BH, twice, stream);
+    launch_fwd<D, 4>(p, BH, twice, scaled_q, stream);
   else if (w >= 2)
-    launch_fwd<D, 2>(p, BH, twice, stream);
+    launch_fwd<D, 2>(p, BH, twice, scaled_q, stream);
   else
-    launch_fwd<D, 1>(p, BH, twice, stream);
+    launch_fwd<D, 1>(p, BH, twice, scaled_q, stream);
 }
 template <int D>
-static void launch_bwd(const BwdParams& p, int BH, hipStream_t stream) {
+static void launch_bwd(const BwdParams& p, int BH, bool scaled_q, hipStream_t stream) {
   const int w = bwd_waves(SplitSize(BH, p.T, D), D);
-  if (p.scaled_q)
+  if (scaled_q)
     launch_bwd_split<D, 4, true>(p, BH, stream);
   else if (w >= 4)
     launch_bwd_split<D, 4>(p, BH, stream);
@@ -980,20 +986,20 @@ static void launch_bwd(const BwdParams& p, int BH, hipStream_t stream) {
     launch_bwd_split<D, 1>(p, BH, stream);
 }
 
-void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream) {
+void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, bool scaled_q, hipStream_t stream) {
   LaunchScope scope("attn_fwd_f16", stream);
   switch (D) {
-    case 32: launch_fwd<32>(p, B * p.H, stream); break;
-    case 64: launch_fwd<64>(p, B * p.H, stream); break;
-    case 128: launch_fwd<128>(p, B * p.H, stream); break;
+    case 32: launch_fwd<32>(p, B * p.H, scaled_q, stream); break;
+    case 64: launch_fwd<64>(p, B * p.H, scaled_q, stream); break;
+    case 128: launch_fwd<128>(p, B * p.H, scaled_q, stream); break;
   }
 }
-void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream) {
+void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, bool scaled_q, hipStream_t stream) {
   LaunchScope scope("attn_bwd_f16", stream);
   switch (D) {
-    case 32: launch_bwd<32>(p, B * p.H, stream); break;
-    case 64: launch_bwd<64>(p, B * p.H, stream); break;
-    case 128: launch_bwd<128>(p, B * p.H, stream); break;
+    case 32: launch_bwd<32>(p, B * p.H, scaled_q, stream); break;
+    case 64: launch_bwd<64>(p, B * p.H, scaled_q, stream); break;
+    case 128: launch_bwd<128>(p, B * p.H, scaled_q, stream); break;
   }
 }
 

@@ -17,16 +17,19 @@
 // dQ, dK and dV are reproducible bit for bit.
 //
 // A wave's first loads and its merge cost it some 10 K clocks; blocks are dealt so that every XCD has
-// the same number of them also when the heads are not a multiple of eight (map_block_even).
+// the same number of them also when the heads are not a multiple of eight (map_block_even), and, while all are resident
+// at once, so that the CUs have even totals (paired_block; 24 x 256 x 32 backward 11.3 -> 10.3 us, 12 x 512 x 32 17.4 ->
+// 14.4, forward 24 x 512 x 64 17.9 -> 14.3; not at head width 128, where one workgroup fills a CU and the index
+// arithmetic costs the forward 6 %).
 //
 // A product costs 64 clocks of matrix pipe per two elements of D (v_mfma_f32_32x32x2_f32), so the
 // pipe is the bound as long as a wave's blocks arrive in time.  The operand whose block is asked for
 // last is the one that the next stage needs second, so that both requests are covered by a product
 // (2048 clocks at D = 64).
 //
-// us, forward / backward, 128-row kernels -> these: 24 heads x 256 x 32 15.6 / 26.9 -> 5.9 / 11.3, 12 x 512 x 64
-// 41 / 66 -> 14 / 32, 12 x 1024 x 64 77 / 119 -> 28 / 67, 3 x 4096 x 32 191 / 337 -> 55 / 129, 8 x 256 x 128 48 / 98
-// -> 16 / 31.
+// us, forward / backward, 128-row kernels -> these: 24 heads x 256 x 32 15.6 / 26.9 -> 5.8 / 10.1, 12 x 512 x 64
+// 41 / 66 -> 14 / 32, 12 x 1024 x 64 77 / 119 -> 23 / 67, 3 x 4096 x 32 191 / 337 -> 55 / 129, 8 x 256 x 128 48 / 98
+// -> 15 / 29.
 #include <algorithm>
 
 #include "attn_f32_blocks.h"
@@ -38,7 +41,7 @@ namespace {
 // ---- forward ----
 
 template <int D, int W>
-__global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f32_split_kernel(FwdParams p, int BH, int n_blocks) {
+__global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f32_split_kernel(FwdParams p, int BH, int n_blocks, int cus) {
   using C = Split32<D>;
   constexpr int KH = C::KH, DB = C::DB;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -46,7 +49,7 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5, T = p.T;
   int bh, rank;
-  if (!map_block_even(blockIdx.x, n_blocks, BH, &bh, &rank)) return;
+  if (!map_block_even(D == 128 ? blockIdx.x : paired_block(blockIdx.x, gridDim.x, cus), n_blocks, BH, &bh, &rank)) return;
   const int qb = n_blocks - 1 - rank;  // longest rows first
   const int b = bh / p.H, h = bh % p.H;
   const float* K = (const float*)p.k + b * p.sk.b + h * p.sk.h;
@@ -66,9 +69,9 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
 #pragma unroll
   for (int k = 0; k < KH; ++k) qf[k] *= p.scale_log2;
 
-  floatx16 oacc[DB];
+  floatx16 oacc[1][DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) oacc[db] = ZERO16;
+  for (int db = 0; db < DB; ++db) oacc[0][db] = ZERO16;
   // The reference m of a row's exponentials is the maximum of its first block, and moves when a later
   // score exceeds it by more than 2^8: `ref` is -m in the layout of the products, which start from it, so
   // that the usual stage has no subtraction and no rescaling (some 60 of 110 vector instructions).
@@ -100,7 +103,7 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
       const float alpha = fast_exp2(m - m_new);  // the first block's scales zeros
       l *= alpha;
 #pragma unroll
-      for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+      for (int db = 0; db < DB; ++db) oacc[0][db] *= alpha;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         s[r] -= kLazy ? m_new - m : m_new;
@@ -120,7 +123,7 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
       wait_vmcnt<C::NI>();  // V
     else
       wait_vmcnt<0>();
-    accumulate<D>(oacc, v_blk, s, lane);
+    accumulate<D>(oacc[0], v_blk, s, lane);
     if (more) {
       settle_lds_reads();
       load_block<D>(V, svt, 32 * (kb + W), T, v_blk, lane);
@@ -136,14 +139,19 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
     stat_m[wave * 32 + lane] = m;
     stat_l[wave * 32 + lane] = l;
   }
-  __syncthreads();
-  float M = -INFINITY, L = 0.f;
+  settle_lds_reads();
+  leave_sums<D, W, 1, 2 * C::BB>(oacc, k_blk, lane);
+  float M = -INFINITY, L = 0.f, weight[W];
 #pragma unroll
   for (int w = 0; w < W; ++w) M = fmaxf(M, stat_m[w * 32 + (lane & 31)]);
 #pragma unroll
-  for (int w = 0; w < W; ++w) L += stat_l[w * 32 + (lane & 31)] * fast_exp2(stat_m[w * 32 + (lane & 31)] - M);
-  float* orow = (float*)p.o + b * p.so.b + h * p.so.h + (int64_t)min(qrow, T - 1) * p.so.t;
-  merge_store<D, W>(oacc, fast_exp2(m - M), 1.f / L, orow, qrow < T, (float*)smem, wave, lane);
+  for (int w = 0; w < W; ++w) {
+    weight[w] = fast_exp2(stat_m[w * 32 + (lane & 31)] - M);
+    L += stat_l[w * 32 + (lane & 31)] * weight[w];
+  }
+  float* const orow = (float*)p.o + b * p.so.b + h * p.so.h + (int64_t)min(qrow, T - 1) * p.so.t;
+  const float inv = 1.f / L;
+  store_sums<D, W, 1, 2 * C::BB, true>(oacc, lds_address(smem), weight, &inv, &orow, qrow < T, wave, lane);
   if (wave == 0 && g == 0 && qrow < T) p.lse[(int64_t)bh * T + qrow] = (M + fast_log2(L)) * kLn2;
 }
 
@@ -184,9 +192,9 @@ __device__ __forceinline__ void split32_dq(const BwdParams& p, int bh, int qb, c
 #pragma unroll
   for (int k = 0; k < KH; ++k) qf[k] *= p.scale_log2;
 
-  floatx16 dq[DB];
+  floatx16 dq[1][DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dq[db] = ZERO16;
+  for (int db = 0; db < DB; ++db) dq[0][db] = ZERO16;
   for (; kb <= qb; kb += W) {
     const bool more = kb + W <= qb;
     wait_vmcnt<C::NI>();  // V; K's block may be on its way
@@ -207,14 +215,17 @@ __device__ __forceinline__ void split32_dq(const BwdParams& p, int bh, int qb, c
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = fast_exp2(s[r] + lse2) * (dp[r] + nd);
-    accumulate<D>(dq, k_blk, s, lane);
+    accumulate<D>(dq[0], k_blk, s, lane);
     if (more) {
       settle_lds_reads();
       load_block<D>(K, skt, 32 * (kb + W), T, k_blk, lane);
     }
   }
-  float* row = (float*)p.dq + b * p.sdq.b + h * p.sdq.h + (int64_t)qread * p.sdq.t;
-  merge_store<D, W>(dq, 1.f, p.scale, row, qrow < T, (float*)smem, wave, lane);
+  float* const row = (float*)p.dq + b * p.sdq.b + h * p.sdq.h + (int64_t)qread * p.sdq.t;
+  const float mul = p.scale;
+  settle_lds_reads();
+  leave_sums<D, W, 1, 2 * C::BB>(dq, k_blk, lane);
+  store_sums<D, W, 1, 2 * C::BB>(dq, lds_address(smem), nullptr, &mul, &row, qrow < T, wave, lane);
 }
 
 template <int D, int W>
@@ -246,9 +257,9 @@ __device__ __forceinline__ void split32_dkdv(const BwdParams& p, int bh, int kb,
 #pragma unroll
   for (int k = 0; k < KH; ++k) kf[k] *= p.scale_log2;
 
-  floatx16 dk[DB], dv[DB];
+  floatx16 acc[2][DB];  // dK, dV
 #pragma unroll
-  for (int db = 0; db < DB; ++db) dk[db] = dv[db] = ZERO16;
+  for (int db = 0; db < DB; ++db) acc[0][db] = acc[1][db] = ZERO16;
   for (; qb < n_blocks; qb += W) {
     const bool more = qb + W < n_blocks;
     const int row = 32 * qb + (lane & 31), read = min(row, T - 1);
@@ -274,33 +285,35 @@ __device__ __forceinline__ void split32_dkdv(const BwdParams& p, int bh, int kb,
       s[r] = fast_exp2(s[r]);
       dp[r] = s[r] * (dp[r] + d[r]);
     }
-    accumulate<D>(dk, q_blk, dp, lane);
+    accumulate<D>(acc[0], q_blk, dp, lane);
     if (more) {
       settle_lds_reads();
       lse_row = lse[min(32 * (qb + W) + (lane & 31), T - 1)];
       load_block<D>(Q, sqt, 32 * (qb + W), T, q_blk, lane);
     }
-    accumulate<D>(dv, do_blk, s, lane);
+    accumulate<D>(acc[1], do_blk, s, lane);
     if (more) {
       settle_lds_reads();
       load_block<D>(dO, sdot, 32 * (qb + W), T, do_blk, lane);
     }
   }
-  float* dv_row = (float*)p.dv + b * p.sdv.b + h * p.sdv.h + (int64_t)kread * p.sdv.t;
-  float* dk_row = (float*)p.dk + b * p.sdk.b + h * p.sdk.h + (int64_t)kread * p.sdk.t;
-  merge_store<D, W>(dv, 1.f, 1.f, dv_row, krow < T, (float*)smem, wave, lane);
-  merge_store<D, W>(dk, 1.f, p.scale, dk_row, krow < T, (float*)smem, wave, lane);
+  float* const row[2] = {(float*)p.dk + b * p.sdk.b + h * p.sdk.h + (int64_t)kread * p.sdk.t,
+                         (float*)p.dv + b * p.sdv.b + h * p.sdv.h + (int64_t)kread * p.sdv.t};
+  const float mul[2] = {p.scale, 1.f};
+  settle_lds_reads();
+  leave_sums<D, W, 2, 2 * C::BB>(acc, q_blk, lane);
+  store_sums<D, W, 2, 2 * C::BB>(acc, lds_address(smem), nullptr, mul, row, krow < T, wave, lane);
 }
 
 // Ranks alternate between the roles, longest first: rank 2 r is the dK/dV block of keys 32 r ..,
 // rank 2 r + 1 the dQ block as many rows from the end.
 template <int D, int W>
-__global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f32_split_kernel(BwdParams p, int BH, int n_blocks) {
+__global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f32_split_kernel(BwdParams p, int BH, int n_blocks, int cus) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bh, rank;
-  if (!map_block_even(blockIdx.x, 2 * n_blocks, BH, &bh, &rank)) return;
+  if (!map_block_even(D == 128 ? blockIdx.x : paired_block(blockIdx.x, gridDim.x, cus), 2 * n_blocks, BH, &bh, &rank)) return;
   if (rank & 1)
     split32_dq<D, W>(first_argument<BwdParams>(), bh, n_blocks - 1 - (rank >> 1), smem, wave, lane);
   else
@@ -315,7 +328,10 @@ void launch_fwd_split(const FwdParams& p, int BH, hipStream_t stream) {
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
   const int n_blocks = (p.T + 31) / 32;
-  hipLaunchKernelGGL(kernel, dim3(map_even_blocks(n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
+  const int grid = map_even_blocks(n_blocks, BH);
+  static PairedState paired;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), lds, stream, p, BH, n_blocks,
+                     paired_cus(paired, kernel, 64 * W, lds, grid));
 }
 template <int D, int W>
 void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
@@ -325,7 +341,10 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
   if (!attr_set) allow_lds(kernel, lds);
   attr_set = true;
   const int n_blocks = (p.T + 31) / 32;
-  hipLaunchKernelGGL(kernel, dim3(map_even_blocks(2 * n_blocks, BH)), dim3(64 * W), lds, stream, p, BH, n_blocks);
+  const int grid = map_even_blocks(2 * n_blocks, BH);
+  static PairedState paired;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * W), lds, stream, p, BH, n_blocks,
+                     paired_cus(paired, kernel, 64 * W, lds, grid));
 }
 
 }  // namespace

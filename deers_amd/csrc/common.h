@@ -248,7 +248,6 @@ struct FwdParams {
   Strides3 sq, sk, sv, so;
   int H, T;
   float scale_log2;  // scale * log2(e)
-  int scaled_q;      // f16, 32 rows per workgroup: scores from f16(Q * scale_log2), not from Q
 };
 
 // Whether the single-launch f16 backward runs its dQ groups shortest first: when a group
@@ -274,7 +273,6 @@ struct BwdParams {
   Strides3 sq, sk, sv, so, sdo, sdq, sdk, sdv;
   int H, T;
   float scale, scale_log2;
-  int scaled_q;  // as in FwdParams: what the forward that made lse did
 };
 
 struct DecodeParams {
@@ -307,7 +305,7 @@ __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH
   const int whole = BH >> 3, rest = BH & 7;
   // remaining heads' blocks of rank < k on this XCD: t = rank * rest + head, dealt to XCD t % 8
   auto dealt = [&](int k) { return k * rest > xcd ? (k * rest - xcd + 7) >> 3 : 0; };
-  int k = (int)((unsigned)idx * 8u / (unsigned)BH);  // idx * 8 <= the block id, which fits
+  int k = (int)((int64_t)idx * 8 / BH);
   while (whole * (k + 1) + dealt(k + 1) <= idx) ++k;
   while (k > 0 && whole * k + dealt(k) > idx) --k;
   if (k >= n_ranks) return false;
@@ -320,6 +318,37 @@ __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH
   return true;
 }
 __host__ __device__ inline int map_even_blocks(int n_ranks, int BH) { return 8 * (n_ranks * (BH >> 3) + (n_ranks * (BH & 7) + 7) / 8); }
+
+// Block ids for launches whose workgroups are all resident at once, more than one to a CU.  The dispatcher deals an
+// XCD's blocks to its `cus` CUs in turn, so that blocks i, i + cus, .. of an XCD share a CU: longest first, the longest of
+// all would meet on the CUs with one workgroup more than the others.  Here those CUs begin with the shorter ones of
+// the first round, and every second round runs from the other end.  Returns the id in the order of length that block
+// `id` of `grid` takes; cus == 0: itself.
+__host__ __device__ inline int paired_block(int id, int grid, int cus) {
+  if (cus == 0) return id;
+  const int n = grid >> 3, i = id >> 3, round = i / cus, r = i - round * cus;
+  const int last = (n - 1) / cus, more = n - last * cus;  // the CUs r < more have last + 1 workgroups
+  int at = i;
+  if (round == 0) at = r < more ? cus - more + r : r - more;
+  else if (round & 1) at = (round == last ? n : (round + 1) * cus) - 1 - r;
+  return (at << 3) | (id & 7);
+}
+// The CUs of an XCD if that order applies to a launch of `grid` workgroups of this kernel, otherwise 0.  `state` is the
+// caller's static, one per kernel (launches are serialised by the caller).
+struct PairedState { int cus = -1, per_cu = 0; };
+template <typename Kernel>
+inline int paired_cus(PairedState& state, Kernel kernel, int threads, size_t lds, int grid) {
+  if (state.cus < 0) {
+    int dev = 0, all = 0;
+    const bool known = hipGetDevice(&dev) == hipSuccess &&
+                       hipDeviceGetAttribute(&all, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+                       hipOccupancyMaxActiveBlocksPerMultiprocessor(&state.per_cu, kernel, threads, lds) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    state.cus = known ? all / 8 : 0;
+  }
+  const int n = grid >> 3;
+  return n > state.cus && n <= state.per_cu * state.cus ? state.cus : 0;
+}
 
 // The kernel's first argument, fetched where it is asked for.  In a kernel whose branches are roles with
 // arguments of their own, the arguments of all roles fetched before the branch do not fit the scalar

@@ -30,8 +30,9 @@ void launch_attn_fwd_f32(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, hipStream_t stream);
 bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
-void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, hipStream_t stream);
-void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, hipStream_t stream);
+// scaled_q: scores from f16(Q * scale * log2(e)), as the 128-row kernels form them, not from Q
+void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, bool scaled_q, hipStream_t stream);
+void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, bool scaled_q, hipStream_t stream);
 int64_t attn_bwd_f32_default_ds_limit();
 int attn_bwd_f32_heads(int64_t BH, int64_t T, int64_t D, int64_t limit);
 size_t attn_bwd_f32_ds_bytes(int heads, int64_t T);
@@ -753,9 +754,8 @@ int deers_rocm_attn_fwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
   p.H = (int)H; p.T = (int)T;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
-  p.scaled_q = !deers::attn_bwd_f16_split_takes(B * H, T, D);
   if (dtype == DEERS_ROCM_F16 && deers::attn_fwd_f16_split_takes(B * H, T, D))
-    deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+    deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, !deers::attn_bwd_f16_split_takes(B * H, T, D), g_rt.stream);
   else if (dtype == DEERS_ROCM_F16)
     deers::launch_attn_fwd_f16(p, (int)B, (int)D, g_rt.stream);
   else if (deers::attn_fwd_f32_split_takes(B * H, T, D))
@@ -793,11 +793,10 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.H = (int)H; p.T = (int)T;
   p.scale = scale;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
-  p.scaled_q = !deers::attn_bwd_f16_split_takes(B * H, T, D);
   // the forms for launches that cannot fill the device need no workspace and hand nothing over
   // (the test hook of the hand-over asks for the form that does)
   if (dtype == DEERS_ROCM_F16 && !g_rt.bwd_skip_producers && deers::attn_bwd_f16_split_takes(B * H, T, D)) {
-    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, false, g_rt.stream);
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }
@@ -833,7 +832,7 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   bool capturing;
   if (int rc = stream_captures(&capturing)) return rc;
   if (capturing && (flags_grow || ws_bytes > g_rt.workspace.bytes)) {
-    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, g_rt.stream);
+    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, /*scaled_q=*/true, g_rt.stream);
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }
