@@ -44,6 +44,9 @@ template <int D, int W>
 __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f32_split_kernel(FwdParams p, int BH, int n_blocks, int cus) {
   using C = Split32<D>;
   constexpr int KH = C::KH, DB = C::DB;
+  // More than 256 registers in all, so that a SIMD takes one wave: with 208 a CU's workgroups of one or two waves come to lie two
+  // on a SIMD, beside idle ones (12 heads x 2094 x 128 227 us, 149 so; 48 x 1024 197 / 136).
+  if constexpr (D == 128) asm volatile("" ::: "a63");
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
