@@ -277,10 +277,11 @@ struct BwdParams {
 
 struct DecodeParams {
   const void* q; const void* k; const void* v; void* o;
-  float* part_o; float* part_ml;  // split partials: [B*H, splits, D], [B*H, splits, 2]
+  float* part_o; float* part_ml;  // split partials: [B*H - 8*whole, splits, D], [B*H - 8*whole, splits, 2]
   int64_t skb, skh, skl;          // cache strides (elements)
-  int BH, H, L, splits, chunk;
-  int* arrived;  // per head: splits that have written their partial, zero between launches; null: merge by a second launch
+  int BH, H, L;
+  int whole, splits, chunk;  // heads of an XCD that one workgroup each attends over; the others' splits, of `chunk` rows
+  int* arrived;  // per split head: splits that have written their partial, zero between launches; null: merge by a second launch
   float scale_log2;
   // append form: the new token's projections [B,H,D] by element strides in_b, in_h, the
   // D/2 cos / sin entries of its position; its rotated key and its value become cache

@@ -41,7 +41,7 @@ bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D);
 void launch_attn_fwd_f32_split(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f32_split(const BwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_decode_f16(const DecodeParams& p, int B, int D, bool append, hipStream_t stream);
-int decode_pick_splits(int64_t BH, int64_t L, int64_t D, int* chunk);
+int decode_pick_whole(int64_t BH, int64_t L, int64_t D, int* splits, int* chunk);
 void launch_fill(int dtype_f16, void* dst, size_t n, float value, hipStream_t stream);
 void launch_add(int dtype_f16, const void* a, const void* b, void* out, size_t n,
                 hipStream_t stream);
@@ -866,12 +866,13 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
 
 // Where the splits of a decode call's heads meet: the partials in the workspace (or in `ws`, if that is given),
 // and the arrival counters for a merge inside the launch.  Those are null where a second launch merges:
-// splits that may not share an XCD, more of them than `merge_most`, or a call that may run beside another one (a
+// splits that may not share an XCD, or a call that may run beside another one (a
 // captured graph), since calls that overlap would count each other's arrivals.
-static int decode_meeting(deers::DecodeParams* p, int64_t D, void* ws, int merge_most) {
+static int decode_meeting(deers::DecodeParams* p, int64_t D, void* ws) {
   if (p->splits == 1) return DEERS_ROCM_OK;  // nothing to merge
-  const size_t part_o = (size_t)p->BH * p->splits * D * sizeof(float);
-  const size_t part_ml = (size_t)p->BH * p->splits * 2 * sizeof(float);
+  const size_t heads = p->BH - 8 * p->whole;
+  const size_t part_o = heads * p->splits * D * sizeof(float);
+  const size_t part_ml = heads * p->splits * 2 * sizeof(float);
   bool capturing;
   if (ws) {
     if (part_o + part_ml > kScratchBytes)
@@ -885,7 +886,7 @@ static int decode_meeting(deers::DecodeParams* p, int64_t D, void* ws, int merge
   }
   p->part_o = static_cast<float*>(ws);
   p->part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + part_o);
-  if (p->BH <= kDecodeCounters && p->splits <= merge_most && !capturing && same_xcd_handover_now())
+  if (heads <= kDecodeCounters && !capturing && same_xcd_handover_now())
     p->arrived = g_decode_arrivals;
   return DEERS_ROCM_OK;
 }
@@ -912,14 +913,10 @@ static int attn_decode_impl(const char* what, bool no_alloc, int dtype, const vo
       (reinterpret_cast<uintptr_t>(v_cache) & 15) || (reinterpret_cast<uintptr_t>(q) & 15) ||
       (reinterpret_cast<uintptr_t>(o) & 15))
     return fail(DEERS_ROCM_ERR_LAYOUT, "%s: cache rows, q and o must be 16-byte aligned", what);
-  int chunk = 0;
-  const int splits = deers::decode_pick_splits(B * H, L, D, &chunk);
   p.q = q; p.k = k_cache; p.v = v_cache; p.o = o;
-  p.BH = (int)(B * H); p.H = (int)H; p.L = (int)L; p.splits = splits; p.chunk = chunk;
-  // The entry point that allocates nothing has merged by a second launch from the beginning; inside the
-  // launch pays for up to four splits (1 head x 500 x 64 6.5 -> 4.0 us, 48 x 2000 x 64 9.2 -> 8.9), and with many
-  // short ones it does not (12 x 2000 x 64 in 16 splits 6.2 -> 7.1).
-  if (int rc = decode_meeting(&p, D, no_alloc ? g_scratch_ptr : nullptr, no_alloc ? 4 : splits)) return rc;
+  p.BH = (int)(B * H); p.H = (int)H; p.L = (int)L;
+  p.whole = deers::decode_pick_whole(B * H, L, D, &p.splits, &p.chunk);
+  if (int rc = decode_meeting(&p, D, no_alloc ? g_scratch_ptr : nullptr)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, false, g_rt.stream);
   HIP_TRY(hipGetLastError());
@@ -975,13 +972,12 @@ int deers_rocm_attn_decode_append(int dtype, const void* q, const void* k, const
     if ((uintptr_t)ptr & 15) return fail(DEERS_ROCM_ERR_LAYOUT, "attn_decode_append: pointers must be 16-byte aligned");
   deers::DecodeParams p{};
   p.skb = cache_strides[0]; p.skh = cache_strides[1]; p.skl = cache_strides[2];
-  int chunk = 0;
-  const int splits = deers::decode_pick_splits(B * H, pos, D, &chunk);  // over the rows already cached
   p.k = k_cache; p.v = v_cache; p.o = o;
   p.q_in = q; p.k_in = k; p.v_in = v; p.cos_row = cos_row; p.sin_row = sin_row;
   p.in_b = in_strides[0]; p.in_h = in_strides[1];
-  p.BH = (int)(B * H); p.H = (int)H; p.L = (int)pos; p.splits = splits; p.chunk = chunk;
-  if (int rc = decode_meeting(&p, D, nullptr, splits)) return rc;
+  p.BH = (int)(B * H); p.H = (int)H; p.L = (int)pos;
+  p.whole = deers::decode_pick_whole(B * H, pos, D, &p.splits, &p.chunk);  // over the rows already cached
+  if (int rc = decode_meeting(&p, D, nullptr)) return rc;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
   deers::launch_attn_decode_f16(p, (int)B, (int)D, true, g_rt.stream);
   HIP_TRY(hipGetLastError());
