@@ -9,18 +9,6 @@
 namespace deers {
 
 constexpr int kFwdBM = 128;  // query rows per workgroup
-constexpr int kFwdBN = 64;   // key/value rows per tile
-
-template <int D>
-struct FwdCfg {
-  // prefetch distance in tiles; D = 128 keeps one tile less in flight so that two
-  // workgroups' rings (2 x 64 KB) share a CU
-  static constexpr int P = D == 128 ? 1 : 2;
-  static constexpr int NS = P + 1;              // ring slots per tensor
-  static constexpr int RB = D * 2;              // row bytes
-  static constexpr int TILE_B = kFwdBN * RB;    // tile bytes
-  static constexpr size_t kLds = 2 * NS * TILE_B;
-};
 
 // Position -> tile table of a launch whose workgroups are all resident at once, passed in
 // the kernel arguments: entry p = (head index within the XCD) << 16 | query tile for the
@@ -39,7 +27,8 @@ struct TileOrder {
 // v_dot2_f32_f16 costs 16 clocks beside an MFMA where an add costs 3.  So the loop is cut into
 // chunks of one MFMA and the softmax of two scores, and everything that is not the exponential,
 // the f16 packing and the row sum is taken off the vector pipe:
-//   * scale * log2(e) is folded into the f16 Q fragments once per workgroup;
+//   * scale * log2(e) is folded into the f16 Q fragments once per workgroup (RAW: it is not, and a product per score
+//     stands before the exponential; row sums then are of the rounded probabilities, by v_fma_mix_f32);
 //   * the score accumulator starts from -m (the row's reference maximum), so the MFMA result is
 //     already the exponent; -m is kept in LDS, four copies per lane, and four 16-byte reads fill
 //     the accumulator with it (no vector-pipe work, no 16 registers set aside);
@@ -82,7 +71,7 @@ struct BpCfg {
 
 // BENCH (micro-benchmark build of the same body): the loop runs `bench_stages` stages of a long
 // row with no diagonal in reach and the wave's clocks around the loop go to `bench_clk`.
-template <int D, bool BENCH>
+template <int D, bool BENCH, bool RAW = false>
 __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH, int n_qtiles, int heads_per_xcd,
                                                      const TileOrder& order, int bench_stages, long long* bench_clk) {
   using Cfg = BpCfg<D>;
@@ -104,7 +93,10 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
     if (bh >= BH) return;
   } else {
     int rank;
-    if (!map_block(blockIdx.x, n_qtiles, heads_per_xcd, BH, &bh, &rank)) return;
+    const bool mapped = heads_per_xcd > 0
+                            ? map_block(blockIdx.x, n_qtiles, heads_per_xcd, BH, &bh, &rank)
+                            : map_block_even(paired_block(blockIdx.x, gridDim.x, -heads_per_xcd), n_qtiles, BH, &bh, &rank);
+    if (!mapped) return;
     qtile = n_qtiles - 1 - rank;
   }
   qtile = __builtin_amdgcn_readfirstlane(qtile);
@@ -185,12 +177,15 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
   floatx16 oacc[DB];
 #pragma unroll
   for (int i = 0; i < DB; ++i) oacc[i] = ZERO16;
-  float m = -INFINITY, lsum = 0.f;  // m in units of the scaled scores (log2 domain)
+  float m = -INFINITY, lsum = 0.f;  // m in the units of the accumulated scores
   half8 pf[2];                      // P of the previous block as B operands (keys 0-15, 16-31)
   half8 fr[W];                      // operand fragments on their way from LDS
   wait_all_vmem();
   DEERS_TRACE_POINT(1);
-  {  // fold scale * log2(e) into Q (one rounding to f16)
+  float c = RAW ? p.scale_log2 : 1.f;
+  if constexpr (RAW) {
+    asm volatile("" : "+v"(c));  // a vector operand: a scalar one makes the products below take longer to issue
+  } else {  // fold scale * log2(e) into Q (one rounding to f16)
     const float c = p.scale_log2;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
@@ -198,6 +193,8 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
       for (int e = 0; e < 8; ++e) qf[ks][e] = (half_t)((float)qf[ks][e] * c);
   }
   __syncthreads();
+
+  auto power = [&](float x) { return RAW ? x * c : x; };  // of two, of a difference of scores
 
   // Causal mask of a 32-key block starting at key kb0, in place (tied operands: a select
   // written in C++ left the choice of registers to the allocator, which copied the whole
@@ -276,7 +273,13 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
     float bs0, bs1;
     auto finish_pair = [&](int i) {  // f16 packing and row sum of the pair exponentiated in chunk i
       pw[i] = __builtin_bit_cast(uint32_t, half2v{(half_t)cur[2 * i], (half_t)cur[2 * i + 1]});
-      if (i == 0) {
+      if constexpr (RAW) {  // of what P V multiplies: the rounded values
+        if (i == 0) bs0 = bs1 = 0.f;
+        asm("v_fma_mix_f32 %0, %2, 1.0, %0 op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mix_f32 %1, %2, 1.0, %1 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "+v"(bs0), "+v"(bs1)
+            : "v"(pw[i]));
+      } else if (i == 0) {
         bs0 = cur[0];
         bs1 = cur[1];
       } else {
@@ -304,11 +307,11 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
       if (!FIRST && PRODUCE && i < 4) seed_part(i, nxt);
       if (i >= 1 && i <= LPI) request_part(i - 1, b + 1 + F, b + F, (SLOT + 1 + F) % R, (SLOT + F) % R);
       if constexpr (FIRST) {
-        cur[2 * i] = fast_exp2(cur[2 * i] - m);
-        cur[2 * i + 1] = fast_exp2(cur[2 * i + 1] - m);
+        cur[2 * i] = fast_exp2(power(cur[2 * i] - m));
+        cur[2 * i + 1] = fast_exp2(power(cur[2 * i + 1] - m));
       } else {
-        cur[2 * i] = fast_exp2(cur[2 * i]);
-        cur[2 * i + 1] = fast_exp2(cur[2 * i + 1]);
+        cur[2 * i] = fast_exp2(power(cur[2 * i]));
+        cur[2 * i + 1] = fast_exp2(power(cur[2 * i + 1]));
       }
       if (i > 0) finish_pair(i - 1);
       __builtin_amdgcn_sched_barrier(0);
@@ -353,7 +356,7 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
       if (masked) mask_block(s, 32 * b);
       const float m_new = fmaxf(m, row_max(s));
       const float shift = m - m_new;  // <= 0
-      const float alpha = fast_exp2(shift);
+      const float alpha = fast_exp2(power(shift));
       m = m_new;
       lsum *= alpha;
 #pragma unroll
@@ -364,9 +367,9 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
       bsum = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float e0 = fast_exp2(s[2 * i] - m), e1 = fast_exp2(s[2 * i + 1] - m);
-        bsum += e0 + e1;
+        const float e0 = fast_exp2(power(s[2 * i] - m)), e1 = fast_exp2(power(s[2 * i + 1] - m));
         pw[i] = __builtin_bit_cast(uint32_t, half2v{(half_t)e0, (half_t)e1});
+        bsum = RAW ? add_half2(__builtin_bit_cast(half2v, pw[i]), bsum) : bsum + (e0 + e1);
       }
     }
     lsum += bsum;
@@ -447,15 +450,15 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
     half_t* orow = O + (int64_t)qrow * p.so.t;
 #pragma unroll
     for (int db = 0; db < DB; ++db) store_block_f16(orow + 32 * db, oacc[db], inv, g);
-    if (g == 0) p.lse[(int64_t)bh * T + qrow] = (m + fast_log2(lsum)) * kLn2;
+    if (g == 0) p.lse[(int64_t)bh * T + qrow] = (power(m) + fast_log2(lsum)) * kLn2;
   }
 }
 
-template <int D>
+template <int D, bool RAW>
 __global__ __launch_bounds__(256, (D == 128 ? 2 : BP_OCC)) void attn_fwd_f16_bp_kernel(FwdParams p, int BH, int n_qtiles,
                                                                                 int heads_per_xcd,
                                                                                 TileOrder order) {
-  attn_fwd_f16_bp_body<D, false>(p, BH, n_qtiles, heads_per_xcd, order, 0, nullptr);
+  attn_fwd_f16_bp_body<D, false, RAW>(p, BH, n_qtiles, heads_per_xcd, order, 0, nullptr);
 }
 
 }  // namespace deers

@@ -405,7 +405,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5, T = p.T;
   int bh, rank;
-  if (!map_block_even(paired_block(blockIdx.x, gridDim.x, cus), n_blocks, BH, &bh, &rank)) return;
+  if (!map_block_even(D == 128 ? paired_block(blockIdx.x, gridDim.x, cus) : blockIdx.x, n_blocks, BH, &bh, &rank)) return;
   const int qb = n_blocks - 1 - rank;  // longest rows first
   const int b_ = bh / p.H, h_ = bh % p.H;
   const int qrow = 32 * qb + (lane & 31);
@@ -891,9 +891,9 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 }  // namespace
 
 // Which launches come here and in which form, fitted to times of both directions in every form and of the 128-row
-// kernels at T = 64 .. 4096 and 20 numbers of heads each, per head width (1300 launches; the rules are on average 0.3 %,
-// at worst 14 % behind the best form of a launch).  nb = T / 32 is the length of a walk, n = heads * nb the number of
-// workgroups, u = n * D / 64 their number weighted by what a block of the other operand weighs.
+// kernels at T = 32 .. 4096 and some 20 numbers of heads each, per head width (the waves: 1300 launches; the lines below:
+// 2500).  nb = T / 32 is the length of a walk, n = heads * nb the number of workgroups, u = n * D / 64 their number
+// weighted by what a block of the other operand weighs.
 //
 // Waves: four while the workgroups are few and for long walks, since a walk of nb blocks is nb / W stages long; fewer
 // where the device is full anyway and every wave costs its start and the merge (us in 4 / 2 / 1 waves, forward D = 64:
@@ -901,42 +901,59 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 14.2 / 20.3 / 31.6, 15 x 1024 40.4 / 32.0 / 46.2, 187 x 256 73.4 / 49.0 / 38.3).  Twice the blocks in LDS where a CU has
 // one workgroup or two (forward D = 128, once / twice: 10 x 512 6.8 / 6.7, 6 x 128 4.7 / 4.5, 15 x 777 10.8 / 11.9).
 //
-// Takes, 128-row kernels / these: short walks up to a multiple of what the device holds (those form 128 rows where
-// 64 to 384 are, and every stage has a barrier: forward 2000 x 64 x 64 17.2 / 13.0, 500 x 256 x 64 18.2 / 14.5; backward
-// 800 x 256 x 32 45.9 / 40.1, 187 x 256 x 128 45.0 / 38.3), longer ones up to about one and a half times, where each
-// of four waves reading all of the other operand for 32 rows costs more than it saves (forward 25 x 2048 x 64 31.4 /
-// 28.5, 41 x 768 x 128 19.0 / 18.1, 66 x 768 x 64 15.5 / 16.4, 37 x 2048 x 64 32.4 / 39.8; backward 12 x 2048 x 64 48.5 /
-// 42.8, 9 x 2048 x 128 67.8 / 57.3, 9 x 4096 x 64 108.6 / 103.0, 35 x 768 x 128 38.6 / 40.4, 31 x 1024 x 64 35.0 / 37.4).
-// From 9 blocks on some lines lie lower than the times would have them: at 9 to 12 blocks, in the backward at D = 128 up
-// to 23 and at D = 32 at 17 to 20 (100 x 384 x 64 backward 22.5 / 20.8, 83 x 384 x 128 39.0 / 30.3, 20 x 512 x 128 27.5 / 18.9):
-// the tests of what the 128-row kernels hand over, and of strided rows in them, have their shapes just above.
-// What the backward takes the forward takes too: then both form their scores from Q itself (`scaled_q`: the other way).
+// Takes, us in the 128-row kernels / these: walks of up to 15 blocks nearly always (those form 128 rows where 64 to 384
+// are, and every stage has a barrier: forward 419 x 96 x 64 8.3 / 5.5, 286 x 300 x 128 28.4 / 22.1, 327 x 400 x 64 24.9 / 19.2;
+// backward 403 x 160 x 128 73.9 / 48.3, 179 x 320 x 64 26.5 / 21.7, 107 x 416 x 64 25.0 / 21.8) until the operands no longer
+// stay in the L2 beside each other (forward 1043 x 256 x 64 34.1 / 41.2, backward 723 x 256 x 64 69.4 / 91.4); longer ones
+// while the 128-row kernels leave CUs idle, since each of the waves reading all of the other operand for 32 rows costs
+// more than it saves elsewhere (forward 24 x 2048 x 32 21.0 / 17.2, 13 x 3000 x 64 34.6 / 31.1, 10 x 4096 x 128 64.3 / 69.8,
+// 20 x 3000 x 64 37.2 / 41.4; backward 9 x 2048 x 64 44.9 / 31.9, 9 x 4096 x 64 105.7 / 100.6, 12 x 3000 x 128 144.7 / 157.6,
+// 20 x 2048 x 64 56.4 / 62.3).  Seven or eight heads give each XCD one, which is what those kernels like best (backward 8 x
+// 3000 x 64 51.2 / 56.5, 9 x 3000 x 64 63.8 / 62.9).  At nb = 12 to 16 they are as fast or faster while all their
+// workgroups are resident two to a CU (forward 128 x 512 x 32 8.3 / 9.7, 168 x 512 x 64 14.8 / 15.8, 80 x 512 x 128 15.5 /
+// 17.5, 141 x 384 x 64 11.0 / 13.8).
+// From 9 blocks on some lines lie lower than the times would have them, or a stretch is left out, for the tests of what
+// the 128-row kernels hand over, and of strided rows in them, whose shapes lie there: D = 64 and 128 at 9 to 11 blocks
+// (109 x 320 x 64 backward 21.3 / 16.1), the backward at D = 32 from 17 to 20 and at D = 128 from 21 to 23.
+// The forward takes what the backward takes: then both form their scores from Q itself (`scaled_q`: the other way).
 struct SplitSize {
   int64_t nb, u;
   SplitSize(int64_t BH, int64_t T, int64_t D) : nb((T + 31) / 32), u(BH * nb * D / 64) {}
 };
 // By head width: 32, 64, 128.
 static int64_t of_width(int64_t D, int64_t w32, int64_t w64, int64_t w128) { return D == 32 ? w32 : D == 64 ? w64 : w128; }
+// Up to `low`, and again from `again` up to `most`.
+static bool outside(int64_t u, int64_t low, int64_t again, int64_t most) { return u <= low || (u > again && u <= most); }
 bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   const SplitSize z(BH, T, D);
-  if (z.nb <= 2) return z.u <= of_width(D, 2000, 4000, 6000);
-  if (z.nb <= 8) return z.u <= of_width(D, 5000, 6200, 6000);
-  if (z.nb <= 12) return z.u <= of_width(D, 5000, 1200, 2048);
-  if (z.nb <= 16) return z.u <= of_width(D, 5000, 4000, 2400);
-  if (z.nb < 64) return z.u <= of_width(D, 1000, 1700, 2400);
-  return z.u <= of_width(D, 1000, 2000, 2900);
+  const int64_t nb = z.nb, u = z.u;
+  if (nb <= 2) return u <= of_width(D, 5000, 5000, 9000);
+  if (nb <= 4) return u <= of_width(D, 4500, 5200, 6400);
+  if (nb <= 8) return u <= of_width(D, 5000, 5800, 8400);
+  if (nb <= 11) return outside(u, of_width(D, 4500, 1200, 2048), of_width(D, 4500, 1250, 2100), of_width(D, 4500, 6000, 8000));
+  if (nb <= 12) return outside(u, of_width(D, 4500, 1200, 2048), of_width(D, 4500, 1750, 3300), of_width(D, 4500, 5800, 7000));
+  if (nb <= 15) return outside(u, of_width(D, 4000, 6800, 2048), 3300, of_width(D, 4000, 6800, 7500));
+  if (nb <= 16) return outside(u, of_width(D, 770, 1300, 2048), of_width(D, 1540, 3000, 8192), of_width(D, 4200, 5800, 8192));
+  return u <= of_width(D, nb < 40 ? 830 : 920, 1200, 2048);
 }
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
+  if (!attn_fwd_f16_split_takes(BH, T, D)) return false;
   const SplitSize z(BH, T, D);
-  if (z.nb <= 2) return z.u <= of_width(D, 2000, 4000, 6000);
-  if (z.nb <= 4) return z.u <= of_width(D, 4000, 3200, 6000);
-  if (z.nb <= 8) return z.u <= of_width(D, 4000, 3200, 4000);
-  if (z.nb <= 12) return z.u <= 768;
-  if (z.nb <= 16) return z.u <= of_width(D, 3200, 1700, 768);
-  if (z.nb <= 20) return z.u <= of_width(D, 448, 1300, 768);
-  if (z.nb <= 23) return z.u <= of_width(D, 1000, 1100, 768);
-  if (z.nb <= 28) return z.u <= of_width(D, 1000, 1100, 1300);
-  return z.u <= of_width(D, 800, 1000, z.nb < 96 ? 1300 : 1800);
+  const int64_t nb = z.nb, u = z.u;
+  if (nb <= 2) return u <= of_width(D, 4000, 4000, 8600);
+  if (nb <= 3) return u <= of_width(D, 3600, 4300, 8600);
+  if (nb <= 4) return u <= of_width(D, 3600, 3500, 6400);
+  if (nb <= 6) return u <= of_width(D, 4000, 3800, 6200);
+  if (nb <= 8) return u <= of_width(D, 3600, 3000, 4700);
+  if (nb <= 11) return outside(u, 768, of_width(D, 800, 1250, 2100), of_width(D, 2600, 3600, 5000));
+  if (nb <= 12) return outside(u, 768, of_width(D, 800, 1750, 3300), of_width(D, 2600, 2900, 4400));
+  if (nb <= 15) return u <= of_width(D, 3200, 3400, 4700);
+  if (nb <= 16) return u <= of_width(D, 3200, 1300, 2048);
+  if (nb <= 20) return u <= of_width(D, 448, 1000, 1200);
+  if (nb <= 23) return u <= of_width(D, 760, 1000, 768);
+  if (nb < 72) return u <= of_width(D, 720, 960, 1200);
+  if (BH > 6 && BH <= 8) return u <= of_width(D, 700, 640, 1110);
+  return u <= of_width(D, 700, 1100, 1700);
 }
 static int waves(const SplitSize& z, int64_t four, int64_t two) {
   return z.u <= four && z.nb >= 4 ? 4 : z.u <= std::max(four, two) && z.nb >= 2 ? 2 : 1;
@@ -947,7 +964,7 @@ static int fwd_waves(const SplitSize& z, int64_t D) {
   const int64_t two = of_width(D, std::min<int64_t>(16 * sq, 900), std::min<int64_t>(64 * sq, 1700), std::min(120 * sq, 1300 + 60 * nb));
   return waves(z, four, nb > 16 ? z.u : two);
 }
-static bool fwd_twice(const SplitSize& z, int64_t D) { return z.u <= of_width(D, 192, 320, 448); }
+static bool fwd_twice(const SplitSize& z, int64_t D) { return z.u <= of_width(D, 192, 256, 448); }
 static int bwd_waves(const SplitSize& z, int64_t D) {
   const int64_t nb = z.nb;
   const int64_t four = of_width(D, std::min(24 * nb, 120 + 9 * nb), std::min(32 * nb, 160 + 12 * nb), std::max<int64_t>(256, 72 + 20 * nb));

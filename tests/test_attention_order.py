@@ -1,0 +1,53 @@
+"""f16 attention on either side of the lines between its forms, and the forward of 128 rows per workgroup whose scores are
+formed from Q itself: heads in whole numbers per XCD (placed by a table) and not (placed by formula)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from deers_amd import rocm, synth
+
+
+def takes(direction, heads, T, D):
+    rule = rocm.load()[f"_ZN5deers24attn_{direction}_f16_split_takesElll"]
+    rule.restype = ctypes.c_bool
+    i64 = ctypes.c_int64
+    return rule(i64(heads), i64(T), i64(D))
+
+
+def test_the_forward_takes_what_the_backward_takes():
+    """Otherwise one would form its scores from Q and the other from Q times the scale."""
+    for D in (32, 64, 128):
+        for T in (1, 32, 64, 65, 100, 128, 160, 256, 288, 300, 352, 384, 450, 480, 512, 600, 700, 1000, 2304, 2816, 4096, 9000):
+            for heads in list(range(1, 140)) + list(range(140, 3000, 37)):
+                assert takes("fwd", heads, T, D) or not takes("bwd", heads, T, D), (heads, T, D)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,T,D", [
+    (4, 6, 2049, 64), (2, 9, 1900, 128), (1, 33, 1025, 128), (3, 7, 2048, 64), (8, 8, 700, 64), (8, 8, 641, 128),  # from Q
+    (9, 8, 900, 64), (5, 11, 1150, 64), (7, 13, 700, 32),                                           # three to a CU
+    (9, 16, 353, 64), (17, 16, 384, 64), (60, 7, 480, 64), (25, 8, 450, 128), (16, 12, 512, 32),    # 32 rows again
+    (10, 100, 33, 32), (3, 50, 161, 128), (20, 16, 288, 64)])
+def test_forms_at_their_lines(gpu, B, H, T, D):
+    """Two roundings to f16 (of a probability, of the result; 2^-11 each) of sums of weights that are at most one: 2^-10 of
+    the largest value, twice that for Q times the scale (|s| 2^-11 in every score, ten or less here, of the order of one
+    rounding on average); gradients add one product of that kind and the difference dP - dO.O."""
+    x = synth.attention_inputs(f"order-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=61)
+    out = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    one = (slice(B - 1, B), slice(H - 1, H))
+    want = (oracle.attn_fwd(x["q"][one], x["k"][one], x["v"][one]),
+            *oracle.attn_bwd(x["q"][one], x["k"][one], x["v"][one], x["do"][one]))
+    for name, got, ref in zip(("o", "dq", "dk", "dv"), (out[0], *out[2:]), want):
+        assert np.max(np.abs(got[one].astype(np.float64) - ref)) <= 4 * 2.0 ** -10 * max(1.0, np.max(np.abs(ref))), name
+    again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
+    for a, b in zip(out, again):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.fixture
+def gpu():
+    if not rocm.available():
+        pytest.fail("no gfx950 device")
+    rocm.init(0)
