@@ -301,18 +301,16 @@ struct SkinnyPrefetch {
 // Block ids for launches of few heads, where whole heads per XCD leave XCDs idle (12 heads: 2, 2, 2, 2,
 // 1, 1, 1, 1): BH / 8 whole heads per XCD, and the blocks of the BH % 8 remaining heads dealt to all
 // XCDs in turn.  An XCD's list is still ordered by rank.  The grid is map_even_blocks(n_ranks, BH).
+// An XCD's blocks of ranks below k are (k * BH + 7 - xcd) / 8: it holds every eighth of the blocks in order of rank.
 __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH, int* bh, int* rank) {
-  const int xcd = block_id & 7, idx = block_id >> 3;
-  const int whole = BH >> 3, rest = BH & 7;
-  // remaining heads' blocks of rank < k on this XCD: t = rank * rest + head, dealt to XCD t % 8
-  auto dealt = [&](int k) { return k * rest > xcd ? (k * rest - xcd + 7) >> 3 : 0; };
-  int k = (int)((int64_t)idx * 8 / BH);
-  while (whole * (k + 1) + dealt(k + 1) <= idx) ++k;
-  while (k > 0 && whole * k + dealt(k) > idx) --k;
+  const int xcd = block_id & 7, whole = BH >> 3, rest = BH & 7;
+  const int k = (int)((unsigned)block_id / (unsigned)BH);
   if (k >= n_ranks) return false;
-  const int in_rank = idx - (whole * k + dealt(k)), extra = dealt(k + 1) - dealt(k);
+  // remaining heads' blocks of rank < k on this XCD: t = rank * rest + head, dealt to XCD t % 8
+  const int dealt = (k * rest + 7 - xcd) >> 3, extra = (((k + 1) * rest + 7 - xcd) >> 3) - dealt;
+  const int in_rank = (block_id >> 3) - (whole * k + dealt);
   if (in_rank < extra)
-    *bh = 8 * whole + (8 * (dealt(k) + in_rank) + xcd) % rest;
+    *bh = 8 * whole + (8 * (dealt + in_rank) + xcd) % rest;
   else
     *bh = (in_rank - extra) * 8 + xcd;
   *rank = k;
@@ -349,6 +347,18 @@ inline int paired_cus(PairedState& state, Kernel kernel, int threads, size_t lds
   }
   const int n = grid >> 3;
   return n > state.cus && n <= state.per_cu * state.cus ? state.cus : 0;
+}
+
+// Fetches the first BYTES of a kernel's arguments at its start.  They come from memory that no cache has yet, a line of
+// 64 bytes at a time; left alone the compiler asks for them where they are used, and the trips follow each other.
+template <int BYTES>
+__device__ __forceinline__ void fetch_arguments() {
+  const auto ptr = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int LINES = (BYTES + 63) / 64, LAST = LINES - 1;
+  static_assert(LINES <= 8);
+  asm volatile("" ::"s"(ptr[0]), "s"(ptr[16 * (LAST < 1 ? LAST : 1)]), "s"(ptr[16 * (LAST < 2 ? LAST : 2)]),
+               "s"(ptr[16 * (LAST < 3 ? LAST : 3)]), "s"(ptr[16 * (LAST < 4 ? LAST : 4)]), "s"(ptr[16 * (LAST < 5 ? LAST : 5)]),
+               "s"(ptr[16 * (LAST < 6 ? LAST : 6)]), "s"(ptr[16 * LAST]));
 }
 
 // The kernel's first argument, fetched where it is asked for.  In a kernel whose branches are roles with

@@ -37,6 +37,7 @@ struct RopeParams {
 // INVERSE = true : src is the gradient of the rotated heads, dst the projection grad.
 template <typename T, bool INVERSE>
 __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
+  fetch_arguments<sizeof(RopeParams)>();
   typedef typename Vec16<T>::type V;
   constexpr int N = Vec16<T>::N;
   const int half_chunks = p.D / 2 / N;  // 16-byte chunks in half a row
@@ -71,6 +72,7 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
 // tests/gpt.rs:38-49) or rows that are not 16-byte aligned.  Same arithmetic and rounding.
 template <typename T, bool INVERSE>
 __global__ __launch_bounds__(256) void rope_pair_kernel(RopeParams p) {
+  fetch_arguments<sizeof(RopeParams)>();
   const int half = p.D / 2;
   const int64_t total = (int64_t)p.B * p.T * p.H * half;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total;
@@ -106,6 +108,7 @@ struct DecodeQkvParams {
 };
 template <typename T>
 __global__ __launch_bounds__(256) void decode_qkv_kernel(DecodeQkvParams p) {
+  fetch_arguments<sizeof(DecodeQkvParams)>();
   typedef typename Vec16<T>::type V;
   constexpr int N = Vec16<T>::N;
   const int half_chunks = p.D / 2 / N;

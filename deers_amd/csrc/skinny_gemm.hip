@@ -59,6 +59,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
                                                               int64_t w_block_stride, int main_blocks,
                                                               const char* __restrict__ next_w,
                                                               int next_tiles, int next_tile_bytes) {
+  fetch_arguments<120>();
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int)blockIdx.x >= main_blocks) {
