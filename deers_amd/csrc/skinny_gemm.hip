@@ -31,6 +31,9 @@
 //          a row-major W is 64 bytes out of every row, and fetched from HBM (a generation
 //          step cycles through more weights and cache than the last-level cache holds) such
 //          scattered pieces cost 2-3 us per launch more than the same bytes in one run.
+// A product of this size is a chain of latencies: its arguments, the first chunk, the waves' sums, the meeting.  us with
+// arguments from memory, divisions by S and sums by single dwords through LDS, and as it is (32 rows, packed): 768 x 2304
+// 4.19 -> 3.79, 768 x 768 3.94 -> 3.36, 3072 x 768 5.91 -> 5.67, 1024 x 256 4.82 -> 4.08.
 // Shapes: K a multiple of 256 (every wave then owns whole chunks), N a multiple of 8,
 // rows 16-byte aligned; the caller falls back to the library otherwise.
 #include "common.h"
@@ -50,16 +53,17 @@ constexpr int kSkLds = kSkWaves * kSkWaveBytes;  // 96 KB
 constexpr int kSkGather = 4;                     // splits whose partials the last arrival has in flight
 constexpr int kSkPieceBytes = 256 * 64;          // prefetch unit: 256 rows of a packed tile
 
+// The first 56 bytes of the arguments are in scalar registers when a wave starts (-amdgpu-kernarg-preload-count): what the
+// first requests need is among them.  `form`: M, S << 8, packed << 16.  k_per_wave is a
+// multiple of 64.
 template <bool ACCUMULATE, int PROLOGUE>
-__global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __restrict__ x, int64_t ldx,
-                                                              const half_t* __restrict__ W, int64_t ldw,
-                                                              half_t* __restrict__ y, int64_t ldy, int M,
-                                                              int N, int K, int S, float* __restrict__ partial,
-                                                              int* __restrict__ counters, float eps,
-                                                              int64_t w_block_stride, int main_blocks,
-                                                              const char* __restrict__ next_w,
-                                                              int next_tiles, int next_tile_bytes) {
-  fetch_arguments<120>();
+__global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __restrict__ x, const half_t* __restrict__ W,
+                                                              half_t* __restrict__ y, int64_t ldy, int ldx, int ldw,
+                                                              int N, int k_per_wave, int form, int main_blocks,
+                                                              float* __restrict__ partial, int* __restrict__ counters,
+                                                              float eps, int next_tiles, int next_tile_bytes,
+                                                              const char* __restrict__ next_w) {
+  const int M = form & 255, S = (form >> 8) & 255, K = k_per_wave * (S * kSkWaves);
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int)blockIdx.x >= main_blocks) {
@@ -93,11 +97,12 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
   // block id -> (column block, K split): the S splits of a column block share id % 8
   const int n_col_blocks = (N + 31) / 32;
   const int xcd = blockIdx.x & 7, t_id = blockIdx.x >> 3;
-  const int split = t_id % S;
-  const int col_block = (t_id / S) * 8 + xcd;
+  // t_id / S, exact: S > 1 only with fewer than 96 column blocks, far from where the rounding could reach 0.5 / S
+  const int group = __builtin_amdgcn_readfirstlane((int)(((float)t_id + 0.5f) * __builtin_amdgcn_rcpf((float)S)));  
+  const int split = t_id - group * S;
+  const int col_block = group * 8 + xcd;
   if (col_block >= n_col_blocks) return;
   const int n0 = col_block * 32;
-  const int k_per_wave = K / (S * kSkWaves);               // a multiple of 64
   const int n_chunks = k_per_wave / (16 * kSkStepsPerChunk);
   const int k_begin = (split * kSkWaves + wave) * k_per_wave;
   const uint32_t lds_wave = lds_address(smem) + wave * kSkWaveBytes;
@@ -116,7 +121,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
     x_lane_off[i] = (uint32_t)((min(8 * i + (lane >> 3), M - 1) * ldx + 8 * ((lane & 7) ^ (lane >> 3))) * 2);
   // row-major W: the block's 32 columns start 32 elements after the previous block's, rows
   // ldw apart; packed W ([column block][K][32]): blocks K*32 apart, rows 32 apart
-  const half_t* w_base = W + col_block * w_block_stride;
+  const half_t* w_base = W + (int64_t)col_block * (form >> 16 ? K * 32 : 32);
 
   auto issue = [&](int chunk) {
     const uint32_t dst = lds_wave + (chunk % kSkRing) * kSkChunkBytes;
@@ -180,20 +185,25 @@ __global__ __launch_bounds__(256) void skinny_gemm_f16_kernel(const half_t* __re
 
   // ---- reduce the four waves' partial sums (fixed order) and write 16 bytes per lane ----
   __syncthreads();  // every wave is done with its ring: reuse the start of LDS
-  float* red = (float*)smem;  // [wave][reg][lane]
+  float* red = (float*)smem;  // [wave][reg / 4][lane][reg % 4]
 #pragma unroll
-  for (int r = 0; r < 16; ++r) red[(wave * 16 + r) * 64 + lane] = acc[r];
+  for (int q = 0; q < 4; ++q)
+    *(floatx4*)(red + ((wave * 4 + q) * 64 + lane) * 4) = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
   float* red_sq = red + kSkWaves * 16 * 64;  // [wave][lane]
   if constexpr (PROLOGUE == kSkinnyRmsNorm) red_sq[wave * 64 + lane] = sum_sq;
   __syncthreads();
   float s[8];
   if (wave < 2) {
+    floatx4 t[kSkWaves][2];
+#pragma unroll
+    for (int w = 0; w < kSkWaves; ++w)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) t[w][q] = *(const floatx4*)(red + ((w * 4 + 2 * rp + q) * 64 + lane) * 4);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      float t = red[(0 * 16 + 8 * rp + e) * 64 + lane];
+      s[e] = t[0][e / 4][e % 4];
 #pragma unroll
-      for (int w = 1; w < kSkWaves; ++w) t += red[(w * 16 + 8 * rp + e) * 64 + lane];
-      s[e] = t;
+      for (int w = 1; w < kSkWaves; ++w) s[e] += t[w][e / 4][e % 4];
     }
     if constexpr (PROLOGUE == kSkinnyRmsNorm) {
       // row m's sum of squares: both lane halves of all four waves, in a fixed order
@@ -331,9 +341,9 @@ static void launch_one(const void* x, int64_t ldx, const void* w, int64_t ldw, v
   const int pieces = next.w ? (int)(next.k / 256) : 0;  // K % 256 == 0 for every weight the kernel takes
   const dim3 grid((unsigned)(main_blocks + 8 * ((next_tiles + 7) / 8) * pieces));
   hipLaunchKernelGGL((skinny_gemm_f16_kernel<ACCUMULATE, PROLOGUE>), grid, dim3(256), kSkLds, stream,
-                     (const half_t*)x, ldx, (const half_t*)w, packed ? (int64_t)32 : ldw, (half_t*)y, ldy, m, n, k,
-                     splits, partial, counters, eps, packed ? (int64_t)k * 32 : (int64_t)32, main_blocks,
-                     (const char*)next.w, next_tiles, (int)(next.k * 64));
+                     (const half_t*)x, (const half_t*)w, (half_t*)y, ldy, (int)ldx, packed ? 32 : (int)ldw, n, k / (splits * kSkWaves),
+                     m | splits << 8 | (int)packed << 16, main_blocks, partial, counters, eps, next_tiles,
+                     (int)(next.k * 64), (const char*)next.w);
 }
 
 // prologue: kSkinnyPlain, kSkinnyRmsNorm (splits must be 1) or kSkinnyReluSq; packed: w is
