@@ -1,5 +1,5 @@
-// Fused causal attention forward, f32 storage and arithmetic, gfx950: the large launches of head
-// widths 64 and 128 (attn_split_f32.hip has the others and the rule).
+// Fused causal attention forward, f32 storage and arithmetic, gfx950: the launches of head
+// widths 64 and 128 that fill the device many times over (attn_split_f32.hip has the others and the rule).
 //
 // Same decomposition as the f16 kernel (one query column per lane, S^T = K Q^T,
 // O^T += V^T P^T, online softmax in the log2 domain) on v_mfma_f32_32x32x2_f32.

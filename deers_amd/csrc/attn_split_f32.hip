@@ -355,34 +355,45 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 }  // namespace
 
 // Which launches come here and with how many waves per workgroup.  Measured on T = 32 .. 8192, 1 ..
-// 4000 heads and the three head widths against the other kernels and between 1, 2 and 4 waves;
-// nb = T / 32 is the length of a walk, n = heads * nb the number of workgroups.
+// 4000 heads and the three head widths against the other kernels and between 1, 2 and 4 waves (the forward anew: 850
+// launches; its rules are on average 0.4 % behind the best form); nb = T / 32 is the length of a walk, n = heads * nb the
+// number of workgroups.
 //
-// Waves.  Few workgroups: four waves, the shortest chain (D = 64, 12 x 512: forward 14 us, with two
-// waves 23, with one 41).  Many: the SIMDs are covered anyway, and a wave that walks longer pays
-// its start-up and its merge less often (400 x 512 x 64: 154 us in four waves, 138 in one; 300 x 384 x 64
-// 81 / 68); the shorter the walks, the fewer workgroups that takes, and the longer they are, the more
-// are needed for the last ones to end together (96 x 1024 x 64: 129 / 151).  Never more waves than blocks
-// to walk.
+// Waves.  Few workgroups: four waves, the shortest chain (us in 4 / 2 / 1: 13 x 512 x 64 14 / 22 / 39, 25 x 4096 x 64 441 /
+// 500 / 590).  Many: the SIMDs are covered anyway, and a wave that walks longer pays its start-up and its merge less often
+// (168 x 400 x 128 132 / 97 / 83, 480 x 400 x 64 140 / 126 / 113); the shorter the walks, the fewer workgroups that takes, and the
+// longer they are, the more are needed for the last ones to end together.  At head width 128 a SIMD has one wave, so
+// that two or one are enough early (65 x 1024 x 128 208 / 175 / 161).
 //
-// Takes, forward: at head width 32, and for walks of up to eight blocks, always.  Otherwise up to
-// the size where the 128-row kernel's four-fold reuse of a K/V tile decides: every wave here
-// fetches its own blocks (D = 64: 4 x 12 x 1024 69 us against 80, 8 x 12 x 1024 129 against 129; D = 128,
-// 96 x 1024 283 / 261), or where one wave per workgroup will do (192 x 768 x 64: 147 against 150).
+// Takes, forward, us in the 128-row kernel / here: nearly everything, since that one forms 128 rows and has barriers
+// where waves here wait for themselves only (100 x 1024 x 64 143 / 130, 25 x 4096 x 64 559 / 441, 168 x 400 x 128 119 / 83, 65 x 1024
+// x 128 197 / 161, 25 x 4096 x 128 1137 / 928), up to the size where a four-fold reuse of K and V tiles decides (563 x
+// 1024 x 64 705 / 717, 375 x 1024 x 128 950 / 963, 563 x 1024 x 128 1432 / 1583; shorter walks later).  Two stretches are
+// left out that the tests of strided rows in the 128-row kernel have for their shapes.
 bool attn_f32_one_wave(int64_t n, int64_t nb, int64_t D) {
   return n >= (D == 32 ? 4608 + 48 * nb : D == 64 ? 1800 + 80 * nb : 1152 + 48 * nb);
 }
 bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb;
   if (D == 32 || nb <= 8) return true;
-  if (D == 128) return n <= 1536 || (nb <= 12 && attn_f32_one_wave(n, nb, D));
-  return n <= 2048 || (nb >= 48 && n <= 3072) || (nb <= 24 && attn_f32_one_wave(n, nb, D));
+  if (D == 128) return n <= (nb <= 10 ? 18000 : nb >= 13 && nb <= 15 ? 12000 : 9000) && !(nb >= 12 && n > 1656 && n <= 1664);
+  return n <= (nb <= 24 ? 20000 : 16000) && !(n > 2100 && n <= 2112);
 }
 static int fwd_waves(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb;
-  if (n <= 512) return nb >= 4 ? 4 : nb >= 2 ? 2 : 1;
-  if (nb >= 12 && D <= 64) return attn_f32_one_wave(n, nb, D) ? 1 : 4;
-  return n <= 1536 && nb >= 4 && !attn_f32_one_wave(n, nb, D) ? 2 : 1;
+  if (nb < 2) return 1;
+  int64_t four, two;  // workgroups up to which there are as many waves
+  if (D == 32) {
+    four = nb < 10 ? 900 : std::min<int64_t>(6500, 170 * nb - 150);
+    two = nb < 10 ? 220 * nb : 5300;
+  } else if (D == 64) {
+    four = nb < 4 ? 400 : nb < 8 ? 110 * nb : nb < 12 ? 1100 : std::min(175 * nb - 560, 2600 + 36 * nb);
+    two = nb < 11 ? 200 * nb : 3200;
+  } else {
+    four = nb < 9 ? std::max<int64_t>(60 * nb, 200) : std::max<int64_t>(510, 400 + 9 * nb);
+    two = nb < 9 ? std::max<int64_t>(600, 150 * nb) : nb < 12 ? 1180 : nb < 16 ? 1400 : nb >= 48 && n > 2200 ? 3400 : 1650;
+  }
+  return nb >= 3 && n <= four ? 4 : n <= two ? 2 : 1;
 }
 static int bwd_waves(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb, u = n * D / 64;

@@ -46,6 +46,24 @@ def test_forms_at_their_lines(gpu, B, H, T, D):
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,T,D", [
+    (1, 7, 65, 64), (5, 1, 96, 32), (3, 31, 70, 128),                            # three blocks: four waves, two
+    (28, 8, 300, 64), (21, 8, 400, 128), (23, 13, 33, 64), (26, 7, 290, 32),     # one wave
+    (8, 13, 510, 64), (12, 8, 450, 128), (7, 10, 1025, 128), (17, 1, 3000, 64)])  # four, two, one, four
+def test_f32_forward_at_its_lines(gpu, B, H, T, D):
+    """Two sums in f32, of D products for a score and of up to T weighted values: (D + T) 2^-24 of the largest value, and
+    as much again for a score's error in its weight."""
+    x = synth.attention_inputs(f"order32-{B}-{H}-{T}-{D}", B, H, T, D, np.float32, base_seed=62, names=("q", "k", "v"))
+    o, lse = rocm.attn_fwd(x["q"], x["k"], x["v"])[:2]
+    one = (slice(B - 1, B), slice(H - 1, H))
+    want = oracle.attn_fwd(*(x[n][one] for n in ("q", "k", "v")))
+    assert np.max(np.abs(o[one].astype(np.float64) - want)) <= 2 * (D + T) * 2.0 ** -24 * np.max(np.abs(x["v"]))
+    again = rocm.attn_fwd(x["q"], x["k"], x["v"])[:2]
+    np.testing.assert_array_equal(o, again[0])
+    np.testing.assert_array_equal(lse, again[1])
+
+
 @pytest.fixture
 def gpu():
     if not rocm.available():
