@@ -23,11 +23,11 @@
 //   needs cost several times the whole stream.)  Where the splits may not share an
 //   XCD a second tiny kernel merges: same order, same bits.  It costs two microseconds more (12 heads
 //   x 700 x 64 7.4 us, 4.8 in the launch; 12 x 6000 x 64 8.5 / 7.9).
-//   A short call is a chain of latencies: the launch, the query, the tile, the reductions, the meeting.  us per call with
-//   lane exchanges through LDS, a wait for all of a tile before the next was requested, row addresses by 64-bit
-//   products and the partials read in batches of eight, and as it is: 12 heads x 200 x 64 4.8 -> 3.9, 12 x 1500 x 64 6.7 ->
-//   5.8, 12 x 6000 x 64 9.1 -> 7.9, 112 x 2000 x 64 13.1 -> 12.0, 192 x 2000 x 64 18.6 -> 16.6; appending:
-//   12 x 600 x 64 5.7 -> 5.0, 32 x 400 x 32 5.8 -> 4.4, 384 x 600 x 64 12.7 -> 12.0.
+//   A short call is a chain of latencies: the launch, its arguments, the query, the tile, the reductions, the meeting.  us per
+//   call with lane exchanges through LDS, a wait for all of a tile before the next was requested, row addresses by 64-bit
+//   products, arguments fetched where they are used and the partials read in batches of eight, and as it is: 12 heads x
+//   200 x 64 4.4 -> 3.2, 12 x 1500 x 64 6.7 -> 5.8, 12 x 6000 x 64 9.0 -> 8.0, 112 x 2000 x 64 13.1 -> 12.1, 192 x 2000 x 64 18.6 ->
+//   16.7; appending: 12 x 600 x 64 5.7 -> 4.7, 32 x 400 x 32 5.8 -> 4.2, 384 x 600 x 64 12.7 -> 11.7.
 //
 //   Append form (a generation step): instead of a ready query the kernel takes the new
 //   token's q, k, v projections, rotates q and k at the token's position (the
