@@ -198,10 +198,12 @@ __device__ __forceinline__ void attn_fwd_f16_bp_body(const FwdParams& p, int BH,
 
   // Causal mask of a 32-key block starting at key kb0, in place (tied operands: a select
   // written in C++ left the choice of registers to the allocator, which copied the whole
-  // accumulator in every stage, masked or not).
+  // accumulator in every stage, masked or not).  The compiler does not see that the asm text reads
+  // and writes what a matrix instruction may still be producing: the wait states (12) stand here.
   auto mask_block = [&](floatx16& s, int kb0) {
     const int dist = qrow - 4 * g - kb0;
     const float ninf = -INFINITY;
+    asm volatile("s_nop 15" : "+v"(s));
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       asm volatile("v_cmp_gt_i32_e32 vcc, %2, %1\n\tv_cndmask_b32_e32 %0, %0, %3, vcc"
