@@ -74,7 +74,7 @@ template <int D>
 __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void attn_bwd_f16_bp_kernel(BwdParams p, int BH, int n_blocks,
                                                                                  int heads_per_xcd, int first_id,
                                                                                  int dq_short_first) {
-  fetch_arguments<sizeof(BwdParams) + 20>();
+  fetch_arguments<decltype(attn_bwd_f16_bp_kernel<D>)>();
   const int group_wgs = 8 * heads_per_xcd;
   const int per_role = heads_per_xcd ? n_blocks * group_wgs : map_even_blocks(n_blocks, BH);
   const int id = (int)blockIdx.x + first_id;

@@ -37,7 +37,7 @@ namespace {
 // padded to t_pad per head (-inf and 0 there).  Reads O and dO once: 11 us for 96 x 1024 x 64, 4.5 TB/s.
 template <int D>
 __global__ __launch_bounds__(256) void attn_bwd_prep_f32_kernel(BwdParams p, int64_t rows) {
-  fetch_arguments<sizeof(BwdParams) + 8>();
+  fetch_arguments<decltype(attn_bwd_prep_f32_kernel<D>)>();
   constexpr int LPR = D / 4;  // lanes per row, 16 bytes each
   const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LPR;  // of [B*H][t_pad]
   const int part = threadIdx.x % LPR;
@@ -68,7 +68,7 @@ __host__ __device__ __forceinline__ int64_t ds_block(int qb, int kb) { return (i
 template <int D, int W>
 __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f32_dkdv_kernel(BwdParams p, int bh0, int BH,
                                                                                          int n_blocks, char* ds) {
-  fetch_arguments<sizeof(BwdParams) + 24>();
+  fetch_arguments<decltype(attn_bwd_f32_dkdv_kernel<D, W>)>();
   using C = Split32<D>;
   constexpr int KH = C::KH, DB = C::DB;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -168,7 +168,7 @@ struct DqPass {
 template <int D, int W>
 __global__ __launch_bounds__(64 * W) void attn_bwd_f32_dq_kernel(BwdParams p, int bh0, int BH, int n_blocks,
                                                                  const char* ds) {
-  fetch_arguments<sizeof(BwdParams) + 24>();
+  fetch_arguments<decltype(attn_bwd_f32_dq_kernel<D, W>)>();
   using C = Split32<D>;
   using S = DqPass<D, W>;
   constexpr int DB = C::DB;

@@ -221,7 +221,7 @@ __device__ __forceinline__ half_t merge_splits(const DecodeParams& p, int bh, in
 
 template <int D, bool APPEND>
 __global__ __launch_bounds__(256) void attn_decode_f16_kernel(DecodeParams p) {
-  fetch_arguments<sizeof(DecodeParams)>();
+  fetch_arguments<decltype(attn_decode_f16_kernel<D, APPEND>)>();
   constexpr int LPR = D / 8;            // lanes per cache row
   constexpr int GROUPS = 256 / LPR;         // row groups per workgroup
   constexpr int TILE = GROUPS * kDecRowsPerIt;
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(256) void attn_decode_f16_kernel(DecodeParams p) {
 // The merge as a launch of its own, where the splits of a head may not meet in one L2.
 template <int D>
 __global__ __launch_bounds__(D) void attn_decode_merge_kernel(DecodeParams p) {
-  fetch_arguments<sizeof(DecodeParams)>();
+  fetch_arguments<decltype(attn_decode_merge_kernel<D>)>();
   const int bh = 8 * p.whole + blockIdx.x, d = threadIdx.x;
   ((half_t*)p.o)[(int64_t)bh * D + d] = merge_splits<D>(p, bh, d);
 }

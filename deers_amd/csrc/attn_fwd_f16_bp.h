@@ -460,7 +460,7 @@ template <int D, bool RAW>
 __global__ __launch_bounds__(256, (D == 128 ? 2 : BP_OCC)) void attn_fwd_f16_bp_kernel(FwdParams p, int BH, int n_qtiles,
                                                                                 int heads_per_xcd,
                                                                                 TileOrder order) {
-  fetch_arguments<sizeof(FwdParams) + 16>();
+  fetch_first_arguments<decltype(attn_fwd_f16_bp_kernel<D, RAW>), 4>();
   attn_fwd_f16_bp_body<D, false, RAW>(p, BH, n_qtiles, heads_per_xcd, order, 0, nullptr);
 }
 

@@ -39,7 +39,7 @@ template <int D, int BN>
 __global__ __launch_bounds__(256, 2) void attn_fwd_f32_kernel(FwdParams p, int BH, int n_qtiles,
                                                            int heads_per_xcd, const int* lists,
                                                            int max_len) {
-  fetch_arguments<sizeof(FwdParams) + 28>();
+  fetch_arguments<decltype(attn_fwd_f32_kernel<D, BN>)>();
   constexpr int LD = D + 4;   // LDS row stride in floats
   constexpr int KH = D / 2;   // contraction steps (2 elements of D per MFMA)
   constexpr int DB = D / 32;

@@ -401,7 +401,7 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
   using C = SplitCfg<D>;
   constexpr int KS = C::KS, DB = C::DB, A = kSplitAhead, kWave = (DOUBLE ? 4 : 2) * C::BB;
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  fetch_arguments<sizeof(FwdParams) + 16>();
+  fetch_arguments<decltype(attn_fwd_f16_split_kernel<D, W, DOUBLE>)>();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5, T = p.T;
@@ -853,7 +853,7 @@ __device__ __forceinline__ void split_dkdv_body(const BwdParams& p, int bh, int 
 template <int D, int W, bool SCALED_Q>
 __global__ __launch_bounds__(64 * W, D == 128 ? 1 : 2) void attn_bwd_f16_split_kernel(BwdParams p, int BH, int n_blocks) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  fetch_arguments<sizeof(BwdParams) + 8>();
+  fetch_arguments<decltype(attn_bwd_f16_split_kernel<D, W, SCALED_Q>)>();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bh, rank;

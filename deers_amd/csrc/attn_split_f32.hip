@@ -42,7 +42,7 @@ namespace {
 
 template <int D, int W>
 __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f32_split_kernel(FwdParams p, int BH, int n_blocks, int cus) {
-  fetch_arguments<sizeof(FwdParams) + 12>();
+  fetch_arguments<decltype(attn_fwd_f32_split_kernel<D, W>)>();
   using C = Split32<D>;
   constexpr int KH = C::KH, DB = C::DB;
   // More than 256 registers in all, so that a SIMD takes one wave: with 208 a CU's workgroups of one or two waves come to lie two
@@ -313,7 +313,7 @@ __device__ __forceinline__ void split32_dkdv(const BwdParams& p, int bh, int kb,
 // rank 2 r + 1 the dQ block as many rows from the end.
 template <int D, int W>
 __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_bwd_f32_split_kernel(BwdParams p, int BH, int n_blocks, int cus) {
-  fetch_arguments<sizeof(BwdParams) + 12>();
+  fetch_arguments<decltype(attn_bwd_f32_split_kernel<D, W>)>();
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

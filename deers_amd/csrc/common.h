@@ -349,9 +349,18 @@ inline int paired_cus(PairedState& state, Kernel kernel, int threads, size_t lds
   return n > state.cus && n <= state.per_cu * state.cus ? state.cus : 0;
 }
 
-// Fetches the first BYTES of a kernel's arguments at its start.  They come from memory that no cache has yet, a line of
-// 64 bytes at a time; left alone the compiler asks for them where they are used, and the trips follow each other.
-template <int BYTES>
+// Where the first `count` arguments of a kernel end: each at its own alignment, as in a struct.
+template <typename... Args>
+constexpr int argument_bytes(void (*)(Args...), int count = sizeof...(Args)) {
+  constexpr int size[] = {(int)sizeof(Args)...}, align[] = {(int)alignof(Args)...};
+  int end = 0;
+  for (int i = 0; i < count; ++i) end = (end + align[i] - 1) / align[i] * align[i] + size[i];
+  return end;
+}
+// Fetches the arguments of a kernel, KERNEL its type, which calls this at its start (fetch_first_arguments: the first COUNT of
+// them).  They come from memory that no cache has yet, a line of 64 bytes at a time; left alone the compiler asks for them
+// where they are used, and the trips follow each other.
+template <typename KERNEL, int BYTES = argument_bytes((KERNEL*)nullptr)>
 __device__ __forceinline__ void fetch_arguments() {
   const auto ptr = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
   constexpr int LINES = (BYTES + 63) / 64, LAST = LINES - 1;
@@ -359,6 +368,10 @@ __device__ __forceinline__ void fetch_arguments() {
   asm volatile("" ::"s"(ptr[0]), "s"(ptr[16 * (LAST < 1 ? LAST : 1)]), "s"(ptr[16 * (LAST < 2 ? LAST : 2)]),
                "s"(ptr[16 * (LAST < 3 ? LAST : 3)]), "s"(ptr[16 * (LAST < 4 ? LAST : 4)]), "s"(ptr[16 * (LAST < 5 ? LAST : 5)]),
                "s"(ptr[16 * (LAST < 6 ? LAST : 6)]), "s"(ptr[16 * LAST]));
+}
+template <typename KERNEL, int COUNT>
+__device__ __forceinline__ void fetch_first_arguments() {
+  fetch_arguments<KERNEL, argument_bytes((KERNEL*)nullptr, COUNT)>();
 }
 
 // The kernel's first argument, fetched where it is asked for.  In a kernel whose branches are roles with

@@ -443,7 +443,7 @@ template <typename T, int GROUP, int NREG, int NLDS, bool GRAD>
 __global__ __launch_bounds__(kRegBlockOf(GROUP), NLDS ? 8 : 1) void cross_entropy_fwd_kernel(
     const T* logits, const int64_t* targets, float* row_lse, float* row_loss, T* dlogits, float inv_n,
     int64_t n_rows, int width, int* error_flag) {
-  fetch_arguments<72>();
+  fetch_arguments<decltype(cross_entropy_fwd_kernel<T, GROUP, NREG, NLDS, GRAD>)>();
   __shared__ float red_m[16], red_s[16];
   extern __shared__ u32x4 parked[];  // [NLDS][GROUP]
   constexpr int kRows = kRegBlockOf(GROUP) / GROUP;

@@ -37,7 +37,7 @@ struct RopeParams {
 // INVERSE = true : src is the gradient of the rotated heads, dst the projection grad.
 template <typename T, bool INVERSE>
 __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
-  fetch_arguments<sizeof(RopeParams)>();
+  fetch_arguments<decltype(rope_kernel<T, INVERSE>)>();
   typedef typename Vec16<T>::type V;
   constexpr int N = Vec16<T>::N;
   const int half_chunks = p.D / 2 / N;  // 16-byte chunks in half a row
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void rope_kernel(RopeParams p) {
 // tests/gpt.rs:38-49) or rows that are not 16-byte aligned.  Same arithmetic and rounding.
 template <typename T, bool INVERSE>
 __global__ __launch_bounds__(256) void rope_pair_kernel(RopeParams p) {
-  fetch_arguments<sizeof(RopeParams)>();
+  fetch_arguments<decltype(rope_pair_kernel<T, INVERSE>)>();
   const int half = p.D / 2;
   const int64_t total = (int64_t)p.B * p.T * p.H * half;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total;
@@ -108,7 +108,7 @@ struct DecodeQkvParams {
 };
 template <typename T>
 __global__ __launch_bounds__(256) void decode_qkv_kernel(DecodeQkvParams p) {
-  fetch_arguments<sizeof(DecodeQkvParams)>();
+  fetch_arguments<decltype(decode_qkv_kernel<T>)>();
   typedef typename Vec16<T>::type V;
   constexpr int N = Vec16<T>::N;
   const int half_chunks = p.D / 2 / N;

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void unary_compact_kernel(const T* x, T* out, 
 template <typename T, int OP>
 __global__ __launch_bounds__(256) void unary_strided_kernel(const T* x, StridedView v, T* out,
                                                             uint32_t n, float p) {
-  fetch_arguments<24 + sizeof(StridedView)>();
+  fetch_arguments<decltype(unary_strided_kernel<T, OP>)>();
   const uint32_t stride = gridDim.x * 256u;
   for (uint64_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += stride)
     out[i] = (T)unary_fn<OP>((float)x[view_offset(v, (uint32_t)i)], p);
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void binary_compact_kernel(const T* a, const T
 template <typename T, int OP>
 __global__ __launch_bounds__(256) void binary_strided_kernel(const T* a, StridedView va, const T* b,
                                                              StridedView vb, T* out, uint32_t n) {
-  fetch_arguments<28 + 2 * sizeof(StridedView)>();
+  fetch_arguments<decltype(binary_strided_kernel<T, OP>)>();
   const uint32_t stride = gridDim.x * 256u;
   for (uint64_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += stride)
     out[i] = (T)binary_fn<OP>((float)a[view_offset(va, (uint32_t)i)],
@@ -151,7 +151,7 @@ __device__ __forceinline__ Vec16<T> load_chunk(const T* base, const StridedView&
 template <typename T, int OP>
 __global__ __launch_bounds__(256) void unary_rows_kernel(const T* x, StridedView v, T* out,
                                                          uint32_t n_chunks, float p) {
-  fetch_arguments<24 + sizeof(StridedView)>();
+  fetch_arguments<decltype(unary_rows_kernel<T, OP>)>();
   constexpr int kEpc = 16 / sizeof(T);
   const uint32_t stride = gridDim.x * 256u;
   for (uint64_t c = blockIdx.x * 256u + threadIdx.x; c < n_chunks; c += stride) {
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void unary_rows_kernel(const T* x, StridedView
 template <typename T, int OP>
 __global__ __launch_bounds__(256) void binary_rows_kernel(const T* a, StridedView va, const T* b,
                                                           StridedView vb, T* out, uint32_t n_chunks) {
-  fetch_arguments<28 + 2 * sizeof(StridedView)>();
+  fetch_arguments<decltype(binary_rows_kernel<T, OP>)>();
   constexpr int kEpc = 16 / sizeof(T);
   const uint32_t stride = gridDim.x * 256u;
   for (uint64_t c = blockIdx.x * 256u + threadIdx.x; c < n_chunks; c += stride) {

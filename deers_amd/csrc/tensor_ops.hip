@@ -51,7 +51,7 @@ struct CopyView {
 // has merged: 10.8 us = 4.7 TB/s.
 template <typename E, typename I>
 __global__ __launch_bounds__(256) void copy_view_kernel(const E* src, E* dst, CopyView<I> v, I n) {
-  fetch_arguments<16 + sizeof(CopyView<I>) + sizeof(I)>();
+  fetch_arguments<decltype(copy_view_kernel<E, I>)>();
   for (I i = (I)blockIdx.x * 256 + threadIdx.x; i < n; i += (I)gridDim.x * 256) {
     I rem = i, so = 0, dof = 0;
     for (int d = v.ndim - 1; d > 0; --d) {
