@@ -302,7 +302,7 @@ struct SkinnyPrefetch {
 // 1, 1, 1, 1): BH / 8 whole heads per XCD, and the blocks of the BH % 8 remaining heads dealt to all
 // XCDs in turn.  An XCD's list is still ordered by rank.  The grid is map_even_blocks(n_ranks, BH).
 // An XCD's blocks of ranks below k are (k * BH + 7 - xcd) / 8: it holds every eighth of the blocks in order of rank.
-__device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH, int* bh, int* rank) {
+__host__ __device__ __forceinline__ bool map_block_even(int block_id, int n_ranks, int BH, int* bh, int* rank) {
   const int xcd = block_id & 7, whole = BH >> 3, rest = BH & 7;
   const int k = (int)((unsigned)block_id / (unsigned)BH);
   if (k >= n_ranks) return false;
