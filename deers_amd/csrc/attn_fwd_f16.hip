@@ -111,7 +111,7 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
   // others beside them (16 heads x 4096 x 64 in a kernel with 64-row tiles, two workgroups to each CU: 61.5 us, with even
   // totals 58.7).  Beyond that the dispatcher hands out each XCD's list longest first.
   // Up to two workgroups to a CU the scores are formed from Q itself, beyond that from Q times the scale, rounded to
-  // f16: 6 % faster (16 x 4096 x 64 53.1 / 49.2 us), O a quarter further from 64 bits (2.6e-4 / 3.2e-4).
+  // f16: 6 % faster (16 x 4096 x 64 53.1 / 49.2 us), O a quarter further from 64 bits (2.5e-4 / 3.2e-4).
   int n_cu, per_cu;
   resident_capacity<D>(&n_cu, &per_cu);
   const bool raw = D > 32 && (BH + 7) / 8 * n_qtiles <= 2 * n_cu, paired = even && grid / 8 > n_cu && grid / 8 <= per_cu * n_cu;

@@ -47,6 +47,30 @@ def test_forms_at_their_lines(gpu, B, H, T, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,T,D", [(24, 2049, 64), (64, 1024, 64), (33, 1025, 128)])
+def test_the_forward_from_q_is_as_exact_as_one_against_the_true_maximum(gpu, H, T, D):
+    """Relative 2-norm distance from 64 bits, of all rows of some heads: no more than probabilities rounded to f16
+    against the row's true maximum, their sums and a result rounded to f16 have (the largest probability is exact then)."""
+    assert not takes("fwd", H, T, D)
+    x = synth.attention_inputs(f"exact-{H}-{T}-{D}", 1, H, T, D, np.float16, base_seed=63, names=("q", "k", "v"))
+    o = rocm.attn_fwd(x["q"], x["k"], x["v"])[0]
+    future = np.triu(np.ones((T, T), bool), 1)
+    off, bound, size = 0.0, 0.0, 0.0
+    for h in (0, H // 2, H - 1):
+        q, k, v = (x[n][0, h].astype(np.float64) for n in ("q", "k", "v"))
+        s = np.where(future, -np.inf, q @ k.T * float(rocm.default_scale(D)))
+        p = np.exp(s - np.max(s, 1, keepdims=True))
+        want = p @ v / p.sum(1, keepdims=True)
+        rounded = p.astype(np.float16).astype(np.float64)
+        ideal = (rounded @ v / rounded.sum(1, keepdims=True)).astype(np.float16).astype(np.float64)
+        off += np.sum((o[0, h] - want) ** 2)
+        bound += np.sum((ideal - want) ** 2)
+        size += np.sum(want ** 2)
+    print(f"{H} x {T} x {D}: {np.sqrt(off / size):.4g}, true maximum {np.sqrt(bound / size):.4g}", flush=True)
+    assert off <= bound
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,H,T,D", [
     (1, 7, 65, 64), (5, 1, 96, 32), (3, 31, 70, 128),                            # three blocks: four waves, two
     (28, 8, 300, 64), (21, 8, 400, 128), (23, 13, 33, 64), (26, 7, 290, 32),     # one wave
