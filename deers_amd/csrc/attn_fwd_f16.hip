@@ -96,7 +96,7 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) {
     allow_lds(attn_fwd_f16_bp_kernel<D, false>, BpCfg<D>::kLds);
-    allow_lds(attn_fwd_f16_bp_kernel<D, true>, BpCfg<D>::kLds);
+    if constexpr (D > 32) allow_lds(attn_fwd_f16_bp_kernel<D, true>, BpCfg<D>::kLds);
     attr_set = true;
   }
   static const TileOrder kNoTable = [] {
@@ -114,10 +114,14 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
   // f16: 6 % faster (16 x 4096 x 64 53.1 / 49.2 us), O a quarter further from 64 bits (2.5e-4 / 3.2e-4).
   int n_cu, per_cu;
   resident_capacity<D>(&n_cu, &per_cu);
-  const bool raw = D > 32 && (BH + 7) / 8 * n_qtiles <= 2 * n_cu, paired = even && grid / 8 > n_cu && grid / 8 <= per_cu * n_cu;
+  [[maybe_unused]] const bool raw = (BH + 7) / 8 * n_qtiles <= 2 * n_cu;
+  const bool paired = even && grid / 8 > n_cu && grid / 8 <= per_cu * n_cu;
   const TileOrder* order = even ? nullptr : resident_order<D>(heads_per_xcd, p.T, n_cu, per_cu);
-  hipLaunchKernelGGL((raw ? attn_fwd_f16_bp_kernel<D, true> : attn_fwd_f16_bp_kernel<D, false>), dim3(grid), dim3(256),
-                     BpCfg<D>::kLds, stream, p, BH, n_qtiles, paired ? -n_cu : heads_per_xcd, order ? *order : kNoTable);
+  auto kernel = attn_fwd_f16_bp_kernel<D, false>;
+  if constexpr (D > 32)  // (at 32 the 32-row form takes nearly all that have as few)
+    if (raw) kernel = attn_fwd_f16_bp_kernel<D, true>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), BpCfg<D>::kLds, stream, p, BH, n_qtiles, paired ? -n_cu : heads_per_xcd,
+                     order ? *order : kNoTable);
 }
 
 void launch_attn_fwd_f16(const FwdParams& p, int B, int D, hipStream_t stream) {
