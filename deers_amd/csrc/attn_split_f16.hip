@@ -918,6 +918,7 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // the 128-row kernels hand over, and of strided rows in them, whose shapes lie there: D = 64 and 128 at 9 to 11 blocks
 // (109 x 320 x 64 backward 21.3 / 16.1), the backward at D = 32 from 17 to 20 and at D = 128 from 21 to 23.
 // The forward takes what the backward takes: then both form their scores from Q itself (`scaled_q`: the other way).
+extern bool attn_128_rows;  // runtime.hip
 struct SplitSize {
   int64_t nb, u;
   SplitSize(int64_t BH, int64_t T, int64_t D) : nb((T + 31) / 32), u(BH * nb * D / 64) {}
@@ -927,6 +928,7 @@ static int64_t of_width(int64_t D, int64_t w32, int64_t w64, int64_t w128) { ret
 // Up to `low`, and again from `again` up to `most`.
 static bool outside(int64_t u, int64_t low, int64_t again, int64_t most) { return u <= low || (u > again && u <= most); }
 bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
+  if (attn_128_rows) return false;
   const SplitSize z(BH, T, D);
   const int64_t nb = z.nb, u = z.u;
   if (nb <= 2) return u <= of_width(D, 5000, 5000, 9000);

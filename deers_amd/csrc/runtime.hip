@@ -28,6 +28,8 @@ namespace deers {
 void launch_attn_fwd_f16(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_fwd_f32(const FwdParams& p, int B, int D, hipStream_t stream);
 void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, hipStream_t stream);
+// test hook (deers_rocm_debug_attn_128_rows): the rules below leave everything that can be left to the 128-row kernels
+bool attn_128_rows = false;
 bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 // scaled_q: scores from f16(Q * scale * log2(e)), as the 128-row kernels form them, not from Q
@@ -530,6 +532,13 @@ int deers_rocm_debug_bwd_wait(int spin_limit, int skip_producers) {
   if (spin_limit < 1) return fail(DEERS_ROCM_ERR_ARG, "debug_bwd_wait: spin_limit must be >= 1");
   g_rt.bwd_spin_limit = spin_limit;
   g_rt.bwd_skip_producers = skip_producers ? 1 : 0;
+  return DEERS_ROCM_OK;
+}
+
+int deers_rocm_debug_attn_128_rows(int on) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  NEED_INIT();
+  deers::attn_128_rows = on != 0;
   return DEERS_ROCM_OK;
 }
 

@@ -124,6 +124,11 @@ def debug_bwd_wait(spin_limit: int = 1 << 20, skip_producers: bool = False):
     _check(load().deers_rocm_debug_bwd_wait(ctypes.c_int(spin_limit), ctypes.c_int(int(skip_producers))))
 
 
+def debug_attn_128_rows(on: bool):
+    """Test hook: attention calls take the 128-row kernels wherever there is one (see the header)."""
+    _check(load().deers_rocm_debug_attn_128_rows(ctypes.c_int(int(on))))
+
+
 _CODES = {np.float16: F16, np.float32: F32}
 
 

@@ -615,6 +615,12 @@ int deers_rocm_rope_bwd(int dtype, const void* dy, const int64_t* dy_strides,
  * skip_producers 0) restores normal operation.  No counterpart in the reference. */
 int deers_rocm_debug_bwd_wait(int spin_limit, int skip_producers);
 
+/* Test hook for the choice between the attention kernels: with `on` non-zero, forward and f16
+ * backward calls take the kernels with 128 rows per workgroup wherever there is one (f16: every
+ * size; f32: the forward of head widths 64 and 128), so that these can be tested at any size.
+ * 0 restores the choice by size.  No counterpart in the reference. */
+int deers_rocm_debug_attn_128_rows(int on);
+
 #ifdef __cplusplus
 }
 #endif

@@ -11,6 +11,7 @@ import pytest
 
 import oracle
 from deers_amd import rocm, synth
+from forms import rows_128, takes_32_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -384,15 +385,23 @@ def test_elementwise_helper_errors():
         rocm.add_raw(np.float32, None, buf.ptr, buf.ptr, 8)  # null pointer
 
 
-# ---- f16 launches on either side of the line between the two forms (few heads: 32 rows per
-# workgroup, the walk divided among its waves; many heads: 128 rows per workgroup) ----
+# ---- f16 launches of few and of many workgroups: in the form that their size takes, most of them 32 rows per workgroup
+# with the walk divided among its waves, and from two blocks of 128 rows on in the 128-row kernels ----
 
-@pytest.mark.parametrize("B,H,T,D", [
+F16_FORMS = [
     (1, 1, 2, 32), (2, 3, 65, 64), (1, 5, 95, 128), (1, 2, 128, 32), (1, 3, 129, 128), (2, 2, 161, 64),
     (1, 2, 513, 32), (1, 1, 700, 128),                                           # few heads
     (60, 7, 33, 64), (60, 7, 97, 32), (60, 7, 64, 128), (60, 7, 130, 32), (50, 8, 159, 64),  # many
-    (3, 25, 650, 64), (3, 19, 400, 128), (1, 9, 4161, 64)])                      # not whole heads per XCD
-def test_f16_forms_at_the_edges_of_their_blocks(B, H, T, D):
+    (3, 25, 650, 64), (3, 19, 400, 128), (1, 9, 4161, 64)]                       # not whole heads per XCD
+
+
+@pytest.mark.parametrize("rows,B,H,T,D", [("by size", *s) for s in F16_FORMS] + [(128, *s) for s in F16_FORMS if s[2] > 128])
+def test_f16_forms_at_the_edges_of_their_blocks(rows, B, H, T, D):
+    with rows_128(rows == 128):
+        f16_form(B, H, T, D)
+
+
+def f16_form(B, H, T, D):
     x = synth.attention_inputs(f"forms-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=21)
     out = check_case(x, TOL[np.dtype(np.float16)], f"forms {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
     again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
@@ -421,14 +430,23 @@ def test_f16_few_heads_rows_interleaved_over_heads():
     np.testing.assert_array_equal(lse.numpy(), want[1])
 
 
-# ---- f32 launches: 32 rows per workgroup in one, two and four waves, and the 128-row kernels ----
+# ---- f32 launches: 32 rows per workgroup in one, two and four waves, and the forward's 128-row kernels ----
 
-@pytest.mark.parametrize("B,H,T,D", [
+F32_FORMS = [
     (1, 1, 2, 32), (2, 3, 33, 64), (1, 5, 95, 128), (1, 2, 128, 32), (1, 3, 129, 64), (2, 2, 161, 128), (1, 9, 257, 32),
     (1, 1, 700, 128),                                                             # four waves, or a wave per block
     (60, 7, 63, 64), (25, 8, 130, 32), (25, 5, 193, 128), (60, 7, 97, 128), (100, 8, 159, 64),  # two and one
-    (40, 10, 700, 32), (20, 4, 990, 64), (19, 10, 641, 128)])                     # 128 rows
-def test_f32_forms_at_the_edges_of_their_blocks(B, H, T, D):
+    (40, 10, 700, 32), (20, 4, 990, 64), (19, 10, 641, 128)]                     # dS of the backward in memory
+
+
+@pytest.mark.parametrize("rows,B,H,T,D", [("by size", *s) for s in F32_FORMS] +
+                         [(128, *s) for s in F32_FORMS if s[2] > 128 and s[3] > 32])
+def test_f32_forms_at_the_edges_of_their_blocks(rows, B, H, T, D):
+    with rows_128(rows == 128):
+        f32_form(B, H, T, D)
+
+
+def f32_form(B, H, T, D):
     x = synth.attention_inputs(f"forms32-{B}-{H}-{T}-{D}", B, H, T, D, np.float32, base_seed=23)
     out = check_case(x, TOL[np.dtype(np.float32)], f"f32 forms {B}x{H}x{T}x{D}", heads=slice(B - 1, B))
     again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
@@ -527,34 +545,23 @@ def test_f32_gradients_round_at_the_size_of_the_lse_once(B, H, T, D):
     assert (rel <= 12 * 2.0 ** -24).all(), rel
 
 
-# ---- forms by name: the shapes above were chosen before small launches had forms of their own ----
-
-def takes_split(direction, dtype, B, H, T, D):
-    """The library's own rule: whether this launch takes the 32-row form (for the f32 backward: whether it
-    computes S and dP twice)."""
-    import ctypes
-    i64 = ctypes.c_int64
-    if direction == "bwd" and dtype == np.float32:
-        return rocm.load()["_ZN5deers18attn_bwd_f32_headsEllll"](i64(B * H), i64(T), i64(D), i64(2304 << 20)) == 0
-    rule = rocm.load()[f"_ZN5deers24attn_{direction}_f{16 if dtype == np.float16 else 32}_split_takesElll"]
-    rule.restype = ctypes.c_bool
-    return rule(i64(B * H), i64(T), i64(D))
-
+# ---- forms by name ----
 
 @pytest.mark.parametrize("dtype,B,H,T,D", [
     (np.float16, 11, 11, 300, 64), (np.float16, 8, 13, 300, 128), (np.float16, 4, 19, 1000, 32),
-    (np.float16, 9, 13, 1500, 64),                              # tile-pipelined, then block-pipelined forward
+    (np.float16, 9, 13, 1500, 64),                              # from Q itself; from scaled queries
     (np.float32, 17, 4, 990, 64), (np.float32, 13, 8, 500, 128)])
 def test_128_row_kernels_rows_interleaved_over_heads(dtype, B, H, T, D):
     """[B,T,H,D] memory under the logical [B,H,T,D], every operand, in launches that fill the device (f32: the
     backward with dS in memory): same bits as compact."""
-    assert not takes_split("fwd", dtype, B, H, T, D) and not takes_split("bwd", dtype, B, H, T, D)
-    strided_equals_compact(dtype, B, H, T, D)
+    with rows_128():
+        assert not any(takes_32_rows(direction, dtype, B * H, T, D) for direction in ("fwd", "bwd"))
+        strided_equals_compact(dtype, B, H, T, D)
 
 
 @pytest.mark.parametrize("B,H,T,D", [(4, 10, 500, 32), (4, 8, 500, 64), (3, 8, 500, 128)])
 def test_f32_backward_with_ds_in_memory_rows_interleaved_over_heads(B, H, T, D):
-    assert not takes_split("bwd", np.float32, B, H, T, D)
+    assert not takes_32_rows("bwd", np.float32, B * H, T, D)
     strided_equals_compact(np.float32, B, H, T, D)
 
 
@@ -584,7 +591,7 @@ def strided_equals_compact(dtype, B, H, T, D):
 def test_f16_backward_of_heads_dealt_to_all_xcds_at_head_width_128():
     """Nine heads of a long walk: the blocks of the ninth go to every XCD, in two launches."""
     B, H, T, D = 1, 9, 4161, 128
-    assert not takes_split("bwd", np.float16, B, H, T, D)
+    assert not takes_32_rows("bwd", np.float16, B * H, T, D)
     x = synth.attention_inputs("even-bwd-128", B, H, T, D, np.float16, base_seed=53)
     rocm.profile_enable(True)
     out = check_case(x, TOL[np.dtype(np.float16)], "nine heads of 4161 x 128", heads=(slice(0, 1), slice(7, 9)))

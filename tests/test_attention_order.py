@@ -1,27 +1,11 @@
 """f16 attention on either side of the lines between its forms, and the forward of 128 rows per workgroup whose scores are
 formed from Q itself: heads in whole numbers per XCD (placed by a table) and not (placed by formula)."""
-import ctypes
-
 import numpy as np
 import pytest
 
 import oracle
 from deers_amd import rocm, synth
-
-
-def takes(direction, heads, T, D):
-    rule = rocm.load()[f"_ZN5deers24attn_{direction}_f16_split_takesElll"]
-    rule.restype = ctypes.c_bool
-    i64 = ctypes.c_int64
-    return rule(i64(heads), i64(T), i64(D))
-
-
-def test_the_forward_takes_what_the_backward_takes():
-    """Otherwise one would form its scores from Q and the other from Q times the scale."""
-    for D in (32, 64, 128):
-        for T in (1, 32, 64, 65, 100, 128, 160, 256, 288, 300, 352, 384, 450, 480, 512, 600, 700, 1000, 2304, 2816, 4096, 9000):
-            for heads in list(range(1, 140)) + list(range(140, 3000, 37)):
-                assert takes("fwd", heads, T, D) or not takes("bwd", heads, T, D), (heads, T, D)
+from forms import takes_32_rows
 
 
 @pytest.mark.gpu
@@ -51,7 +35,7 @@ def test_forms_at_their_lines(gpu, B, H, T, D):
 def test_the_forward_from_q_is_as_exact_as_one_against_the_true_maximum(gpu, H, T, D):
     """Relative 2-norm distance from 64 bits, of all rows of some heads: no more than probabilities rounded to f16
     against the row's true maximum, their sums and a result rounded to f16 have (the largest probability is exact then)."""
-    assert not takes("fwd", H, T, D)
+    assert not takes_32_rows("fwd", np.float16, H, T, D)
     x = synth.attention_inputs(f"exact-{H}-{T}-{D}", 1, H, T, D, np.float16, base_seed=63, names=("q", "k", "v"))
     o = rocm.attn_fwd(x["q"], x["k"], x["v"])[0]
     future = np.triu(np.ones((T, T), bool), 1)

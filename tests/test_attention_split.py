@@ -1,12 +1,11 @@
 """The f16 attention kernels that give a workgroup 32 rows: every form at the sizes where it can go wrong (a walk of one
 block, of as many blocks as waves and one more, rows past the end of the last block), and the rule that chooses them."""
-import ctypes
-
 import numpy as np
 import pytest
 
 import oracle
 from deers_amd import rocm, synth
+from forms import takes_32_rows
 
 # relative 2-norm error of a result against the f32 oracle on the same f16 inputs: three roundings to f16 on the way
 # (scores' operand or probability, score gradient, result), each 2^-12 / sqrt(3) in the root mean square, and the
@@ -14,18 +13,16 @@ from deers_amd import rocm, synth
 REL = 2 * 3 ** 0.5 * 2.0 ** -12 / 3 ** 0.5
 
 
-def takes(direction, BH, T, D):
-    rule = rocm.load()[f"_ZN5deers24attn_{direction}_f16_split_takesElll"]
-    rule.restype = ctypes.c_bool
-    return rule(*(ctypes.c_int64(v) for v in (BH, T, D)))
+def takes(direction, heads, T, D):
+    return takes_32_rows(direction, np.float16, heads, T, D)
 
 
 def test_what_the_backward_takes_the_forward_takes_too():
     """Both then form their scores from Q itself; otherwise a probability would be recomputed from another score than
     the one it was normalised with."""
     for D in (32, 64, 128):
-        for T in [32 * nb for nb in range(1, 140)] + [8192]:
-            for BH in [int(1.15 ** i) for i in range(70)]:
+        for T in [32 * nb for nb in range(1, 140)] + [8192, 9000]:
+            for BH in sorted({*range(1, 140), *range(140, 3000, 37), *(int(1.15 ** i) for i in range(70))}):
                 assert not takes("bwd", BH, T, D) or takes("fwd", BH, T, D), (BH, T, D)
 
 

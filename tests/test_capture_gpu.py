@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from deers_amd import rocm, synth
+from forms import rows_128, takes_32_rows
 from hipgraph import Graph
 
 pytestmark = pytest.mark.gpu
@@ -97,12 +98,17 @@ def test_a_captured_few_rows_product_and_lookup_replay():
         graph.close()
 
 
-@pytest.mark.parametrize("dtype,B,H,T,D", [(np.float16, 7, 12, 300, 64), (np.float16, 4, 11, 257, 128),
-                                           (np.float16, 2, 3, 300, 64)])
-def test_a_captured_f16_backward_replays(dtype, B, H, T, D):
-    """The first two are launches whose kernels hand statistics over: captured, they are two launches without
-    flags (a replay could be given no fresh epoch); the last is the 32-row form.  Eager backwards of the same and
-    of another geometry between the replays move the epochs on."""
+@pytest.mark.parametrize("B,H,T,D,rows", [(7, 12, 300, 64, 128), (4, 11, 257, 128, 128), (2, 3, 300, 64, 32)])
+def test_a_captured_f16_backward_replays(B, H, T, D, rows):
+    """The 128-row kernels hand statistics over: captured, they are two launches without flags (a replay could be given
+    no fresh epoch).  Eager backwards of the same and of another geometry between the replays move the epochs on."""
+    with rows_128(rows == 128):
+        assert takes_32_rows("bwd", np.float16, B * H, T, D) == (rows == 32)
+        captured_backward(B, H, T, D)
+
+
+def captured_backward(B, H, T, D):
+    dtype = np.float16
     x = synth.attention_inputs(f"cap-bwd-{B}-{H}-{T}-{D}", B, H, T, D, dtype, base_seed=45)
     want = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
     ins = [rocm.DeviceBuffer.from_numpy(a) for a in (x["q"], x["k"], x["v"], want[0], want[1], x["do"])]

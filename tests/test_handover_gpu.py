@@ -13,6 +13,7 @@ import pytest
 
 import oracle
 from deers_amd import rocm, synth
+from forms import rows_128
 
 
 def test_policy_takes_same_xcd_handover_only_on_a_whole_unmasked_mi355x():
@@ -39,6 +40,13 @@ def gpu():
     rocm.set_handover_mode(-1)
 
 
+@pytest.fixture
+def backward_hands_over(gpu):
+    """The 128-row kernels at every size: the 32-row form hands nothing over."""
+    with rows_128():
+        yield
+
+
 @pytest.mark.gpu
 def test_device_policy_matches_the_device(gpu):
     # the boxes these tests run on are whole MI355X: 256 CUs, no mask
@@ -47,7 +55,7 @@ def test_device_policy_matches_the_device(gpu):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,T,D", [(2, 3, 300, 64), (1, 2, 129, 32), (1, 2, 257, 128), (3, 5, 1000, 64)])
-def test_two_launch_backward_equals_single_launch_bit_for_bit(gpu, B, H, T, D):
+def test_two_launch_backward_equals_single_launch_bit_for_bit(backward_hands_over, B, H, T, D):
     x = synth.attention_inputs(f"handover-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=11)
     rocm.set_handover_mode(rocm.HANDOVER_SAME_XCD)
     one = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
@@ -62,7 +70,7 @@ def test_two_launch_backward_equals_single_launch_bit_for_bit(gpu, B, H, T, D):
 
 
 @pytest.mark.gpu
-def test_more_than_64_query_blocks_per_head(gpu):
+def test_more_than_64_query_blocks_per_head(backward_hands_over):
     """A dK/dV workgroup polls its flags one per lane: 66 query blocks take a second round of
     the 64-lane poll.  Single launch against two launches bit for bit, and one whole head
     against the oracle."""
@@ -120,7 +128,7 @@ def test_decode_splits_merged_in_the_launch_or_after_it_give_the_same_bits(gpu, 
 
 
 @pytest.mark.gpu
-def test_a_wait_that_runs_out_is_reported_and_then_cleared(gpu):
+def test_a_wait_that_runs_out_is_reported_and_then_cleared(backward_hands_over):
     B, H, T, D = 1, 2, 200, 64
     x = synth.attention_inputs("handover-giveup", B, H, T, D, np.float16, base_seed=12)
     good = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
@@ -146,7 +154,7 @@ def test_a_wait_that_runs_out_is_reported_and_then_cleared(gpu):
 
 
 @pytest.mark.gpu
-def test_captured_backward_replays_correctly(gpu):
+def test_captured_backward_replays_correctly(backward_hands_over):
     """A replayed graph cannot be given a fresh hand-over epoch, so a backward that is being
     captured takes the two-launch form without the flags.  The captured backward is replayed
     three times, with eager backwards of another geometry and synchronisations between the
@@ -232,9 +240,8 @@ def test_decode_with_two_workgroups_on_a_compute_unit(gpu, B, H, L, D):
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,H,T,D", [(14, 11, 300, 32), (6, 9, 520, 32), (7, 12, 300, 64), (4, 11, 257, 128),
                                      (2, 9, 700, 128)])
-def test_backward_kernels_with_a_hand_over_give_the_same_bits_in_two_launches(gpu, B, H, T, D):
-    """Launches beyond the 32-row form, which hands nothing over, at every head width; the kernels are named by
-    what they were launched as."""
+def test_backward_kernels_with_a_hand_over_give_the_same_bits_in_two_launches(backward_hands_over, B, H, T, D):
+    """Every head width; the kernels are named by what they were launched as."""
     x = synth.attention_inputs(f"handover128-{B}-{H}-{T}-{D}", B, H, T, D, np.float16, base_seed=18)
     outs = []
     for mode, names in ((rocm.HANDOVER_SAME_XCD, {"attn_bwd_f16"}),
