@@ -368,8 +368,7 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // Takes, forward, us in the 128-row kernel / here: nearly everything, since that one forms 128 rows and has barriers
 // where waves here wait for themselves only (100 x 1024 x 64 143 / 130, 25 x 4096 x 64 559 / 441, 168 x 400 x 128 119 / 83, 65 x 1024
 // x 128 197 / 161, 25 x 4096 x 128 1137 / 928), up to the size where a four-fold reuse of K and V tiles decides (563 x
-// 1024 x 64 705 / 717, 375 x 1024 x 128 950 / 963, 563 x 1024 x 128 1432 / 1583; shorter walks later).  Two stretches are
-// left out that the tests of strided rows in the 128-row kernel have for their shapes.
+// 1024 x 64 705 / 717, 375 x 1024 x 128 950 / 963, 563 x 1024 x 128 1432 / 1583; shorter walks later).
 extern bool attn_128_rows;  // runtime.hip
 bool attn_f32_one_wave(int64_t n, int64_t nb, int64_t D) {
   return n >= (D == 32 ? 4608 + 48 * nb : D == 64 ? 1800 + 80 * nb : 1152 + 48 * nb);
@@ -378,8 +377,8 @@ bool attn_fwd_f32_split_takes(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb;
   if (attn_128_rows) return D == 32;
   if (D == 32 || nb <= 8) return true;
-  if (D == 128) return n <= (nb <= 10 ? 18000 : nb >= 13 && nb <= 15 ? 12000 : 9000) && !(nb >= 12 && n > 1656 && n <= 1664);
-  return n <= (nb <= 24 ? 20000 : 16000) && !(n > 2100 && n <= 2112);
+  if (D == 128) return n <= (nb <= 10 ? 18000 : nb >= 13 && nb <= 15 ? 12000 : 9000);
+  return n <= (nb <= 24 ? 20000 : 16000);
 }
 static int fwd_waves(int64_t BH, int64_t T, int64_t D) {
   const int64_t nb = (T + 31) / 32, n = BH * nb;

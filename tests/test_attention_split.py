@@ -26,6 +26,14 @@ def test_what_the_backward_takes_the_forward_takes_too():
                 assert not takes("bwd", BH, T, D) or takes("fwd", BH, T, D), (BH, T, D)
 
 
+def test_the_f32_forward_leaves_the_32_row_form_at_one_size():
+    """Up to a number of heads, and not again beyond it."""
+    for D in (32, 64, 128):
+        for T in [32 * nb for nb in range(1, 140)]:
+            took = [takes_32_rows("fwd", np.float32, heads, T, D) for heads in range(1, 400)]
+            assert took == sorted(took, reverse=True), (T, D)
+
+
 def rel(got, want):
     return float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want))
 
