@@ -913,10 +913,7 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 20 x 2048 x 64 56.4 / 62.3).  Seven or eight heads give each XCD one, which is what those kernels like best (backward 8 x
 // 3000 x 64 51.2 / 56.5, 9 x 3000 x 64 63.8 / 62.9).  At nb = 12 to 16 they are as fast or faster while all their
 // workgroups are resident two to a CU (forward 128 x 512 x 32 8.3 / 9.7, 168 x 512 x 64 14.8 / 15.8, 80 x 512 x 128 15.5 /
-// 17.5, 141 x 384 x 64 11.0 / 13.8).
-// From 9 blocks on some lines lie lower than the times would have them, or a stretch is left out, for the tests of what
-// the 128-row kernels hand over, and of strided rows in them, whose shapes lie there: D = 64 and 128 at 9 to 11 blocks
-// (109 x 320 x 64 backward 21.3 / 16.1), the backward at D = 32 from 17 to 20 and at D = 128 from 21 to 23.
+// 17.5, 124 x 372 x 64 10.6 / 11.8, but 108 x 372 x 64 10.3 / 9.7, 148 x 372 x 64 12.3 / 11.3).
 // The forward takes what the backward takes: then both form their scores from Q itself (`scaled_q`: the other way).
 extern bool attn_128_rows;  // runtime.hip
 struct SplitSize {
@@ -934,8 +931,8 @@ bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   if (nb <= 2) return u <= of_width(D, 5000, 5000, 9000);
   if (nb <= 4) return u <= of_width(D, 4500, 5200, 6400);
   if (nb <= 8) return u <= of_width(D, 5000, 5800, 8400);
-  if (nb <= 11) return outside(u, of_width(D, 4500, 1200, 2048), of_width(D, 4500, 1250, 2100), of_width(D, 4500, 6000, 8000));
-  if (nb <= 12) return outside(u, of_width(D, 4500, 1200, 2048), of_width(D, 4500, 1750, 3300), of_width(D, 4500, 5800, 7000));
+  if (nb <= 11) return u <= of_width(D, 4500, 6000, 8000);
+  if (nb <= 12) return outside(u, of_width(D, 4500, 1350, 2048), of_width(D, 4500, 1660, 3300), of_width(D, 4500, 5800, 7000));
   if (nb <= 15) return outside(u, of_width(D, 4000, 6800, 2048), 3300, of_width(D, 4000, 6800, 7500));
   if (nb <= 16) return outside(u, of_width(D, 770, 1300, 2048), of_width(D, 1540, 3000, 8192), of_width(D, 4200, 5800, 8192));
   return u <= of_width(D, nb < 40 ? 830 : 920, 1200, 2048);
@@ -949,12 +946,12 @@ bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   if (nb <= 4) return u <= of_width(D, 3600, 3500, 6400);
   if (nb <= 6) return u <= of_width(D, 4000, 3800, 6200);
   if (nb <= 8) return u <= of_width(D, 3600, 3000, 4700);
-  if (nb <= 11) return outside(u, 768, of_width(D, 800, 1250, 2100), of_width(D, 2600, 3600, 5000));
-  if (nb <= 12) return outside(u, 768, of_width(D, 800, 1750, 3300), of_width(D, 2600, 2900, 4400));
+  if (nb <= 11) return u <= of_width(D, 2600, 3600, 5000);
+  if (nb <= 12) return u <= of_width(D, 2600, 2900, 4400);
   if (nb <= 15) return u <= of_width(D, 3200, 3400, 4700);
   if (nb <= 16) return u <= of_width(D, 3200, 1300, 2048);
-  if (nb <= 20) return u <= of_width(D, 448, 1000, 1200);
-  if (nb <= 23) return u <= of_width(D, 760, 1000, 768);
+  if (nb <= 20) return u <= of_width(D, 700, 1000, 1200);
+  if (nb <= 23) return u <= of_width(D, 760, 1000, 1200);
   if (nb < 72) return u <= of_width(D, 720, 960, 1200);
   if (BH > 6 && BH <= 8) return u <= of_width(D, 700, 640, 1110);
   return u <= of_width(D, 700, 1100, 1700);

@@ -34,6 +34,19 @@ def test_the_f32_forward_leaves_the_32_row_form_at_one_size():
             assert took == sorted(took, reverse=True), (T, D)
 
 
+def test_the_f16_lines_follow_the_lengths_around_them():
+    """Walks of up to 11 blocks leave the 32-row form at one size, and the backward's line does not drop by more than a
+    tenth between longer walks and others a few blocks longer."""
+    for D in (32, 64, 128):
+        for nb in range(1, 12):
+            for direction in ("fwd", "bwd"):
+                took = [takes(direction, heads, 32 * nb, D) for heads in range(1, 1500)]
+                assert took == sorted(took, reverse=True), (direction, nb, D)
+        line = [max(heads for heads in range(1, 200) if takes("bwd", heads, 32 * nb, D)) * nb for nb in range(17, 30)]
+        for i in range(len(line) - 6):  # a head is up to 29 workgroups
+            assert line[i] + 29 >= 0.9 * max(line[i:i + 7]), (D, 17 + i, line)
+
+
 def rel(got, want):
     return float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want))
 
