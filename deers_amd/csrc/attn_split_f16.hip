@@ -991,11 +991,15 @@ static void launch_fwd(const FwdParams& p, int BH, bool scaled_q, hipStream_t st
   else
     launch_fwd<D, 1>(p, BH, twice, scaled_q, stream);
 }
+// Scaled queries: captured launches that the 128-row kernel would have, larger than what comes here in four waves (in
+// four 300 x 256 x 128 119.7 us, in one 67.3; 30 x 1300 x 128 in four 109.6, in two 88.0).
 template <int D>
 static void launch_bwd(const BwdParams& p, int BH, bool scaled_q, hipStream_t stream) {
   const int w = bwd_waves(SplitSize(BH, p.T, D), D);
-  if (scaled_q)
-    launch_bwd_split<D, 4, true>(p, BH, stream);
+  if (scaled_q && w >= 2)
+    launch_bwd_split<D, 2, true>(p, BH, stream);
+  else if (scaled_q)
+    launch_bwd_split<D, 1, true>(p, BH, stream);
   else if (w >= 4)
     launch_bwd_split<D, 4>(p, BH, stream);
   else if (w >= 2)

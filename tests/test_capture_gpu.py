@@ -1,4 +1,6 @@
 """Calls captured into a HIP graph and replayed between the program's own eager calls."""
+import multiprocessing
+
 import numpy as np
 import pytest
 
@@ -166,3 +168,41 @@ def test_a_captured_f16_backward_without_workspace_or_flags():
         for run in runs[1:]:
             for a, b in zip(run, runs[0]):
                 np.testing.assert_array_equal(a, b)
+
+
+# BH, T, D, waves: launches of the 128-row kernel, in the form that needs neither its workspace nor its flags
+FIRST_CAPTURED = [(300, 256, 128, 1), (60, 1024, 64, 2), (70, 700, 32, 2), (30, 1300, 128, 2), (200, 600, 64, 1)]
+
+
+def capture_first():
+    """In a process that has run no backward before, so that every capture finds neither."""
+    import oracle
+    rocm.init(0)
+    for BH, T, D, waves in FIRST_CAPTURED:
+        print(f"captured first: {BH} x {T} x {D}", flush=True)
+        assert not takes_32_rows("bwd", np.float16, BH, T, D)
+        x = synth.attention_inputs(f"cap-first-{BH}-{T}-{D}", 1, BH, T, D, np.float16, base_seed=46)
+        o, lse = rocm.attn_fwd(x["q"], x["k"], x["v"])
+        ins = [rocm.DeviceBuffer.from_numpy(a) for a in (x["q"], x["k"], x["v"], o, lse, x["do"])]
+        grads = [rocm.DeviceBuffer((1, BH, T, D), np.float16) for _ in range(3)]
+        graph = Graph(lambda: rocm.attn_bwd_raw(np.float16, *(b.ptr for b in ins + grads), 1, BH, T, D, rocm.default_scale(D)))
+        assert graph.threads() == [64 * waves], (graph.threads(), waves)
+        one = (slice(0, 1), slice(BH - 1, BH))
+        refs = oracle.attn_bwd(*(x[n][one] for n in ("q", "k", "v", "do")))
+        for _ in range(2):
+            for g in grads:
+                rocm.fill_raw(np.float16, g.ptr, BH * T * D, float("nan"))
+            graph.launch()
+            for got, ref in zip(grads, refs):
+                assert np.max(np.abs(got.numpy()[one].astype(np.float64) - ref)) <= 5e-3
+        graph.close()
+
+
+def test_a_backward_that_is_captured_first_has_as_many_waves_as_its_size_asks_for():
+    """One where many workgroups of short walks cover the device, two for longer ones."""
+    child = multiprocessing.get_context("spawn").Process(target=capture_first)
+    child.start()
+    child.join(100)
+    if child.is_alive():
+        child.kill()
+    assert child.exitcode == 0
