@@ -387,8 +387,13 @@ constexpr int kSplitAhead = 4;  // fragments on their way from LDS: a read takes
 // one each, asked for again as soon as they have been read: half the LDS, for launches in which several waves of a
 // SIMD cover each other's waits.
 // One wave: Q passes through V's block, V is asked for after it (a third more workgroups per CU).
+// DOUBLE at D = 32: K's rows go straight into registers a stage ahead (kSplitKDirect) and V is asked for when the stage
+// begins: the stage is a chain of waits, and this takes the read of K from LDS off it and gives V all of it (3 heads x
+// 2038 9.50 -> 8.41 us, 8 x 502 4.32 -> 4.07).
 template <int D, int W, bool DOUBLE>
 constexpr bool kSplitQInV = W == 1 && !DOUBLE && !kSplitDirect<D>;
+template <int D, bool DOUBLE>
+constexpr bool kSplitKDirect = kSplitDirect<D> && DOUBLE;
 template <int D, int W, bool DOUBLE>
 constexpr size_t split_fwd_lds() {  // blocks of every wave, as large as its accumulators; Q's block; m and l of every wave
   static_assert(2 * SplitCfg<D>::BB >= SplitMerge<D, W>::kWaveBytes, "the merge takes the blocks' place");
@@ -420,9 +425,18 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
   else
     split_load_resident<D, W, 1>(p.q, p.sq, p.q, p.sq, b_, h_, 32 * qb, T, q_blk, wave, lane);
   const SplitStream<D> K(p.k, p.sk, b_, h_, T, lane), V(p.v, p.sv, b_, h_, T, lane);
+  constexpr bool kKDirect = kSplitKDirect<D, DOUBLE>;
+  const SplitRowDots<D> k_rows(p.sk, T, lane);
+  const rsrc_t k_rsrc = k_rows.rsrc(p.k, p.sk, b_, h_, T);
+  half8 kf[KS];
   int kb = wave;
   if (kb <= qb) {
-    K.request_all(kb, p.k, p.sk, b_, h_, T, ring, lane);
+    if constexpr (kKDirect) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[ks] = k_rows.load(k_rsrc, ks, kb);
+    } else {
+      K.request_all(kb, p.k, p.sk, b_, h_, T, ring, lane);
+    }
     if (!kQInV) V.request_all(kb, p.v, p.sv, b_, h_, T, ring + C::BB, lane);
   }
   const float c = scaled_q ? 1.f : p.scale_log2;
@@ -462,14 +476,24 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
       else if constexpr (n < KS + 2 * DB)
         f[n % A] = at.col((n - KS) / DB, (n - KS) % DB, C::BB);
     };
-    split_for<(DOUBLE || A < KS ? A : KS)>(fetch);
+    half8 k_next[KS];
+    if constexpr (kKDirect) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) k_next[ks] = k_rows.load(k_rsrc, ks, next);
+      split_for<2 * DB>([&](auto i) { fetch(std::integral_constant<int, KS + decltype(i)::value>()); });
+    } else {
+      split_for<(DOUBLE || A < KS ? A : KS)>(fetch);
+    }
     floatx16 s = ZERO16;
     DEERS_SPLIT_CHUNK_END();
     split_for<KS>([&](auto i) {
       constexpr int ks = decltype(i)::value;
-      s = mfma_f16(f[ks % A], qf[ks], s);
-      if constexpr (DOUBLE || ks + A < KS) fetch(std::integral_constant<int, ks + A>());
-      if constexpr (DOUBLE && ks % 2 == 0) K.template request<ks>(next, ring + other);
+      s = mfma_f16(kKDirect ? kf[ks] : f[ks % A], qf[ks], s);
+      if constexpr (!kKDirect && (DOUBLE || ks + A < KS)) fetch(std::integral_constant<int, ks + A>());
+      if constexpr (kKDirect && ks % 2 == 0)
+        V.template request<ks>(next, ring + other + C::BB);
+      else if constexpr (DOUBLE && ks % 2 == 0)
+        K.template request<ks>(next, ring + other);
       DEERS_SPLIT_CHUNK_END();
     });
     if (!DOUBLE && more) {  // K's block has been read
@@ -513,9 +537,13 @@ __global__ __launch_bounds__(64 * W, 2) void attn_fwd_f16_split_kernel(FwdParams
       constexpr int n = decltype(i)::value;
       oacc[0][n % DB] = mfma_f16(f[(KS + n) % A], pf[n / DB], oacc[0][n % DB]);
       fetch(std::integral_constant<int, KS + n + A>());
-      if constexpr (DOUBLE && n % 2 == 0) V.template request<n>(next, ring + other + C::BB);
+      if constexpr (!kKDirect && DOUBLE && n % 2 == 0) V.template request<n>(next, ring + other + C::BB);
       DEERS_SPLIT_CHUNK_END();
     });
+    if constexpr (kKDirect) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kf[ks] = k_next[ks];
+    }
     if constexpr (DOUBLE) {
       at.move(other - slot);
       slot = other;
@@ -901,7 +929,11 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // where the device is full anyway and every wave costs its start and the merge (us in 4 / 2 / 1 waves, forward D = 64:
 // 12 x 512 5.8 / 7.7 / 11.1, 62 x 512 11.6 / 9.1 / 12.3, 200 x 256 11.5 / 11.0 / 8.8; backward D = 128: 6 x 768
 // 14.2 / 20.3 / 31.6, 15 x 1024 40.4 / 32.0 / 46.2, 187 x 256 73.4 / 49.0 / 38.3).  Twice the blocks in LDS where a CU has
-// one workgroup or two (forward D = 128, once / twice: 10 x 512 6.8 / 6.7, 6 x 128 4.7 / 4.5, 15 x 777 10.8 / 11.9).
+// one workgroup or two (forward D = 128, once / twice: 10 x 512 6.8 / 6.7, 6 x 128 4.7 / 4.5, 15 x 777 10.8 / 11.9; D = 32
+// 8 x 2038 9.4 / 8.6, 12 x 1500 7.9 / 7.4, 16 x 1494 8.3 / 8.5).  The
+// forward at D = 32: four up to some 90 heads, walks of three blocks included, and two up to 250, of two blocks up to
+// 120 (us in 4 / 2 / 1: 50 x 86 3.0 / 3.4 / 3.5, 120 x 54 3.0 / 3.0 / 3.2, 130 x 54 3.4 / 3.4 / 3.2, 240 x 86 4.2 / 3.6 /
+// 3.8, 90 x 246 4.4 / 4.8 / 5.9, 250 x 150 5.6 / 4.6 / 4.9, 300 x 150 6.1 / 5.3 / 5.1).
 //
 // Takes, us in the 128-row kernels / these: walks of up to 15 blocks nearly always (those form 128 rows where 64 to 384
 // are, and every stage has a barrier: forward 419 x 96 x 64 8.3 / 5.5, 286 x 300 x 128 28.4 / 22.1, 327 x 400 x 64 24.9 / 19.2;
@@ -956,16 +988,17 @@ bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   if (BH > 6 && BH <= 8) return u <= of_width(D, 700, 640, 1110);
   return u <= of_width(D, 700, 1100, 1700);
 }
-static int waves(const SplitSize& z, int64_t four, int64_t two) {
-  return z.u <= four && z.nb >= 4 ? 4 : z.u <= std::max(four, two) && z.nb >= 2 ? 2 : 1;
+static int waves(const SplitSize& z, int64_t four, int64_t two, int64_t shortest = 4) {
+  return z.u <= four && z.nb >= shortest ? 4 : z.u <= std::max(four, two) && z.nb >= 2 ? 2 : 1;
 }
 static int fwd_waves(const SplitSize& z, int64_t D) {
   const int64_t nb = z.nb, sq = nb * nb;
-  const int64_t four = of_width(D, 40 * nb, std::min(90 * nb, 700 + 25 * nb), std::min(160 * nb, 780 + 27 * nb));
-  const int64_t two = of_width(D, std::min<int64_t>(16 * sq, 900), std::min<int64_t>(64 * sq, 1700), std::min(120 * sq, 1300 + 60 * nb));
-  return waves(z, four, nb > 16 ? z.u : two);
+  const int64_t four = of_width(D, (nb < 5 ? 45 : 50) * nb, std::min(90 * nb, 700 + 25 * nb), std::min(160 * nb, 780 + 27 * nb));
+  const int64_t two = of_width(D, nb < 3 ? 120 : std::min<int64_t>(125 * nb, 900), std::min<int64_t>(64 * sq, 1700),
+                               std::min(120 * sq, 1300 + 60 * nb));
+  return waves(z, four, nb > 16 ? z.u : two, D == 32 ? 3 : 4);
 }
-static bool fwd_twice(const SplitSize& z, int64_t D) { return z.u <= of_width(D, 192, 256, 448); }
+static bool fwd_twice(const SplitSize& z, int64_t D) { return z.u <= of_width(D, 300, 256, 448); }
 static int bwd_waves(const SplitSize& z, int64_t D) {
   const int64_t nb = z.nb;
   const int64_t four = of_width(D, std::min(24 * nb, 120 + 9 * nb), std::min(32 * nb, 160 + 12 * nb), std::max<int64_t>(256, 72 + 20 * nb));

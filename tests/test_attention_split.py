@@ -6,6 +6,7 @@ import pytest
 import oracle
 from deers_amd import rocm, synth
 from forms import takes_32_rows
+from hipgraph import Graph
 
 # relative 2-norm error of a result against the f32 oracle on the same f16 inputs: three roundings to f16 on the way
 # (scores' operand or probability, score gradient, result), each 2^-12 / sqrt(3) in the root mean square, and the
@@ -74,6 +75,26 @@ def test_every_form_matches_the_oracle(BH, T, D):
             assert np.max(np.abs(g[few])) <= 2.0 ** -8
         else:
             assert rel(g[few], want) <= REL, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("BH,T,waves", [(100, 54, 2), (150, 54, 1), (50, 86, 4), (150, 86, 2), (300, 86, 1), (90, 118, 4),
+                                        (200, 150, 2), (90, 246, 4), (250, 246, 1)])
+def test_short_walks_at_head_width_32_have_the_waves_that_are_fastest(BH, T, waves):
+    """Read from the captured launch; its result like any other's."""
+    x = synth.attention_inputs(f"split-waves-{BH}-{T}", 1, BH, T, 32, np.float16, base_seed=64, names=("q", "k", "v"))
+    q, k, v = (rocm.DeviceBuffer.from_numpy(x[n]) for n in ("q", "k", "v"))
+    o, lse = rocm.DeviceBuffer((1, BH, T, 32), np.float16), rocm.DeviceBuffer((1, BH, T), np.float32)
+    graph = Graph(lambda: rocm.attn_fwd_raw(np.float16, q.ptr, k.ptr, v.ptr, o.ptr, lse.ptr, 1, BH, T, 32, rocm.default_scale(32)))
+    try:
+        assert graph.threads() == [64 * waves]
+        for _ in range(2):
+            rocm.fill_raw(np.float16, o.ptr, BH * T * 32, float("nan"))
+            graph.launch()
+            few = (slice(None), sorted({0, BH // 2, BH - 1}))
+            assert rel(o.numpy()[few], oracle.attn_fwd(x["q"][few], x["k"][few], x["v"][few])) <= REL
+    finally:
+        graph.close()
 
 
 @pytest.mark.gpu
