@@ -70,11 +70,11 @@ constexpr int kBwdBlk = 128;  // rows owned by a workgroup (keys in dK/dV, queri
 // One of the roles fetches its own arguments, so that those of both need not fit the scalar registers before the
 // branch (backward, us, both roles' before it / one fetches / each fetches: 8 x 12 x 1024 x 64 63.3 / 61.7 / 61.9, 8 x
 // 12 x 1024 x 128 135.6 / 133.1 / 133.4, 16 x 8192 x 128 906.0 / 907.1 / 909.2).
-template <int D>
+template <int D, bool RAW>
 __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void attn_bwd_f16_bp_kernel(BwdParams p, int BH, int n_blocks,
                                                                                  int heads_per_xcd, int first_id,
                                                                                  int dq_short_first) {
-  fetch_arguments<decltype(attn_bwd_f16_bp_kernel<D>)>();
+  fetch_arguments<decltype(attn_bwd_f16_bp_kernel<D, RAW>)>();
   const int group_wgs = 8 * heads_per_xcd;
   const int per_role = heads_per_xcd ? n_blocks * group_wgs : map_even_blocks(n_blocks, BH);
   const int id = (int)blockIdx.x + first_id;
@@ -83,11 +83,11 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void attn_bwd_f16_bp_kernel(
     int at = id;
     if (dq_short_first) at = (n_blocks - 1 - id / group_wgs) * group_wgs + id % group_wgs;
     if (map_block(at, n_blocks, heads_per_xcd, BH, &bh, &rank))
-      bwd_dq_f16_bp_body<D>(p, __builtin_amdgcn_readfirstlane(bh), n_blocks - 1 - __builtin_amdgcn_readfirstlane(rank),
+      bwd_dq_f16_bp_body<D, RAW>(p, __builtin_amdgcn_readfirstlane(bh), n_blocks - 1 - __builtin_amdgcn_readfirstlane(rank),
                             n_blocks, blockIdx.x);
   } else {
     if (map_block(id - per_role, n_blocks, heads_per_xcd, BH, &bh, &rank))
-      bwd_dkdv_f16_bp_body<D>(first_argument<BwdParams>(), __builtin_amdgcn_readfirstlane(bh), __builtin_amdgcn_readfirstlane(rank), n_blocks,
+      bwd_dkdv_f16_bp_body<D, RAW>(first_argument<BwdParams>(), __builtin_amdgcn_readfirstlane(bh), __builtin_amdgcn_readfirstlane(rank), n_blocks,
                               blockIdx.x);
   }
 }
@@ -100,7 +100,7 @@ static bool bwd_even(int BH, int T, int D) {
   return T >= 4096 && (int64_t)T * D >= 262144 && 80 * ((BH + 7) / 8) >= 11 * BH;
 }
 
-template <int D>
+template <int D, bool RAW>
 static void launch_bwd_f16_d(const BwdParams& p, int B, int mode, hipStream_t stream) {
   const int BH = B * p.H;
   const int n_blocks = (p.T + kBwdBlk - 1) / kBwdBlk;
@@ -109,7 +109,7 @@ static void launch_bwd_f16_d(const BwdParams& p, int B, int mode, hipStream_t st
   const int heads_per_xcd = even ? 0 : (BH + 7) / 8;
   const int per_role = even ? map_even_blocks(n_blocks, BH) : 8 * n_blocks * heads_per_xcd;
   typedef void (*Kernel)(BwdParams, int, int, int, int, int);
-  const Kernel kernel = attn_bwd_f16_bp_kernel<D>;
+  const Kernel kernel = attn_bwd_f16_bp_kernel<D, RAW>;
   const size_t lds = BwdBpCfg<D>::kLds;
   static bool attr_set = false;  // launches are serialised by the caller
   if (!attr_set) allow_lds(kernel, lds);
@@ -152,11 +152,22 @@ static void launch_bwd_f16_d(const BwdParams& p, int B, int mode, hipStream_t st
 // mode 1: both roles in one grid with the flag hand-over (needs workgroup id % 8 == XCD);
 // mode 0: two launches in stream order; mode 2: only the dK/dV half of the single launch
 // (host-side test of the bounded wait: nobody publishes, every wait runs out).
-void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, hipStream_t stream) {
+// from_q: scores from Q itself, as that launch's forward formed them (never at head width 32).
+void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, bool from_q, hipStream_t stream) {
   switch (D) {
-    case 32: launch_bwd_f16_d<32>(p, B, mode, stream); break;
-    case 64: launch_bwd_f16_d<64>(p, B, mode, stream); break;
-    case 128: launch_bwd_f16_d<128>(p, B, mode, stream); break;
+    case 32: launch_bwd_f16_d<32, false>(p, B, mode, stream); break;
+    case 64:
+      if (from_q)
+        launch_bwd_f16_d<64, true>(p, B, mode, stream);
+      else
+        launch_bwd_f16_d<64, false>(p, B, mode, stream);
+      break;
+    case 128:
+      if (from_q)
+        launch_bwd_f16_d<128, true>(p, B, mode, stream);
+      else
+        launch_bwd_f16_d<128, false>(p, B, mode, stream);
+      break;
   }
 }
 

@@ -19,7 +19,11 @@
 //     queries (its dK sum is rescaled by ln 2 at the end).  The forward folds the scale into its
 //     queries the same way, so all three kernels exponentiate bit-identical scores: with the
 //     scale folded into K in the dK/dV role instead, its scores differed from the forward's by up
-//     to |S| * 2^-11, a dominant probability by 0.2 %, and dK of a peaked row by 6e-3;
+//     to |S| * 2^-11, a dominant probability by 0.2 %, and dK of a peaked row by 6e-3.
+//     RAW: where the forward formed its scores from Q itself, both roles do (and the row statistic is
+//     -LSE / scale); a product per score then stands before the exponential (16 x 4096 x 64 123.3 -> 126.2 us,
+//     12 x 4096 x 128 200.9 -> 205.2; relative distance from 64 bits of dQ 3.8e-4 -> 3.0e-4, dK 4.4e-4 -> 3.0e-4, dV
+//     3.6e-4 -> 2.9e-4, largest error of dV over 60 launches 5.6e-3 -> 2.8e-3);
 //   * the S accumulator starts from -LSE*log2(e) and the dP accumulator from -delta (row values
 //     read from LDS straight into the accumulator registers in the dK/dV role, 16-register
 //     constants in the dQ role), so P = exp2(S) and dS = P * dP;
@@ -78,7 +82,7 @@ __device__ __forceinline__ uint32_t pack_pair_f16(float a, float b) {
 // ---------------------------------------------------------------------------
 // dK / dV
 // ---------------------------------------------------------------------------
-template <int D>
+template <int D, bool RAW>
 __device__ __forceinline__ void bwd_dkdv_f16_bp_body(const BwdParams& p, int bh, int kvblk, int n_own,
                                                      [[maybe_unused]] int trace_row) {
   using Cfg = BwdBpCfg<D>;
@@ -98,7 +102,9 @@ __device__ __forceinline__ void bwd_dkdv_f16_bp_body(const BwdParams& p, int bh,
   const int T = p.T;
   DEERS_TRACE_POINT(0);  // key block 0 walks the most queries
   const int b_ = bh / p.H, h_ = bh % p.H;
-  // the queries as the dQ role scaled them (f16(Q * scale * log2(e)), compact rows)
+  [[maybe_unused]] float c = p.scale_log2;
+  if constexpr (RAW) asm volatile("" : "+v"(c));  // a vector operand: a scalar one makes the products take longer to issue
+  // the queries as the dQ role left them (f16(Q * scale * log2(e)), or Q itself; compact rows)
   const half_t* Q = (const half_t*)p.qs + (int64_t)bh * p.t_pad * D;
   const half_t* K = (const half_t*)p.k + b_ * p.sk.b + h_ * p.sk.h;
   const half_t* V = (const half_t*)p.v + b_ * p.sv.b + h_ * p.sv.h;
@@ -342,7 +348,7 @@ __device__ __forceinline__ void bwd_dkdv_f16_bp_body(const BwdParams& p, int bh,
       }
       if (!FIRST && PRODUCE && i < 8) seed_part(i, sn, dpn, NSLOT);
       if (i >= 1 && i <= LPI) request_part(i - 1, n + 1 + F, RSLOT);
-      s[i] = fast_exp2(s[i]);
+      s[i] = fast_exp2(RAW ? s[i] * c : s[i]);
       if (i > 0) dp[i - 1] = s[i - 1] * dp[i - 1];
       if (i > 2 && (i & 1)) finish_pair((i - 3) >> 1);
       __builtin_amdgcn_sched_barrier(0);
@@ -443,7 +449,7 @@ __device__ __forceinline__ void bwd_dkdv_f16_bp_body(const BwdParams& p, int bh,
     half_t* dvrow = dV + (int64_t)kvrow * p.sdv.t;
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
-      store_block_f16(dkrow + 32 * db, dkacc[db], kLn2, g);  // sum of dS * Q * scale * log2(e)
+      store_block_f16(dkrow + 32 * db, dkacc[db], RAW ? p.scale : kLn2, g);  // sum of dS * Q (* scale * log2(e))
       store_block_f16(dvrow + 32 * db, dvacc[db], 1.f, g);
     }
   }
@@ -453,7 +459,7 @@ __device__ __forceinline__ void bwd_dkdv_f16_bp_body(const BwdParams& p, int bh,
 // ---------------------------------------------------------------------------
 // dQ
 // ---------------------------------------------------------------------------
-template <int D>
+template <int D, bool RAW>
 __device__ __forceinline__ void bwd_dq_f16_bp_body(const BwdParams& p, int bh, int qtile, int n_own,
                                                    [[maybe_unused]] int trace_row) {
   using Cfg = BwdBpCfg<D>;
@@ -541,7 +547,7 @@ __device__ __forceinline__ void bwd_dq_f16_bp_body(const BwdParams& p, int bh, i
       for (int e = 0; e < 8; ++e) dsum += (float)dof[ks][e] * (float)of[ks][e];
     if (qrow >= T) dsum = 0.f;
     nd = -pair_sum(dsum);
-    nl2 = qrow < T ? -lse_row * kLog2e : -INFINITY;
+    nl2 = qrow < T ? -lse_row * (RAW ? 1.f / p.scale : kLog2e) : -INFINITY;
     if (g == 0 && qrow < p.t_pad) {
       p.lse2[(int64_t)bh * p.t_pad + qrow] = nl2;
       p.negdelta[(int64_t)bh * p.t_pad + qrow] = nd;
@@ -601,17 +607,18 @@ __device__ __forceinline__ void bwd_dq_f16_bp_body(const BwdParams& p, int bh, i
   half8 dsf[2];
   half8 fr[W];
   wait_all_vmem();
-  {
-    const float c = p.scale_log2;
+  [[maybe_unused]] float c = p.scale_log2;
+  if constexpr (RAW) {
+    asm volatile("" : "+v"(c));
+  } else {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int e = 0; e < 8; ++e) qf[ks][e] = (half_t)((float)qf[ks][e] * c);
   }
-  // The scaled queries go to the workspace: the dK/dV role forms its scores from these very
-  // values, as the forward did, so that all three exponentiate identical scores (with the
-  // scale folded into K there instead, scores differed by up to |S| * 2^-11 and a dominant
-  // probability by 0.2 %).
+  // The queries go to the workspace: the dK/dV role forms its scores from these very values, as
+  // the forward did, so that all three exponentiate identical scores (with the scale folded
+  // into K there instead, scores differed by up to |S| * 2^-11 and a dominant probability by 0.2 %).
   if (qrow < T) {
     half_t* qs = (half_t*)p.qs + ((int64_t)bh * p.t_pad + qrow) * D + 8 * g;
 #pragma unroll
@@ -670,7 +677,7 @@ __device__ __forceinline__ void bwd_dq_f16_bp_body(const BwdParams& p, int bh, i
           fr[mi % W] = fetch2(mi + W - NMS, SLOT);
       }
       if (i >= 1 && i <= LPI) request_part(i - 1, n + 1 + F, RSLOT);
-      s[i] = fast_exp2(s[i]);
+      s[i] = fast_exp2(RAW ? s[i] * c : s[i]);
       if (i > 0) dp[i - 1] = s[i - 1] * dp[i - 1];
       if (i > 2 && (i & 1)) finish_pair((i - 3) >> 1);
       __builtin_amdgcn_sched_barrier(0);

@@ -85,7 +85,7 @@ static const TileOrder* resident_order(int heads_per_xcd, int T, int n_cu, int p
 }
 
 template <int D>
-static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
+static void launch_fwd_f16_d(const FwdParams& p, int B, bool from_q, hipStream_t stream) {
   const int BH = B * p.H;
   const int n_qtiles = (p.T + kFwdBM - 1) / kFwdBM;
   // heads that the XCDs cannot share out whole (9 x 8192 x 128: 218 us with two heads on one XCD, 163
@@ -110,25 +110,38 @@ static void launch_fwd_f16_d(const FwdParams& p, int B, hipStream_t stream) {
   // tiles of some heads are dealt to all XCDs.  Longest first instead, the CUs that have two get the longest ones and
   // others beside them (16 heads x 4096 x 64 in a kernel with 64-row tiles, two workgroups to each CU: 61.5 us, with even
   // totals 58.7).  Beyond that the dispatcher hands out each XCD's list longest first.
-  // Up to two workgroups to a CU the scores are formed from Q itself, beyond that from Q times the scale, rounded to
-  // f16: 6 % faster (16 x 4096 x 64 53.1 / 49.2 us), O a quarter further from 64 bits (2.5e-4 / 3.2e-4).
   int n_cu, per_cu;
   resident_capacity<D>(&n_cu, &per_cu);
-  [[maybe_unused]] const bool raw = (BH + 7) / 8 * n_qtiles <= 2 * n_cu;
   const bool paired = even && grid / 8 > n_cu && grid / 8 <= per_cu * n_cu;
   const TileOrder* order = even ? nullptr : resident_order<D>(heads_per_xcd, p.T, n_cu, per_cu);
   auto kernel = attn_fwd_f16_bp_kernel<D, false>;
-  if constexpr (D > 32)  // (at 32 the 32-row form takes nearly all that have as few)
-    if (raw) kernel = attn_fwd_f16_bp_kernel<D, true>;
+  if constexpr (D > 32)
+    if (from_q) kernel = attn_fwd_f16_bp_kernel<D, true>;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), BpCfg<D>::kLds, stream, p, BH, n_qtiles, paired ? -n_cu : heads_per_xcd,
                      order ? *order : kNoTable);
 }
 
-void launch_attn_fwd_f16(const FwdParams& p, int B, int D, hipStream_t stream) {
+bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);  // attn_split_f16.hip
+bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
+
+// Whether a launch's scores are formed from Q itself, or from Q * scale * log2(e) rounded to f16.  Forward and backward
+// ask the same question: a probability that is recomputed from another score than it was normalised with is off by
+// up to |S| * 2^-11, dV of a peaked row by more than 5e-3.
+//   both in the 32-row form       from Q (a product per score costs them nothing)
+//   128 rows, D = 64 and 128      from Q up to two workgroups to a CU, beyond that from scaled queries, 6 % faster
+//                                 (forward 16 x 4096 x 64 53.1 / 49.2 us; O 2.5e-4 / 3.2e-4 from 64 bits, relative)
+//   else                          from scaled queries: the 128-row backward after a 32-row forward, and head width 32
+// The 128-row backward starts from -LSE / scale: not for scales whose reciprocal leaves f32.
+bool attn_f16_from_q(int64_t BH, int64_t T, int64_t D, float scale) {
+  if (attn_fwd_f16_split_takes(BH, T, D)) return attn_bwd_f16_split_takes(BH, T, D);
+  return D > 32 && (BH + 7) / 8 * ((T + kFwdBM - 1) / kFwdBM) <= 64 && scale >= 0x1p-60f;
+}
+
+void launch_attn_fwd_f16(const FwdParams& p, int B, int D, bool from_q, hipStream_t stream) {
   switch (D) {
-    case 32: launch_fwd_f16_d<32>(p, B, stream); break;
-    case 64: launch_fwd_f16_d<64>(p, B, stream); break;
-    case 128: launch_fwd_f16_d<128>(p, B, stream); break;
+    case 32: launch_fwd_f16_d<32>(p, B, from_q, stream); break;
+    case 64: launch_fwd_f16_d<64>(p, B, from_q, stream); break;
+    case 128: launch_fwd_f16_d<128>(p, B, from_q, stream); break;
   }
 }
 

@@ -21,8 +21,8 @@
 // The walked operands pass through LDS, rows and transposed fragments from the same blocks; what a workgroup owns is
 // loaded once through LDS as well, by all its waves.  All three form the scores from Q and apply scale * log2e to the
 // f32 sums; where the 128-row backward follows the forward (or, in a captured launch, the 128-row forward has gone
-// before), from f16(Q * scale * log2e) as that does (scaled_q), so that a probability is recomputed from the score it
-// was normalised with.  Partial sums are added in wave order: results are reproducible bit for bit.
+// before), from what that takes, Q or f16(Q * scale * log2e): a probability is recomputed from the score it was
+// normalised with (attn_f16_from_q).  Partial sums are added in wave order: results are reproducible bit for bit.
 //
 // What bounds a launch: the start of a workgroup (2 us of loads that depend on nothing but its number), the stages of
 // its longest wave (1.0 us at D = 128 and 0.6 us at D = 64 in the backward, for 0.5 and 0.25 us of matrix
@@ -946,7 +946,7 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 3000 x 64 51.2 / 56.5, 9 x 3000 x 64 63.8 / 62.9).  At nb = 12 to 16 they are as fast or faster while all their
 // workgroups are resident two to a CU (forward 128 x 512 x 32 8.3 / 9.7, 168 x 512 x 64 14.8 / 15.8, 80 x 512 x 128 15.5 /
 // 17.5, 124 x 372 x 64 10.6 / 11.8, but 108 x 372 x 64 10.3 / 9.7, 148 x 372 x 64 12.3 / 11.3).
-// The forward takes what the backward takes: then both form their scores from Q itself (`scaled_q`: the other way).
+// The forward takes what the backward takes: then both form their scores from Q itself.
 extern bool attn_128_rows;  // runtime.hip
 struct SplitSize {
   int64_t nb, u;
@@ -1027,11 +1027,11 @@ static void launch_fwd(const FwdParams& p, int BH, bool scaled_q, hipStream_t st
 // Scaled queries: captured launches that the 128-row kernel would have, larger than what comes here in four waves (in
 // four 300 x 256 x 128 119.7 us, in one 67.3; 30 x 1300 x 128 in four 109.6, in two 88.0).
 template <int D>
-static void launch_bwd(const BwdParams& p, int BH, bool scaled_q, hipStream_t stream) {
+static void launch_bwd(const BwdParams& p, int BH, bool from_q, hipStream_t stream) {
   const int w = bwd_waves(SplitSize(BH, p.T, D), D);
-  if (scaled_q && w >= 2)
+  if (!from_q && w >= 2)
     launch_bwd_split<D, 2, true>(p, BH, stream);
-  else if (scaled_q)
+  else if (!from_q)
     launch_bwd_split<D, 1, true>(p, BH, stream);
   else if (w >= 4)
     launch_bwd_split<D, 4>(p, BH, stream);
@@ -1041,20 +1041,20 @@ static void launch_bwd(const BwdParams& p, int BH, bool scaled_q, hipStream_t st
     launch_bwd_split<D, 1>(p, BH, stream);
 }
 
-void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, bool scaled_q, hipStream_t stream) {
+void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, bool from_q, hipStream_t stream) {
   LaunchScope scope("attn_fwd_f16", stream);
   switch (D) {
-    case 32: launch_fwd<32>(p, B * p.H, scaled_q, stream); break;
-    case 64: launch_fwd<64>(p, B * p.H, scaled_q, stream); break;
-    case 128: launch_fwd<128>(p, B * p.H, scaled_q, stream); break;
+    case 32: launch_fwd<32>(p, B * p.H, !from_q, stream); break;
+    case 64: launch_fwd<64>(p, B * p.H, !from_q, stream); break;
+    case 128: launch_fwd<128>(p, B * p.H, !from_q, stream); break;
   }
 }
-void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, bool scaled_q, hipStream_t stream) {
+void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, bool from_q, hipStream_t stream) {
   LaunchScope scope("attn_bwd_f16", stream);
   switch (D) {
-    case 32: launch_bwd<32>(p, B * p.H, scaled_q, stream); break;
-    case 64: launch_bwd<64>(p, B * p.H, scaled_q, stream); break;
-    case 128: launch_bwd<128>(p, B * p.H, scaled_q, stream); break;
+    case 32: launch_bwd<32>(p, B * p.H, from_q, stream); break;
+    case 64: launch_bwd<64>(p, B * p.H, from_q, stream); break;
+    case 128: launch_bwd<128>(p, B * p.H, from_q, stream); break;
   }
 }
 

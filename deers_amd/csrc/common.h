@@ -261,8 +261,8 @@ struct BwdParams {
   // workspace, rows padded to a multiple of 64 per head (t_pad), written by the dQ role (f32: by a
   // launch of its own) and read by the dK/dV role: lse2 = -LSE*log2(e) (-inf in the padding), negdelta =
   // -rowsum(dO o O) (0 in the padding), and, f16, qs = f16(Q * scale * log2(e)), [B*H][t_pad][D]
-  // compact: the scaled queries the forward and the dQ role form their scores from, so that
-  // all three kernels exponentiate the same scores
+  // compact: the queries the forward and the dQ role form their scores from, so that all three
+  // kernels exponentiate the same scores (from Q itself: qs = Q, lse2 = -LSE / scale)
   float* lse2; float* negdelta; void* qs; int t_pad;
   // ready[bh * n_blocks + q_block] == epoch once the lse2 / negdelta rows of that 128-row
   // query block are published (f16 path, hand-over inside one launch); epoch 0: the flags

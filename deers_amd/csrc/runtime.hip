@@ -25,16 +25,17 @@
 #include "storage_ops.h"
 
 namespace deers {
-void launch_attn_fwd_f16(const FwdParams& p, int B, int D, hipStream_t stream);
+// from_q: scores from Q itself, not from f16(Q * scale * log2(e)); the answer of attn_f16_from_q
+void launch_attn_fwd_f16(const FwdParams& p, int B, int D, bool from_q, hipStream_t stream);
 void launch_attn_fwd_f32(const FwdParams& p, int B, int D, hipStream_t stream);
-void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, hipStream_t stream);
+void launch_attn_bwd_f16(const BwdParams& p, int B, int D, int mode, bool from_q, hipStream_t stream);
 // test hook (deers_rocm_debug_attn_128_rows): the rules below leave everything that can be left to the 128-row kernels
 bool attn_128_rows = false;
 bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D);
-// scaled_q: scores from f16(Q * scale * log2(e)), as the 128-row kernels form them, not from Q
-void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, bool scaled_q, hipStream_t stream);
-void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, bool scaled_q, hipStream_t stream);
+bool attn_f16_from_q(int64_t BH, int64_t T, int64_t D, float scale);
+void launch_attn_fwd_f16_split(const FwdParams& p, int B, int D, bool from_q, hipStream_t stream);
+void launch_attn_bwd_f16_split(const BwdParams& p, int B, int D, bool from_q, hipStream_t stream);
 int64_t attn_bwd_f32_default_ds_limit();
 int attn_bwd_f32_heads(int64_t BH, int64_t T, int64_t D, int64_t limit);
 size_t attn_bwd_f32_ds_bytes(int heads, int64_t T);
@@ -763,10 +764,11 @@ int deers_rocm_attn_fwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
   p.H = (int)H; p.T = (int)T;
   p.scale_log2 = (float)((double)scale * 1.4426950408889634);
+  const bool from_q = dtype == DEERS_ROCM_F16 && deers::attn_f16_from_q(B * H, T, D, scale);
   if (dtype == DEERS_ROCM_F16 && deers::attn_fwd_f16_split_takes(B * H, T, D))
-    deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, !deers::attn_bwd_f16_split_takes(B * H, T, D), g_rt.stream);
+    deers::launch_attn_fwd_f16_split(p, (int)B, (int)D, from_q, g_rt.stream);
   else if (dtype == DEERS_ROCM_F16)
-    deers::launch_attn_fwd_f16(p, (int)B, (int)D, g_rt.stream);
+    deers::launch_attn_fwd_f16(p, (int)B, (int)D, from_q, g_rt.stream);
   else if (deers::attn_fwd_f32_split_takes(B * H, T, D))
     deers::launch_attn_fwd_f32_split(p, (int)B, (int)D, g_rt.stream);
   else
@@ -805,7 +807,7 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   // the forms for launches that cannot fill the device need no workspace and hand nothing over
   // (the test hook of the hand-over asks for the form that does)
   if (dtype == DEERS_ROCM_F16 && !g_rt.bwd_skip_producers && deers::attn_bwd_f16_split_takes(B * H, T, D)) {
-    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, false, g_rt.stream);
+    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, /*from_q=*/true, g_rt.stream);
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }
@@ -838,10 +840,11 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   // A launch that is being captured into a graph gets no fresh epoch on replay: it takes the
   // two-launch form with the flags switched off (epoch 0; the dQ role still clears its flags).  Where the
   // workspace or the flags would have to grow, which a capture does not allow, the form that needs neither.
+  const bool from_q = deers::attn_f16_from_q(B * H, T, D, scale);
   bool capturing;
   if (int rc = stream_captures(&capturing)) return rc;
   if (capturing && (flags_grow || ws_bytes > g_rt.workspace.bytes)) {
-    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, /*scaled_q=*/true, g_rt.stream);
+    deers::launch_attn_bwd_f16_split(p, (int)B, (int)D, from_q, g_rt.stream);
     HIP_TRY(hipGetLastError());
     return DEERS_ROCM_OK;
   }
@@ -868,7 +871,7 @@ int deers_rocm_attn_bwd(int dtype, const void* q, const int64_t* q_strides, cons
   p.t_pad = (int)t_pad;
   if (single_launch) g_rt.bwd_error_armed = true;
   const int mode = !single_launch ? 0 : (g_rt.bwd_skip_producers ? 2 : 1);
-  deers::launch_attn_bwd_f16(p, (int)B, (int)D, mode, g_rt.stream);
+  deers::launch_attn_bwd_f16(p, (int)B, (int)D, mode, from_q, g_rt.stream);
   HIP_TRY(hipGetLastError());
   return DEERS_ROCM_OK;
 }
