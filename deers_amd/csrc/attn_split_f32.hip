@@ -104,7 +104,8 @@ __global__ __launch_bounds__(64 * W, Split32<D>::kWavesPerSimd) void attn_fwd_f3
     const float top = pair_max(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])));
     if (!kLazy || first || __any(top > 8.f)) {
       const float m_new = kLazy ? m + (first ? top : fmaxf(top, 0.f)) : fmaxf(m, top);
-      const float alpha = fast_exp2(m - m_new);  // the first block's scales zeros
+      // the first block's scales zeros: by no more than one, where all of its scores lie far below zero
+      const float alpha = fast_exp2(fminf(m - m_new, 0.f));
       l *= alpha;
 #pragma unroll
       for (int db = 0; db < DB; ++db) oacc[0][db] *= alpha;

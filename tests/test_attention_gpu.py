@@ -12,6 +12,7 @@ import pytest
 import oracle
 from deers_amd import rocm, synth
 from forms import rows_128, takes_32_rows
+from hipgraph import Graph
 
 pytestmark = pytest.mark.gpu
 
@@ -480,6 +481,39 @@ def f32_form(B, H, T, D):
     again = rocm.attn_fwd_bwd(x["q"], x["k"], x["v"], x["do"])
     for a, b in zip(out, again):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("H,T,D,waves", [(4, 288, 32, 4), (110, 288, 32, 2), (230, 288, 32, 1), (4, 288, 64, 4), (130, 288, 64, 2),
+                                         (210, 288, 64, 1), (4, 288, 128, 4), (3, 65, 32, 4), (3, 40, 64, 2), (2, 1, 32, 1)])
+def test_f32_forward_of_blocks_whose_scores_all_lie_far_below_zero(H, T, D, waves):
+    """Every key of a block of 32 shifts the scores by -100 to -1000, another one in each block, so that some waves begin
+    with a maximum far below zero, rise or fall from there, and row 0 has nothing else.  A score is a sum of D products
+    of one large and D - 1 usual ones: rounded to sqrt(D) 2^-24 of its size in the root mean square, which is the
+    relative error of a probability and of O; four times that."""
+    x = synth.attention_inputs(f"far-below-{H}-{T}-{D}", 1, H, T, D, np.float32, base_seed=66, names=("q", "k", "v"))
+    scale = float(rocm.default_scale(D))
+    shift = -np.array([100, 1000, 300, 200, 1000, 150, 120, 90, 400], np.float32)[np.arange(T) // 32]
+    x["q"][..., 0] = 1
+    x["k"][..., 0] = shift / scale
+    q, k, v = (rocm.DeviceBuffer.from_numpy(x[n]) for n in ("q", "k", "v"))
+    o, lse = rocm.DeviceBuffer((1, H, T, D), np.float32), rocm.DeviceBuffer((1, H, T), np.float32)
+    graph = Graph(lambda: rocm.attn_fwd_raw(np.float32, q.ptr, k.ptr, v.ptr, o.ptr, lse.ptr, 1, H, T, D, rocm.default_scale(D)))
+    try:
+        assert graph.threads() == [64 * waves]
+        graph.launch()
+        got, got_lse = o.numpy(), lse.numpy()
+    finally:
+        graph.close()
+    assert np.isfinite(got).all() and np.isfinite(got_lse).all()
+    rounding = D ** 0.5 * 2.0 ** -24 * 1000
+    for h in (0, H - 1):
+        q, k, v = (x[n][0, h].astype(np.float64) for n in ("q", "k", "v"))
+        s = np.where(np.triu(np.ones((T, T), bool), 1), -np.inf, q @ k.T * scale)
+        top = np.max(s, 1, keepdims=True)
+        p = np.exp(s - top)
+        want, want_lse = p @ v / p.sum(1, keepdims=True), top[:, 0] + np.log(p.sum(1))
+        assert np.linalg.norm(got[0, h] - want) <= 4 * rounding * np.linalg.norm(want)
+        assert np.max(np.abs(got_lse[0, h] - want_lse)) <= 4 * rounding
 
 
 def test_f32_few_heads_rows_interleaved_over_heads():
