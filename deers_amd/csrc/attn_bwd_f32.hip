@@ -176,7 +176,7 @@ __global__ __launch_bounds__(64 * W) void attn_bwd_f32_dq_kernel(BwdParams p, in
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bh, rank;
-  if (!map_block_even(blockIdx.x, n_blocks, BH, &bh, &rank)) return;
+  if (!map_block_even_by_search(blockIdx.x, n_blocks, BH, &bh, &rank)) return;
   bh = __builtin_amdgcn_readfirstlane(bh);
   const int qb = __builtin_amdgcn_readfirstlane(n_blocks - 1 - rank);  // longest rows first
   const char* ds_row = ds + ((int64_t)bh * ds_block(n_blocks, 0) + ds_block(qb, 0)) * kDsBlock;

@@ -13,9 +13,10 @@ PROGRAM = r"""
 #include "common.h"
 extern "C" int block(int id, int grid, int cus) { return deers::paired_block(id, grid, cus); }
 extern "C" int even_blocks(int n_ranks, int heads) { return deers::map_even_blocks(n_ranks, heads); }
-extern "C" int even(int id, int n_ranks, int heads) {
+extern "C" int even(int id, int n_ranks, int heads, int by_search) {
   int head, rank;
-  return deers::map_block_even(id, n_ranks, heads, &head, &rank) ? rank * heads + head : -1;
+  const auto map = by_search ? deers::map_block_even_by_search : deers::map_block_even;
+  return map(id, n_ranks, heads, &head, &rank) ? rank * heads + head : -1;
 }
 """
 
@@ -62,5 +63,6 @@ def test_blocks_of_heads_that_the_xcds_cannot_share_out_whole(maps):
                     lists[head % 8].append(rank * heads + head)
             grid = maps.even_blocks(n_ranks, heads)
             assert grid == 8 * max(map(len, lists))
-            taken = [[maps.even(8 * i + xcd, n_ranks, heads) for i in range(grid // 8)] for xcd in range(8)]
-            assert taken == [x + [-1] * (grid // 8 - len(x)) for x in lists], (heads, n_ranks)
+            for by_search in (0, 1):
+                taken = [[maps.even(8 * i + xcd, n_ranks, heads, by_search) for i in range(grid // 8)] for xcd in range(8)]
+                assert taken == [x + [-1] * (grid // 8 - len(x)) for x in lists], (heads, n_ranks)
