@@ -227,11 +227,13 @@ int deers_rocm_attn_decode(int dtype,
  * counterpart in the reference.  Same arguments, same kernels and bit-identical results;
  * the split partial results live in a fixed 512 KiB device array that is part of the
  * library image, so the call performs no hipMalloc / hipFree and never grows a
- * workspace.  A problem whose partials (B*H*splits*(D+2) floats, only when heads are
- * split over workgroups, i.e. B*H <= 168) would not fit is rejected with
- * DEERS_ROCM_ERR_ARG.  All calls on a device share the one array: calls that overlap
- * on the device (other streams, other processes' copies aside) would race; the library
- * stream runs them in order. */
+ * workspace.  Heads are split over workgroups in calls of up to 168 heads (B*H), and in larger
+ * ones of up to 128 heads beyond a multiple of 256, where the last heads are: the partials take
+ * n*splits*(D+2) floats for n split heads, 256 KiB at most, and a call whose partials would not
+ * fit is rejected with DEERS_ROCM_ERR_ARG.  All calls on a device share that array and the
+ * counters by which a head's splits meet, deers_rocm_attn_decode's among them: calls of such head
+ * counts that overlap on the device (other streams, other processes' copies aside) would race;
+ * the library stream runs them in order. */
 int deers_rocm_attn_decode_noalloc(int dtype,
                                    const void* q,
                                    const void* k_cache, const void* v_cache,
