@@ -316,11 +316,12 @@ __host__ __device__ __forceinline__ bool map_block_even(int block_id, int n_rank
   *rank = k;
   return true;
 }
-// The same map by a search for the rank, as the dQ pass of the f32 backward has it: it costs a start some hundred
-// instructions more and no launch alone any time, but with it a device that is at its power limit runs faster.  Found by timing
-// (forward and backward of 96 x 1024 x 64 f32, us, closed form / this, on three devices: 475 / 463, 435.1 / 428.0, 421.2 /
-// 420.5; 112 x 1024 x 64 552 / 540, 509.7 / 500.2, 486.1 / 485.9); waiting as long, dividing in 64 bits and other alignments of
-// the code do not do it, nor does it in the dK/dV pass, and no counter of instructions, LDS or caches differs.
+// The same map by a search for the rank, as the dQ pass of the f32 backward has it: a start some hundred instructions
+// longer (24 x 1000 x 64 alone 93.3 -> 93.7 us), but with it a device that is at its power limit runs faster.  Found by timing, and
+// not explained: forward and backward of 96 x 1024 x 64 f32, us, closed form / this, on three devices 475 / 464 (there with
+// both passes so), 435.1 / 428.0, 421.2 / 420.5; 112 x 1024 x 64 552 / 541, 509.7 / 500.2, 486.1 / 485.9.  Waiting as long, dividing
+// in 64 bits or another alignment of the code does not do it, nor does this map in the dK/dV pass alone, and no counter of
+// instructions, LDS or caches differs.
 __host__ __device__ __forceinline__ bool map_block_even_by_search(int block_id, int n_ranks, int BH, int* bh, int* rank) {
   const int xcd = block_id & 7, idx = block_id >> 3;
   const int whole = BH >> 3, rest = BH & 7;
