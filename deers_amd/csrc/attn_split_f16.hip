@@ -944,9 +944,12 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 20 x 3000 x 64 37.2 / 41.4; backward 9 x 2048 x 64 44.9 / 31.9, 9 x 4096 x 64 105.7 / 100.6, 12 x 3000 x 128 144.7 / 157.6,
 // 20 x 2048 x 64 56.4 / 62.3).  Seven or eight heads give each XCD one, which is what those kernels like best (backward 8 x
 // 3000 x 64 51.2 / 56.5, 9 x 3000 x 64 63.8 / 62.9).  At nb = 12 to 16 they are as fast or faster while all their
-// workgroups are resident two to a CU (forward 128 x 512 x 32 8.3 / 9.7, 168 x 512 x 64 14.8 / 15.8, 80 x 512 x 128 15.5 /
+// workgroups are resident two to a CU (forward 168 x 512 x 64 14.8 / 15.8, 80 x 512 x 128 15.5 /
 // 17.5, 124 x 372 x 64 10.6 / 11.8, but 108 x 372 x 64 10.3 / 9.7, 148 x 372 x 64 12.3 / 11.3).
 // The forward takes what the backward takes: then both form their scores from Q itself.
+// At D = 32 from 16 blocks on the forward's line lies where its error does, not its time: the 128-row kernel's reference moves
+// late and P is rounded against it (O from 64 bits, 128 rows / here: 31 x 2425 3.24e-4 / 3.12e-4, 75 x 1024 3.27e-4 / 3.11e-4; us
+// 23.6 / 26.2, 12.8 / 14.4).  At 16 blocks the backward comes along: 120 x 512 8.5 / 9.5, with it 26.8 / 24.3.
 extern bool attn_128_rows;  // runtime.hip
 struct SplitSize {
   int64_t nb, u;
@@ -966,8 +969,8 @@ bool attn_fwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   if (nb <= 11) return u <= of_width(D, 4500, 6000, 8000);
   if (nb <= 12) return outside(u, of_width(D, 4500, 1350, 2048), of_width(D, 4500, 1660, 3300), of_width(D, 4500, 5800, 7000));
   if (nb <= 15) return outside(u, of_width(D, 4000, 6800, 2048), 3300, of_width(D, 4000, 6800, 7500));
-  if (nb <= 16) return outside(u, of_width(D, 770, 1300, 2048), of_width(D, 1540, 3000, 8192), of_width(D, 4200, 5800, 8192));
-  return u <= of_width(D, nb < 40 ? 830 : 920, 1200, 2048);
+  if (nb <= 16) return outside(u, of_width(D, 1200, 1300, 2048), of_width(D, 1540, 3000, 8192), of_width(D, 4200, 5800, 8192));
+  return u <= of_width(D, 1200, 1200, 2048);
 }
 bool attn_bwd_f16_split_takes(int64_t BH, int64_t T, int64_t D) {
   if (!attn_fwd_f16_split_takes(BH, T, D)) return false;

@@ -48,28 +48,51 @@ def test_forms_at_their_lines(gpu, B, H, T, D):
         np.testing.assert_array_equal(a, b)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("H,T,D", [(24, 2049, 64), (64, 1024, 64), (33, 1025, 128)])
-def test_the_forward_from_q_is_as_exact_as_one_against_the_true_maximum(gpu, H, T, D):
-    """Relative 2-norm distance from 64 bits, of all rows of some heads: no more than probabilities rounded to f16
-    against the row's true maximum, their sums and a result rounded to f16 have (the largest probability is exact then)."""
-    assert not takes_32_rows("fwd", np.float16, H, T, D)
+def far_from_64_bits(H, T, D):
+    """Relative 2-norm distance from 64 bits, of all rows of some heads: of the forward's O, and of one whose probabilities are
+    rounded to f16 against the row's true maximum (the largest is exact then) and summed so, as is its result."""
     x = synth.attention_inputs(f"exact-{H}-{T}-{D}", 1, H, T, D, np.float16, base_seed=63, names=("q", "k", "v"))
     o = rocm.attn_fwd(x["q"], x["k"], x["v"])[0]
     future = np.triu(np.ones((T, T), bool), 1)
-    off, bound, size = 0.0, 0.0, 0.0
+    scale = float(rocm.default_scale(D))
+    off, ideal_off, size = 0.0, 0.0, 0.0
     for h in (0, H // 2, H - 1):
         q, k, v = (x[n][0, h].astype(np.float64) for n in ("q", "k", "v"))
-        s = np.where(future, -np.inf, q @ k.T * float(rocm.default_scale(D)))
-        p = np.exp(s - np.max(s, 1, keepdims=True))
-        want = p @ v / p.sum(1, keepdims=True)
-        rounded = p.astype(np.float16).astype(np.float64)
-        ideal = (rounded @ v / rounded.sum(1, keepdims=True)).astype(np.float16).astype(np.float64)
+
+        def attend(s, dtype):
+            s = np.where(future, -np.inf, s)
+            p = np.exp(s - np.max(s, 1, keepdims=True)).astype(dtype).astype(np.float64)
+            return (p @ v / p.sum(1, keepdims=True)).astype(dtype).astype(np.float64)
+
+        want = attend(q @ k.T * scale, np.float64)
+        if scores_from_q(H, T, D):
+            s = q @ k.T * scale
+        else:
+            log2_scale = np.float32(scale / np.log(2))
+            s = (x["q"][0, h].astype(np.float32) * log2_scale).astype(np.float16).astype(np.float64) @ k.T * np.log(2)
         off += np.sum((o[0, h] - want) ** 2)
-        bound += np.sum((ideal - want) ** 2)
+        ideal_off += np.sum((attend(s, np.float16) - want) ** 2)
         size += np.sum(want ** 2)
-    print(f"{H} x {T} x {D}: {np.sqrt(off / size):.4g}, true maximum {np.sqrt(bound / size):.4g}", flush=True)
-    assert off <= bound
+    off, ideal_off = np.sqrt(off / size), np.sqrt(ideal_off / size)
+    print(f"{H} x {T} x {D}: {off:.4g}, true maximum {ideal_off:.4g}", flush=True)
+    return off, ideal_off
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,T,D", [(24, 2049, 64), (64, 1024, 64), (33, 1025, 128)])
+def test_the_forward_from_q_is_as_exact_as_one_against_the_true_maximum(gpu, H, T, D):
+    assert not takes_32_rows("fwd", np.float16, H, T, D)
+    off, ideal = far_from_64_bits(H, T, D)
+    assert off <= ideal
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,T", [(31, 2425), (75, 1024), (45, 1500), (110, 510)])
+def test_forwards_at_head_width_32_that_are_as_exact_as_one_against_the_true_maximum(gpu, H, T):
+    """Launches that the 128-row kernel, whose reference moves late, would have 2 to 3 per cent further off."""
+    assert takes_32_rows("fwd", np.float16, H, T, 32)
+    off, ideal = far_from_64_bits(H, T, 32)
+    assert off <= ideal
 
 
 @pytest.mark.gpu
