@@ -363,7 +363,8 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // Waves.  Few workgroups: four waves, the shortest chain (us in 4 / 2 / 1: 13 x 512 x 64 14 / 22 / 39, 25 x 4096 x 64 441 /
 // 500 / 590).  Many: the SIMDs are covered anyway, and a wave that walks longer pays its start-up and its merge less often
 // (168 x 400 x 128 132 / 97 / 83, 480 x 400 x 64 140 / 126 / 113); the shorter the walks, the fewer workgroups that takes, and the
-// longer they are, the more are needed for the last ones to end together.  At head width 128 a SIMD has one wave, so
+// longer they are, the more are needed for the last ones to end together (in 4 / 1: 90 x 2395 x 32 269 / 296, 30 x 8192 x 32 988 /
+// 1068).  At head width 128 a SIMD has one wave, so
 // that two or one are enough early (65 x 1024 x 128 208 / 175 / 161).
 //
 // Takes, forward, us in the 128-row kernel / here: nearly everything, since that one forms 128 rows and has barriers
@@ -386,7 +387,7 @@ static int fwd_waves(int64_t BH, int64_t T, int64_t D) {
   if (nb < 2) return 1;
   int64_t four, two;  // workgroups up to which there are as many waves
   if (D == 32) {
-    four = nb < 10 ? 900 : std::min<int64_t>(6500, 170 * nb - 150);
+    four = nb < 10 ? 900 : std::min<int64_t>(std::max<int64_t>(6500, 4608 + 48 * nb), 170 * nb - 150);
     two = nb < 10 ? 220 * nb : 5300;
   } else if (D == 64) {
     four = nb < 4 ? 400 : nb < 8 ? 110 * nb : nb < 12 ? 1100 : std::min(175 * nb - 560, 2600 + 36 * nb);
