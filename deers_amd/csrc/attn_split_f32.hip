@@ -364,7 +364,9 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 500 / 590).  Many: the SIMDs are covered anyway, and a wave that walks longer pays its start-up and its merge less often
 // (168 x 400 x 128 132 / 97 / 83, 480 x 400 x 64 140 / 126 / 113); the shorter the walks, the fewer workgroups that takes, and the
 // longer they are, the more are needed for the last ones to end together (in 4 / 1: 90 x 2395 x 32 269 / 296, 30 x 8192 x 32 988 /
-// 1068).  At head width 128 a SIMD has one wave, so
+// 1068).  Walks of up to 12 blocks were timed on a grid of their own: in 4 / 2 / 1 312 x 121 x 32 10.4 / 8.5 / 9.4, 235 x 89 x 32 7.3 / 5.9 / 6.9,
+// 152 x 185 x 128 41.8 / 28.7 / 33.5, 258 x 57 x 128 25.3 / 17.7 / 14.5; a line at 256 or 512 is where the device's SIMDs have taken as many waves as
+// they hold (122 x 123 x 64, 488 workgroups of four waves, 9.9 and of two 10.7).  At head width 128 a SIMD has one wave, so
 // that two or one are enough early (65 x 1024 x 128 208 / 175 / 161).
 //
 // Takes, forward, us in the 128-row kernel / here: nearly everything, since that one forms 128 rows and has barriers
@@ -387,14 +389,14 @@ static int fwd_waves(int64_t BH, int64_t T, int64_t D) {
   if (nb < 2) return 1;
   int64_t four, two;  // workgroups up to which there are as many waves
   if (D == 32) {
-    four = nb < 10 ? 900 : std::min<int64_t>(std::max<int64_t>(6500, 4608 + 48 * nb), 170 * nb - 150);
-    two = nb < 10 ? 220 * nb : 5300;
+    four = nb < 4 ? 350 : nb < 10 ? std::min(180 * nb, 560 + 66 * nb) : std::min<int64_t>(std::max<int64_t>(6500, 4608 + 48 * nb), 170 * nb - 150);
+    two = nb < 3 ? 330 : nb < 10 ? std::min<int64_t>(350 * nb - 50, 2500) : nb < 12 && n > 230 * nb && n <= 3750 ? 0 : nb < 16 ? 5300 : 7000;
   } else if (D == 64) {
-    four = nb < 4 ? 400 : nb < 8 ? 110 * nb : nb < 12 ? 1100 : std::min(175 * nb - 560, 2600 + 36 * nb);
-    two = nb < 11 ? 200 * nb : 3200;
+    four = nb < 4 ? 330 : nb < 5 ? (n > 440 ? 512 : 256) : nb < 8 ? std::min<int64_t>(110 * nb, 650) : nb < 9 ? 900 : nb < 12 ? 1100 : std::min(175 * nb - 560, 2600 + 36 * nb);
+    two = nb < 3 ? 350 : nb < 4 ? 800 : nb < 11 ? std::min<int64_t>(200 * nb, 1800) : 3200;
   } else {
-    four = nb < 9 ? std::max<int64_t>(60 * nb, 200) : std::max<int64_t>(510, 400 + 9 * nb);
-    two = nb < 9 ? std::max<int64_t>(600, 150 * nb) : nb < 12 ? 1180 : nb < 16 ? 1400 : nb >= 48 && n > 2200 ? 3400 : 1650;
+    four = nb < 9 ? std::max<int64_t>(60 * nb, 256) : std::max<int64_t>(510, 400 + 9 * nb);
+    two = nb < 3 ? 512 : nb < 4 ? 800 : nb < 9 ? std::max<int64_t>(1000, 150 * nb) : nb < 12 ? 1300 : nb < 16 ? 1400 : nb >= 48 && n > 2200 ? 3400 : 1650;
   }
   return nb >= 3 && n <= four ? 4 : n <= two ? 2 : 1;
 }

@@ -483,7 +483,7 @@ def f32_form(B, H, T, D):
         np.testing.assert_array_equal(a, b)
 
 
-@pytest.mark.parametrize("H,T,D,waves", [(4, 288, 32, 4), (110, 288, 32, 2), (230, 288, 32, 1), (4, 288, 64, 4), (130, 288, 64, 2),
+@pytest.mark.parametrize("H,T,D,waves", [(4, 288, 32, 4), (150, 288, 32, 2), (290, 288, 32, 1), (4, 288, 64, 4), (130, 288, 64, 2),
                                          (210, 288, 64, 1), (4, 288, 128, 4), (3, 65, 32, 4), (3, 40, 64, 2), (2, 1, 32, 1)])
 def test_f32_forward_of_blocks_whose_scores_all_lie_far_below_zero(H, T, D, waves):
     """Every key of a block of 32 shifts the scores by -100 to -1000, another one in each block, so that some waves begin
