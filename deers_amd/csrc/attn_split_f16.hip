@@ -930,7 +930,7 @@ void launch_bwd_split(const BwdParams& p, int BH, hipStream_t stream) {
 // 12 x 512 5.8 / 7.7 / 11.1, 62 x 512 11.6 / 9.1 / 12.3, 200 x 256 11.5 / 11.0 / 8.8; backward D = 128: 6 x 768
 // 14.2 / 20.3 / 31.6, 15 x 1024 40.4 / 32.0 / 46.2, 187 x 256 73.4 / 49.0 / 38.3).  Twice the blocks in LDS where a CU has
 // one workgroup or two (forward D = 128, once / twice: 10 x 512 6.8 / 6.7, 6 x 128 4.7 / 4.5, 15 x 777 10.8 / 11.9; D = 32
-// 8 x 2038 9.4 / 8.6, 12 x 1500 7.9 / 7.4, 16 x 1494 8.3 / 8.5).  The
+// 8 x 2038 9.4 / 8.6, 12 x 1500 7.9 / 7.4, 5 x 4096 16.7 / 15.8, 12 x 2048 10.4 / 10.7).  The
 // forward at D = 32: four up to some 90 heads, walks of three blocks included, and two up to 250, of two blocks up to
 // 120 (us in 4 / 2 / 1: 50 x 86 3.0 / 3.4 / 3.5, 120 x 54 3.0 / 3.0 / 3.2, 130 x 54 3.4 / 3.4 / 3.2, 240 x 86 4.2 / 3.6 /
 // 3.8, 90 x 246 4.4 / 4.8 / 5.9, 250 x 150 5.6 / 4.6 / 4.9, 300 x 150 6.1 / 5.3 / 5.1).
@@ -1001,7 +1001,7 @@ static int fwd_waves(const SplitSize& z, int64_t D) {
                                std::min(120 * sq, 1300 + 60 * nb));
   return waves(z, four, nb > 16 ? z.u : two, D == 32 ? 3 : 4);
 }
-static bool fwd_twice(const SplitSize& z, int64_t D) { return z.u <= of_width(D, 300, 256, 448); }
+static bool fwd_twice(const SplitSize& z, int64_t D) { return z.u <= of_width(D, 340, 256, 448); }
 static int bwd_waves(const SplitSize& z, int64_t D) {
   const int64_t nb = z.nb;
   const int64_t four = of_width(D, std::min(24 * nb, 120 + 9 * nb), std::min(32 * nb, 160 + 12 * nb), std::max<int64_t>(256, 72 + 20 * nb));
